@@ -69,7 +69,7 @@ def step_bytes(k: float, passes: int = 3) -> float:
     return 300.0 + 16.0 * passes + 108.0 * k
 
 
-KERNELS = ("grid_setup", "keys", "radix_pass", "reorder", "cell_table", "density", "forces", "pressure_sph",
+KERNELS = ("grid_setup", "keys", "cell_table", "place", "reorder", "density", "forces", "pressure_sph",
            "pci_density", "mlp_seed", "pci_pressure", "integrate")
 
 

@@ -128,7 +128,6 @@ struct lps_ctx {
     uint32_t next_id = 0;   // id of the next particle added (ids number particles in order of arrival)
     uint32_t cap_n = 0;     // allocated slot capacity
     uint32_t cell_cap = 0;  // allocated cell-table entries (plus one sentinel)
-    uint32_t passes = 0;    // radix passes for cell_cap
     int cur = 0;            // which state buffer holds the sorted state
     uint64_t steps = 0;
     bool have_step = false; // a step has produced grid/fields
@@ -138,17 +137,16 @@ struct lps_ctx {
     uint8_t* first[2] = {};
     uint32_t* id[2] = {};
     float* pprev[2] = {};
-    uint32_t *keysA = nullptr, *valsA = nullptr, *keysB = nullptr, *valsB = nullptr;
+    uint32_t *keys = nullptr, *rank = nullptr;  // cell and place of arrival in it, before the sort
+    uint2* placed = nullptr;                    // (index, key) in the cells' slots, by arrival
     uint32_t *skeys = nullptr, *perm = nullptr;
-    uint32_t* hist = nullptr;
-    uint32_t* digit_total = nullptr;
     uint32_t* bbox_part = nullptr;
     float4 *posrho = nullptr, *force = nullptr, *fp = nullptr, *xpred[2] = {};
     float4* xq = nullptr;  // predicted-density pass: (prediction, p / rho*^2) [cap_n + LPS_STENCIL_PAD]
     float *press = nullptr, *q = nullptr, *rho_pred = nullptr;
     uint32_t *mk_mask = nullptr, *mk_ok = nullptr;  // recorded candidate masks [LPS_MC_ROWS][cap_n], flags
     uint2* mk_cq = nullptr;                         // compact predictions [cap_n + LPS_STENCIL_PAD]
-    uint32_t *run_end = nullptr, *cell_lb = nullptr, *block_max = nullptr;
+    uint32_t *cell_count = nullptr, *cell_lb = nullptr, *tile_sum = nullptr;  // counts are zero between steps
     float* tables = nullptr;
     lps_box* boxes = nullptr;
     lps_sphere* spheres = nullptr;
@@ -386,12 +384,10 @@ int ensure_cells(lps_ctx* c, uint32_t cap) {
     c->epoch++;
     int st;
     if ((st = dalloc(&c->cell_lb, (size_t)cap + 1))) return st;
-    if ((st = dalloc(&c->run_end, (size_t)cap + 1))) return st;
-    if ((st = dalloc(&c->block_max, lps_dev::cell_blocks(cap) + 1))) return st;
-    HIPC(hipMemsetAsync(c->run_end, 0, sizeof(uint32_t) * ((size_t)cap + 1), c->stream));
+    if ((st = dalloc(&c->cell_count, (size_t)cap + 1))) return st;
+    if ((st = dalloc(&c->tile_sum, lps_dev::cell_blocks(cap) + 1))) return st;
+    HIPC(hipMemsetAsync(c->cell_count, 0, sizeof(uint32_t) * ((size_t)cap + 1), c->stream));
     c->cell_cap = cap;
-    const uint32_t bits = cap > 1 ? 32u - (uint32_t)__builtin_clz(cap - 1) : 1u;
-    c->passes = (bits + 7) / 8;
     return LPS_OK;
 }
 
@@ -408,14 +404,11 @@ int ensure_particles(lps_ctx* c, uint32_t n) {
         if ((st = dalloc(&c->pprev[b], n))) return st;
         if ((st = dalloc(&c->xpred[b], (size_t)n + LPS_STENCIL_PAD))) return st;
     }
-    if ((st = dalloc(&c->keysA, n))) return st;
-    if ((st = dalloc(&c->valsA, n))) return st;
-    if ((st = dalloc(&c->keysB, n))) return st;
-    if ((st = dalloc(&c->valsB, n))) return st;
+    if ((st = dalloc(&c->keys, n))) return st;
+    if ((st = dalloc(&c->rank, n))) return st;
+    if ((st = dalloc(&c->placed, n))) return st;
     if ((st = dalloc(&c->skeys, n))) return st;
     if ((st = dalloc(&c->perm, n))) return st;
-    if ((st = dalloc(&c->hist, (size_t)256 * lps_dev::radix_tiles(n)))) return st;
-    if ((st = dalloc(&c->digit_total, 256))) return st;
     if ((st = dalloc(&c->bbox_part, (size_t)LPS_BBOX_PART * lps_dev::bbox_parts(n)))) return st;
     if ((st = dalloc(&c->posrho, (size_t)n + LPS_STENCIL_PAD))) return st;
     if ((st = dalloc(&c->force, n))) return st;
@@ -443,11 +436,10 @@ void free_all(lps_ctx* c) {
         dfree(c->pos[b]); dfree(c->vel[b]); dfree(c->vh[b]); dfree(c->first[b]);
         dfree(c->id[b]); dfree(c->pprev[b]); dfree(c->xpred[b]);
     }
-    dfree(c->keysA); dfree(c->valsA); dfree(c->keysB); dfree(c->valsB);
-    dfree(c->skeys); dfree(c->perm); dfree(c->hist); dfree(c->digit_total); dfree(c->bbox_part);
+    dfree(c->keys); dfree(c->rank); dfree(c->placed); dfree(c->skeys); dfree(c->perm); dfree(c->bbox_part);
     dfree(c->posrho); dfree(c->force); dfree(c->fp); dfree(c->press); dfree(c->q); dfree(c->xq); dfree(c->rho_pred);
     dfree(c->mk_mask); dfree(c->mk_ok); dfree(c->mk_cq);
-    dfree(c->run_end); dfree(c->cell_lb); dfree(c->block_max);
+    dfree(c->cell_count); dfree(c->cell_lb); dfree(c->tile_sum);
     dfree(c->tables); dfree(c->boxes); dfree(c->spheres); dfree(c->planes); dfree(c->grid);
     dfree(c->d_mlp); dfree(c->d_mlp_packed); dfree(c->feat); dfree(c->seed); dfree(c->coll_x); dfree(c->coll_t);
     dfree(c->d_grad); dfree(c->d_m1); dfree(c->d_m2); dfree(c->d_loss); dfree(c->d_stats);
@@ -497,8 +489,8 @@ lps_dev::PhysArgs phys_args(lps_ctx* c, const SimConst& k) {
     return a;
 }
 
-// Grid build of one step: keys, sort, reorder (state flips to the other
-// buffer), cell table.
+// Grid build of one step: keys, cell table, placement, reorder (state flips to
+// the other buffer).
 void enqueue_grid(lps_ctx* c) {
     const hipStream_t s = c->stream;
     const uint32_t n = c->n;
@@ -508,38 +500,34 @@ void enqueue_grid(lps_ctx* c) {
     }
     {
         Timed t(c, "keys");
-        lps_dev::launch_keys(s, c->pos[c->cur], n, c->grid, scenes(c), c->keysA, c->valsA, c->block_max, c->hist);
+        lps_dev::launch_keys(s, c->pos[c->cur], n, c->grid, scenes(c), c->keys, c->rank, c->cell_count);
     }
-    for (uint32_t p = 0; p < c->passes; p++) {
-        Timed t(c, "radix_pass");
-        const bool even = (p & 1u) == 0u;
-        lps_dev::launch_radix_pass(s, even ? c->keysA : c->keysB, even ? c->valsA : c->valsB,
-                                   even ? c->keysB : c->keysA, even ? c->valsB : c->valsA, n, 8u * p, c->grid,
-                                   c->hist, c->digit_total);
+    {
+        Timed t(c, "cell_table");
+        lps_dev::launch_cell_table(s, c->cell_count, c->grid, c->tile_sum, c->cell_lb, c->cell_cap);
+    }
+    {
+        Timed t(c, "place");
+        lps_dev::launch_place(s, c->keys, c->rank, n, c->grid, c->cell_lb, c->placed);
     }
     {
         Timed t(c, "reorder");
         lps_dev::ReorderArgs r;
         const int a = c->cur, b = 1 - c->cur;
-        r.keysA = c->keysA; r.valsA = c->valsA; r.keysB = c->keysB; r.valsB = c->valsB;
+        r.placed = c->placed;
+        r.cell_lb = c->cell_lb;
         r.n = n;
         r.g = c->grid;
         r.pos_in = c->pos[a]; r.vel_in = c->vel[a]; r.vh_in = c->vh[a]; r.first_in = c->first[a];
         r.id_in = c->id[a]; r.pprev_in = c->pprev[a];
         r.pos_out = c->pos[b]; r.vel_out = c->vel[b]; r.vh_out = c->vh[b]; r.first_out = c->first[b];
         r.id_out = c->id[b]; r.pprev_out = c->pprev[b];
-        r.run_end = c->run_end;
-        r.tile_max = c->block_max;
         r.skeys = c->skeys;
         r.perm = c->perm;
         r.sc = scenes(c);
         r.cq = c->mk_cq;
         lps_dev::launch_reorder(s, r);
         c->cur = b;
-    }
-    {
-        Timed t(c, "cell_table");
-        lps_dev::launch_cell_table(s, c->run_end, c->grid, c->block_max, c->cell_lb, c->cell_cap);
     }
 }
 

@@ -11,8 +11,6 @@
 #include "lps.h"
 
 #define LPS_BLOCK 256           // threads per block for particle kernels (4 wave64)
-#define LPS_RADIX_ITEMS 4       // keys per thread per radix tile
-#define LPS_RADIX_TILE (LPS_BLOCK * LPS_RADIX_ITEMS)
 #define LPS_SCAN_ITEMS 4       // cells per thread in the cell-table scan
 #define LPS_SCAN_TILE (LPS_BLOCK * LPS_SCAN_ITEMS)
 #define LPS_MAX_ITER_SLOTS 64   // per-correction error slots, used as a ring: correction k owns slot (k - 1) % 64
@@ -76,8 +74,6 @@ struct DevGrid {
     float spacing;           // cell size h (SPHSolver.cpp:1031)
     uint32_t nscenes;
     uint32_t total_cells;    // sum over scenes of cells + 1 (the empty-slot cell)
-    uint32_t key_bits;       // bits of (total_cells - 1): radix passes beyond are skipped
-    uint32_t passes_done;    // radix passes executed this step
     uint32_t status;         // lps_status of the step; kernels no-op when non-zero
     uint32_t cells_needed;   // total cells requested when status == GRID_OVERFLOW
     uint32_t steps_ok;       // steps whose grid set-up succeeded, minus failed loops (monotone)

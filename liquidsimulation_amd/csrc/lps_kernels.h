@@ -40,8 +40,9 @@ struct NbMasks {
 };
 
 struct ReorderArgs {
-    const uint32_t *keysA, *valsA, *keysB, *valsB;
-    uint32_t n;
+    const uint2* placed;     // (index, key) of each cell's particles in the cell's slots, by arrival
+    const uint32_t* cell_lb;
+    uint32_t n;              // slots (whole blocks)
     const DevGrid* g;
     const float4 *pos_in, *vel_in, *vh_in;
     const uint8_t* first_in;
@@ -51,8 +52,6 @@ struct ReorderArgs {
     uint8_t* first_out;
     uint32_t* id_out;
     float* pprev_out;
-    uint32_t* run_end;
-    uint32_t* tile_max;  // per-tile maxima of the run ends (cell-table scan tiles)
     uint32_t* skeys;
     uint32_t* perm;
     Scenes sc;            // slot -> scene (for the compact copy's grid)
@@ -90,16 +89,16 @@ void launch_scene_energy(hipStream_t s, const Scenes& sc, const uint32_t* part, 
 // to energy[2 * scene .. + 1] when energy is given
 void launch_grid_setup(hipStream_t s, DevGrid* g, const Scenes& sc, const uint32_t* part, float h, uint32_t cell_cap,
                        double* energy);
-// keys, and the first radix pass's histogram into hist (that pass skips its own)
+// cell keys, places of arrival in the cells, and the particles per cell (zero before; launch_cell_table clears
+// them); n: slots (whole blocks)
 void launch_keys(hipStream_t s, const float4* pos, uint32_t n, const DevGrid* g, const Scenes& sc, uint32_t* keys,
-                 uint32_t* vals, uint32_t* tile_max, uint32_t* hist);
-uint32_t radix_tiles(uint32_t n);
-void launch_radix_pass(hipStream_t s, const uint32_t* kin, const uint32_t* vin, uint32_t* kout, uint32_t* vout,
-                       uint32_t n, uint32_t shift, DevGrid* g, uint32_t* hist, uint32_t* digit_total);
-void launch_reorder(hipStream_t s, const ReorderArgs& a);
+                 uint32_t* rank, uint32_t* count);
 uint32_t cell_blocks(uint32_t cell_cap);
-void launch_cell_table(hipStream_t s, uint32_t* run_end, const DevGrid* g, uint32_t* block_max, uint32_t* cell_lb,
+void launch_cell_table(hipStream_t s, uint32_t* count, const DevGrid* g, uint32_t* tile_sum, uint32_t* cell_lb,
                        uint32_t cell_cap);
+void launch_place(hipStream_t s, const uint32_t* keys, const uint32_t* rank, uint32_t n, const DevGrid* g,
+                  const uint32_t* cell_lb, uint2* placed);
+void launch_reorder(hipStream_t s, const ReorderArgs& a);
 void launch_density(hipStream_t s, const PhysArgs& a, float* press, float* q);
 void launch_forces(hipStream_t s, const PhysArgs& a, float4* xpred, const float* pprev, float* feat);
 void launch_pressure_sph(hipStream_t s, const PhysArgs& a, const float* q);

@@ -1,8 +1,8 @@
 // lps_kernels.hip -- hand-written gfx950 kernels of the SPH/PCISPH step.
 //
 // One launch per phase of PhysicSolver::update (LiquidPhysics/src/PhysicSolver.cpp:12-21):
-//   grid      k_grid_one (or k_scene_grid + k_grid_finish), k_keys,
-//             k_radix_{hist,scan,scatter} x P, k_reorder (+ run-end marks), k_cell_scan
+//   grid      k_grid_one (or k_scene_grid + k_grid_finish), k_keys, k_cell_scan,
+//             k_place, k_reorder
 //   density   k_density
 //   forces    k_forces (+ first PCISPH prediction)
 //   pressure  SPH: k_pressure_sph;  PCISPH: {k_pci_density, k_pci_pressure (+ the
@@ -53,18 +53,6 @@ __device__ __forceinline__ float wave_sum_f32(float v) {
 __device__ __forceinline__ double wave_sum_f64(double v) {
     for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
     return v;
-}
-
-// 64-lane mask of the lanes holding the same 8-bit digit (8 ballots).
-__device__ __forceinline__ uint64_t match_digit(uint32_t d, uint64_t active) {
-    uint64_t peers = active;
-#pragma unroll
-    for (int b = 0; b < 8; b++) {
-        const int bit = (d >> b) & 1u;
-        const uint64_t m = __ballot(bit);
-        peers &= bit ? m : ~m;
-    }
-    return peers;
 }
 
 // LDS copies of the kernel tables, staged by a workgroup of NT threads.  A
@@ -969,9 +957,6 @@ __device__ __forceinline__ void grid_finish_block(DevGrid* g, const lps_dev::Sce
     g->cells_needed = total > 0xFFFFFFFFull ? 0xFFFFFFFFu : (uint32_t)total;
     if (!status && total > (uint64_t)cell_cap) status = LPS_ERR_GRID_OVERFLOW;
     g->total_cells = status ? 1u : (uint32_t)total;
-    const uint32_t cm1 = g->total_cells - 1u;
-    g->key_bits = cm1 ? 32u - (uint32_t)__clz(cm1) : 0u;
-    g->passes_done = 0u;
     g->status = status;
     g->running = S.count;
     g->iterations = 0u;
@@ -999,328 +984,210 @@ __global__ __launch_bounds__(LPS_BLOCK) void k_grid_one(DevGrid* g, lps_dev::Sce
     grid_finish_block(g, S, h, cell_cap);
 }
 
-// calcGridIndices (SPHKernels.cl:66-82) within the scene's grid, offset by the
-// scene's first cell; empty slots get the scene's empty-slot cell so they sort
-// after its particles.
-// Cell keys (calcGridIndices), one radix tile of LPS_RADIX_TILE slots per
-// block in the radix kernels' item order, and the tile's histogram of the
-// first digit (the first radix pass then starts at its scan).
-__global__ __launch_bounds__(LPS_BLOCK) void k_keys(const float4* __restrict__ pos, uint32_t n, const DevGrid* g,
+// ---- sort by cell: a counting sort
+//
+// k_keys counts each cell's particles and gives every particle its place of
+// arrival in its cell (one returning atomic per run of equal keys in a wave);
+// k_cell_scan turns the counts into the cell table; k_place lists every cell's
+// particles by arrival; k_reorder puts them into index order within the cell
+// (each counts the cell's particles of smaller index) and gathers the state.
+// The order of arrival varies from run to run, the result does not: it is the
+// stable sort of radixSort (SPHKernels.cl:84-146).
+//
+// Against the stable radix sort with 8-bit digits that it replaced, it moves
+// every key once instead of once per digit and needs five launches for the
+// sort and cell table instead of 3 P + 2 (P = 2 at 16,000 particles, 3 from
+// about 100,000 on); each is bound by its chain of a few dependent memory
+// round trips (about 5 us whatever the size up to 524,288 particles), so their
+// number is what counts: 33 -> 25 us per step at 16,000 particles, 72 -> 33 at
+// 524,288, 172 -> 88 at 2,097,152.  Counting whole tiles with atomics in k_keys
+// too, to save k_tile_sum, took 49 us at 151,219 particles instead of 5 (many
+// waves on few counters).
+// Its cost grows with the square of a cell's particles in k_reorder, as every
+// stencil pass's does.
+
+// Cell keys (calcGridIndices, SPHKernels.cl:66-82) within the scene's grid,
+// offset by the scene's first cell; empty slots get the scene's empty-slot
+// cell so they follow its particles.  run[i] is the place of arrival in the
+// cell, count[cell] the counts.
+__global__ __launch_bounds__(LPS_BLOCK) void k_keys(const float4* __restrict__ pos, const DevGrid* g,
                                                     lps_dev::Scenes S, uint32_t* __restrict__ keys,
-                                                    uint32_t* __restrict__ vals, uint32_t* __restrict__ tile_max,
-                                                    uint32_t* __restrict__ hist, uint32_t ntiles) {
+                                                    uint32_t* __restrict__ rank, uint32_t* __restrict__ count) {
     if (step_dead(g)) return;
-    __shared__ uint32_t cnt[256];
-    cnt[threadIdx.x] = 0u;
-    // the cell table's per-tile maxima of the run ends start at zero; the
-    // reorder writes those of the non-empty tiles
-    const uint32_t ncell_tiles = (g->total_cells + LPS_SCAN_TILE) / LPS_SCAN_TILE;
-    for (uint32_t b = blockIdx.x * LPS_BLOCK + threadIdx.x; b < ncell_tiles; b += gridDim.x * LPS_BLOCK)
-        tile_max[b] = 0u;
-    __syncthreads();
-    const uint32_t tile = blockIdx.x;
-    // the tile's four positions are loaded before any key is formed
-    float4 p[LPS_RADIX_ITEMS];
-#pragma unroll
-    for (uint32_t r = 0; r < LPS_RADIX_ITEMS; r++) {
-        const uint32_t i = tile * LPS_RADIX_TILE + r * LPS_BLOCK + threadIdx.x;
-        p[r] = i < n ? pos[i] : make_float4(0.f, 0.f, 0.f, 0.f);
+    const uint32_t lb = blockIdx.x, i = lb * LPS_BLOCK + threadIdx.x, lane = lane_id();
+    const float4 p = pos[i];
+    const BlockScene B = block_scene(S, lb);
+    const SceneGrid* sg = S.grid + B.s;
+    const GridView G = grid_view(g, sg);
+    uint32_t key = G.base + sg->cells;
+    if (i < B.info.slot0 + B.info.count) {
+        const uint32_t xg = (uint32_t)truncf((p.x + G.off0) / G.gs);
+        const uint32_t yg = (uint32_t)truncf((p.y + G.off1) / G.gs);
+        const uint32_t zg = (uint32_t)truncf((p.z + G.off2) / G.gs);
+        key = G.base + xg + (uint32_t)G.gx * yg + G.gxy * zg;
     }
-    // the scene and grid of each of the tile's particle blocks (slot i lies
-    // in block i / LPS_BLOCK, uniform over a round), all loaded before the
-    // first key is formed
-    // (blocks past the last one read the last one's, unused)
-    uint32_t sidx[LPS_RADIX_ITEMS], kend[LPS_RADIX_ITEMS], kempty[LPS_RADIX_ITEMS];
-    GridView Gr[LPS_RADIX_ITEMS];
-#pragma unroll
-    for (uint32_t r = 0; r < LPS_RADIX_ITEMS; r++)
-        sidx[r] = S.block_scene[min((tile * LPS_RADIX_TILE + r * LPS_BLOCK) / LPS_BLOCK, S.nblocks - 1u)];
-#pragma unroll
-    for (uint32_t r = 0; r < LPS_RADIX_ITEMS; r++) {
-        const SceneGrid* sg = S.grid + sidx[r];
-        kend[r] = S.info[sidx[r]].slot0 + S.info[sidx[r]].count;
-        kempty[r] = sg->cell_base + sg->cells;
-        Gr[r] = grid_view(g, sg);
+    keys[i] = key;
+    // the particles are in the last step's sorted order, so most of a cell's
+    // lie in consecutive lanes: the first lane of a run of equal keys counts
+    // the whole run
+    const uint32_t before = (uint32_t)__shfl_up((int)key, 1, 64);
+    const uint64_t heads = __ballot(lane == 0u || key != before);
+    const uint64_t upto = ~0ull >> (63u - lane);
+    const uint32_t head = 63u - (uint32_t)__clzll((long long)(heads & upto));
+    uint32_t base = 0u;
+    if (lane == head) {
+        const uint64_t later = heads & ~upto;
+        const uint32_t end = later ? (uint32_t)__ffsll((long long)later) - 1u : 64u;
+        base = atomicAdd(&count[key], end - lane);
     }
-#pragma unroll
-    for (uint32_t r = 0; r < LPS_RADIX_ITEMS; r++) {
-        const uint32_t i = tile * LPS_RADIX_TILE + r * LPS_BLOCK + threadIdx.x;
-        const bool valid = i < n;
-        uint32_t key = 0u;
-        if (valid) {
-            key = kempty[r];
-            if (i < kend[r]) {
-                const GridView& G = Gr[r];
-                const uint32_t xg = (uint32_t)truncf((p[r].x + G.off0) / G.gs);
-                const uint32_t yg = (uint32_t)truncf((p[r].y + G.off1) / G.gs);
-                const uint32_t zg = (uint32_t)truncf((p[r].z + G.off2) / G.gs);
-                key = G.base + xg + (uint32_t)G.gx * yg + G.gxy * zg;
-            }
-            keys[i] = key;
-            vals[i] = i;
-        }
-        const uint32_t d = key & 0xFFu;
-        const uint64_t act = __ballot(valid);
-        const uint64_t peers = match_digit(d, act);
-        if (valid && lane_id() == (uint32_t)__ffsll((long long)peers) - 1u) atomicAdd(&cnt[d], (uint32_t)__popcll(peers));
-    }
-    __syncthreads();
-    hist[threadIdx.x * ntiles + tile] = cnt[threadIdx.x];
+    rank[i] = (uint32_t)__shfl((int)base, (int)head, 64) + lane - head;
 }
 
-// ---- stable LSD radix sort by key, 8-bit digits, reduce-then-scan ----------
-// A pass is skipped when its digit is above the key width of this step's
-// cell count; skipped passes leave the result in the buffer given by the
-// parity of passes_done.
-__global__ __launch_bounds__(LPS_BLOCK) void k_radix_hist(const uint32_t* __restrict__ keys, uint32_t n,
-                                                          uint32_t shift, const DevGrid* g,
-                                                          uint32_t* __restrict__ hist, uint32_t ntiles) {
-    if (step_dead(g) || shift >= g->key_bits) return;
-    __shared__ uint32_t cnt[256];
-    const uint32_t tile = blockIdx.x;
-    // the tile's keys load before the counters are cleared
-    uint32_t kr[LPS_RADIX_ITEMS];
-#pragma unroll
-    for (uint32_t r = 0; r < LPS_RADIX_ITEMS; r++) {
-        const uint32_t idx = tile * LPS_RADIX_TILE + r * LPS_BLOCK + threadIdx.x;
-        kr[r] = idx < n ? keys[idx] : 0u;
-    }
-    cnt[threadIdx.x] = 0u;
-    __syncthreads();
-#pragma unroll
-    for (uint32_t r = 0; r < LPS_RADIX_ITEMS; r++) {
-        const uint32_t idx = tile * LPS_RADIX_TILE + r * LPS_BLOCK + threadIdx.x;
-        const bool valid = idx < n;
-        const uint32_t d = valid ? (kr[r] >> shift) & 0xFFu : 0u;
-        const uint64_t act = __ballot(valid);
-        const uint64_t peers = match_digit(d, act);
-        if (valid && lane_id() == (uint32_t)__ffsll((long long)peers) - 1u) atomicAdd(&cnt[d], (uint32_t)__popcll(peers));
-    }
-    __syncthreads();
-    hist[threadIdx.x * ntiles + tile] = cnt[threadIdx.x];
-}
-
-// Exclusive scan of each digit's per-tile counts (one block per digit); the
-// digit totals are scanned by every scatter block.  Together this is the
-// bucket-major scan of the reference (SPHSolver.cpp:1069-1078).
-__global__ __launch_bounds__(LPS_BLOCK) void k_radix_scan(uint32_t* __restrict__ hist, uint32_t ntiles,
-                                                          uint32_t* __restrict__ digit_total, DevGrid* g,
-                                                          uint32_t shift) {
-    if (step_dead(g) || shift >= g->key_bits) return;
-    __shared__ uint32_t wsum[LPS_BLOCK / 64];
-    const uint32_t d = blockIdx.x, t = threadIdx.x, lane = lane_id(), w = t >> 6;
-    uint32_t* row = hist + d * ntiles;
-    uint32_t carry = 0;
-    for (uint32_t base = 0; base < ntiles; base += LPS_BLOCK) {
-        const uint32_t k = base + t;
-        const uint32_t v = k < ntiles ? row[k] : 0u;
-        uint32_t incl = v;
-        for (int off = 1; off < 64; off <<= 1) {
-            const uint32_t y = (uint32_t)__shfl_up((int)incl, off, 64);
-            if (lane >= (uint32_t)off) incl += y;
-        }
-        if (lane == 63) wsum[w] = incl;
-        __syncthreads();
-        uint32_t wpre = 0, tot = 0;
-        for (uint32_t q = 0; q < LPS_BLOCK / 64; q++) {
-            if (q < w) wpre += wsum[q];
-            tot += wsum[q];
-        }
-        if (k < ntiles) row[k] = carry + wpre + incl - v;
-        carry += tot;
-        __syncthreads();
-    }
-    if (t == 0) {
-        digit_total[d] = carry;
-        if (d == 0) g->passes_done += 1u;
-    }
-}
-
-// Stable scatter of one tile: items are taken in index order (round-major,
-// then wave, then lane); ranks within a wave come from the digit match mask,
-// across waves and rounds from per-digit running offsets in LDS.
-__global__ __launch_bounds__(LPS_BLOCK) void k_radix_scatter(const uint32_t* __restrict__ kin,
-                                                             const uint32_t* __restrict__ vin,
-                                                             uint32_t* __restrict__ kout, uint32_t* __restrict__ vout,
-                                                             uint32_t n, uint32_t shift, const DevGrid* g,
-                                                             const uint32_t* __restrict__ hist, uint32_t ntiles,
-                                                             const uint32_t* __restrict__ digit_total) {
-    if (step_dead(g) || shift >= g->key_bits) return;
-    __shared__ uint32_t s_off[256];
-    __shared__ uint32_t s_w[LPS_BLOCK / 64][256];
-    __shared__ uint32_t s_ws[LPS_BLOCK / 64];
-    const uint32_t t = threadIdx.x, w = t >> 6, lane = lane_id();
-    const uint32_t tile = blockIdx.x;
-    // every load of the block issues before its first barrier: the digit
-    // totals, this tile's offsets and its items
-    const uint32_t v = digit_total[t];
-    const uint32_t tile_off = hist[t * ntiles + tile];
-    uint32_t kr[LPS_RADIX_ITEMS], vr[LPS_RADIX_ITEMS];
-#pragma unroll
-    for (uint32_t r = 0; r < LPS_RADIX_ITEMS; r++) {
-        const uint32_t idx = tile * LPS_RADIX_TILE + r * LPS_BLOCK + t;
-        kr[r] = idx < n ? kin[idx] : 0u;
-        vr[r] = idx < n ? vin[idx] : 0u;
-    }
-    {
-        // exclusive scan of the 256 digit totals
-        uint32_t incl = v;
-        for (int off = 1; off < 64; off <<= 1) {
-            const uint32_t y = (uint32_t)__shfl_up((int)incl, off, 64);
-            if (lane >= (uint32_t)off) incl += y;
-        }
-        if (lane == 63) s_ws[w] = incl;
-        __syncthreads();
-        uint32_t wpre = 0;
-        for (uint32_t q = 0; q < w; q++) wpre += s_ws[q];
-        s_off[t] = tile_off + wpre + incl - v;
-    }
-    for (uint32_t k = 0; k < LPS_BLOCK / 64; k++) s_w[k][t] = 0u;
-    __syncthreads();
-    const uint64_t lt = (lane == 0) ? 0ull : (~0ull >> (64u - lane));
-#pragma unroll
-    for (uint32_t r = 0; r < LPS_RADIX_ITEMS; r++) {
-        const uint32_t idx = tile * LPS_RADIX_TILE + r * LPS_BLOCK + t;
-        const bool valid = idx < n;
-        const uint32_t key = kr[r], val = vr[r];
-        const uint32_t d = (key >> shift) & 0xFFu;
-        const uint64_t act = __ballot(valid);
-        const uint64_t peers = match_digit(d, act);
-        const uint32_t rank = (uint32_t)__popcll(peers & lt);
-        if (valid && rank == 0u) s_w[w][d] = (uint32_t)__popcll(peers);
-        __syncthreads();
-        {
-            uint32_t base = s_off[t];
-            for (uint32_t k = 0; k < LPS_BLOCK / 64; k++) {
-                const uint32_t c = s_w[k][t];
-                s_w[k][t] = base;
-                base += c;
-            }
-            s_off[t] = base;
-        }
-        __syncthreads();
-        if (valid) {
-            const uint32_t dst = s_w[w][d] + rank;
-            kout[dst] = key;
-            vout[dst] = val;
-        }
-        __syncthreads();
-        for (uint32_t k = 0; k < LPS_BLOCK / 64; k++) s_w[k][t] = 0u;
-        __syncthreads();
-    }
-}
-
-// Gather the state into sorted order (the payload moves of permuteParticles,
-// SPHKernels.cl:108-146, done once) and mark the end of every run of equal
-// keys for the cell table.  On a failed step the copy is the identity so the
-// state survives the buffer flip.
-__global__ __launch_bounds__(LPS_BLOCK) void k_reorder(
-    const uint32_t* __restrict__ keysA, const uint32_t* __restrict__ valsA, const uint32_t* __restrict__ keysB,
-    const uint32_t* __restrict__ valsB, uint32_t n, const DevGrid* g, const float4* __restrict__ pos_in,
-    const float4* __restrict__ vel_in, const float4* __restrict__ vh_in, const uint8_t* __restrict__ first_in,
-    const uint32_t* __restrict__ id_in, const float* __restrict__ pprev_in, float4* __restrict__ pos_out,
-    float4* __restrict__ vel_out, float4* __restrict__ vh_out, uint8_t* __restrict__ first_out,
-    uint32_t* __restrict__ id_out, float* __restrict__ pprev_out, uint32_t* __restrict__ run_end,
-    uint32_t* __restrict__ skeys_out, uint32_t* __restrict__ perm_out, lps_dev::Scenes S, uint2* __restrict__ cq,
-    uint32_t* __restrict__ tile_max, uint32_t nlogical) {
-    const uint32_t lb = xcd_block(nlogical);
-    if (lb == UINT_MAX) return;
-    const uint32_t i = lb * LPS_BLOCK + threadIdx.x;
-    if (i >= n) return;
-    const bool dead = step_dead(g);
-    uint32_t j = i;
-    if (!dead) {
-        const bool b = (g->passes_done & 1u) != 0u;
-        const uint32_t* keys = b ? keysB : keysA;
-        const uint32_t* vals = b ? valsB : valsA;
-        j = vals[i];
-        const uint32_t k = keys[i];
-        skeys_out[i] = k;
-        perm_out[i] = j;
-        if (i == n - 1u || keys[i + 1u] != k) {
-            run_end[k] = i + 1u;
-            // the last run of a cell-table tile holds the tile's largest run
-            // end (keys are sorted): one plain store per non-empty tile
-            if (i == n - 1u || keys[i + 1u] / LPS_SCAN_TILE != k / LPS_SCAN_TILE) tile_max[k / LPS_SCAN_TILE] = i + 1u;
-        }
-    }
-    const float4 p = pos_in[j];
-    pos_out[i] = p;
-    if (!dead) {
-        // the density pass filters candidates on this copy (slots of one
-        // block belong to one scene)
-        const BlockScene B = block_scene(S, lb);
-        const GridView G = grid_view(g, S.grid + B.s);
-        cq[i] = quantize(p.x, p.y, p.z, G, compact_scale(G));
-    }
-    vel_out[i] = vel_in[j];
-    vh_out[i] = vh_in[j];
-    first_out[i] = first_in[j];
-    id_out[i] = id_in[j];
-    if (pprev_in) pprev_out[i] = pprev_in[j];
-}
-
-// Cell table = exclusive max-scan of the run ends: LB[c] = #keys < c, the
-// cellList of buildCellList (SPHKernels.cl:148-186), with LB[cells] = n.  The
-// run-end marks are cleared as they are consumed.  block_max holds each
-// tile's largest run end (0 for an empty tile), written by the reorder after
-// k_keys cleared it.
-__global__ __launch_bounds__(LPS_BLOCK) void k_cell_scan(uint32_t* __restrict__ run_end, const DevGrid* g,
-                                                         const uint32_t* __restrict__ block_max,
-                                                         uint32_t* __restrict__ cell_lb) {
+// Particles of each tile of LPS_SCAN_TILE cells.
+__global__ __launch_bounds__(LPS_BLOCK) void k_tile_sum(const uint32_t* __restrict__ count, const DevGrid* g,
+                                                        uint32_t* __restrict__ tile_sum) {
+    static_assert(LPS_SCAN_ITEMS == 4, "one uint4 of counts per thread");
     if (step_dead(g)) return;
     const uint32_t total = g->total_cells + 1u;
     const uint32_t base = blockIdx.x * LPS_SCAN_TILE;
     if (base >= total) return;
     __shared__ uint32_t s[LPS_BLOCK / 64];
-    __shared__ uint32_t s_carry;
-    const uint32_t t = threadIdx.x, lane = lane_id(), w = t >> 6;
-    // carry = max of the previous blocks
-    uint32_t c0 = 0;
-    for (uint32_t k = t; k < blockIdx.x; k += LPS_BLOCK) c0 = max(c0, block_max[k]);
-    c0 = wave_max_u32(c0);
-    if (lane == 0) s[w] = c0;
-    __syncthreads();
-    if (t == 0) {
-        uint32_t r = 0;
-        for (uint32_t k = 0; k < LPS_BLOCK / 64; k++) r = max(r, s[k]);
-        s_carry = r;
+    const uint32_t c = base + threadIdx.x * LPS_SCAN_ITEMS;
+    uint32_t v = 0u;
+    if (c + 3u < total) {
+        const uint4 q = *reinterpret_cast<const uint4*>(count + c);
+        v = q.x + q.y + q.z + q.w;
+    } else {
+        for (uint32_t k = c; k < total; k++) v += count[k];
     }
+    for (int off = 32; off > 0; off >>= 1) v += (uint32_t)__shfl_xor((int)v, off, 64);
+    if (lane_id() == 0u) s[threadIdx.x >> 6] = v;
     __syncthreads();
-    uint32_t carry = s_carry;
+    if (threadIdx.x == 0u) {
+        for (uint32_t k = 1; k < LPS_BLOCK / 64; k++) v += s[k];
+        tile_sum[blockIdx.x] = v;
+    }
+}
+
+// Cell table = exclusive sum of the counts: LB[c] = #keys < c, the cellList of
+// buildCellList (SPHKernels.cl:148-186), with LB[cells] = n.  The counts are
+// cleared as they are consumed.
+__global__ __launch_bounds__(LPS_BLOCK) void k_cell_scan(uint32_t* __restrict__ count, const DevGrid* g,
+                                                         const uint32_t* __restrict__ tile_sum,
+                                                         uint32_t* __restrict__ cell_lb) {
+    if (step_dead(g)) return;
+    const uint32_t total = g->total_cells + 1u;
+    const uint32_t base = blockIdx.x * LPS_SCAN_TILE;
+    if (base >= total) return;
+    __shared__ uint32_t s_pre[LPS_BLOCK / 64], s_in[LPS_BLOCK / 64];
+    const uint32_t t = threadIdx.x, lane = lane_id(), w = t >> 6;
     // thread t owns cells base + t*ITEMS .. +ITEMS (contiguous)
     const uint32_t c_begin = base + t * LPS_SCAN_ITEMS;
     uint32_t v[LPS_SCAN_ITEMS];
-    uint32_t local = 0;
 #pragma unroll
-    for (uint32_t k = 0; k < LPS_SCAN_ITEMS; k++) {
-        const uint32_t c = c_begin + k;
-        v[k] = (c < total) ? run_end[c] : 0u;
-        local = max(local, v[k]);
-    }
-    // exclusive max-scan of `local` across the block
+    for (uint32_t k = 0; k < LPS_SCAN_ITEMS; k++) v[k] = c_begin + k < total ? count[c_begin + k] : 0u;
+    // the cells of all tiles before this one
+    uint32_t pre = 0u;
+#pragma unroll 4
+    for (uint32_t k = t; k < blockIdx.x; k += LPS_BLOCK) pre += tile_sum[k];
+    uint32_t local = 0u;
+#pragma unroll
+    for (uint32_t k = 0; k < LPS_SCAN_ITEMS; k++) local += v[k];
     uint32_t incl = local;
     for (int off = 1; off < 64; off <<= 1) {
         const uint32_t y = (uint32_t)__shfl_up((int)incl, off, 64);
-        if (lane >= (uint32_t)off) incl = max(incl, y);
+        if (lane >= (uint32_t)off) incl += y;
+        pre += (uint32_t)__shfl_xor((int)pre, off, 64);
     }
-    uint32_t excl = (uint32_t)__shfl_up((int)incl, 1, 64);
-    if (lane == 0) excl = 0u;
+    if (lane == 63u) {
+        s_pre[w] = pre;
+        s_in[w] = incl;
+    }
     __syncthreads();
-    if (lane == 63) s[w] = incl;
-    __syncthreads();
-    uint32_t wprefix = 0;
-    for (uint32_t k = 0; k < w; k++) wprefix = max(wprefix, s[k]);
-    uint32_t run = max(carry, max(wprefix, excl));
+    uint32_t run = incl - local;
+    for (uint32_t k = 0; k < LPS_BLOCK / 64; k++) run += s_pre[k] + (k < w ? s_in[k] : 0u);
 #pragma unroll
     for (uint32_t k = 0; k < LPS_SCAN_ITEMS; k++) {
         const uint32_t c = c_begin + k;
         if (c < total) {
             cell_lb[c] = run;
-            if (v[k]) run_end[c] = 0u;
+            if (v[k]) count[c] = 0u;
         }
-        run = max(run, v[k]);
+        run += v[k];
     }
+}
+
+// Every cell's particles (index, key) in the cell's slots, by arrival.
+__global__ __launch_bounds__(LPS_BLOCK) void k_place(const uint32_t* __restrict__ keys,
+                                                     const uint32_t* __restrict__ rank, const DevGrid* g,
+                                                     const uint32_t* __restrict__ cell_lb,
+                                                     uint2* __restrict__ placed) {
+    const uint32_t i = blockIdx.x * LPS_BLOCK + threadIdx.x;
+    const uint32_t key = keys[i], r = rank[i];
+    if (step_dead(g)) return;
+    placed[cell_lb[key] + r] = make_uint2(i, key);
+}
+
+// The stable order within each cell, and the state gathered into it (the
+// payload moves of permuteParticles, SPHKernels.cl:108-146, done once): thread
+// s takes the particle placed in slot s and writes it to the cell's first slot
+// plus the number of the cell's particles of smaller index, a slot of the same
+// cell, so a wave's writes stay together.  On a failed step the copy is the identity so the state survives
+// the buffer flip.
+__global__ __launch_bounds__(LPS_BLOCK) void k_reorder(
+    const uint2* __restrict__ placed, const uint32_t* __restrict__ cell_lb, const DevGrid* g,
+    const float4* __restrict__ pos_in, const float4* __restrict__ vel_in, const float4* __restrict__ vh_in,
+    const uint8_t* __restrict__ first_in, const uint32_t* __restrict__ id_in, const float* __restrict__ pprev_in,
+    float4* __restrict__ pos_out, float4* __restrict__ vel_out, float4* __restrict__ vh_out,
+    uint8_t* __restrict__ first_out, uint32_t* __restrict__ id_out, float* __restrict__ pprev_out,
+    uint32_t* __restrict__ skeys_out, uint32_t* __restrict__ perm_out, lps_dev::Scenes S, uint2* __restrict__ cq,
+    uint32_t nlogical) {
+    const uint32_t lb = xcd_block(nlogical);
+    if (lb == UINT_MAX) return;
+    const uint32_t s = lb * LPS_BLOCK + threadIdx.x;
+    const bool dead = step_dead(g);
+    uint32_t i = s, d = s, key = 0u;
+    if (!dead) {
+        const uint2 own = placed[s];
+        i = own.x;
+        key = own.y;
+    }
+    const float4 p = pos_in[i], v = vel_in[i], h = vh_in[i];
+    const uint8_t f = first_in[i];
+    const uint32_t id = id_in[i];
+    const float pp = pprev_in[i];
+    if (!dead) {
+        const BlockScene B = block_scene(S, lb);
+        const SceneGrid* sg = S.grid + B.s;
+        const GridView G = grid_view(g, sg);
+        // empty slots follow all particles of their scene before and after
+        // the sort: they keep their places
+        d = i;
+        if (key != G.base + sg->cells) {
+            const uint32_t b = cell_lb[key], e = cell_lb[key + 1u];
+            d = b;
+            // four of the cell's entries at a time (the last one repeats,
+            // uncounted, past the cell's end)
+            for (uint32_t t = b; t < e; t += 4u) {
+                uint32_t o[4];
+#pragma unroll
+                for (uint32_t k = 0; k < 4u; k++) o[k] = placed[min(t + k, e - 1u)].x;
+#pragma unroll
+                for (uint32_t k = 0; k < 4u; k++) d += t + k < e && o[k] < i ? 1u : 0u;
+            }
+        }
+        // the density pass filters candidates on this copy (slots of one
+        // block belong to one scene)
+        cq[d] = quantize(p.x, p.y, p.z, G, compact_scale(G));
+        skeys_out[d] = key;
+        perm_out[d] = i;
+    }
+    pos_out[d] = p;
+    vel_out[d] = v;
+    vh_out[d] = h;
+    first_out[d] = f;
+    id_out[d] = id;
+    pprev_out[d] = pp;
 }
 
 // ============================================================= physics ====
@@ -2471,37 +2338,31 @@ void launch_grid_setup(hipStream_t s, DevGrid* g, const Scenes& sc, const uint32
     }
 }
 
-uint32_t radix_tiles(uint32_t n) { return cdiv(n, LPS_RADIX_TILE); }
-
 void launch_keys(hipStream_t s, const float4* pos, uint32_t n, const DevGrid* g, const Scenes& sc, uint32_t* keys,
-                 uint32_t* vals, uint32_t* tile_max, uint32_t* hist) {
-    const uint32_t nt = radix_tiles(n);
-    k_keys<<<nt, LPS_BLOCK, 0, s>>>(pos, n, g, sc, keys, vals, tile_max, hist, nt);
-}
-
-void launch_radix_pass(hipStream_t s, const uint32_t* kin, const uint32_t* vin, uint32_t* kout, uint32_t* vout,
-                       uint32_t n, uint32_t shift, DevGrid* g, uint32_t* hist, uint32_t* digit_total) {
-    const uint32_t nt = radix_tiles(n);
-    // the first digit's histogram comes from the key kernel
-    if (shift != 0u) k_radix_hist<<<nt, LPS_BLOCK, 0, s>>>(kin, n, shift, g, hist, nt);
-    k_radix_scan<<<256, LPS_BLOCK, 0, s>>>(hist, nt, digit_total, g, shift);
-    k_radix_scatter<<<nt, LPS_BLOCK, 0, s>>>(kin, vin, kout, vout, n, shift, g, hist, nt, digit_total);
-}
-
-void launch_reorder(hipStream_t s, const ReorderArgs& a) {
-    const uint32_t nl = cdiv(a.n, LPS_BLOCK);
-    k_reorder<<<xcd_grid(nl), LPS_BLOCK, 0, s>>>(a.keysA, a.valsA, a.keysB, a.valsB, a.n, a.g, a.pos_in, a.vel_in,
-                                                 a.vh_in, a.first_in, a.id_in, a.pprev_in, a.pos_out, a.vel_out,
-                                                 a.vh_out, a.first_out, a.id_out, a.pprev_out, a.run_end,
-                                                 a.skeys, a.perm, a.sc, a.cq, a.tile_max, nl);
+                 uint32_t* rank, uint32_t* count) {
+    k_keys<<<cdiv(n, LPS_BLOCK), LPS_BLOCK, 0, s>>>(pos, g, sc, keys, rank, count);
 }
 
 uint32_t cell_blocks(uint32_t cell_cap) { return cdiv(cell_cap + 1u, LPS_SCAN_TILE); }
 
-void launch_cell_table(hipStream_t s, uint32_t* run_end, const DevGrid* g, uint32_t* block_max, uint32_t* cell_lb,
+void launch_cell_table(hipStream_t s, uint32_t* count, const DevGrid* g, uint32_t* tile_sum, uint32_t* cell_lb,
                        uint32_t cell_cap) {
     const uint32_t nb = cell_blocks(cell_cap);
-    k_cell_scan<<<nb, LPS_BLOCK, 0, s>>>(run_end, g, block_max, cell_lb);
+    k_tile_sum<<<nb, LPS_BLOCK, 0, s>>>(count, g, tile_sum);
+    k_cell_scan<<<nb, LPS_BLOCK, 0, s>>>(count, g, tile_sum, cell_lb);
+}
+
+void launch_place(hipStream_t s, const uint32_t* keys, const uint32_t* rank, uint32_t n, const DevGrid* g,
+                  const uint32_t* cell_lb, uint2* placed) {
+    k_place<<<cdiv(n, LPS_BLOCK), LPS_BLOCK, 0, s>>>(keys, rank, g, cell_lb, placed);
+}
+
+void launch_reorder(hipStream_t s, const ReorderArgs& a) {
+    const uint32_t nl = cdiv(a.n, LPS_BLOCK);
+    k_reorder<<<xcd_grid(nl), LPS_BLOCK, 0, s>>>(a.placed, a.cell_lb, a.g, a.pos_in, a.vel_in, a.vh_in,
+                                                 a.first_in, a.id_in, a.pprev_in, a.pos_out, a.vel_out, a.vh_out,
+                                                 a.first_out, a.id_out, a.pprev_out, a.skeys, a.perm, a.sc, a.cq,
+                                                 nl);
 }
 
 void launch_density(hipStream_t s, const PhysArgs& a, float* press, float* q) {
