@@ -193,10 +193,10 @@ int lps_get_scene_stats(lps_ctx* ctx, lps_step_stats* stats /* [nscenes] */, uin
  * of the two correction kernels (256 runs a 256-slot particle block per
  * workgroup, 128 and 64 split it over 2 or 4); lanes_per_particle: lanes of
  * a wave that share one particle's neighbour walk in the stencil kernels (1,
- * or 4: a quad splits the candidates and adds the terms in the one-lane
- * order; 0 chooses 4 below 512 particle blocks of 256 slots, else 1; the
- * correction workgroup size then applies only with 1; with several scenes, 0
- * also gives quads to the corrections that run fewer than 512 blocks).
+ * or 4: several lanes, a quad or in the smallest scenes a team of 16, split
+ * the candidates and add the terms in the one-lane order; 0 chooses 4 below
+ * 512 particle blocks of 256 slots, else 1; the correction workgroup size then
+ * applies only with 1; with several scenes, 0 also gives quads to the corrections that run fewer than 512 blocks).
  * lps_autotune times `steps` steps of every combination from the current
  * state (4 lanes only below 2048 particle blocks, 0 only with several scenes
  * and at least 512 blocks), restores the state (the run continues exactly as

@@ -145,6 +145,7 @@ struct lps_ctx {
     float4* xq = nullptr;  // predicted-density pass: (prediction, p / rho*^2) [cap_n + LPS_STENCIL_PAD]
     float *press = nullptr, *q = nullptr, *rho_pred = nullptr;
     uint32_t *mk_mask = nullptr, *mk_ok = nullptr;  // recorded candidate masks [LPS_MC_ROWS][cap_n], flags
+    uint32_t *nb_list = nullptr, *nb_count = nullptr;  // recorded neighbour lists of the team kernels
     uint2* mk_cq = nullptr;                         // compact predictions [cap_n + LPS_STENCIL_PAD]
     uint32_t *cell_count = nullptr, *cell_lb = nullptr, *tile_sum = nullptr;  // counts are zero between steps
     float* tables = nullptr;
@@ -422,6 +423,9 @@ int ensure_particles(lps_ctx* c, uint32_t n) {
     if ((st = dalloc(&c->mk_mask, (size_t)LPS_MC_ROWS * n))) return st;
     if ((st = dalloc(&c->mk_ok, n))) return st;
     if ((st = dalloc(&c->mk_cq, (size_t)n + LPS_STENCIL_PAD))) return st;
+    const size_t nt = std::min<size_t>(n, (size_t)LPS_TEAM_BLOCKS * LPS_BLOCK);
+    if ((st = dalloc(&c->nb_list, nt * LPS_NB_LIST))) return st;
+    if ((st = dalloc(&c->nb_count, nt))) return st;
     // every replaying pass follows its recording pass; until then no slot
     // counts as recorded
     HIPC(hipMemsetAsync(c->mk_ok, 0, sizeof(uint32_t) * n, c->stream));
@@ -438,7 +442,7 @@ void free_all(lps_ctx* c) {
     }
     dfree(c->keys); dfree(c->rank); dfree(c->placed); dfree(c->skeys); dfree(c->perm); dfree(c->bbox_part);
     dfree(c->posrho); dfree(c->force); dfree(c->fp); dfree(c->press); dfree(c->q); dfree(c->xq); dfree(c->rho_pred);
-    dfree(c->mk_mask); dfree(c->mk_ok); dfree(c->mk_cq);
+    dfree(c->mk_mask); dfree(c->mk_ok); dfree(c->mk_cq); dfree(c->nb_list); dfree(c->nb_count);
     dfree(c->cell_count); dfree(c->cell_lb); dfree(c->tile_sum);
     dfree(c->tables); dfree(c->boxes); dfree(c->spheres); dfree(c->planes); dfree(c->grid);
     dfree(c->d_mlp); dfree(c->d_mlp_packed); dfree(c->feat); dfree(c->seed); dfree(c->coll_x); dfree(c->coll_t);
@@ -459,10 +463,24 @@ lps_dev::Scenes scenes(const lps_ctx* c) {
                            c->d_actlist};
 }
 
-// Whether the stencil kernels give each particle a quad of lanes.  By
-// default below 512 particle blocks (131,072 slots): one lane per particle
-// then fills at most two waves per SIMD.
-bool quad_lanes(const lps_ctx* c) { return c->lanes == 4u || (c->lanes == 0u && c->n / LPS_BLOCK < 512u); }
+// Whether the stencil kernels give each particle several lanes.  By default
+// below 512 particle blocks (131,072 slots): one lane per particle then fills
+// at most two waves per SIMD.
+bool several_lanes(const lps_ctx* c) { return c->lanes == 4u || (c->lanes == 0u && c->n / LPS_BLOCK < 512u); }
+
+// How many lanes: a team of 16, or a quad.  Microseconds per step of a dam
+// break, 16 lanes against 4 (and 1):
+//   SPH     4,394 particles 44 : 82,  16,000 50 : 92 (171),  65,536 85 : 109
+//           (155),  128,000 129 : 153 (158): teams at every size they may run
+//   PCISPH  4,394 121 : 231,  16,000 223 : 377 (618),  31,250 486 : 567 (893),
+//           65,536 905 : 709 (905): teams up to 160 particle blocks, where the
+//           two cross; a team's density pass costs more per particle, and
+//           PCISPH runs one per correction
+uint32_t stencil_lanes(const lps_ctx* c) {
+    if (!several_lanes(c)) return 1u;
+    const uint32_t most = c->params.method == LPS_METHOD_SPH ? LPS_TEAM_BLOCKS : 160u;
+    return c->n / LPS_BLOCK <= most ? 16u : 4u;
+}
 
 lps_dev::PhysArgs phys_args(lps_ctx* c, const SimConst& k) {
     lps_dev::PhysArgs a;
@@ -485,7 +503,8 @@ lps_dev::PhysArgs phys_args(lps_ctx* c, const SimConst& k) {
     a.mk.stride = c->cap_n;
     a.mk.cq = c->mk_cq;
     a.c = k;
-    a.quad = quad_lanes(c) ? 1u : 0u;
+    a.nl = lps_dev::NbLists{c->nb_list, c->nb_count};
+    a.lanes = stencil_lanes(c);
     return a;
 }
 
@@ -775,7 +794,7 @@ StepResult enqueue_step(lps_ctx* c, float dt, bool seeded, bool feat_on) {
         if (state != 0u) break;
         k_known = kw;
         if (kw >= kmax) break;
-        if (c->lanes == 0u && f[4] < 512u) ac.quad = 1u;
+        if (c->lanes == 0u && f[4] < 512u && ac.lanes == 1u) ac.lanes = 4u;
     }
     {
         Timed t(c, "integrate");
@@ -1446,7 +1465,7 @@ int lps_get_tuning(lps_ctx* c, lps_tuning* t) {
     t->lookahead = c->lookahead;
     t->ms_per_step = 0.f;
     t->correction_threads = c->corr_threads;
-    t->lanes_per_particle = quad_lanes(c) ? 4u : 1u;
+    t->lanes_per_particle = several_lanes(c) ? 4u : 1u;
     return LPS_OK;
 }
 

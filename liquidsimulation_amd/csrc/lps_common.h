@@ -138,6 +138,12 @@ static inline __host__ __device__ float o2f(uint32_t u) {
 // candidates; a replaying pass filters any further candidates live.
 #define LPS_MC_ROWS 9
 
+// Neighbours per particle that the team kernels record (512 bytes per slot; a
+// resting fluid has about 30).
+#define LPS_NB_LIST 128u
+// Particle blocks up to which the stencil kernels may run 16 lanes per particle.
+#define LPS_TEAM_BLOCKS 512u
+
 // Position arrays scanned by the stencils carry this many padding entries:
 // the candidate filter reads whole groups of eight past a row's end.
 #define LPS_STENCIL_PAD 8

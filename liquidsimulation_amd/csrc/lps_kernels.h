@@ -39,6 +39,14 @@ struct NbMasks {
                        // density pass), then each prediction (read by the predicted-density pass)
 };
 
+// Neighbours recorded by the team kernels' density passes for the passes over
+// the same positions: per slot the number of accepted candidates (the particle
+// itself among them) and, in visiting order, the first LPS_NB_LIST of them.
+struct NbLists {
+    uint32_t* nb;      // [slots][LPS_NB_LIST]
+    uint32_t* count;   // [slots]
+};
+
 struct ReorderArgs {
     const uint2* placed;     // (index, key) of each cell's particles in the cell's slots, by arrival
     const uint32_t* cell_lb;
@@ -75,7 +83,8 @@ struct PhysArgs {
     const lps_plane* planes;
     NbMasks mk;
     SimConst c;
-    uint32_t quad;        // 1: density, forces and SPH pressure give each particle a quad of lanes
+    NbLists nl;           // for 16 lanes per particle
+    uint32_t lanes;       // lanes per particle of the stencil kernels: 1, 4 or 16
 };
 
 // per-block partial records (bounding box and energies) of a state

@@ -2224,6 +2224,667 @@ __global__ __launch_bounds__(LPS_BLOCK) void k_pci_pressure_q(
     if (lps_div::tiny_coord(xn.x, xn.y, xn.z)) g->tiny_pred = 1u;
 }
 
+// ===================================================== team stencils ====
+// Small scenes: a team of 16 lanes (a DPP row) per particle.  A stencil pass
+// over a few thousand particles is a chain of memory round trips, not work:
+// walking the nine rows of the stencil one after the other, as the one-lane
+// kernels do, waits for the cell table, the candidates and the kept
+// candidates' data in every row.  A team waits for each of them once.  Times
+// per launch, quads -> teams: density 18.7 -> 9.8, forces 18.6 -> 5.2, SPH
+// pressure 16.7 -> 4.8 us at 512 particles; 22.5 -> 13.0, 26.9 -> 7.7, 24.1 ->
+// 6.8 us in the 16k SPH dam break; predicted density 19.0 -> 12.4, its
+// pressure pass 17.0 -> 8.1 us in the 16k PCISPH one.
+// * lanes 0 to 8 load the ranges of the nine rows together, and a prefix sum
+//   numbers the candidates of the whole stencil;
+// * the density passes test the numbered candidates 64 at a time (four loads
+//   in flight per lane) with the exact squared distance, and append the
+//   accepted ones in order (ballot and bit count) to the team's list in LDS;
+// * the lists are also recorded in memory, so the passes over the same
+//   positions (forces, pressure) start from the list itself: one load gives
+//   16 neighbours, one gather their data;
+// * 16 lanes compute the terms of 16 neighbours, which are then added in
+//   order, either by every lane (row broadcasts; up to three sums) or by one
+//   lane per sum from LDS.
+// Accepted pairs and order of additions are those of for_neighbors; a lane
+// without a neighbour contributes +0, which leaves sums that start at +0
+// unchanged (they are never -0).  A particle with more neighbours than a
+// recorded list holds makes its wave's passes scan the candidates again.
+// All 64 lanes stay active until the end of the walk.
+constexpr uint32_t LPS_TEAM = 16u;
+
+__device__ __forceinline__ uint32_t team_lane() { return threadIdx.x & (LPS_TEAM - 1u); }
+
+// Lane K of the team's value on every lane of the team (row_newbcast).
+template <int K>
+__device__ __forceinline__ uint32_t team_bcast(uint32_t v) {
+    return (uint32_t)__builtin_amdgcn_mov_dpp((int)v, 0x150 + K, 0xF, 0xF, false);
+}
+template <int K>
+__device__ __forceinline__ float team_bcast(float v) {
+    return __uint_as_float(team_bcast<K>(__float_as_uint(v)));
+}
+
+// LDS of one wave is written and read by its own lanes, in program order.
+__device__ __forceinline__ void wave_lds_fence() {
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+}
+
+__device__ __forceinline__ uint32_t max_over_teams(uint32_t v) {
+    v = max(v, (uint32_t)__shfl_xor((int)v, 16, 64));
+    return max(v, (uint32_t)__shfl_xor((int)v, 32, 64));
+}
+
+// The candidates of a team's stencil, numbered in visiting order: number f of
+// row r (the largest r with pre[r] <= f) is slot f + off[r].
+struct TeamRows {
+    uint32_t pre[9], off[9], total;
+};
+
+__device__ __forceinline__ TeamRows team_rows(const GridView& G, const uint32_t* __restrict__ lb, float ax, float ay,
+                                              float az, bool valid) {
+    const uint32_t lane = team_lane();
+    const int xg = (int)truncf((ax + G.off0) / G.gs);
+    const int yg = (int)truncf((ay + G.off1) / G.gs);
+    const int zg = (int)truncf((az + G.off2) / G.gs);
+    const int x0 = max(xg - 1, 0), x1 = min(xg + 1, G.gx - 1);
+    const int z = zg - 1 + (int)(lane / 3u), y = yg - 1 + (int)(lane % 3u);
+    uint32_t b = 0u, n = 0u;
+    if (valid && lane < 9u && z >= 0 && z < G.gz && y >= 0 && y < G.gy) {
+        const uint32_t base = G.base + (uint32_t)G.gx * (uint32_t)y + G.gxy * (uint32_t)z;
+        b = lb[base + (uint32_t)x0];
+        n = lb[base + (uint32_t)x1 + 1u] - b;
+    }
+    // inclusive prefix sum over the row of lanes (row_shr 1, 2, 4, 8)
+    uint32_t s = n;
+    s += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)s, 0x111, 0xF, 0xF, false);
+    s += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)s, 0x112, 0xF, 0xF, false);
+    s += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)s, 0x114, 0xF, 0xF, false);
+    s += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)s, 0x118, 0xF, 0xF, false);
+    const uint32_t pre = s - n, off = b - pre;
+    TeamRows R;
+    R.pre[0] = 0u;
+    R.off[0] = team_bcast<0>(off);
+    R.pre[1] = team_bcast<1>(pre);
+    R.off[1] = team_bcast<1>(off);
+    R.pre[2] = team_bcast<2>(pre);
+    R.off[2] = team_bcast<2>(off);
+    R.pre[3] = team_bcast<3>(pre);
+    R.off[3] = team_bcast<3>(off);
+    R.pre[4] = team_bcast<4>(pre);
+    R.off[4] = team_bcast<4>(off);
+    R.pre[5] = team_bcast<5>(pre);
+    R.off[5] = team_bcast<5>(off);
+    R.pre[6] = team_bcast<6>(pre);
+    R.off[6] = team_bcast<6>(off);
+    R.pre[7] = team_bcast<7>(pre);
+    R.off[7] = team_bcast<7>(off);
+    R.pre[8] = team_bcast<8>(pre);
+    R.off[8] = team_bcast<8>(off);
+    R.total = team_bcast<15>(s);
+    return R;
+}
+
+// Every candidate of the stencil in visiting order, 64 per team and trip:
+// room() before each trip (the lists then take 64 more), take(accepted, j,
+// s2, number of the team's accepted lanes before this one, and in all) for
+// every 16.
+template <class Room, class Take>
+__device__ __forceinline__ void team_scan(const TeamRows& R, const float4* __restrict__ xs, uint32_t i, float px,
+                                          float py, float pz, float s_max, Room&& room, Take&& take) {
+    const uint32_t lane = team_lane(), shift = threadIdx.x & 48u;
+    const uint32_t last = max_over_teams(R.total);
+    for (uint32_t f0 = 0u; f0 < last; f0 += 64u) {
+        room();
+        uint32_t j[4];
+        float4 q[4];
+#pragma unroll
+        for (uint32_t u = 0; u < 4u; u++) {
+            const uint32_t f = f0 + 16u * u + lane;
+            uint32_t o = R.off[0];
+#pragma unroll
+            for (int r = 1; r < 9; r++) o = f >= R.pre[r] ? R.off[r] : o;
+            j[u] = f < R.total ? f + o : i;  // without a candidate: the particle itself, not taken
+            q[u] = xs[j[u]];
+        }
+#pragma unroll
+        for (uint32_t u = 0; u < 4u; u++) {
+            const float dx = q[u].x - px, dy = q[u].y - py, dz = q[u].z - pz;
+            const float s2 = dx * dx + dy * dy + dz * dz;
+            const bool ok = f0 + 16u * u + lane < R.total && s2 <= s_max;
+            const uint32_t m = (uint32_t)(__ballot(ok) >> shift) & 0xFFFFu;
+            take(ok, j[u], s2, (uint32_t)__popc(m & ((1u << lane) - 1u)), (uint32_t)__popc(m));
+        }
+    }
+}
+
+// The exact table index from s2 = d^2 (no threshold table).
+__device__ __forceinline__ uint32_t team_index(float s2, bool qidx, float div, float inv_div) {
+    const float d = sqrt_rn(s2);
+    return qidx ? table_index_q(d, div, inv_div) : min((uint32_t)(d / div), (uint32_t)(LPS_TABLE_SIZE - 1));
+}
+
+// acc[a] += the team's NT terms in lane order, `left` of them (uniform over the wave) at most.
+template <int NT>
+struct TeamSum {
+    static constexpr bool kLds = NT > 3;  // one lane per sum instead of every lane
+    float v[kLds ? 1 : NT];
+    __device__ __forceinline__ TeamSum() {
+        for (float& f : v) f = 0.f;
+    }
+    __device__ __forceinline__ void add(const float (&t)[NT], uint32_t left, float* s_t) {
+        if constexpr (kLds) {
+            const uint32_t lane = team_lane();
+#pragma unroll
+            for (int a = 0; a < NT; a++) s_t[a * LPS_TEAM + lane] = t[a];
+            wave_lds_fence();
+            const float4* r = reinterpret_cast<const float4*>(s_t + min(lane, (uint32_t)(NT - 1)) * LPS_TEAM);
+#pragma unroll
+            for (uint32_t k = 0; k < 4u; k++) {
+                const float4 w = r[k];
+                v[0] += w.x;
+                v[0] += w.y;
+                v[0] += w.z;
+                v[0] += w.w;
+            }
+            wave_lds_fence();
+        } else {
+            step<0>(t);
+            if (left > 4u) step<4>(t);
+            if (left > 8u) step<8>(t);
+            if (left > 12u) step<12>(t);
+        }
+    }
+    template <int K>
+    __device__ __forceinline__ void step(const float (&t)[NT]) {
+#pragma unroll
+        for (int a = 0; a < NT; a++) v[a] += team_bcast<K>(t[a]);
+#pragma unroll
+        for (int a = 0; a < NT; a++) v[a] += team_bcast<K + 1>(t[a]);
+#pragma unroll
+        for (int a = 0; a < NT; a++) v[a] += team_bcast<K + 2>(t[a]);
+#pragma unroll
+        for (int a = 0; a < NT; a++) v[a] += team_bcast<K + 3>(t[a]);
+    }
+    // the sums on every lane of the team
+    __device__ __forceinline__ void get(float (&out)[NT]) const {
+#pragma unroll
+        for (int a = 0; a < NT; a++) out[a] = kLds ? __shfl(v[0], a, 16) : v[kLds ? 0 : a];
+    }
+};
+
+constexpr uint32_t LPS_PENDING = 128u;  // entries of a team's list in LDS
+
+// Sum of W over the stencil of (px, py, pz), cells around the anchor of R;
+// records the accepted list.  s_list: the team's LPS_PENDING floats.
+__device__ __forceinline__ float team_density(const TeamRows& R, const float4* __restrict__ xs, uint32_t i, float px,
+                                              float py, float pz, const SimConst& c, const float* sW, float* s_list,
+                                              const lps_dev::NbLists& L, bool valid) {
+    const uint32_t lane = team_lane();
+    const bool qidx = index_q_ok(c.div);
+    uint32_t* __restrict__ out = L.nb + (size_t)i * LPS_NB_LIST;
+    uint32_t pend = 0u, done = 0u;
+    TeamSum<1> sum;
+    auto flush = [&]() {
+        const uint32_t last = max_over_teams(pend);
+        wave_lds_fence();
+        for (uint32_t t = 0u; t < last; t += LPS_TEAM) {
+            const bool ok = t + lane < pend;
+            const float s2 = ok ? s_list[t + lane] : 0.f;
+            const float w = sW[team_index(s2, qidx, c.div, c.inv_div)];
+            const float term[1] = {ok ? w : 0.f};
+            sum.add(term, last - t, nullptr);
+        }
+        wave_lds_fence();
+        done += pend;
+        pend = 0u;
+    };
+    team_scan(
+        R, xs, i, px, py, pz, c.s_max,
+        [&]() {
+            if (__any(pend > LPS_PENDING - 64u)) flush();
+        },
+        [&](bool ok, uint32_t j, float s2, uint32_t before, uint32_t all) {
+            const uint32_t at = pend + before;
+            if (ok) {
+                s_list[at] = s2;
+                if (done + at < LPS_NB_LIST) out[done + at] = j;
+            }
+            pend += all;
+        });
+    flush();
+    if (valid && lane == 0u) L.count[i] = done;
+    return sum.v[0];
+}
+
+// The terms of every recorded neighbour (or, where a list of the wave was too
+// short, of every accepted candidate) of particle i, summed in order:
+// term(ok, j, x_j, s2, pre(j), x_j - x_i, t) writes the terms (zeros when not
+// ok).  `count` is the recorded count (0 for an empty slot), s_list the team's
+// LPS_PENDING words, s_t its NT * 16 floats.
+template <int NT, class Rows, class Pre, class Term>
+__device__ __forceinline__ void team_replay(const lps_dev::NbLists& L, uint32_t count, uint32_t first_nb, Rows&& rows,
+                                            const float4* __restrict__ xs, uint32_t i, float px, float py, float pz,
+                                            const SimConst& c, uint32_t* s_list, float* s_t, Pre&& pre, Term&& term,
+                                            TeamSum<NT>& sum) {
+    const uint32_t lane = team_lane();
+    auto visit = [&](bool ok, uint32_t j, uint32_t left) {
+        const float4 q = xs[j];
+        const auto pv = pre(j);
+        const float dx = q.x - px, dy = q.y - py, dz = q.z - pz;
+        const float s2 = dx * dx + dy * dy + dz * dz;
+        float t[NT];
+        term(ok, j, q, s2, pv, make_float3(dx, dy, dz), t);
+        sum.add(t, left, s_t);
+    };
+    if (!__any(count > LPS_NB_LIST)) {
+        const uint32_t* __restrict__ nb = L.nb + (size_t)i * LPS_NB_LIST;
+        const uint32_t last = max_over_teams(count);
+        uint32_t next = first_nb;
+        for (uint32_t t = 0u; t < last; t += LPS_TEAM) {
+            const bool ok = t + lane < count;
+            const uint32_t j = ok ? next : i;
+            if (t + LPS_TEAM < last) next = nb[t + LPS_TEAM + lane];
+            visit(ok, j, last - t);
+        }
+        return;
+    }
+    const TeamRows R = rows();
+    uint32_t pend = 0u;
+    auto flush = [&]() {
+        const uint32_t last = max_over_teams(pend);
+        wave_lds_fence();
+        for (uint32_t t = 0u; t < last; t += LPS_TEAM) {
+            const bool ok = t + lane < pend;
+            visit(ok, ok ? s_list[t + lane] : i, last - t);
+        }
+        wave_lds_fence();
+        pend = 0u;
+    };
+    team_scan(
+        R, xs, i, px, py, pz, c.s_max,
+        [&]() {
+            if (__any(pend > LPS_PENDING - 64u)) flush();
+        },
+        [&](bool ok, uint32_t j, float, uint32_t before, uint32_t all) {
+            if (ok) s_list[pend + before] = j;
+            pend += all;
+        });
+    flush();
+}
+
+// The particle of a team kernel's thread: launch block lb covers LPS_BLOCK /
+// 16 particles, 16 lanes each.
+__device__ __forceinline__ uint32_t team_particle(uint32_t lb) {
+    return lb * (LPS_BLOCK / LPS_TEAM) + threadIdx.x / LPS_TEAM;
+}
+
+// k_density with a team per particle.
+__global__ __launch_bounds__(LPS_BLOCK) void k_density_t(const float4* __restrict__ pos, const DevGrid* g,
+                                                         lps_dev::Scenes S, const uint32_t* __restrict__ cell_lb,
+                                                         SimConst c, const float* __restrict__ tables,
+                                                         float4* __restrict__ posrho, float* __restrict__ press,
+                                                         float* __restrict__ q, lps_dev::NbLists L,
+                                                         uint32_t nlogical) {
+    if (step_dead(g)) return;
+    const uint32_t lb = xcd_block(nlogical);
+    if (lb == UINT_MAX) return;
+    const uint32_t i = team_particle(lb);
+    const float4 xi = pos[i];
+    TableSlice<LPS_BLOCK, LPS_TABLE_SIZE> W;
+    W.load(tables);
+    const BlockScene B = block_scene(S, i / LPS_BLOCK);
+    __shared__ float sW[LPS_TABLE_SIZE];
+    __shared__ float s_list[LPS_BLOCK / LPS_TEAM][LPS_PENDING];
+    const GridView G = grid_view(g, S.grid + B.s);
+    const bool valid = i < B.info.slot0 + B.info.count;
+    const TeamRows R = team_rows(G, cell_lb, xi.x, xi.y, xi.z, valid);
+    W.store(sW);
+    __syncthreads();
+    const float sum =
+        team_density(R, pos, i, xi.x, xi.y, xi.z, c, sW, s_list[threadIdx.x / LPS_TEAM], L, valid);
+    if (!valid || team_lane() != 0u) return;
+    const float rho = c.mass * sum;
+    float p = c.stiffness * (rho - c.rest_density);
+    if (p < 0.f) p *= c.npf;
+    posrho[i] = make_float4(xi.x, xi.y, xi.z, rho);
+    press[i] = p;
+    q[i] = p / (rho * rho);
+}
+
+// k_forces with a team per particle.
+template <bool FEAT>
+__global__ __launch_bounds__(LPS_BLOCK) void k_forces_t(
+    const float4* __restrict__ posrho, const float4* __restrict__ vel, const float4* __restrict__ vh,
+    const uint8_t* __restrict__ first, DevGrid* g, const uint32_t* __restrict__ cell_lb, SimConst c0,
+    const float* __restrict__ tables, const lps_box* __restrict__ boxes0, const lps_sphere* __restrict__ spheres0,
+    const lps_plane* __restrict__ planes0, float4* __restrict__ force, float4* __restrict__ xpred,
+    const float* __restrict__ pprev, float* __restrict__ feat, lps_dev::Scenes S, lps_dev::NbMasks mk,
+    lps_dev::NbLists L,
+    uint32_t nlogical) {
+    if (step_dead(g)) return;
+    const uint32_t lb = xcd_block(nlogical);
+    if (lb == UINT_MAX) return;
+    const uint32_t i = team_particle(lb);
+    const uint32_t nb0 = L.nb[(size_t)i * LPS_NB_LIST + team_lane()];
+    const float4 xi = posrho[i];
+    const float4 vi = vel[i];
+    const uint32_t listed = L.count[i];
+    const float4 vhi = vh[i];
+    const bool is_first = first[i] != 0;
+    const BlockScene B = block_scene(S, i / LPS_BLOCK);
+    __shared__ float sW1[LPS_TABLE_SIZE], sW2[LPS_TABLE_SIZE], sV2[LPS_TABLE_SIZE];
+    {
+        TableSlice<LPS_BLOCK, LPS_TABLE_SIZE> a, b, v;
+        a.load(tables + 1 * LPS_TABLE_SIZE);
+        b.load(tables + 2 * LPS_TABLE_SIZE);
+        v.load(tables + 4 * LPS_TABLE_SIZE);
+        a.store(sW1);
+        b.store(sW2);
+        v.store(sV2);
+    }
+    __syncthreads();
+    const GridView G = grid_view(g, S.grid + B.s);
+    const SimConst c = scene_const(c0, B.info);
+    const bool valid = i < B.info.slot0 + B.info.count;
+    const bool qidx = index_q_ok(c.div);
+    const float ri = xi.w;
+    // snx, sny, snz, lc, vfx, vfy, vfz, then (features) nb, dv
+    constexpr int NT = FEAT ? 9 : 7;
+    __shared__ uint32_t s_list[LPS_BLOCK / LPS_TEAM][LPS_PENDING];
+    __shared__ __align__(16) float s_t[LPS_BLOCK / LPS_TEAM][NT * LPS_TEAM];
+    TeamSum<NT> sum;
+    team_replay<NT>(L, valid ? listed : 0u, nb0, [&]() { return team_rows(G, cell_lb, xi.x, xi.y, xi.z, valid); },
+                    posrho, i, xi.x, xi.y, xi.z, c, s_list[threadIdx.x / LPS_TEAM], s_t[threadIdx.x / LPS_TEAM],
+                    [&](uint32_t j) { return vel[j]; },
+                    [&](bool ok, uint32_t j, const float4& xj, float s2, const float4& vj, const float3&,
+                               float (&t)[NT]) {
+        if (!ok) {
+#pragma unroll
+            for (int a = 0; a < NT; a++) t[a] = 0.f;
+            return;
+        }
+        const uint32_t idx = team_index(s2, qidx, c.div, c.inv_div);
+        const float rj = xj.w;
+        const float w1 = sW1[idx], wv = sV2[idx];
+        float n[8] = {(xi.x - xj.x) * w1, (xi.y - xj.y) * w1, (xi.z - xj.z) * w1, sW2[idx],
+                      (vj.x - vi.x) * wv, (vj.y - vi.y) * wv, (vj.z - vi.z) * wv, 0.f};
+        constexpr int NQ = FEAT ? 8 : 7;
+        if constexpr (FEAT)
+            n[7] = ((vj.x - vi.x) * (xi.x - xj.x) + (vj.y - vi.y) * (xi.y - xj.y) + (vj.z - vi.z) * (xi.z - xj.z)) * w1;
+        uint32_t key = lps_div::num_key(n[0]);
+        for (int a = 1; a < NQ; a++) key = min(key, lps_div::num_key(n[a]));
+        if (rj < 0x1p40f && lps_div::div_rn_ok(rj, key)) {
+            const float y = lps_div::rcp_rn(rj);
+            for (int a = 0; a < NQ; a++) n[a] = lps_div::div_rn(n[a], rj, y);
+        } else {
+            for (int a = 0; a < NQ; a++) n[a] = n[a] / rj;
+        }
+        const bool other = i != j;
+        t[0] = n[0];
+        t[1] = n[1];
+        t[2] = n[2];
+        t[3] = n[3];
+        t[4] = other ? n[4] : 0.f;
+        t[5] = other ? n[5] : 0.f;
+        t[6] = other ? n[6] : 0.f;
+        if constexpr (FEAT) {
+            t[7] = other ? 1.f : 0.f;
+            t[8] = other ? n[7] : 0.f;
+        }
+    }, sum);
+    float acc[NT];
+    sum.get(acc);
+    if (!valid || team_lane() != 0u) return;
+    float snx = acc[0], sny = acc[1], snz = acc[2];
+    const float lc = acc[3], vfx = acc[4], vfy = acc[5], vfz = acc[6];
+    float fx = c.gravity[0] * ri, fy = c.gravity[1] * ri, fz = c.gravity[2] * ri;
+    snx *= c.mass; sny *= c.mass; snz *= c.mass;
+    const float snl = sqrtf(snx * snx + sny * sny + snz * snz);
+    if constexpr (FEAT) {
+        float* fr = feat + i;
+        const size_t fs = mk.stride;
+        fr[0 * fs] = ri / c.rest_density - 1.f;
+        fr[1 * fs] = acc[7] * (1.f / 32.f);
+        fr[2 * fs] = acc[8] * c.mass * c.dt;
+        fr[3 * fs] = snx * c.h;
+        fr[4 * fs] = sny * c.h;
+        fr[5 * fs] = snz * c.h;
+        fr[6 * fs] = snl * c.h;
+        fr[7 * fs] = pprev[i] / (c.delta * c.rest_density);
+        fr[8 * fs] = sqrtf(vi.x * vi.x + vi.y * vi.y + vi.z * vi.z) * c.dt / c.h;
+        fr[9 * fs] = is_first ? 1.f : 0.f;
+    }
+    if (snl > c.st_threshold) {
+        const float k = -c.surface_tension * lc * c.mass;
+        fx += (snx / snl) * k;
+        fy += (sny / snl) * k;
+        fz += (snz / snl) * k;
+    }
+    fx += vfx * c.viscosity * c.mass;
+    fy += vfy * c.viscosity * c.mass;
+    fz += vfz * c.viscosity * c.mass;
+    force[i] = make_float4(fx, fy, fz, 0.f);
+    if (xpred) {
+        const float4 xo = make_float4(xi.x, xi.y, xi.z, 0.f);
+        const float4 xp = predict(xo, vi, vhi, is_first, fx + 0.f, fy + 0.f, fz + 0.f, ri, c,
+                                  boxes0 + B.info.box0, spheres0 + B.info.sphere0, planes0 + B.info.plane0);
+        xpred[i] = xp;
+        if (lps_div::tiny_coord(xp.x, xp.y, xp.z)) g->tiny_pred = 1u;
+        if constexpr (FEAT) {
+            const float ex = xp.x - xo.x, ey = xp.y - xo.y, ez = xp.z - xo.z;
+            feat[(size_t)10 * mk.stride + i] = sqrtf(ex * ex + ey * ey + ez * ez) / c.h;
+        }
+    }
+}
+
+// k_pressure_sph with a team per particle.
+__global__ __launch_bounds__(LPS_BLOCK) void k_pressure_sph_t(const float4* __restrict__ posrho,
+                                                              const float* __restrict__ q, const DevGrid* g,
+                                                              const uint32_t* __restrict__ cell_lb, SimConst c,
+                                                              const float* __restrict__ tables,
+                                                              float4* __restrict__ force, lps_dev::Scenes S,
+                                                              lps_dev::NbLists L, uint32_t nlogical) {
+    if (step_dead(g)) return;
+    const uint32_t lb = xcd_block(nlogical);
+    if (lb == UINT_MAX) return;
+    const uint32_t i = team_particle(lb);
+    const uint32_t nb0 = L.nb[(size_t)i * LPS_NB_LIST + team_lane()];
+    const float4 xi = posrho[i];
+    const float tf = q[i];
+    const uint32_t listed = L.count[i];
+    const BlockScene B = block_scene(S, i / LPS_BLOCK);
+    __shared__ float sP1[LPS_TABLE_SIZE];
+    {
+        TableSlice<LPS_BLOCK, LPS_TABLE_SIZE> a;
+        a.load(tables + 3 * LPS_TABLE_SIZE);
+        a.store(sP1);
+    }
+    __syncthreads();
+    const bool valid = i < B.info.slot0 + B.info.count;
+    const GridView G = grid_view(g, S.grid + B.s);
+    const bool fastdiv = c.s_max < 0x1p78f;  // accepted pairs have d < 2^40
+    const bool qidx = index_q_ok(c.div);
+    __shared__ uint32_t s_list[LPS_BLOCK / LPS_TEAM][LPS_PENDING];
+    TeamSum<3> sum;
+    team_replay<3>(L, valid ? listed : 0u, nb0, [&]() { return team_rows(G, cell_lb, xi.x, xi.y, xi.z, valid); },
+                   posrho, i, xi.x, xi.y, xi.z, c, s_list[threadIdx.x / LPS_TEAM], nullptr,
+                   [&](uint32_t j) { return q[j]; },
+                   [&](bool ok, uint32_t j, const float4&, float s2, float qj, const float3& dl, float (&t)[3]) {
+        if (!ok || i == j) {
+            t[0] = t[1] = t[2] = 0.f;
+            return;
+        }
+        const float d = sqrt_rn(s2);
+        float ux, uy, uz;
+        pair_dir<false>(dl, d, i, j, fastdiv, ux, uy, uz);
+        const float w = sP1[qidx ? table_index_q(d, c.div, c.inv_div) : min((uint32_t)(d / c.div), (uint32_t)(LPS_TABLE_SIZE - 1))];
+        const float sc = tf + qj;
+        t[0] = ux * sc * w;
+        t[1] = uy * sc * w;
+        t[2] = uz * sc * w;
+    }, sum);
+    float acc[3];
+    sum.get(acc);
+    if (!valid || team_lane() != 0u) return;
+    float4 f = force[i];
+    f.x += (-acc[0]) * c.mass * xi.w;
+    f.y += (-acc[1]) * c.mass * xi.w;
+    f.z += (-acc[2]) * c.mass * xi.w;
+    force[i] = f;
+}
+
+// k_pci_density with a team per particle: a workgroup of 256 threads takes a
+// 16-slot piece of an active particle block.
+template <bool FEAT>
+__global__ __launch_bounds__(LPS_BLOCK) void k_pci_density_t(
+    const float4* __restrict__ pos, const float4* __restrict__ xpred, DevGrid* g, const uint32_t* __restrict__ cell_lb,
+    SimConst c, const float* __restrict__ tables, float* __restrict__ rho_pred, float* __restrict__ press,
+    float4* __restrict__ xq, uint32_t k, float* __restrict__ feat, const float4* __restrict__ posrho,
+    lps_dev::Scenes S, lps_dev::NbMasks mk, lps_dev::NbLists nl, uint32_t nlogical) {
+    const uint32_t slot = (k - 1u) % LPS_MAX_ITER_SLOTS;
+    if (step_dead(g) || g->running == 0u) return;
+    const uint32_t L = g->list_of[k % LPS_MAX_ITER_SLOTS];
+    uint32_t s0 = 0u;
+    const uint32_t lb = active_piece<LPS_BLOCK / LPS_TEAM>(g, S, L, s0);
+    if (lb == UINT_MAX) return;
+    __shared__ float sW[LPS_TABLE_SIZE];
+    __shared__ float s_list[LPS_BLOCK / LPS_TEAM][LPS_PENDING];
+    __shared__ uint32_t s_max[LPS_BLOCK / 64];
+    TableSlice<LPS_BLOCK, LPS_TABLE_SIZE> W;
+    W.load(tables);
+    // the slot's own state loads while the tables are staged (every slot of
+    // an active piece lies within the allocated slots)
+    const uint32_t i = s0 + threadIdx.x / LPS_TEAM;
+    const float4 xa = pos[i];
+    const float4 xi = xpred[i];
+    const BlockScene B = block_scene(S, lb);
+    const GridView G = grid_view(g, S.grid + B.s);
+    const bool valid = i < B.info.slot0 + B.info.count;
+    const TeamRows R = team_rows(G, cell_lb, xa.x, xa.y, xa.z, valid);
+    W.store(sW);
+    __syncthreads();
+    const float sum =
+        team_density(R, xpred, i, xi.x, xi.y, xi.z, c, sW, s_list[threadIdx.x / LPS_TEAM], nl, valid);
+    uint32_t ebits = 0;
+    if (valid) {
+        if (team_lane() == 0u) {
+            const float rp = c.mass * sum;
+            float e = rp - c.rest_density;
+            float dp = c.delta * e;
+            if (dp < 0.f) {
+                dp *= c.npf;
+                e *= c.npf;
+            }
+            const SceneGrid* sg = S.grid + B.s;
+            const size_t ob = (size_t)sg->buf_of[k % LPS_MAX_ITER_SLOTS] * mk.stride;
+            const float pold =
+                k == 1u ? 0.f : press[(size_t)sg->buf_of[(k - 1u) % LPS_MAX_ITER_SLOTS] * mk.stride + i];
+            const float p = pold + dp;
+            rho_pred[ob + i] = rp;
+            press[ob + i] = p;
+            xq[i] = make_float4(xi.x, xi.y, xi.z, p / (rp * rp));
+            if (FEAT && k == 1u) {
+                float* fr = feat + i;
+                const size_t fs = mk.stride;
+                const float e1 = rp / c.rest_density - 1.f;
+                fr[11 * fs] = e1;
+                fr[12 * fs] = fmaxf(e1, 0.f);
+                fr[13 * fs] = dp / (c.delta * c.rest_density);
+                fr[14 * fs] = (rp - posrho[i].w) / c.rest_density;
+                fr[15 * fs] = e1 * e1 * 100.f;
+            }
+            ebits = __float_as_uint(fabsf(e));
+        }
+    }
+    ebits = wave_max_u32(ebits);
+    if (lane_id() == 0) s_max[threadIdx.x >> 6] = ebits;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        uint32_t m = 0;
+        for (uint32_t w = 0; w < LPS_BLOCK / 64; w++) m = max(m, s_max[w]);
+        if (m) atomicMax(&S.grid[B.s].err_bits[slot], m);
+    }
+}
+
+// k_pci_pressure with a team per particle.
+__global__ __launch_bounds__(LPS_BLOCK) void k_pci_pressure_t(
+    const float4* __restrict__ pos, const float4* __restrict__ xq, const float* __restrict__ rho_pred, DevGrid* g,
+    const uint32_t* __restrict__ cell_lb, SimConst c0, const float* __restrict__ tables, float4* __restrict__ fp,
+    const float4* __restrict__ force, const float4* __restrict__ posrho, const float4* __restrict__ vel,
+    const float4* __restrict__ vh, const uint8_t* __restrict__ first, const lps_box* __restrict__ boxes0,
+    const lps_sphere* __restrict__ spheres0, const lps_plane* __restrict__ planes0, float4* __restrict__ xpred_next,
+    uint32_t k, lps_dev::Scenes S, lps_dev::NbMasks mk, lps_dev::NbLists nl, LoopRule rule, uint32_t* __restrict__ host_flag,
+    uint32_t nlogical) {
+    if (blockIdx.x == 0) loop_rule_block(g, S, k, rule, c0.rest_density, host_flag);
+    if (step_dead(g)) return;
+    uint32_t s0 = 0u;
+    const uint32_t lb = active_piece<LPS_BLOCK / LPS_TEAM>(g, S, g->list_of[k % LPS_MAX_ITER_SLOTS], s0);
+    if (lb == UINT_MAX) return;
+    // the slot's own state loads while the tables are staged; the
+    // predicted-density pass's (prediction, p / rho*^2)
+    const uint32_t i = s0 + threadIdx.x / LPS_TEAM;
+    const uint32_t nb0 = nl.nb[(size_t)i * LPS_NB_LIST + team_lane()];
+    const float4 xa = pos[i];
+    const float4 xi = xq[i];
+    const uint32_t listed = nl.count[i];
+    const float4 f = force[i];
+    const float4 xr = posrho[i];
+    const float4 vi = vel[i];
+    const float4 vhi = vh[i];
+    const bool is_first = first[i] != 0;
+    const BlockScene B = block_scene(S, lb);
+    const uint32_t stop = S.grid[B.s].stop_iter;
+    if (stop != 0u && stop < k) return;
+    const bool fastdiv = c0.s_max < 0x1p78f;
+    const bool nocheck = fastdiv && g->tiny_pred == 0u;
+    const bool qidx = index_q_ok(c0.div);
+    __shared__ float sP1[LPS_TABLE_SIZE];
+    {
+        TableSlice<LPS_BLOCK, LPS_TABLE_SIZE> a;
+        a.load(tables + 3 * LPS_TABLE_SIZE);
+        a.store(sP1);
+    }
+    __syncthreads();
+    const bool valid = i < B.info.slot0 + B.info.count;
+    const GridView G = grid_view(g, S.grid + B.s);
+    const SimConst c = scene_const(c0, B.info);
+    const float tf = xi.w;
+    __shared__ uint32_t s_list[LPS_BLOCK / LPS_TEAM][LPS_PENDING];
+    TeamSum<3> sum;
+    team_replay<3>(nl, valid ? listed : 0u, nb0, [&]() { return team_rows(G, cell_lb, xa.x, xa.y, xa.z, valid); }, xq,
+                   i, xi.x, xi.y, xi.z, c, s_list[threadIdx.x / LPS_TEAM], nullptr, [](uint32_t) { return 0; },
+                   [&](bool ok, uint32_t j, const float4& xqj, float s2, int, const float3& dl, float (&t)[3]) {
+        if (!ok || i == j) {
+            t[0] = t[1] = t[2] = 0.f;
+            return;
+        }
+        const float d = sqrt_rn(s2);
+        float ux, uy, uz;
+        if (nocheck)
+            pair_dir<true>(dl, d, i, j, fastdiv, ux, uy, uz);
+        else
+            pair_dir<false>(dl, d, i, j, fastdiv, ux, uy, uz);
+        const float w = sP1[qidx ? table_index_q(d, c.div, c.inv_div) : min((uint32_t)(d / c.div), (uint32_t)(LPS_TABLE_SIZE - 1))];
+        const float sc = tf + xqj.w;
+        t[0] = ux * sc * w;
+        t[1] = uy * sc * w;
+        t[2] = uz * sc * w;
+    }, sum);
+    float acc[3];
+    sum.get(acc);
+    if (!valid || team_lane() != 0u) return;
+    const size_t ob = (size_t)S.grid[B.s].buf_of[k % LPS_MAX_ITER_SLOTS] * mk.stride;
+    const float ri = rho_pred[ob + i];
+    const float4 f4 = make_float4((-acc[0]) * c.mass * ri, (-acc[1]) * c.mass * ri, (-acc[2]) * c.mass * ri, 0.f);
+    fp[ob + i] = f4;
+    const float4 xn = predict(make_float4(xr.x, xr.y, xr.z, 0.f), vi, vhi, is_first, f.x + f4.x,
+                              f.y + f4.y, f.z + f4.z, xr.w, c, boxes0 + B.info.box0, spheres0 + B.info.sphere0,
+                              planes0 + B.info.plane0);
+    xpred_next[i] = xn;
+    if (lps_div::tiny_coord(xn.x, xn.y, xn.z)) g->tiny_pred = 1u;
+}
+
 // integrate (SPHKernels.cl:424-455) + pciAddPressureForce (SPHKernels.cl:880-890)
 // + handleCollisions (SPHKernels.cl:457-486); accumulates the bounding box of
 // the new positions for the next step.
@@ -2367,7 +3028,13 @@ void launch_reorder(hipStream_t s, const ReorderArgs& a) {
 
 void launch_density(hipStream_t s, const PhysArgs& a, float* press, float* q) {
     const uint32_t nl = cdiv(a.c.n, LPS_BLOCK);
-    if (a.quad) {
+    if (a.lanes == LPS_TEAM) {
+        const uint32_t nt = nl * LPS_TEAM;
+        k_density_t<<<xcd_grid(nt), LPS_BLOCK, 0, s>>>(a.pos, a.g, a.sc, a.cell_lb, a.c, a.tables, a.posrho, press, q,
+                                                      a.nl, nt);
+        return;
+    }
+    if (a.lanes == LPS_QUAD) {
         const uint32_t nq = nl * LPS_QUAD;
         k_density_q<<<xcd_grid(nq), LPS_BLOCK, 0, s>>>(a.pos, a.g, a.sc, a.cell_lb, a.c, a.tables, a.posrho, press, q,
                                                       a.mk, nq);
@@ -2379,7 +3046,15 @@ void launch_density(hipStream_t s, const PhysArgs& a, float* press, float* q) {
 
 void launch_forces(hipStream_t s, const PhysArgs& a, float4* xpred, const float* pprev, float* feat) {
     const uint32_t nl = cdiv(a.c.n, LPS_BLOCK);
-    if (a.quad) {
+    if (a.lanes == LPS_TEAM) {
+        const uint32_t nt = nl * LPS_TEAM;
+        auto kern = feat ? k_forces_t<true> : k_forces_t<false>;
+        kern<<<xcd_grid(nt), LPS_BLOCK, 0, s>>>(a.posrho, a.vel, a.vh, a.first, a.g, a.cell_lb, a.c, a.tables,
+                                                a.boxes, a.spheres, a.planes, a.force, xpred, pprev, feat, a.sc, a.mk,
+                                                a.nl, nt);
+        return;
+    }
+    if (a.lanes == LPS_QUAD) {
         const uint32_t nq = nl * LPS_QUAD;
         auto kern = feat ? k_forces_q<true> : k_forces_q<false>;
         kern<<<xcd_grid(nq), LPS_BLOCK, 0, s>>>(a.posrho, a.vel, a.vh, a.first, a.g, a.cell_lb, a.c, a.tables,
@@ -2394,7 +3069,13 @@ void launch_forces(hipStream_t s, const PhysArgs& a, float4* xpred, const float*
 
 void launch_pressure_sph(hipStream_t s, const PhysArgs& a, const float* q) {
     const uint32_t nl = cdiv(a.c.n, LPS_BLOCK);
-    if (a.quad) {
+    if (a.lanes == LPS_TEAM) {
+        const uint32_t nt = nl * LPS_TEAM;
+        k_pressure_sph_t<<<xcd_grid(nt), LPS_BLOCK, 0, s>>>(a.posrho, q, a.g, a.cell_lb, a.c, a.tables, a.force, a.sc,
+                                                           a.nl, nt);
+        return;
+    }
+    if (a.lanes == LPS_QUAD) {
         const uint32_t nq = nl * LPS_QUAD;
         k_pressure_sph_q<<<xcd_grid(nq), LPS_BLOCK, 0, s>>>(a.posrho, q, a.g, a.cell_lb, a.c, a.tables, a.force, a.sc,
                                                            a.mk, nq);
@@ -2415,7 +3096,14 @@ static void pci_density_wg(hipStream_t s, const PhysArgs& a, const float4* xpred
 
 void launch_pci_density(hipStream_t s, const PhysArgs& a, const float4* xpred, float* rho_pred, float* press,
                         float4* xq, uint32_t k, float* feat, uint32_t threads) {
-    if (a.quad) {
+    if (a.lanes == LPS_TEAM) {
+        const uint32_t nl = cdiv(a.c.n, LPS_BLOCK);
+        auto kern = (feat && k == 1u) ? k_pci_density_t<true> : k_pci_density_t<false>;
+        kern<<<xcd_grid(nl * LPS_TEAM), LPS_BLOCK, 0, s>>>(a.pos, xpred, a.g, a.cell_lb, a.c, a.tables, rho_pred, press,
+                                                          xq, k, feat, a.posrho, a.sc, a.mk, a.nl, nl);
+        return;
+    }
+    if (a.lanes == LPS_QUAD) {
         const uint32_t nl = cdiv(a.c.n, LPS_BLOCK);
         auto kern = (feat && k == 1u) ? k_pci_density_q<true> : k_pci_density_q<false>;
         kern<<<xcd_grid(nl * LPS_QUAD), LPS_BLOCK, 0, s>>>(a.pos, xpred, a.g, a.cell_lb, a.c, a.tables, rho_pred, press,
@@ -2439,7 +3127,14 @@ static void pci_pressure_wg(hipStream_t s, const PhysArgs& a, const float4* xq, 
 void launch_pci_pressure(hipStream_t s, const PhysArgs& a, const float4* xq, const float* rho_pred, float4* fp,
                          float4* xpred_next, uint32_t k, const LoopRule& rule, uint32_t* host_flag,
                          uint32_t threads) {
-    if (a.quad) {
+    if (a.lanes == LPS_TEAM) {
+        const uint32_t nl = cdiv(a.c.n, LPS_BLOCK);
+        k_pci_pressure_t<<<xcd_grid(nl * LPS_TEAM), LPS_BLOCK, 0, s>>>(
+            a.pos, xq, rho_pred, a.g, a.cell_lb, a.c, a.tables, fp, a.force, a.posrho, a.vel, a.vh, a.first, a.boxes,
+            a.spheres, a.planes, xpred_next, k, a.sc, a.mk, a.nl, rule, host_flag, nl);
+        return;
+    }
+    if (a.lanes == LPS_QUAD) {
         const uint32_t nl = cdiv(a.c.n, LPS_BLOCK);
         k_pci_pressure_q<<<xcd_grid(nl * LPS_QUAD), LPS_BLOCK, 0, s>>>(
             a.pos, xq, rho_pred, a.g, a.cell_lb, a.c, a.tables, fp, a.force, a.posrho, a.vel, a.vh, a.first, a.boxes,
