@@ -13,7 +13,11 @@
 #define LPS_BLOCK 256           // threads per block for particle kernels (4 wave64)
 #define LPS_SCAN_ITEMS 4       // cells per thread in the cell-table scan
 #define LPS_SCAN_TILE (LPS_BLOCK * LPS_SCAN_ITEMS)
-#define LPS_MAX_ITER_SLOTS 64   // per-correction error slots, used as a ring: correction k owns slot (k - 1) % 64
+#define LPS_MAX_ITER_SLOTS 64   // per-correction slots (buffers, block lists, host flags), used as a ring
+// Maximum error of a correction: sub-maxima per scene, 64 bytes apart, in two
+// sets that the corrections use in turn
+#define LPS_ERR_SUBS 16u
+#define LPS_ERR_STRIDE 16u
 // host flag words per correction slot: state, corrections, error bits,
 // converged, particle blocks the next correction runs (then unused)
 #define LPS_FLAG_WORDS 8
@@ -64,9 +68,6 @@ struct SceneGrid {
     // the loop rule of correction k - 1 chose as neither that correction's nor
     // the best one's, so the best correction's inputs survive until the stop.
     uint8_t buf_of[LPS_MAX_ITER_SLOTS];
-    // max |e_i| (float bits) of correction k in slot (k - 1) % 64; the loop
-    // rule of correction k clears the slot of correction k + 1
-    uint32_t err_bits[LPS_MAX_ITER_SLOTS];
 };
 
 // Global state of the current step.

@@ -21,7 +21,14 @@ struct Scenes {
     uint32_t count;
     uint32_t nblocks;        // particle blocks (slots / LPS_BLOCK)
     uint32_t* act_list;      // [2][nblocks] active-block lists of the correction kernels
+    uint32_t* err;           // [count][2][LPS_ERR_SUBS] max |e_i| (float bits), LPS_ERR_STRIDE words apart
 };
+
+// The sub-maxima of correction k's error in a scene; the loop rule of
+// correction k clears those of correction k + 1.
+__device__ __forceinline__ uint32_t* err_slot(const Scenes& S, uint32_t scene, uint32_t k) {
+    return S.err + ((size_t)scene * 2u + (k & 1u)) * (LPS_ERR_SUBS * LPS_ERR_STRIDE);
+}
 
 // Candidate masks recorded by one neighbour pass for the next pass over the
 // same positions and cells (k_density -> k_forces / k_pressure_sph,

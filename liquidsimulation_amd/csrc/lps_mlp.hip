@@ -298,7 +298,10 @@ __global__ __launch_bounds__(LPS_BLOCK) __attribute__((amdgpu_waves_per_eu(4))) 
         // The test is uniform over the block, so the whole block leaves
         // before the barrier or none of it does.
         const uint32_t s = sc.block_scene[blockIdx.x];
-        const uint32_t eb = sc.grid[s].err_bits[0];
+        const uint32_t* err = lps_dev::err_slot(sc, s, 1u);
+        uint32_t eb = 0u;
+#pragma unroll
+        for (uint32_t u = 0; u < LPS_ERR_SUBS; u++) eb = max(eb, err[u * LPS_ERR_STRIDE]);
         if (eb >= 0x7F800000u || (1u >= rule.min_iter && __uint_as_float(eb) / rest_density < rule.tol) ||
             1u >= rule.max_iter)
             return;
