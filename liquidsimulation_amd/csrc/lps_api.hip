@@ -323,6 +323,7 @@ SimConst make_const(const lps_ctx* c, float dt, float delta) {
     k.nsphere = 0;
     k.nplane = 0;
     k.cell_cap = c->cell_cap;
+    k.quick_forces = c->der.quick_forces;
     return k;
 }
 
@@ -546,6 +547,7 @@ void enqueue_grid(lps_ctx* c) {
         r.perm = c->perm;
         r.sc = scenes(c);
         r.cq = c->mk_cq;
+        r.tiny_key = c->der.tiny_key;
         lps_dev::launch_reorder(s, r);
         c->cur = b;
     }

@@ -83,6 +83,8 @@ struct DevGrid {
     uint32_t final_err;      // max over scenes of the last correction's max |e| (float bits)
     uint32_t converged;      // every scene met the tolerance
     uint32_t tiny_pred;      // a prediction of this step has a coordinate in (0, 2^-56)
+    uint32_t odd_state;      // a nonzero coordinate or velocity component of the step's state is below the
+                             // magnitude of Derived::tiny_key, or a density outside [2^-78, 2^40)
     // Correction kernels run only the particle blocks of scenes whose loop
     // is still running.  Two block lists alternate; list_of[k % 64] names the
     // list of correction k (both of its passes).  Entries are written once per
@@ -120,6 +122,7 @@ struct SimConst {
     uint32_t n;
     uint32_t nbox, nsphere, nplane;
     uint32_t cell_cap;  // allocated cell-table entries (excluding the sentinel)
+    uint32_t quick_forces;  // Derived::quick_forces
 };
 
 // orderable encoding of floats for atomic min/max (monotone for non-NaN)
@@ -156,6 +159,12 @@ static inline __host__ __device__ float o2f(uint32_t u) {
 // Host-side derived quantities (lps_host.cpp).
 struct Derived {
     float h, div, mass, s_max, s_relax, inv_div;
+    // The force passes skip the range checks of their quotients' numerators
+    // while the state's coordinates and velocities are 0 or >= tau in
+    // magnitude: their differences are then 0 or >= tau 2^-23, and the products
+    // with table entries of at least 2^e 0 or >= tau 2^(e - 23) >= 2^-80.
+    uint32_t tiny_key;      // 2 bits(tau) - 1 (see lps_div::num_key), tau = 2^-56 or 2^(-56 - e) for e < 0
+    uint32_t quick_forces;  // such a tau of at most 2^-16 exists
     float tables[5][LPS_TABLE_SIZE];  // W, W', W'' (poly6), spiky', viscosity''
     // thr[k] (k = 1..1000): smallest float s >= 0 whose lookup index
     // min(trunc(sqrtf(s) / div), 1000) is >= k; thr[0] = 0, thr[1001] = +inf.

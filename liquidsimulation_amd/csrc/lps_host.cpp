@@ -66,6 +66,18 @@ void lps_compute_derived(const lps_params* p, Derived* d) {
     }
     d->h = r;
     d->div = step;
+    float least = INFINITY, least2 = INFINITY;  // of W' and the Laplacian (factors), of W'' (a numerator itself)
+    for (int i = 0; i <= kSubdivision; i++) {
+        for (int k : {1, 4})
+            if (d->tables[k][i] != 0.f) least = std::min(least, std::fabs(d->tables[k][i]));
+        if (d->tables[2][i] != 0.f) least2 = std::min(least2, std::fabs(d->tables[2][i]));
+    }
+    const int e = std::isfinite(least) ? std::min(std::ilogb(least), 0) : 0;
+    d->quick_forces = e >= -40 && least2 >= 0x1p-80f ? 1u : 0u;
+    const float tau = std::ldexp(1.f, -56 - std::max(e, -40));
+    uint32_t bits;
+    std::memcpy(&bits, &tau, sizeof(float));
+    d->tiny_key = 2u * bits - 1u;
     if (p->mass_override > 0.f) {
         d->mass = p->mass_override;
     } else {

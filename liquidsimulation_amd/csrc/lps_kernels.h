@@ -58,7 +58,7 @@ struct ReorderArgs {
     const uint2* placed;     // (index, key) of each cell's particles in the cell's slots, by arrival
     const uint32_t* cell_lb;
     uint32_t n;              // slots (whole blocks)
-    const DevGrid* g;
+    DevGrid* g;
     const float4 *pos_in, *vel_in, *vh_in;
     const uint8_t* first_in;
     const uint32_t* id_in;
@@ -71,6 +71,7 @@ struct ReorderArgs {
     uint32_t* perm;
     Scenes sc;            // slot -> scene (for the compact copy's grid)
     uint2* cq;            // compact copy of pos_out for the density pass's filter
+    uint32_t tiny_key;    // Derived::tiny_key
 };
 
 // Buffers shared by the physics kernels of one step (sorted order).

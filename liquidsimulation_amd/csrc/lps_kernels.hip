@@ -450,12 +450,12 @@ __device__ __forceinline__ void for_neighbors_masked(const GridView& G, const ui
 // are those of for_neighbors_masked in MC_REPLAY mode; a plane where some lane
 // of the wave has no recorded masks or a row longer than one window of 32
 // candidates is walked row by row as there.
-template <int VB, class Acc, class Pre, class F>
+// SELF: the particle itself is visited too.
+template <int VB, bool SELF, class Pre, class F>
 __device__ __forceinline__ void for_neighbors_planes(const GridView& G, const uint32_t* __restrict__ lb, float ax,
                                                      float ay, float az, const float4* __restrict__ xs, float px,
                                                      float py, float pz, float s_max, float s_relax,
-                                                     const lps_dev::NbMasks& M, uint32_t i, Acc&& accept_extra,
-                                                     Pre&& pre, F&& fn) {
+                                                     const lps_dev::NbMasks& M, uint32_t i, Pre&& pre, F&& fn) {
     const char* __restrict__ xb = reinterpret_cast<const char*>(xs);
     const int xg = (int)truncf((ax + G.off0) / G.gs);
     const int yg = (int)truncf((ay + G.off1) / G.gs);
@@ -482,6 +482,8 @@ __device__ __forceinline__ void for_neighbors_planes(const GridView& G, const ui
         // one choice for the lanes in this plane
         if (__all(merge)) {
             uint32_t m0 = m[0], m1 = m[1], m2 = m[2];
+            // the particle's own bit lies in the middle row of the middle plane
+            if (!SELF && rz == 1u) m1 &= ~(1u << (i - b[1]));
             while (m0 | m1 | m2) {
                 uint32_t jj[VB];
                 uint32_t cnt = 0u;
@@ -510,11 +512,11 @@ __device__ __forceinline__ void for_neighbors_planes(const GridView& G, const ui
                     const uint32_t j = jj[t];
                     const float dx = q[t].x - px, dy = q[t].y - py, dz = q[t].z - pz;
                     const float s2 = dx * dx + dy * dy + dz * dz;
-                    visit_slot(fn, (uint32_t)t < cnt && s2 <= s_max && accept_extra(j), j, q[t], s2, pv[t],
-                               make_float3(dx, dy, dz));
+                    visit_slot(fn, (uint32_t)t < cnt && s2 <= s_max, j, q[t], s2, pv[t], make_float3(dx, dy, dz));
                 }
             }
         } else {
+            auto accept_extra = [&](uint32_t j) { return SELF || j != i; };
             for (uint32_t ry = 0; ry < 3u; ry++) {
                 const int y = yg - 1 + (int)ry;
                 if (y < 0 || y >= G.gy) continue;
@@ -527,6 +529,14 @@ __device__ __forceinline__ void for_neighbors_planes(const GridView& G, const ui
     }
 }
 
+// v_cvt_u32_f32: truncates, and saturates a negative value or NaN to 0 (which
+// a C conversion leaves undefined).
+__device__ __forceinline__ uint32_t cvt_u32_sat(float f) {
+    uint32_t u;
+    asm("v_cvt_u32_f32 %0, %1" : "=v"(u) : "v"(f));
+    return u;
+}
+
 // Lookup index min(trunc(sqrtf(s2) / div), 1000) of a squared distance
 // s2 <= s_max from the threshold table (see Derived::thr): the hardware
 // square root and 1/div give the quotient to within 5e-4; one below that,
@@ -534,8 +544,8 @@ __device__ __forceinline__ void for_neighbors_planes(const GridView& G, const ui
 // guess is held below 1000, so the index stays in the table for every s2
 // (NaN and +inf included), which the branch-free density visits rely on.
 __device__ __forceinline__ uint32_t table_index(float s2, const float* __restrict__ thr, float inv_div) {
-    const float qa = __builtin_amdgcn_sqrtf(s2) * inv_div - 1e-3f;
-    const uint32_t g = min((uint32_t)fmaxf(qa, 0.f), (uint32_t)(LPS_TABLE_SIZE - 2));
+    const float qa = __builtin_fmaf(__builtin_amdgcn_sqrtf(s2), inv_div, -1e-3f);
+    const uint32_t g = min(cvt_u32_sat(qa), (uint32_t)(LPS_TABLE_SIZE - 2));
     return g + (s2 >= thr[g + 1u] ? 1u : 0u);
 }
 
@@ -576,6 +586,25 @@ __device__ __forceinline__ float sqrt_rn(float s) {
         return r;
     }
     return sqrtf(s);
+}
+
+// d = sqrtf(s) and y = RN(1 / d) from one hardware reciprocal square root y0
+// (within one ulp): g = s y0 and one fused correction give the root, one fused
+// Newton step of y0 on d the reciprocal.  Returns whether both are exact: not
+// below 2^-96 (the residuals lose bits), and not where the first residual is
+// exactly 2^-24, which holds the one significand per exponent whose Newton
+// step lands on a midpoint (d all ones).  tests/rsq_rn_check.hip compares both
+// with the IEEE operations for every float in [2^-96, 2^80).  One
+// transcendental and 6 operations instead of two and 12 (sqrt_rn, rcp_rn):
+// with the particle itself taken out of the walk, k_pci_pressure 58.5 -> 53.0
+// us at 524,288 particles, k_pressure_sph 41.8 -> 34.2 at 151,219.
+__device__ __forceinline__ bool dist_rn(float s, float& d, float& y) {
+    const float y0 = __builtin_amdgcn_rsqf(s);
+    const float g = s * y0;
+    d = __builtin_fmaf(__builtin_fmaf(-g, g, s), 0.5f * y0, g);
+    const float e = __builtin_fmaf(-d, y0, 1.f);
+    y = __builtin_fmaf(e, y0, y0);
+    return s >= 0x1p-96f && e != 0x1p-24f;
 }
 
 // ---------------------------------------------------------- colliders --
@@ -754,6 +783,63 @@ __device__ __forceinline__ void pair_dir(const float3& dl, float d, uint32_t i, 
         uy = i > j ? 1.f : -1.f;
         uz = 0.f;
     }
+}
+
+// Distance and direction (x_i - x_j) / d of an accepted pair.
+template <bool NOCHECK>
+__device__ __forceinline__ float pair_geometry(const float3& dl, float s2, uint32_t i, uint32_t j, bool fastdiv,
+                                               float& ux, float& uy, float& uz) {
+    float d;
+    if constexpr (NOCHECK) {
+        float y;
+        if (dist_rn(s2, d, y)) {
+            ux = lps_div::div_rn(-dl.x, d, y);
+            uy = lps_div::div_rn(-dl.y, d, y);
+            uz = lps_div::div_rn(-dl.z, d, y);
+            return d;
+        }
+    }
+    d = sqrt_rn(s2);
+    pair_dir<NOCHECK>(dl, d, i, j, fastdiv, ux, uy, uz);
+    return d;
+}
+
+// The quotients by rho_j of a pair's force terms, in place.  QUICK: every
+// coordinate and velocity component is 0 or at least the least magnitude that
+// keeps its products with the tables' entries at 2^-80 or above (checked when
+// the state was sorted; Derived::tiny_key), and every density lies in [2^-78,
+// 2^40) (checked by the density pass), so numerators 0 to 6 are 0 or >= 2^-80
+// and y is the density pass's RN(1 / rho_j); the eighth (a product of two
+// differences) is checked here.  Per pair this saves seven checks and the
+// reciprocal: 75.4 -> 70.1 us at 524,288 particles (with features 80.7 -> 71.2),
+// 51.4 -> 42.2 at 151,219 (SPH).
+template <bool QUICK, int NQ>
+__device__ __forceinline__ void force_quotients(float (&n)[8], float rj, float y) {
+    if constexpr (QUICK) {
+#pragma unroll
+        for (int t = 0; t < 7; t++) n[t] = lps_div::div_rn(n[t], rj, y);
+        if constexpr (NQ > 7)
+            n[7] = lps_div::num_key(n[7]) >= lps_div::kNumMin ? lps_div::div_rn(n[7], rj, y) : n[7] / rj;
+    } else {
+        uint32_t key = lps_div::num_key(n[0]);
+        for (int t = 1; t < NQ; t++) key = min(key, lps_div::num_key(n[t]));
+        if (rj < 0x1p40f && lps_div::div_rn_ok(rj, key)) {
+            const float yr = lps_div::rcp_rn(rj);
+            for (int t = 0; t < NQ; t++) n[t] = lps_div::div_rn(n[t], rj, yr);
+        } else {
+            for (int t = 0; t < NQ; t++) n[t] = n[t] / rj;
+        }
+    }
+}
+
+// Writes what the force pass takes from the density pass beside (x, rho): the
+// reciprocal of rho in the spare word of the velocity, or a flag that the
+// quotients need their checks.
+__device__ __forceinline__ void store_rho_rcp(DevGrid* g, float4* __restrict__ vel, uint32_t i, float rho) {
+    if (rho >= 0x1p-78f && rho < 0x1p40f)
+        vel[i].w = lps_div::rcp_rn(rho);
+    else
+        g->odd_state = 1u;
 }
 
 }  // namespace
@@ -967,6 +1053,7 @@ __device__ __forceinline__ void grid_finish_block(DevGrid* g, const lps_dev::Sce
     g->final_err = 0u;
     g->converged = 0u;
     g->tiny_pred = 0u;
+    g->odd_state = 0u;
     g->act_count[0] = S.nblocks;
     g->act_count[1] = 0u;
     g->list_of[1] = 0u;
@@ -1139,13 +1226,13 @@ __global__ __launch_bounds__(LPS_BLOCK) void k_place(const uint32_t* __restrict_
 // cell, so a wave's writes stay together.  On a failed step the copy is the identity so the state survives
 // the buffer flip.
 __global__ __launch_bounds__(LPS_BLOCK) void k_reorder(
-    const uint2* __restrict__ placed, const uint32_t* __restrict__ cell_lb, const DevGrid* g,
+    const uint2* __restrict__ placed, const uint32_t* __restrict__ cell_lb, DevGrid* g,
     const float4* __restrict__ pos_in, const float4* __restrict__ vel_in, const float4* __restrict__ vh_in,
     const uint8_t* __restrict__ first_in, const uint32_t* __restrict__ id_in, const float* __restrict__ pprev_in,
     float4* __restrict__ pos_out, float4* __restrict__ vel_out, float4* __restrict__ vh_out,
     uint8_t* __restrict__ first_out, uint32_t* __restrict__ id_out, float* __restrict__ pprev_out,
     uint32_t* __restrict__ skeys_out, uint32_t* __restrict__ perm_out, lps_dev::Scenes S, uint2* __restrict__ cq,
-    uint32_t nlogical) {
+    uint32_t tiny_key, uint32_t nlogical) {
     const uint32_t lb = xcd_block(nlogical);
     if (lb == UINT_MAX) return;
     const uint32_t s = lb * LPS_BLOCK + threadIdx.x;
@@ -1185,6 +1272,10 @@ __global__ __launch_bounds__(LPS_BLOCK) void k_reorder(
         cq[d] = quantize(p.x, p.y, p.z, G, compact_scale(G));
         skeys_out[d] = key;
         perm_out[d] = i;
+        // the shared-reciprocal quotients of the force passes need checks then
+        const uint32_t least = min(min(min(lps_div::num_key(p.x), lps_div::num_key(p.y)), lps_div::num_key(p.z)),
+                                   min(min(lps_div::num_key(v.x), lps_div::num_key(v.y)), lps_div::num_key(v.z)));
+        if (least < tiny_key) g->odd_state = 1u;
     }
     pos_out[d] = p;
     vel_out[d] = v;
@@ -1198,7 +1289,7 @@ __global__ __launch_bounds__(LPS_BLOCK) void k_reorder(
 // calcDensityPressure (SPHKernels.cl:190-254).  Writes (x, rho) packed for the
 // force pass, the pressure, and q = p / rho^2 (the per-particle term of the
 // SPH pressure force, SPHKernels.cl:383,412).
-__global__ __launch_bounds__(LPS_BLOCK) void k_density(const float4* __restrict__ pos, const DevGrid* g,
+__global__ __launch_bounds__(LPS_BLOCK) void k_density(const float4* __restrict__ pos, DevGrid* g, float4* __restrict__ vel,
                                                        lps_dev::Scenes S, const uint32_t* __restrict__ cell_lb,
                                                        SimConst c, const float* __restrict__ tables,
                                                        float4* __restrict__ posrho, float* __restrict__ press,
@@ -1233,6 +1324,7 @@ __global__ __launch_bounds__(LPS_BLOCK) void k_density(const float4* __restrict_
     float p = c.stiffness * (rho - c.rest_density);
     if (p < 0.f) p *= c.npf;
     posrho[i] = make_float4(xi.x, xi.y, xi.z, rho);
+    store_rho_rcp(g, vel, i, rho);
     press[i] = p;
     q[i] = p / (rho * rho);
 }
@@ -1272,32 +1364,24 @@ __global__ __launch_bounds__(LPS_BLOCK) __attribute__((amdgpu_waves_per_eu(FEAT 
     float snx = 0.f, sny = 0.f, snz = 0.f, lc = 0.f, vfx = 0.f, vfy = 0.f, vfz = 0.f;
     float nb = 0.f, dv = 0.f;  // warm-start features: neighbour count, velocity divergence
     // the density pass recorded this stencil's masks at the same positions
-    for_neighbors_planes<2>(G, cell_lb, xi.x, xi.y, xi.z, posrho, xi.x, xi.y, xi.z, c.s_max, c.s_relax, mk, i,
-                         [](uint32_t) { return true; }, [&](uint32_t j) { return vel[j]; },
-                         [&](uint32_t j, const float4& xj, float s2, const float4& vj, const float3&) {
-        const uint32_t idx = table_index(s2, sT, c.inv_div);
-        const float rj = xj.w;
-        const float w1 = sW1[idx], wv = sV2[idx];
-        // the numerators of every quotient by rho_j (the self pair's velocity
-        // terms are zero and unused)
-        float n[8] = {(xi.x - xj.x) * w1, (xi.y - xj.y) * w1, (xi.z - xj.z) * w1, sW2[idx],
-                      (vj.x - vi.x) * wv, (vj.y - vi.y) * wv, (vj.z - vi.z) * wv, 0.f};
-        constexpr int NQ = FEAT ? 8 : 7;
-        if constexpr (FEAT)
-            n[7] = ((vj.x - vi.x) * (xi.x - xj.x) + (vj.y - vi.y) * (xi.y - xj.y) + (vj.z - vi.z) * (xi.z - xj.z)) * w1;
-        uint32_t key = lps_div::num_key(n[0]);
-        for (int t = 1; t < NQ; t++) key = min(key, lps_div::num_key(n[t]));
-        if (rj < 0x1p40f && lps_div::div_rn_ok(rj, key)) {
-            const float y = lps_div::rcp_rn(rj);
-            for (int t = 0; t < NQ; t++) n[t] = lps_div::div_rn(n[t], rj, y);
-        } else {
-            for (int t = 0; t < NQ; t++) n[t] = n[t] / rj;
-        }
-        snx += n[0];
-        sny += n[1];
-        snz += n[2];
-        lc += n[3];
-        if (i != j) {
+    auto walk = [&](auto quick) {
+        for_neighbors_planes<2, true>(G, cell_lb, xi.x, xi.y, xi.z, posrho, xi.x, xi.y, xi.z, c.s_max, c.s_relax, mk, i,
+                                      [&](uint32_t j) { return vel[j]; },
+                                      [&](uint32_t, const float4& xj, float s2, const float4& vj, const float3& dl) {
+            const uint32_t idx = table_index(s2, sT, c.inv_div);
+            const float w1 = sW1[idx], wv = sV2[idx];
+            // the numerators of every quotient by rho_j; x_i - x_j = -dl but
+            // for the sign of a zero, which the sums cannot tell (they start
+            // at +0), and the self pair's velocity terms are +0
+            const float dvx = vj.x - vi.x, dvy = vj.y - vi.y, dvz = vj.z - vi.z;
+            float n[8] = {-dl.x * w1, -dl.y * w1, -dl.z * w1, sW2[idx], dvx * wv, dvy * wv, dvz * wv, 0.f};
+            constexpr int NQ = FEAT ? 8 : 7;
+            if constexpr (FEAT) n[7] = (dvx * -dl.x + dvy * -dl.y + dvz * -dl.z) * w1;
+            force_quotients<decltype(quick)::value, NQ>(n, xj.w, vj.w);
+            snx += n[0];
+            sny += n[1];
+            snz += n[2];
+            lc += n[3];
             vfx += n[4];
             vfy += n[5];
             vfz += n[6];
@@ -1305,8 +1389,13 @@ __global__ __launch_bounds__(LPS_BLOCK) __attribute__((amdgpu_waves_per_eu(FEAT 
                 nb += 1.f;
                 dv += n[7];
             }
-        }
-    });
+        });
+    };
+    if (c.quick_forces && g->odd_state == 0u)
+        walk(std::true_type{});
+    else
+        walk(std::false_type{});
+    nb -= 1.f;  // the particle itself
     snx *= c.mass; sny *= c.mass; snz *= c.mass;
     const float snl = sqrtf(snx * snx + sny * sny + snz * snz);
     if constexpr (FEAT) {
@@ -1368,23 +1457,23 @@ __global__ __launch_bounds__(LPS_BLOCK) void k_pressure_sph(const float4* __rest
     const float4 xi = posrho[i];
     const float tf = q[i];
     const bool fastdiv = c.s_max < 0x1p78f;  // accepted pairs have d < 2^40
+    const bool quick = fastdiv && g->odd_state == 0u && index_q_ok(c.div);
     float pfx = 0.f, pfy = 0.f, pfz = 0.f;
-    auto pressure = [&](auto qidx) {
-        for_neighbors_planes<2>(G, cell_lb, xi.x, xi.y, xi.z, posrho, xi.x, xi.y, xi.z, c.s_max, c.s_relax, mk, i,
-                             [&](uint32_t j) { return i != j; }, [&](uint32_t j) { return q[j]; },
-                             [&](uint32_t j, const float4&, float s2, float qj, const float3& dl) {
-            const float d = sqrt_rn(s2);
+    auto pressure = [&](auto nocheck) {
+        for_neighbors_planes<2, false>(G, cell_lb, xi.x, xi.y, xi.z, posrho, xi.x, xi.y, xi.z, c.s_max, c.s_relax, mk,
+                                       i, [&](uint32_t j) { return q[j]; },
+                                       [&](uint32_t j, const float4&, float s2, float qj, const float3& dl) {
             float ux, uy, uz;
-            pair_dir<false>(dl, d, i, j, fastdiv, ux, uy, uz);
-            const float w = sP1[decltype(qidx)::value ? table_index_q(d, c.div, c.inv_div)
-                                                      : table_index_d(s2, d, sT, c.inv_div)];
+            const float d = pair_geometry<decltype(nocheck)::value>(dl, s2, i, j, fastdiv, ux, uy, uz);
+            const float w = sP1[decltype(nocheck)::value ? table_index_q(d, c.div, c.inv_div)
+                                                         : table_index_d(s2, d, sT, c.inv_div)];
             const float sc = tf + qj;
             pfx += ux * sc * w;
             pfy += uy * sc * w;
             pfz += uz * sc * w;
         });
     };
-    if (index_q_ok(c.div))
+    if (quick)
         pressure(std::true_type{});
     else
         pressure(std::false_type{});
@@ -1572,7 +1661,7 @@ __device__ __forceinline__ uint32_t quad_particle(uint32_t lb) {
 }
 
 // k_density with a quad per particle.
-__global__ __launch_bounds__(LPS_BLOCK) void k_density_q(const float4* __restrict__ pos, const DevGrid* g,
+__global__ __launch_bounds__(LPS_BLOCK) void k_density_q(const float4* __restrict__ pos, DevGrid* g, float4* __restrict__ vel,
                                                          lps_dev::Scenes S, const uint32_t* __restrict__ cell_lb,
                                                          SimConst c, const float* __restrict__ tables,
                                                          float4* __restrict__ posrho, float* __restrict__ press,
@@ -1607,6 +1696,7 @@ __global__ __launch_bounds__(LPS_BLOCK) void k_density_q(const float4* __restric
     float p = c.stiffness * (rho - c.rest_density);
     if (p < 0.f) p *= c.npf;
     posrho[i] = make_float4(xi.x, xi.y, xi.z, rho);
+    store_rho_rcp(g, vel, i, rho);
     press[i] = p;
     q[i] = p / (rho * rho);
 }
@@ -1634,6 +1724,7 @@ __global__ __launch_bounds__(LPS_BLOCK) void k_forces_q(
     if (i >= B.info.slot0 + B.info.count) return;
     const GridView G = grid_view(g, S.grid + B.s);
     const SimConst c = scene_const(c0, B.info);
+    const bool quick = c.quick_forces && g->odd_state == 0u;
     const float ri = xi.w;
     // snx, sny, snz, lc, vfx, vfy, vfz, then (features) nb, dv
     constexpr int NT = FEAT ? 9 : 7;
@@ -1643,7 +1734,7 @@ __global__ __launch_bounds__(LPS_BLOCK) void k_forces_q(
     for_neighbors_quad<NT>(G, cell_lb, xi.x, xi.y, xi.z, posrho, xi.x, xi.y, xi.z, c.s_max, c.s_relax, mk, i,
                            MC_REPLAY, CompactFilter{}, [](uint32_t) { return true; },
                            [&](uint32_t j) { return vel[j]; },
-                           [&](bool ok, uint32_t j, const float4& xj, float s2, const float4& vj, const float3&,
+                           [&](bool ok, uint32_t j, const float4& xj, float s2, const float4& vj, const float3& dl,
                                float (&t)[NT]) {
         if (!ok) {
 #pragma unroll
@@ -1651,21 +1742,15 @@ __global__ __launch_bounds__(LPS_BLOCK) void k_forces_q(
             return;
         }
         const uint32_t idx = table_index(s2, sT, c.inv_div);
-        const float rj = xj.w;
         const float w1 = sW1[idx], wv = sV2[idx];
-        float n[8] = {(xi.x - xj.x) * w1, (xi.y - xj.y) * w1, (xi.z - xj.z) * w1, sW2[idx],
-                      (vj.x - vi.x) * wv, (vj.y - vi.y) * wv, (vj.z - vi.z) * wv, 0.f};
+        const float dvx = vj.x - vi.x, dvy = vj.y - vi.y, dvz = vj.z - vi.z;
+        float n[8] = {-dl.x * w1, -dl.y * w1, -dl.z * w1, sW2[idx], dvx * wv, dvy * wv, dvz * wv, 0.f};
         constexpr int NQ = FEAT ? 8 : 7;
-        if constexpr (FEAT)
-            n[7] = ((vj.x - vi.x) * (xi.x - xj.x) + (vj.y - vi.y) * (xi.y - xj.y) + (vj.z - vi.z) * (xi.z - xj.z)) * w1;
-        uint32_t key = lps_div::num_key(n[0]);
-        for (int a = 1; a < NQ; a++) key = min(key, lps_div::num_key(n[a]));
-        if (rj < 0x1p40f && lps_div::div_rn_ok(rj, key)) {
-            const float y = lps_div::rcp_rn(rj);
-            for (int a = 0; a < NQ; a++) n[a] = lps_div::div_rn(n[a], rj, y);
-        } else {
-            for (int a = 0; a < NQ; a++) n[a] = n[a] / rj;
-        }
+        if constexpr (FEAT) n[7] = (dvx * -dl.x + dvy * -dl.y + dvz * -dl.z) * w1;
+        if (quick)
+            force_quotients<true, NQ>(n, xj.w, vj.w);
+        else
+            force_quotients<false, NQ>(n, xj.w, vj.w);
         const bool other = i != j;
         t[0] = n[0];
         t[1] = n[1];
@@ -1744,6 +1829,7 @@ __global__ __launch_bounds__(LPS_BLOCK) void k_pressure_sph_q(const float4* __re
     if (i >= B.info.slot0 + B.info.count) return;
     const GridView G = grid_view(g, S.grid + B.s);
     const bool fastdiv = c.s_max < 0x1p78f;  // accepted pairs have d < 2^40
+    const bool nocheck = fastdiv && g->odd_state == 0u;
     const bool qidx = index_q_ok(c.div);
     float acc[3] = {0.f, 0.f, 0.f};
     for_neighbors_quad<3>(G, cell_lb, xi.x, xi.y, xi.z, posrho, xi.x, xi.y, xi.z, c.s_max, c.s_relax, mk, i,
@@ -1754,9 +1840,9 @@ __global__ __launch_bounds__(LPS_BLOCK) void k_pressure_sph_q(const float4* __re
             t[0] = t[1] = t[2] = 0.f;
             return;
         }
-        const float d = sqrt_rn(s2);
         float ux, uy, uz;
-        pair_dir<false>(dl, d, i, j, fastdiv, ux, uy, uz);
+        const float d = nocheck ? pair_geometry<true>(dl, s2, i, j, fastdiv, ux, uy, uz)
+                                : pair_geometry<false>(dl, s2, i, j, fastdiv, ux, uy, uz);
         const float w = sP1[qidx ? table_index_q(d, c.div, c.inv_div) : table_index_d(s2, d, sT, c.inv_div)];
         const float sc = tf + qj;
         t[0] = ux * sc * w;
@@ -2056,13 +2142,12 @@ __global__ __launch_bounds__(WG) __attribute__((amdgpu_waves_per_eu(WG >= 128 ? 
     float pfx = 0.f, pfy = 0.f, pfz = 0.f;
     auto pressure = [&](auto nocheck) {
         // the predicted-density pass of this correction recorded the masks
-        for_neighbors_planes<2>(G, cell_lb, xa.x, xa.y, xa.z, xq, xi.x, xi.y, xi.z, c.s_max, c.s_relax, mk, i,
-                             [&](uint32_t j) { return i != j; }, [](uint32_t) { return 0; },
-                             [&](uint32_t j, const float4& xqj, float s2, int, const float3& dl) {
+        for_neighbors_planes<2, false>(G, cell_lb, xa.x, xa.y, xa.z, xq, xi.x, xi.y, xi.z, c.s_max, c.s_relax, mk, i,
+                                       [](uint32_t) { return 0; },
+                                       [&](uint32_t j, const float4& xqj, float s2, int, const float3& dl) {
             const float qj = xqj.w;
-            const float d = sqrt_rn(s2);
             float ux, uy, uz;
-            pair_dir<decltype(nocheck)::value>(dl, d, i, j, fastdiv, ux, uy, uz);
+            const float d = pair_geometry<decltype(nocheck)::value>(dl, s2, i, j, fastdiv, ux, uy, uz);
             const float w = sP1[decltype(nocheck)::value ? table_index_q(d, c.div, c.inv_div)
                                                          : table_index_d(s2, d, sT, c.inv_div)];
             const float sc = tf + qj;
@@ -2205,12 +2290,9 @@ __global__ __launch_bounds__(LPS_BLOCK) void k_pci_pressure_q(
             t[0] = t[1] = t[2] = 0.f;
             return;
         }
-        const float d = sqrt_rn(s2);
         float ux, uy, uz;
-        if (nocheck)
-            pair_dir<true>(dl, d, i, j, fastdiv, ux, uy, uz);
-        else
-            pair_dir<false>(dl, d, i, j, fastdiv, ux, uy, uz);
+        const float d = nocheck ? pair_geometry<true>(dl, s2, i, j, fastdiv, ux, uy, uz)
+                                : pair_geometry<false>(dl, s2, i, j, fastdiv, ux, uy, uz);
         const float w = sP1[nocheck && qidx ? table_index_q(d, c.div, c.inv_div) : table_index_d(s2, d, sT, c.inv_div)];
         const float sc = tf + xqj.w;
         t[0] = ux * sc * w;
@@ -2528,7 +2610,7 @@ __device__ __forceinline__ uint32_t team_particle(uint32_t lb) {
 }
 
 // k_density with a team per particle.
-__global__ __launch_bounds__(LPS_BLOCK) void k_density_t(const float4* __restrict__ pos, const DevGrid* g,
+__global__ __launch_bounds__(LPS_BLOCK) void k_density_t(const float4* __restrict__ pos, DevGrid* g, float4* __restrict__ vel,
                                                          lps_dev::Scenes S, const uint32_t* __restrict__ cell_lb,
                                                          SimConst c, const float* __restrict__ tables,
                                                          float4* __restrict__ posrho, float* __restrict__ press,
@@ -2556,6 +2638,7 @@ __global__ __launch_bounds__(LPS_BLOCK) void k_density_t(const float4* __restric
     float p = c.stiffness * (rho - c.rest_density);
     if (p < 0.f) p *= c.npf;
     posrho[i] = make_float4(xi.x, xi.y, xi.z, rho);
+    store_rho_rcp(g, vel, i, rho);
     press[i] = p;
     q[i] = p / (rho * rho);
 }
@@ -2596,6 +2679,7 @@ __global__ __launch_bounds__(LPS_BLOCK) void k_forces_t(
     const SimConst c = scene_const(c0, B.info);
     const bool valid = i < B.info.slot0 + B.info.count;
     const bool qidx = index_q_ok(c.div);
+    const bool quick = c.quick_forces && g->odd_state == 0u;
     const float ri = xi.w;
     // snx, sny, snz, lc, vfx, vfy, vfz, then (features) nb, dv
     constexpr int NT = FEAT ? 9 : 7;
@@ -2605,7 +2689,7 @@ __global__ __launch_bounds__(LPS_BLOCK) void k_forces_t(
     team_replay<NT>(L, valid ? listed : 0u, nb0, [&]() { return team_rows(G, cell_lb, xi.x, xi.y, xi.z, valid); },
                     posrho, i, xi.x, xi.y, xi.z, c, s_list[threadIdx.x / LPS_TEAM], s_t[threadIdx.x / LPS_TEAM],
                     [&](uint32_t j) { return vel[j]; },
-                    [&](bool ok, uint32_t j, const float4& xj, float s2, const float4& vj, const float3&,
+                    [&](bool ok, uint32_t j, const float4& xj, float s2, const float4& vj, const float3& dl,
                                float (&t)[NT]) {
         if (!ok) {
 #pragma unroll
@@ -2613,21 +2697,15 @@ __global__ __launch_bounds__(LPS_BLOCK) void k_forces_t(
             return;
         }
         const uint32_t idx = team_index(s2, qidx, c.div, c.inv_div);
-        const float rj = xj.w;
         const float w1 = sW1[idx], wv = sV2[idx];
-        float n[8] = {(xi.x - xj.x) * w1, (xi.y - xj.y) * w1, (xi.z - xj.z) * w1, sW2[idx],
-                      (vj.x - vi.x) * wv, (vj.y - vi.y) * wv, (vj.z - vi.z) * wv, 0.f};
+        const float dvx = vj.x - vi.x, dvy = vj.y - vi.y, dvz = vj.z - vi.z;
+        float n[8] = {-dl.x * w1, -dl.y * w1, -dl.z * w1, sW2[idx], dvx * wv, dvy * wv, dvz * wv, 0.f};
         constexpr int NQ = FEAT ? 8 : 7;
-        if constexpr (FEAT)
-            n[7] = ((vj.x - vi.x) * (xi.x - xj.x) + (vj.y - vi.y) * (xi.y - xj.y) + (vj.z - vi.z) * (xi.z - xj.z)) * w1;
-        uint32_t key = lps_div::num_key(n[0]);
-        for (int a = 1; a < NQ; a++) key = min(key, lps_div::num_key(n[a]));
-        if (rj < 0x1p40f && lps_div::div_rn_ok(rj, key)) {
-            const float y = lps_div::rcp_rn(rj);
-            for (int a = 0; a < NQ; a++) n[a] = lps_div::div_rn(n[a], rj, y);
-        } else {
-            for (int a = 0; a < NQ; a++) n[a] = n[a] / rj;
-        }
+        if constexpr (FEAT) n[7] = (dvx * -dl.x + dvy * -dl.y + dvz * -dl.z) * w1;
+        if (quick)
+            force_quotients<true, NQ>(n, xj.w, vj.w);
+        else
+            force_quotients<false, NQ>(n, xj.w, vj.w);
         const bool other = i != j;
         t[0] = n[0];
         t[1] = n[1];
@@ -2712,6 +2790,7 @@ __global__ __launch_bounds__(LPS_BLOCK) void k_pressure_sph_t(const float4* __re
     const bool valid = i < B.info.slot0 + B.info.count;
     const GridView G = grid_view(g, S.grid + B.s);
     const bool fastdiv = c.s_max < 0x1p78f;  // accepted pairs have d < 2^40
+    const bool nocheck = fastdiv && g->odd_state == 0u;
     const bool qidx = index_q_ok(c.div);
     __shared__ uint32_t s_list[LPS_BLOCK / LPS_TEAM][LPS_PENDING];
     TeamSum<3> sum;
@@ -2723,9 +2802,9 @@ __global__ __launch_bounds__(LPS_BLOCK) void k_pressure_sph_t(const float4* __re
             t[0] = t[1] = t[2] = 0.f;
             return;
         }
-        const float d = sqrt_rn(s2);
         float ux, uy, uz;
-        pair_dir<false>(dl, d, i, j, fastdiv, ux, uy, uz);
+        const float d = nocheck ? pair_geometry<true>(dl, s2, i, j, fastdiv, ux, uy, uz)
+                                : pair_geometry<false>(dl, s2, i, j, fastdiv, ux, uy, uz);
         const float w = sP1[qidx ? table_index_q(d, c.div, c.inv_div) : min((uint32_t)(d / c.div), (uint32_t)(LPS_TABLE_SIZE - 1))];
         const float sc = tf + qj;
         t[0] = ux * sc * w;
@@ -2866,12 +2945,9 @@ __global__ __launch_bounds__(LPS_BLOCK) void k_pci_pressure_t(
             t[0] = t[1] = t[2] = 0.f;
             return;
         }
-        const float d = sqrt_rn(s2);
         float ux, uy, uz;
-        if (nocheck)
-            pair_dir<true>(dl, d, i, j, fastdiv, ux, uy, uz);
-        else
-            pair_dir<false>(dl, d, i, j, fastdiv, ux, uy, uz);
+        const float d = nocheck ? pair_geometry<true>(dl, s2, i, j, fastdiv, ux, uy, uz)
+                                : pair_geometry<false>(dl, s2, i, j, fastdiv, ux, uy, uz);
         const float w = sP1[qidx ? table_index_q(d, c.div, c.inv_div) : min((uint32_t)(d / c.div), (uint32_t)(LPS_TABLE_SIZE - 1))];
         const float sc = tf + xqj.w;
         t[0] = ux * sc * w;
@@ -3030,24 +3106,24 @@ void launch_reorder(hipStream_t s, const ReorderArgs& a) {
     k_reorder<<<xcd_grid(nl), LPS_BLOCK, 0, s>>>(a.placed, a.cell_lb, a.g, a.pos_in, a.vel_in, a.vh_in,
                                                  a.first_in, a.id_in, a.pprev_in, a.pos_out, a.vel_out, a.vh_out,
                                                  a.first_out, a.id_out, a.pprev_out, a.skeys, a.perm, a.sc, a.cq,
-                                                 nl);
+                                                 a.tiny_key, nl);
 }
 
 void launch_density(hipStream_t s, const PhysArgs& a, float* press, float* q) {
     const uint32_t nl = cdiv(a.c.n, LPS_BLOCK);
     if (a.lanes == LPS_TEAM) {
         const uint32_t nt = nl * LPS_TEAM;
-        k_density_t<<<xcd_grid(nt), LPS_BLOCK, 0, s>>>(a.pos, a.g, a.sc, a.cell_lb, a.c, a.tables, a.posrho, press, q,
+        k_density_t<<<xcd_grid(nt), LPS_BLOCK, 0, s>>>(a.pos, a.g, a.vel, a.sc, a.cell_lb, a.c, a.tables, a.posrho, press, q,
                                                       a.nl, nt);
         return;
     }
     if (a.lanes == LPS_QUAD) {
         const uint32_t nq = nl * LPS_QUAD;
-        k_density_q<<<xcd_grid(nq), LPS_BLOCK, 0, s>>>(a.pos, a.g, a.sc, a.cell_lb, a.c, a.tables, a.posrho, press, q,
+        k_density_q<<<xcd_grid(nq), LPS_BLOCK, 0, s>>>(a.pos, a.g, a.vel, a.sc, a.cell_lb, a.c, a.tables, a.posrho, press, q,
                                                       a.mk, nq);
         return;
     }
-    k_density<<<xcd_grid(nl), LPS_BLOCK, 0, s>>>(a.pos, a.g, a.sc, a.cell_lb, a.c, a.tables, a.posrho, press, q, a.mk,
+    k_density<<<xcd_grid(nl), LPS_BLOCK, 0, s>>>(a.pos, a.g, a.vel, a.sc, a.cell_lb, a.c, a.tables, a.posrho, press, q, a.mk,
                                                 nl);
 }
 

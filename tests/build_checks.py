@@ -10,7 +10,8 @@ ROOT = os.path.dirname(HERE)
 BIN = os.path.join(HERE, "_bin")
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 
-CHECKS = {"div_rn_check": "div_rn_check.hip", "bf16_check": "bf16_check.hip"}
+CHECKS = {"div_rn_check": "div_rn_check.hip", "bf16_check": "bf16_check.hip",
+          "rsq_rn_check": "rsq_rn_check.hip"}
 # host programs over the libraries: the C++ layer (include/lps_solver.hpp) against the oracle
 HOST_CHECKS = {"cpp_solver_check": "cpp_solver_check.cpp"}
 
