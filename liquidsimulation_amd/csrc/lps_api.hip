@@ -163,7 +163,7 @@ struct lps_ctx {
     SceneInfo* d_sinfo = nullptr;
     SceneGrid* d_sgrid = nullptr;
     SceneGrid* h_sgrid = nullptr;          // pinned copy for per-scene statistics
-    uint8_t* d_bscene = nullptr;           // scene of every particle block
+    uint32_t* d_bscene = nullptr;          // scene of every particle block
     uint32_t* d_err = nullptr;             // sub-maxima of the corrections' errors per scene
     uint32_t* d_actlist = nullptr;         // [2][blocks] active-block lists of the correction kernels
 
@@ -1116,7 +1116,7 @@ int lps_set_scenes(lps_ctx* c, uint32_t nscenes, const uint32_t* counts, const f
     if ((st = up4(c->vh[0], vhalf))) return st;
     std::vector<uint8_t> f(n, 1);
     std::vector<uint32_t> ids(n, 0xFFFFFFFFu);
-    std::vector<uint8_t> bscene(n / LPS_BLOCK);
+    std::vector<uint32_t> bscene(n / LPS_BLOCK);
     {
         uint32_t r = 0;
         for (uint32_t k = 0; k < nscenes; k++) {
@@ -1125,12 +1125,12 @@ int lps_set_scenes(lps_ctx* c, uint32_t nscenes, const uint32_t* counts, const f
                 ids[si.slot0 + i] = r;
                 if (first) f[si.slot0 + i] = first[r] ? 1 : 0;
             }
-            for (uint32_t b = 0; b < si.padded / LPS_BLOCK; b++) bscene[si.block0 + b] = (uint8_t)k;
+            for (uint32_t b = 0; b < si.padded / LPS_BLOCK; b++) bscene[si.block0 + b] = k;
         }
     }
     HIPC(hipMemcpy(c->first[0], f.data(), n, hipMemcpyHostToDevice));
     HIPC(hipMemcpy(c->id[0], ids.data(), sizeof(uint32_t) * n, hipMemcpyHostToDevice));
-    HIPC(hipMemcpy(c->d_bscene, bscene.data(), n / LPS_BLOCK, hipMemcpyHostToDevice));
+    HIPC(hipMemcpy(c->d_bscene, bscene.data(), sizeof(uint32_t) * (n / LPS_BLOCK), hipMemcpyHostToDevice));
     HIPC(hipMemset(c->pprev[0], 0, sizeof(float) * n));
     HIPC(hipMemset(c->d_sgrid, 0, sizeof(SceneGrid) * nscenes));
     c->n = n;
@@ -1230,7 +1230,7 @@ int lps_add_particles(lps_ctx* c, const float* x, const float* v, const float* v
     if (nslots != c->n) {
         if ((st = dalloc(&c->d_bscene, nslots / LPS_BLOCK))) return st;
         if ((st = dalloc(&c->d_actlist, 2 * (size_t)(nslots / LPS_BLOCK)))) return st;
-        HIPC(hipMemset(c->d_bscene, 0, nslots / LPS_BLOCK));
+        HIPC(hipMemset(c->d_bscene, 0, sizeof(uint32_t) * (nslots / LPS_BLOCK)));
     }
     c->n = nslots;
     c->n_real = (uint32_t)total;

@@ -17,7 +17,7 @@ namespace lps_dev {
 struct Scenes {
     const SceneInfo* info;
     SceneGrid* grid;
-    const uint8_t* block_scene;
+    const uint32_t* block_scene;
     uint32_t count;
     uint32_t nblocks;        // particle blocks (slots / LPS_BLOCK)
     uint32_t* act_list;      // [2][nblocks] active-block lists of the correction kernels
