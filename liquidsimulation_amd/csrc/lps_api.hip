@@ -63,6 +63,13 @@ unsigned char* scratch_ptr(int device) {
     return g_scratch_status[device] == 1 ? static_cast<unsigned char*>(g_scratch_ptr[device]) : nullptr;
 }
 
+// Uploads and readbacks of at most this many bytes go through the context's
+// pinned buffer as one asynchronous copy; larger ones are copied from and to
+// the caller's memory directly (the runtime's own staging is then as fast).
+constexpr size_t LPS_STAGE_BYTES = 1u << 20;
+constexpr size_t LPS_SCENES_BYTES =
+    LPS_MAX_SCENES * sizeof(SceneInfo) + LPS_MAX_COLLIDERS * (sizeof(lps_box) + sizeof(lps_sphere) + sizeof(lps_plane));
+
 struct ProfRec {
     const char* name;
     hipEvent_t a, b;
@@ -167,9 +174,16 @@ struct lps_ctx {
     uint32_t* d_err = nullptr;             // sub-maxima of the corrections' errors per scene
     uint32_t* d_actlist = nullptr;         // [2][blocks] active-block lists of the correction kernels
 
-    // host
-    uint32_t* flags = nullptr;  // pinned, coherent: LPS_FLAG_WORDS words per iteration slot
-    DevGrid* h_grid = nullptr;  // pinned copy
+    // host (the pointers into h_block, one pinned, coherent allocation)
+    uint8_t* h_block = nullptr;
+    uint32_t* flags = nullptr;  // LPS_FLAG_WORDS words per iteration slot
+    DevGrid* h_grid = nullptr;  // copy
+    StepReport* report = nullptr;  // coherent: outcome of the last step enqueued, valid once the stream has drained
+    uint8_t* h_scenes = nullptr;   // LPS_SCENES_BYTES: scene constants and colliders on their way to the device
+    uint8_t* h_stage = nullptr;    // LPS_STAGE_BYTES: small uploads and readbacks
+    uint32_t* h_part = nullptr;    // pinned copy of the per-block records of an upload
+    size_t h_part_cap = 0;
+    uint32_t cap_scenes = 0, cap_blocks = 0;  // allocated entries of the scene and block arrays
     // coherent: per scene kinetic and potential energy of the state entering
     // the last step (written by its grid set-up) or of the current state
     // (lps_get_energy); the warm start's fallback compares consecutive steps
@@ -356,16 +370,18 @@ int upload_tables(lps_ctx* c) {
 
 // Cell-count bound of one scene: particles end every step inside each
 // BOUNDARY box shrunk by the particle radius, so that box bounds the grid; the
-// first step's grid comes from the initial positions.
-uint64_t scene_cell_bound(const lps_ctx* c, const float* x, uint32_t n, const std::vector<lps_box>& boxes) {
+// first step's grid comes from the initial positions, whose bounds (over the
+// finite coordinates) are in the records of the scene's particle blocks.
+uint64_t scene_cell_bound(const lps_ctx* c, const SceneInfo& si, const std::vector<lps_box>& boxes) {
     const float h = c->der.h;
     uint64_t init = 1, bound = 0;
     float mn[3] = {INFINITY, INFINITY, INFINITY}, mx[3] = {-INFINITY, -INFINITY, -INFINITY};
-    for (uint32_t i = 0; i < n; i++)
+    for (uint32_t b = si.block0; b < si.block0 + si.padded / LPS_BLOCK; b++)
         for (int a = 0; a < 3; a++) {
-            if (!std::isfinite(x[3 * i + a])) continue;
-            mn[a] = std::min(mn[a], x[3 * i + a]);
-            mx[a] = std::max(mx[a], x[3 * i + a]);
+            const uint32_t *q = c->h_part + (size_t)LPS_BBOX_PART * b, lo = q[a], hi = q[3 + a];
+            if (lo > hi) continue;  // no finite coordinate in this block
+            mn[a] = std::min(mn[a], o2f(lo));
+            mx[a] = std::max(mx[a], o2f(hi));
         }
     for (int a = 0; a < 3; a++) {
         const double ex = mx[a] >= mn[a] ? ((double)mx[a] - (double)mn[a]) / (double)h : 0.0;
@@ -452,12 +468,10 @@ void free_all(lps_ctx* c) {
     dfree(c->d_sinfo); dfree(c->d_sgrid); dfree(c->d_bscene); dfree(c->d_actlist); dfree(c->d_err);
     if (c->h_sgrid) (void)hipHostFree(c->h_sgrid);
     c->h_sgrid = nullptr;
-    if (c->flags) (void)hipHostFree(c->flags);
-    if (c->h_grid) (void)hipHostFree(c->h_grid);
-    if (c->h_energy) (void)hipHostFree(c->h_energy);
-    c->flags = nullptr;
-    c->h_grid = nullptr;
-    c->h_energy = nullptr;
+    if (c->h_part) (void)hipHostFree(c->h_part);
+    c->h_part = nullptr;
+    if (c->h_block) (void)hipHostFree(c->h_block);
+    c->h_block = nullptr;
 }
 
 lps_dev::Scenes scenes(const lps_ctx* c) {
@@ -756,7 +770,7 @@ StepResult enqueue_step(lps_ctx* c, float dt, bool seeded, bool feat_on) {
         }
         {
             Timed t(c, "integrate");
-            lps_dev::launch_integrate(s, a, nullptr, c->pprev[c->cur], c->press, c->bbox_part);
+            lps_dev::launch_integrate(s, a, nullptr, c->pprev[c->cur], c->press, c->bbox_part, c->report);
         }
         c->last_fp_valid = 0;
         c->feat_valid = c->seed_valid = false;
@@ -801,7 +815,7 @@ StepResult enqueue_step(lps_ctx* c, float dt, bool seeded, bool feat_on) {
     }
     {
         Timed t(c, "integrate");
-        lps_dev::launch_integrate(s, a, c->fp, c->pprev[c->cur], c->press, c->bbox_part);
+        lps_dev::launch_integrate(s, a, c->fp, c->pprev[c->cur], c->press, c->bbox_part, c->report);
     }
     if (feat_on && res.ok && c->coll_stride > 0 && c->coll_rows < c->coll_cap) {
         // training rows: every stride-th particle's features and the
@@ -825,43 +839,105 @@ StepResult enqueue_step(lps_ctx* c, float dt, bool seeded, bool feat_on) {
 }
 
 // Concatenate the scenes' colliders into the device arrays and upload the
-// scene constants (collider ranges, gravity).
+// scene constants (collider ranges, gravity), through the pinned copy: the
+// stream is drained before that is written, and the copies are left to run.
 int upload_scenes(lps_ctx* c) {
     const size_t S = c->h_sinfo.size();
-    std::vector<lps_box> boxes;
-    std::vector<lps_sphere> spheres;
-    std::vector<lps_plane> planes;
+    size_t nbox = 0, nsphere = 0, nplane = 0;
+    for (size_t k = 0; k < S; k++) {
+        nbox += c->s_boxes[k].size();
+        nsphere += c->s_spheres[k].size();
+        nplane += c->s_planes[k].size();
+    }
+    if (nbox > LPS_MAX_COLLIDERS || nsphere > LPS_MAX_COLLIDERS || nplane > LPS_MAX_COLLIDERS) return LPS_ERR_INVALID;
+    HIPC(hipStreamSynchronize(c->stream));
+    SceneInfo* infos = reinterpret_cast<SceneInfo*>(c->h_scenes);
+    lps_box* boxes = reinterpret_cast<lps_box*>(infos + LPS_MAX_SCENES);
+    lps_sphere* spheres = reinterpret_cast<lps_sphere*>(boxes + LPS_MAX_COLLIDERS);
+    lps_plane* planes = reinterpret_cast<lps_plane*>(spheres + LPS_MAX_COLLIDERS);
+    nbox = nsphere = nplane = 0;
     uint32_t real0 = 0;
     for (size_t k = 0; k < S; k++) {
         SceneInfo& si = c->h_sinfo[k];
         si.real0 = real0;
         real0 += si.count;
-        si.box0 = (uint32_t)boxes.size();
+        si.box0 = (uint32_t)nbox;
         si.nbox = (uint32_t)c->s_boxes[k].size();
-        si.sphere0 = (uint32_t)spheres.size();
+        si.sphere0 = (uint32_t)nsphere;
         si.nsphere = (uint32_t)c->s_spheres[k].size();
-        si.plane0 = (uint32_t)planes.size();
+        si.plane0 = (uint32_t)nplane;
         si.nplane = (uint32_t)c->s_planes[k].size();
-        boxes.insert(boxes.end(), c->s_boxes[k].begin(), c->s_boxes[k].end());
-        spheres.insert(spheres.end(), c->s_spheres[k].begin(), c->s_spheres[k].end());
-        planes.insert(planes.end(), c->s_planes[k].begin(), c->s_planes[k].end());
+        for (const lps_box& q : c->s_boxes[k]) boxes[nbox++] = q;
+        for (const lps_sphere& q : c->s_spheres[k]) spheres[nsphere++] = q;
+        for (const lps_plane& q : c->s_planes[k]) planes[nplane++] = q;
         for (int a = 0; a < 3; a++)
             si.gravity[a] = c->s_gravity.empty() ? c->params.gravity[a] : c->s_gravity[3 * k + a];
+        infos[k] = si;
     }
-    if (boxes.size() > LPS_MAX_COLLIDERS || spheres.size() > LPS_MAX_COLLIDERS || planes.size() > LPS_MAX_COLLIDERS)
-        return LPS_ERR_INVALID;
-    if (!boxes.empty())
-        HIPC(hipMemcpyAsync(c->boxes, boxes.data(), sizeof(lps_box) * boxes.size(), hipMemcpyHostToDevice, c->stream));
-    if (!spheres.empty())
-        HIPC(hipMemcpyAsync(c->spheres, spheres.data(), sizeof(lps_sphere) * spheres.size(), hipMemcpyHostToDevice,
-                            c->stream));
-    if (!planes.empty())
-        HIPC(hipMemcpyAsync(c->planes, planes.data(), sizeof(lps_plane) * planes.size(), hipMemcpyHostToDevice,
-                            c->stream));
-    if (c->d_sinfo)
-        HIPC(hipMemcpyAsync(c->d_sinfo, c->h_sinfo.data(), sizeof(SceneInfo) * S, hipMemcpyHostToDevice, c->stream));
-    HIPC(hipStreamSynchronize(c->stream));
+    auto put = [&](void* dst, const void* src, size_t bytes) {
+        return bytes ? hipMemcpyAsync(dst, src, bytes, hipMemcpyHostToDevice, c->stream) : hipSuccess;
+    };
+    HIPC(put(c->boxes, boxes, sizeof(lps_box) * nbox));
+    HIPC(put(c->spheres, spheres, sizeof(lps_sphere) * nsphere));
+    HIPC(put(c->planes, planes, sizeof(lps_plane) * nplane));
+    if (c->d_sinfo) HIPC(put(c->d_sinfo, infos, sizeof(SceneInfo) * S));
     return LPS_OK;
+}
+
+// Arrays per scene and per particle block, grown when needed.
+int ensure_scenes(lps_ctx* c, uint32_t nscenes, uint32_t nblocks) {
+    int st;
+    if (nscenes > c->cap_scenes) {
+        c->epoch++;
+        c->cap_scenes = 0;
+        if ((st = dalloc(&c->d_sinfo, nscenes))) return st;
+        if ((st = dalloc(&c->d_sgrid, nscenes))) return st;
+        if ((st = dalloc(&c->d_err, (size_t)nscenes * 2 * LPS_ERR_SUBS * LPS_ERR_STRIDE))) return st;
+        if (c->h_sgrid) (void)hipHostFree(c->h_sgrid);
+        c->h_sgrid = nullptr;
+        HIPC(hipHostMalloc((void**)&c->h_sgrid, sizeof(SceneGrid) * nscenes, hipHostMallocDefault));
+        c->cap_scenes = nscenes;
+    }
+    if (nblocks > c->cap_blocks) {
+        c->epoch++;
+        c->cap_blocks = 0;
+        if ((st = dalloc(&c->d_bscene, nblocks))) return st;
+        if ((st = dalloc(&c->d_actlist, 2 * (size_t)nblocks))) return st;
+        c->cap_blocks = nblocks;
+    }
+    return LPS_OK;
+}
+
+lps_dev::StateArrays state_arrays(const lps_ctx* c, int b) {
+    return lps_dev::StateArrays{c->pos[b], c->vel[b], c->vh[b], c->first[b], c->id[b], c->pprev[b]};
+}
+
+// Copies a caller's rows to the device, into the pressure-force buffers
+// (scratch between steps; at least 48 bytes per slot, a row takes 37).  The
+// stream has drained.
+int upload_rows(lps_ctx* c, const float* x, const float* v, const float* vhalf, const uint8_t* first, uint32_t n,
+                lps_dev::Rows* out) {
+    const size_t vec = sizeof(float) * 3 * (size_t)n;
+    uint8_t* dev = reinterpret_cast<uint8_t*>(c->fp);
+    const size_t bytes = vec * (1u + (v ? 1u : 0u) + (vhalf ? 1u : 0u)) + (first ? n : 0u);
+    const bool small = bytes <= LPS_STAGE_BYTES;
+    size_t at = 0;
+    hipError_t e = hipSuccess;
+    auto put = [&](const void* src, size_t size) -> uint8_t* {
+        if (!src) return nullptr;
+        uint8_t* d = dev + at;
+        if (small) std::memcpy(c->h_stage + at, src, size);
+        else if (e == hipSuccess) e = hipMemcpyAsync(d, src, size, hipMemcpyHostToDevice, c->stream);
+        at += size;
+        return d;
+    };
+    *out = lps_dev::Rows{};
+    out->x = reinterpret_cast<float*>(put(x, vec));
+    out->v = reinterpret_cast<float*>(put(v, vec));
+    out->vhalf = reinterpret_cast<float*>(put(vhalf, vec));
+    out->first = put(first, n);
+    if (small) e = hipMemcpyAsync(dev, c->h_stage, bytes, hipMemcpyHostToDevice, c->stream);
+    return hip_status(e);
 }
 
 // Real particles of every scene, in slot order, from a full slot array.
@@ -940,12 +1016,29 @@ int lps_create(const lps_params* params, lps_ctx** out) {
         delete c;
         return LPS_ERR_HIP;
     }
-    bool ok = hipMalloc((void**)&c->grid, sizeof(DevGrid)) == hipSuccess &&
-              hipHostMalloc((void**)&c->flags, sizeof(uint32_t) * LPS_FLAG_WORDS * LPS_MAX_ITER_SLOTS,
-                            hipHostMallocCoherent | hipHostMallocMapped) == hipSuccess &&
-              hipHostMalloc((void**)&c->h_grid, sizeof(DevGrid), hipHostMallocDefault) == hipSuccess &&
-              hipHostMalloc((void**)&c->h_energy, sizeof(double) * 2 * LPS_MAX_SCENES,
-                            hipHostMallocCoherent | hipHostMallocMapped) == hipSuccess &&
+    // one pinned block for everything the host shares with the device
+    size_t at = 0;
+    auto carve = [&](size_t bytes) {
+        const size_t here = at;
+        at += (bytes + 255u) / 256u * 256u;
+        return here;
+    };
+    const size_t o_flags = carve(sizeof(uint32_t) * LPS_FLAG_WORDS * LPS_MAX_ITER_SLOTS);
+    const size_t o_grid = carve(sizeof(DevGrid));
+    const size_t o_energy = carve(sizeof(double) * 2 * LPS_MAX_SCENES);
+    const size_t o_report = carve(sizeof(StepReport));
+    const size_t o_scenes = carve(LPS_SCENES_BYTES);
+    const size_t o_stage = carve(LPS_STAGE_BYTES);
+    bool ok = hipHostMalloc((void**)&c->h_block, at, hipHostMallocCoherent | hipHostMallocMapped) == hipSuccess;
+    if (ok) {
+        c->flags = reinterpret_cast<uint32_t*>(c->h_block + o_flags);
+        c->h_grid = reinterpret_cast<DevGrid*>(c->h_block + o_grid);
+        c->h_energy = reinterpret_cast<double*>(c->h_block + o_energy);
+        c->report = reinterpret_cast<StepReport*>(c->h_block + o_report);
+        c->h_scenes = c->h_block + o_scenes;
+        c->h_stage = c->h_block + o_stage;
+    }
+    ok = ok && hipMalloc((void**)&c->grid, sizeof(DevGrid)) == hipSuccess &&
               hipMemsetAsync(c->grid, 0, sizeof(DevGrid), c->stream) == hipSuccess &&
               upload_tables(c) == LPS_OK;
     if (ok) {
@@ -958,6 +1051,7 @@ int lps_create(const lps_params* params, lps_ctx** out) {
         return LPS_ERR_OOM;
     }
     std::memset(c->flags, 0, sizeof(uint32_t) * LPS_FLAG_WORDS * LPS_MAX_ITER_SLOTS);
+    *c->report = StepReport{0u, 0u, 0u};
     *out = c;
     return LPS_OK;
 }
@@ -1062,8 +1156,12 @@ int lps_set_scenes(lps_ctx* c, uint32_t nscenes, const uint32_t* counts, const f
         for (uint32_t k = 0; k < 3 * nscenes; k++)
             if (!std::isfinite(gravity[k])) return LPS_ERR_INVALID;
     const uint32_t n = (uint32_t)slots;
+    const hipStream_t s = c->stream;
+    HIPC(hipStreamSynchronize(s));
     int st = ensure_particles(c, n);
     if (st) return st;
+    // captured graphs hold the sizes and the arrays' addresses
+    if (n != c->n || nscenes != c->h_sinfo.size()) c->epoch++;
     // layout; colliders of scenes that existed before are kept
     c->h_sinfo.assign(nscenes, SceneInfo{});
     c->s_boxes.resize(nscenes);
@@ -1072,8 +1170,6 @@ int lps_set_scenes(lps_ctx* c, uint32_t nscenes, const uint32_t* counts, const f
     if (gravity) c->s_gravity.assign(gravity, gravity + 3 * nscenes);
     else c->s_gravity.clear();
     uint32_t slot = 0;
-    uint64_t cells = 0;
-    size_t off = 0;
     for (uint32_t k = 0; k < nscenes; k++) {
         SceneInfo& si = c->h_sinfo[k];
         si.slot0 = slot;
@@ -1081,66 +1177,38 @@ int lps_set_scenes(lps_ctx* c, uint32_t nscenes, const uint32_t* counts, const f
         si.padded = (counts[k] + LPS_BLOCK - 1u) / LPS_BLOCK * LPS_BLOCK;
         si.block0 = slot / LPS_BLOCK;
         slot += si.padded;
-        cells += scene_cell_bound(c, x + 3 * off, counts[k], c->s_boxes[k]) + 1u;
-        off += counts[k];
     }
-    if ((st = ensure_cells(c, (uint32_t)std::min<uint64_t>(cells, 0x7FFFFFF0ull)))) return st;
-    if ((st = dalloc(&c->d_sinfo, nscenes))) return st;
-    if ((st = dalloc(&c->d_sgrid, nscenes))) return st;
-    if ((st = dalloc(&c->d_err, (size_t)nscenes * 2 * LPS_ERR_SUBS * LPS_ERR_STRIDE))) return st;
-    if ((st = dalloc(&c->d_bscene, n / LPS_BLOCK))) return st;
-    if ((st = dalloc(&c->d_actlist, 2 * (size_t)(n / LPS_BLOCK)))) return st;
-    if (c->h_sgrid) (void)hipHostFree(c->h_sgrid);
-    c->h_sgrid = nullptr;
-    HIPC(hipHostMalloc((void**)&c->h_sgrid, sizeof(SceneGrid) * nscenes, hipHostMallocDefault));
-    // particle arrays in slot order; empty slots at rest at the origin
-    std::vector<float4> buf(n);
-    auto up4 = [&](float4* dst, const float* src) -> int {
-        size_t r0 = 0;  // index of the scene's first particle in the caller's arrays
-        for (uint32_t k = 0; k < nscenes; k++) {
-            const SceneInfo& si = c->h_sinfo[k];
-            for (uint32_t i = 0; i < si.padded; i++) {
-                const size_t r = r0 + i;
-                buf[si.slot0 + i] = (i < si.count && src)
-                                        ? make_float4(src[3 * r], src[3 * r + 1], src[3 * r + 2], 0.f)
-                                        : make_float4(0.f, 0.f, 0.f, 0.f);
-            }
-            r0 += si.count;
-        }
-        HIPC(hipMemcpy(dst, buf.data(), sizeof(float4) * n, hipMemcpyHostToDevice));
-        return LPS_OK;
-    };
-    c->cur = 0;
-    if ((st = up4(c->pos[0], x))) return st;
-    if ((st = up4(c->vel[0], v))) return st;
-    if ((st = up4(c->vh[0], vhalf))) return st;
-    std::vector<uint8_t> f(n, 1);
-    std::vector<uint32_t> ids(n, 0xFFFFFFFFu);
-    std::vector<uint32_t> bscene(n / LPS_BLOCK);
-    {
-        uint32_t r = 0;
-        for (uint32_t k = 0; k < nscenes; k++) {
-            const SceneInfo& si = c->h_sinfo[k];
-            for (uint32_t i = 0; i < si.count; i++, r++) {
-                ids[si.slot0 + i] = r;
-                if (first) f[si.slot0 + i] = first[r] ? 1 : 0;
-            }
-            for (uint32_t b = 0; b < si.padded / LPS_BLOCK; b++) bscene[si.block0 + b] = k;
-        }
-    }
-    HIPC(hipMemcpy(c->first[0], f.data(), n, hipMemcpyHostToDevice));
-    HIPC(hipMemcpy(c->id[0], ids.data(), sizeof(uint32_t) * n, hipMemcpyHostToDevice));
-    HIPC(hipMemcpy(c->d_bscene, bscene.data(), sizeof(uint32_t) * (n / LPS_BLOCK), hipMemcpyHostToDevice));
-    HIPC(hipMemset(c->pprev[0], 0, sizeof(float) * n));
-    HIPC(hipMemset(c->d_sgrid, 0, sizeof(SceneGrid) * nscenes));
+    if ((st = ensure_scenes(c, nscenes, n / LPS_BLOCK))) return st;
     c->n = n;
     c->n_real = (uint32_t)total;
     c->next_id = (uint32_t)total;
+    c->cur = 0;
     c->have_step = false;
-    c->epoch++;
     if ((st = upload_scenes(c))) return st;
-    lps_dev::launch_bbox(c->stream, c->pos[0], c->vel[0], c->der.mass, n, scenes(c), c->bbox_part);
-    HIPC(hipStreamSynchronize(c->stream));
+    if (nscenes > 1u) {
+        std::vector<uint32_t> bscene(n / LPS_BLOCK);
+        for (uint32_t k = 0; k < nscenes; k++)
+            for (uint32_t b = 0; b < c->h_sinfo[k].padded / LPS_BLOCK; b++) bscene[c->h_sinfo[k].block0 + b] = k;
+        HIPC(hipMemcpy(c->d_bscene, bscene.data(), sizeof(uint32_t) * (n / LPS_BLOCK), hipMemcpyHostToDevice));
+    }
+    // the caller's rows as they are, then into the state arrays on the device
+    lps_dev::Rows rows;
+    if ((st = upload_rows(c, x, v, vhalf, first, (uint32_t)total, &rows))) return st;
+    const size_t parts = (size_t)LPS_BBOX_PART * (n / LPS_BLOCK);
+    if (parts > c->h_part_cap) {
+        if (c->h_part) (void)hipHostFree(c->h_part);
+        c->h_part = nullptr;
+        c->h_part_cap = 0;
+        HIPC(hipHostMalloc((void**)&c->h_part, sizeof(uint32_t) * parts, hipHostMallocDefault));
+        c->h_part_cap = parts;
+    }
+    lps_dev::launch_unpack(s, rows, c->der.mass, scenes(c), state_arrays(c, 0), c->bbox_part);
+    HIPC(hipGetLastError());
+    HIPC(hipMemcpyAsync(c->h_part, c->bbox_part, sizeof(uint32_t) * parts, hipMemcpyDeviceToHost, s));
+    HIPC(hipStreamSynchronize(s));
+    uint64_t cells = 0;
+    for (uint32_t k = 0; k < nscenes; k++) cells += scene_cell_bound(c, c->h_sinfo[k], c->s_boxes[k]) + 1u;
+    if ((st = ensure_cells(c, (uint32_t)std::min<uint64_t>(cells, 0x7FFFFFF0ull)))) return st;
     c->e_prev_valid = false;
     c->wf.prev_seeded = -1;  // a new state: its first step pairs with no earlier one
     return LPS_OK;
@@ -1167,6 +1235,7 @@ int lps_add_particles(lps_ctx* c, const float* x, const float* v, const float* v
     const hipStream_t s = c->stream;
     HIPC(hipStreamSynchronize(s));
     int st;
+    bool grown = false;
     if (slots > c->cap_n) {
         // grow by half again, keeping the current state (slots 0 .. old)
         uint64_t cap = std::max<uint64_t>(slots, (uint64_t)c->cap_n + c->cap_n / 2u);
@@ -1196,6 +1265,7 @@ int lps_add_particles(lps_ctx* c, const float* x, const float* v, const float* v
             return e != hipSuccess ? hip_status(e) : st;
         }
         c->cur = 0;
+        grown = true;
         cp(c->pos[0], sp, sizeof(float4) * old); cp(c->vel[0], sv, sizeof(float4) * old);
         cp(c->vh[0], sh, sizeof(float4) * old); cp(c->first[0], sf, old);
         cp(c->id[0], si, sizeof(uint32_t) * old); cp(c->pprev[0], spp, sizeof(float) * old);
@@ -1205,41 +1275,27 @@ int lps_add_particles(lps_ctx* c, const float* x, const float* v, const float* v
     }
     // the new particles take slots old .. total - 1 of the current state
     const int b = c->cur;
-    std::vector<float4> buf(n);
-    auto up4 = [&](float4* dst, const float* src) -> int {
-        for (uint32_t i = 0; i < n; i++)
-            buf[i] = src ? make_float4(src[3 * i], src[3 * i + 1], src[3 * i + 2], 0.f) : make_float4(0.f, 0.f, 0.f, 0.f);
-        HIPC(hipMemcpy(dst + old, buf.data(), sizeof(float4) * n, hipMemcpyHostToDevice));
-        return LPS_OK;
-    };
-    if ((st = up4(c->pos[b], x)) || (st = up4(c->vel[b], v)) || (st = up4(c->vh[b], vhalf))) return st;
-    std::vector<uint8_t> f(n, 1);
-    if (first)
-        for (uint32_t i = 0; i < n; i++) f[i] = first[i] ? 1 : 0;
-    std::vector<uint32_t> ids(n);
-    for (uint32_t i = 0; i < n; i++) ids[i] = c->next_id + i;
-    HIPC(hipMemcpy(c->first[b] + old, f.data(), n, hipMemcpyHostToDevice));
-    HIPC(hipMemcpy(c->id[b] + old, ids.data(), sizeof(uint32_t) * n, hipMemcpyHostToDevice));
-    HIPC(hipMemset(c->pprev[b] + old, 0, sizeof(float) * n));
+    const uint32_t nslots = (uint32_t)slots;
+    if ((st = ensure_scenes(c, 1u, nslots / LPS_BLOCK))) return st;
+    if (nslots != c->n) c->epoch++;  // captured graphs hold the number of slots
+    lps_dev::Rows rows;
+    if ((st = upload_rows(c, x, v, vhalf, first, n, &rows))) return st;
+    lps_dev::launch_append(s, rows, old, n, c->next_id, state_arrays(c, b));
     c->next_id += n;
     // layout: one scene over the grown slot range
-    const uint32_t nslots = (uint32_t)slots;
     SceneInfo& si = c->h_sinfo[0];
     si.count = (uint32_t)total;
     si.padded = nslots;
-    if (nslots != c->n) {
-        if ((st = dalloc(&c->d_bscene, nslots / LPS_BLOCK))) return st;
-        if ((st = dalloc(&c->d_actlist, 2 * (size_t)(nslots / LPS_BLOCK)))) return st;
-        HIPC(hipMemset(c->d_bscene, 0, sizeof(uint32_t) * (nslots / LPS_BLOCK)));
-    }
     c->n = nslots;
     c->n_real = (uint32_t)total;
     c->have_step = false;
     c->last_fp_valid = 0;
     c->feat_valid = c->seed_valid = false;
-    c->epoch++;
     if ((st = upload_scenes(c))) return st;
-    lps_dev::launch_bbox(s, c->pos[b], c->vel[b], c->der.mass, nslots, scenes(c), c->bbox_part);
+    // the blocks before the first new slot keep their records (unless the
+    // storage grew, and the records with it)
+    lps_dev::launch_bbox(s, c->pos[b], c->vel[b], c->der.mass, grown ? 0u : old / LPS_BLOCK, scenes(c), c->bbox_part);
+    HIPC(hipGetLastError());
     HIPC(hipStreamSynchronize(s));
     c->e_prev_valid = false;
     return LPS_OK;
@@ -1302,33 +1358,38 @@ int lps_get_count(lps_ctx* c, uint32_t* n) {
 
 int lps_get_particles(lps_ctx* c, float* x, float* v, float* vhalf, uint8_t* first, uint32_t* id, uint32_t n) {
     if (!c || n != c->n_real || n == 0) return LPS_ERR_INVALID;
-    HIPC(hipStreamSynchronize(c->stream));
-    const uint32_t ns = c->n;
-    std::vector<float4> buf(ns), real(n);
-    auto down4 = [&](float* dst, const float4* src) -> int {
-        if (!dst) return LPS_OK;
-        HIPC(hipMemcpy(buf.data(), src, sizeof(float4) * ns, hipMemcpyDeviceToHost));
-        compact_slots(c, buf, real.data(), 1);
-        for (uint32_t i = 0; i < n; i++) {
-            dst[3 * i] = real[i].x;
-            dst[3 * i + 1] = real[i].y;
-            dst[3 * i + 2] = real[i].z;
-        }
-        return LPS_OK;
-    };
-    int st;
-    if ((st = down4(x, c->pos[c->cur]))) return st;
-    if ((st = down4(v, c->vel[c->cur]))) return st;
-    if ((st = down4(vhalf, c->vh[c->cur]))) return st;
-    if (first) {
-        std::vector<uint8_t> f(ns);
-        HIPC(hipMemcpy(f.data(), c->first[c->cur], ns, hipMemcpyDeviceToHost));
-        compact_slots(c, f, first, 1);
+    // the wanted rows are packed on the device into scratch of the steps (the
+    // recorded masks, 36 bytes per slot, and the sort's placements, 8)
+    const hipStream_t s = c->stream;
+    const size_t vec = sizeof(float) * 3 * (size_t)n;
+    float* rows = reinterpret_cast<float*>(c->mk_mask);
+    uint32_t* words = reinterpret_cast<uint32_t*>(c->placed);
+    lps_dev::Rows dev{};
+    dev.x = x ? rows : nullptr;
+    dev.v = v ? rows + 3 * (size_t)n : nullptr;
+    dev.vhalf = vhalf ? rows + 6 * (size_t)n : nullptr;
+    dev.id = id ? words : nullptr;
+    dev.first = first ? reinterpret_cast<uint8_t*>(words + n) : nullptr;
+    lps_dev::launch_pack(s, state_arrays(c, c->cur), scenes(c), dev);
+    HIPC(hipGetLastError());
+    const struct { void* to; const void* from; size_t bytes; } part[] = {
+        {x, dev.x, vec}, {v, dev.v, vec}, {vhalf, dev.vhalf, vec}, {id, dev.id, sizeof(uint32_t) * (size_t)n},
+        {first, dev.first, n}};
+    size_t all = 0;
+    for (const auto& q : part) all += q.to ? q.bytes : 0u;
+    const bool small = all <= LPS_STAGE_BYTES;
+    size_t at = 0;
+    for (const auto& q : part) {
+        if (!q.to) continue;
+        HIPC(hipMemcpyAsync(small ? c->h_stage + at : q.to, q.from, q.bytes, hipMemcpyDeviceToHost, s));
+        at += q.bytes;
     }
-    if (id) {
-        std::vector<uint32_t> f(ns);
-        HIPC(hipMemcpy(f.data(), c->id[c->cur], sizeof(uint32_t) * ns, hipMemcpyDeviceToHost));
-        compact_slots(c, f, id, 1);
+    HIPC(hipStreamSynchronize(s));
+    at = 0;
+    for (const auto& q : part) {
+        if (!q.to || !small) continue;
+        std::memcpy(q.to, c->h_stage + at, q.bytes);
+        at += q.bytes;
     }
     return LPS_OK;
 }
@@ -1342,9 +1403,8 @@ int lps_step(lps_ctx* c, float dt, uint32_t nsteps, lps_step_stats* stats) {
     // A failed step leaves the state as it was (its kernels no-op and the
     // reorder copies the identity), so after a grid overflow the cell table is
     // grown and the remaining steps are issued again.
-    HIPC(hipMemcpyAsync(c->h_grid, c->grid, sizeof(DevGrid), hipMemcpyDeviceToHost, c->stream));
-    HIPC(hipStreamSynchronize(c->stream));
-    const uint32_t base = c->h_grid->steps_ok;
+    // every call that enqueued steps has waited for the last one's report
+    const uint32_t base = c->report->steps_ok;
     uint32_t completed = 0;
     int retries = 0;
     bool retry_plain = false;
@@ -1382,12 +1442,11 @@ int lps_step(lps_ctx* c, float dt, uint32_t nsteps, lps_step_stats* stats) {
             continue;
         }
         c->e_prev_valid = false;
-        HIPC(hipMemcpyAsync(c->h_grid, c->grid, sizeof(DevGrid), hipMemcpyDeviceToHost, c->stream));
         HIPC(hipStreamSynchronize(c->stream));
-        completed = c->h_grid->steps_ok - base;
-        const uint32_t status = c->h_grid->status;
+        completed = c->report->steps_ok - base;
+        const uint32_t status = c->report->status;
         if (status == LPS_ERR_GRID_OVERFLOW) {
-            const uint32_t need = c->h_grid->cells_needed;
+            const uint32_t need = c->report->cells_needed;
             if (need >= 0x7FFFFFF0u || ++retries > 8) return LPS_ERR_GRID_OVERFLOW;
             int st = ensure_cells(c, need + need / 4 + 64);
             if (st) return st;
@@ -1411,10 +1470,9 @@ int lps_step(lps_ctx* c, float dt, uint32_t nsteps, lps_step_stats* stats) {
     }
     if (pci) {
         // one check per call: every step must have completed on the device
-        HIPC(hipMemcpyAsync(c->h_grid, c->grid, sizeof(DevGrid), hipMemcpyDeviceToHost, c->stream));
         HIPC(hipStreamSynchronize(c->stream));
-        if (c->h_grid->status != 0u) return (int)c->h_grid->status;
-        if (c->h_grid->steps_ok - base != nsteps) return LPS_ERR_HIP;
+        if (c->report->status != 0u) return (int)c->report->status;
+        if (c->report->steps_ok - base != nsteps) return LPS_ERR_HIP;
     }
     if (c->prof) prof_collect(c);
     return LPS_OK;

@@ -94,6 +94,11 @@ struct DevGrid {
     uint32_t list_of[LPS_MAX_ITER_SLOTS];
 };
 
+// What the host checks after a call's steps (coherent host memory).
+struct StepReport {
+    uint32_t status, steps_ok, cells_needed;  // of DevGrid, at the end of the last step
+};
+
 // Per-block partial record: orderable-uint min xyz, max xyz, non-finite flag,
 // then the block's kinetic and potential energy (float bits), one spare word.
 #define LPS_BBOX_PART 10

@@ -95,9 +95,29 @@ struct PhysArgs {
     uint32_t lanes;       // lanes per particle of the stencil kernels: 1, 4 or 16
 };
 
-// per-block partial records (bounding box and energies) of a state
-void launch_bbox(hipStream_t s, const float4* pos, const float4* vel, float mass, uint32_t n, const Scenes& sc,
+// A caller's arrays on the device: n x 3 floats, n bytes, n words (null: absent).
+struct Rows {
+    float *x, *v, *vhalf;
+    uint8_t* first;
+    uint32_t* id;  // readback only
+};
+// One buffer of the state.
+struct StateArrays {
+    float4 *pos, *vel, *vh;
+    uint8_t* first;
+    uint32_t* id;
+    float* pprev;
+};
+
+// per-block partial records (bounding box and energies) of a state, from particle block block0 on
+void launch_bbox(hipStream_t s, const float4* pos, const float4* vel, float mass, uint32_t block0, const Scenes& sc,
                  uint32_t* part);
+// the state of all scenes from the caller's rows, its records, and zeroed scene grids
+void launch_unpack(hipStream_t s, const Rows& in, float mass, const Scenes& sc, const StateArrays& a, uint32_t* part);
+// n particles appended at slot `at` (no records)
+void launch_append(hipStream_t s, const Rows& in, uint32_t at, uint32_t n, uint32_t id0, const StateArrays& a);
+// the wanted rows of the real particles, scenes back to back
+void launch_pack(hipStream_t s, const StateArrays& a, const Scenes& sc, const Rows& out);
 uint32_t bbox_parts(uint32_t n);
 // per-scene kinetic and potential energy from the partial records to
 // out[2 * scene], out[2 * scene + 1] (coherent host memory)
@@ -177,9 +197,10 @@ void launch_pci_pressure(hipStream_t s, const PhysArgs& a, const float4* xq, con
                          float4* xpred_next, uint32_t k, const LoopRule& rule, uint32_t* host_flag, uint32_t threads);
 // PCISPH (fp given): fp and press hold three buffers of a.mk.stride slots;
 // each scene reads the one its loop applied (SceneGrid::final_buf).  SPH:
-// press is the density pass's pressure.  pprev receives the applied pressure.
+// press is the density pass's pressure.  pprev receives the applied pressure,
+// report (coherent host memory) the step's outcome.
 void launch_integrate(hipStream_t s, const PhysArgs& a, const float4* fp, float* pprev, const float* press,
-                      uint32_t* bbox_part);
+                      uint32_t* bbox_part, StepReport* report);
 // positions of the real particles, scenes back to back, to dst[r * stride + 0..2]
 void launch_export_positions(hipStream_t s, const float4* pos, uint32_t n, const Scenes& sc, float* dst,
                              uint32_t stride);

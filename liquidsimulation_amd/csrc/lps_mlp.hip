@@ -297,7 +297,7 @@ __global__ __launch_bounds__(LPS_BLOCK) __attribute__((amdgpu_waves_per_eu(4))) 
         // <= 1; the stall rule cannot stop a loop at its first correction).
         // The test is uniform over the block, so the whole block leaves
         // before the barrier or none of it does.
-        const uint32_t s = sc.block_scene[blockIdx.x];
+        const uint32_t s = sc.count == 1u ? 0u : sc.block_scene[blockIdx.x];
         const uint32_t* err = lps_dev::err_slot(sc, s, 1u);
         uint32_t eb = 0u;
 #pragma unroll
