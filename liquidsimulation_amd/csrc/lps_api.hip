@@ -29,11 +29,13 @@
 // Scratch memory of lps_mlp_grad_noalloc: one array per GPU, held until the
 // process ends.  Layout (bytes): staged features [LPS_NOALLOC_MAX_ROWS][16]
 // floats, staged targets [LPS_NOALLOC_MAX_ROWS] floats, gradient
-// accumulators [LPS_MLP_PARAMS] floats (padded to 256 bytes), loss [1].
+// [LPS_MLP_PARAMS] floats (padded to 256 bytes), loss [1] (padded), the
+// blocks' gradient sums.
 #define LPS_NOALLOC_X_BYTES ((size_t)LPS_NOALLOC_MAX_ROWS * LPS_MLP_IN * sizeof(float))
 #define LPS_NOALLOC_T_BYTES ((size_t)LPS_NOALLOC_MAX_ROWS * sizeof(float))
 #define LPS_NOALLOC_G_BYTES ((((size_t)LPS_MLP_PARAMS * sizeof(float)) + 255u) / 256u * 256u)
-#define LPS_NOALLOC_BYTES (LPS_NOALLOC_X_BYTES + LPS_NOALLOC_T_BYTES + LPS_NOALLOC_G_BYTES + 256u)
+#define LPS_NOALLOC_PART (LPS_NOALLOC_X_BYTES + LPS_NOALLOC_T_BYTES + LPS_NOALLOC_G_BYTES + 256u)
+#define LPS_NOALLOC_BYTES (LPS_NOALLOC_PART + (size_t)LPS_GRAD_BLOCKS * LPS_GRAD_STRIDE * sizeof(float))
 static __device__ __align__(256) unsigned char scratch[LPS_NOALLOC_BYTES];
 
 namespace {
@@ -69,6 +71,10 @@ unsigned char* scratch_ptr(int device) {
 constexpr size_t LPS_STAGE_BYTES = 1u << 20;
 constexpr size_t LPS_SCENES_BYTES =
     LPS_MAX_SCENES * sizeof(SceneInfo) + LPS_MAX_COLLIDERS * (sizeof(lps_box) + sizeof(lps_sphere) + sizeof(lps_plane));
+
+// Device rows of the network's host calls kept between calls (64 MiB); larger
+// batches take an allocation of their own.
+constexpr size_t LPS_ROWS_KEPT = 16u << 20;
 
 struct ProfRec {
     const char* name;
@@ -210,6 +216,9 @@ struct lps_ctx {
     float *coll_x = nullptr, *coll_t = nullptr;
     uint64_t coll_cap = 0, coll_rows = 0;
     uint32_t coll_stride = 1, coll_offset = 0;
+    float* d_part = nullptr;  // the blocks' gradient sums
+    float* d_rows = nullptr;  // rows of lps_mlp_forward and lps_mlp_grad, kept up to LPS_ROWS_KEPT floats
+    size_t rows_cap = 0;
     float *d_grad = nullptr, *d_m1 = nullptr, *d_m2 = nullptr, *d_loss = nullptr;
     double* d_stats = nullptr;
 
@@ -464,7 +473,7 @@ void free_all(lps_ctx* c) {
     dfree(c->cell_count); dfree(c->cell_lb); dfree(c->tile_sum);
     dfree(c->tables); dfree(c->boxes); dfree(c->spheres); dfree(c->planes); dfree(c->grid);
     dfree(c->d_mlp); dfree(c->d_mlp_packed); dfree(c->feat); dfree(c->seed); dfree(c->coll_x); dfree(c->coll_t);
-    dfree(c->d_grad); dfree(c->d_m1); dfree(c->d_m2); dfree(c->d_loss); dfree(c->d_stats);
+    dfree(c->d_part); dfree(c->d_rows); dfree(c->d_grad); dfree(c->d_m1); dfree(c->d_m2); dfree(c->d_loss); dfree(c->d_stats);
     dfree(c->d_sinfo); dfree(c->d_sgrid); dfree(c->d_bscene); dfree(c->d_actlist); dfree(c->d_err);
     if (c->h_sgrid) (void)hipHostFree(c->h_sgrid);
     c->h_sgrid = nullptr;
@@ -1848,10 +1857,41 @@ int lps_mlp_collected(lps_ctx* c, uint64_t* rows) {
 
 namespace {
 
+// Device memory for the rows of one call: the context's buffer, or an
+// allocation that ends with the call.  The stream is drained before either is
+// given back.
+struct HostRows {
+    lps_ctx* c;
+    float* p = nullptr;
+    int st = LPS_OK;
+    bool own = false;
+    HostRows(lps_ctx* ctx, size_t floats) : c(ctx) {
+        if (floats > LPS_ROWS_KEPT) {
+            own = true;
+            st = dalloc(&p, floats);
+            return;
+        }
+        if (floats > c->rows_cap) {
+            c->rows_cap = 0;
+            if ((st = dalloc(&c->d_rows, floats))) return;
+            c->rows_cap = floats;
+        }
+        p = c->d_rows;
+    }
+    ~HostRows() {
+        if (st) return;
+        (void)hipStreamSynchronize(c->stream);
+        if (own) dfree(p);
+    }
+    HostRows(const HostRows&) = delete;
+    HostRows& operator=(const HostRows&) = delete;
+};
+
 int ensure_train_buffers(lps_ctx* c) {
     int st;
     if (!c->d_mlp && (st = dalloc(&c->d_mlp, LPS_MLP_PARAMS + 2 * LPS_MLP_IN))) return st;
     if (!c->d_mlp_packed && (st = dalloc(&c->d_mlp_packed, lps_dev::mlp_packed_bytes()))) return st;
+    if (!c->d_part && (st = dalloc(&c->d_part, (size_t)LPS_GRAD_BLOCKS * LPS_GRAD_STRIDE))) return st;
     if (!c->d_grad && (st = dalloc(&c->d_grad, LPS_MLP_PARAMS))) return st;
     if (!c->d_m1 && (st = dalloc(&c->d_m1, LPS_MLP_PARAMS))) return st;
     if (!c->d_m2 && (st = dalloc(&c->d_m2, LPS_MLP_PARAMS))) return st;
@@ -1902,8 +1942,8 @@ int lps_mlp_train(lps_ctx* c, const lps_mlp_train_cfg* cfg, float* epoch_loss) {
         // feature normalisation (mean, 1/std; constant features get weight 0)
         // and target scale (root mean square of the targets)
         HIPC(hipMemsetAsync(c->d_stats, 0, sizeof(double) * 4 * LPS_MLP_IN, s));
-        lps_dev::launch_feature_stats(s, c->coll_x, N, LPS_MLP_IN, c->d_stats);
-        lps_dev::launch_feature_stats(s, c->coll_t, N, 1, c->d_stats + 2 * LPS_MLP_IN);
+        lps_dev::launch_feature_stats(s, c->coll_x, N, c->d_stats);
+        lps_dev::launch_target_stats(s, c->coll_t, N, c->d_stats + 2 * LPS_MLP_IN);
         double h[4 * LPS_MLP_IN];
         HIPC(hipMemcpyAsync(h, c->d_stats, sizeof(h), hipMemcpyDeviceToHost, s));
         HIPC(hipStreamSynchronize(s));
@@ -1921,7 +1961,6 @@ int lps_mlp_train(lps_ctx* c, const lps_mlp_train_cfg* cfg, float* epoch_loss) {
     HIPC(hipMemcpyAsync(c->d_mlp, c->mlp_w.data(), sizeof(float) * LPS_MLP_PARAMS, hipMemcpyHostToDevice, s));
     HIPC(hipMemcpyAsync(c->d_mlp + LPS_MLP_PARAMS, c->mlp_fscale.data(), sizeof(float) * 2 * LPS_MLP_IN,
                         hipMemcpyHostToDevice, s));
-    HIPC(hipMemsetAsync(c->d_grad, 0, sizeof(float) * LPS_MLP_PARAMS, s));
     HIPC(hipMemsetAsync(c->d_m1, 0, sizeof(float) * LPS_MLP_PARAMS, s));
     HIPC(hipMemsetAsync(c->d_m2, 0, sizeof(float) * LPS_MLP_PARAMS, s));
     const lps_dev::MlpArgs m = mlp_args(c);
@@ -1939,12 +1978,11 @@ int lps_mlp_train(lps_ctx* c, const lps_mlp_train_cfg* cfg, float* epoch_loss) {
             const uint64_t start = b * cfg->batch;
             const uint32_t rows = (uint32_t)std::min<uint64_t>(cfg->batch, N - start);
             const lps_dev::RowMap rm{nullptr, start, mul, add, N};
-            lps_dev::launch_mlp_grad(s, m, c->coll_x, c->coll_t, rm, rows, cfg->over_weight, c->d_grad, c->d_loss);
             const double u = (double)t / std::max(total - 1.0, 1.0);
             const float lr = (float)(cfg->lr_final + 0.5 * (cfg->lr - cfg->lr_final) * (1.0 + std::cos(3.14159265358979323846 * u)));
             ++t;
-            lps_dev::launch_adam(s, c->d_mlp, c->d_grad, c->d_m1, c->d_m2, LPS_MLP_PARAMS, lr, cfg->beta1, cfg->beta2,
-                                 cfg->eps, t);
+            lps_dev::launch_train_step(s, m, c->coll_x, c->coll_t, rm, rows, cfg->over_weight, c->d_part, c->d_loss,
+                                       c->d_mlp, c->d_m1, c->d_m2, lr, cfg->beta1, cfg->beta2, cfg->eps, t);
         }
         float loss = 0.f;
         HIPC(hipMemcpyAsync(&loss, c->d_loss, sizeof(float), hipMemcpyDeviceToHost, s));
@@ -1969,20 +2007,15 @@ int lps_mlp_train(lps_ctx* c, const lps_mlp_train_cfg* cfg, float* epoch_loss) {
 int lps_mlp_forward(lps_ctx* c, const float* x, uint32_t n, float* y) {
     if (!c || !x || !y || n == 0) return LPS_ERR_INVALID;
     if (!c->mlp_loaded) return LPS_ERR_STATE;
-    float *dx = nullptr, *dy = nullptr;
-    int st = dalloc(&dx, (size_t)n * LPS_MLP_IN);
-    if (!st) st = dalloc(&dy, n);
-    if (!st && hipMemcpy(dx, x, sizeof(float) * LPS_MLP_IN * (size_t)n, hipMemcpyHostToDevice) != hipSuccess)
-        st = LPS_ERR_HIP;
-    if (!st) {
-        lps_dev::launch_mlp_forward(c->stream, c->d_mlp_packed, dx, n, dy);
-        if (hipMemcpyAsync(y, dy, sizeof(float) * n, hipMemcpyDeviceToHost, c->stream) != hipSuccess ||
-            hipStreamSynchronize(c->stream) != hipSuccess)
-            st = LPS_ERR_HIP;
-    }
-    dfree(dx);
-    dfree(dy);
-    return st;
+    HostRows rows(c, (size_t)n * (LPS_MLP_IN + 1));
+    if (rows.st) return rows.st;
+    float* dx = rows.p;
+    float* dy = rows.p + (size_t)n * LPS_MLP_IN;
+    HIPC(hipMemcpyAsync(dx, x, sizeof(float) * LPS_MLP_IN * (size_t)n, hipMemcpyHostToDevice, c->stream));
+    lps_dev::launch_mlp_forward(c->stream, c->d_mlp_packed, dx, n, dy);
+    HIPC(hipMemcpyAsync(y, dy, sizeof(float) * n, hipMemcpyDeviceToHost, c->stream));
+    HIPC(hipStreamSynchronize(c->stream));
+    return LPS_OK;
 }
 
 int lps_mlp_grad(lps_ctx* c, const float* x, const float* t, uint32_t n, float over_weight, float* grad,
@@ -1992,31 +2025,23 @@ int lps_mlp_grad(lps_ctx* c, const float* x, const float* t, uint32_t n, float o
     if (!c->mlp_loaded) return LPS_ERR_STATE;
     int st = ensure_train_buffers(c);
     if (st) return st;
-    float *dx = nullptr, *dt = nullptr;
-    if ((st = dalloc(&dx, (size_t)n * LPS_MLP_IN)) || (st = dalloc(&dt, n))) {
-        dfree(dx);
-        return st;
-    }
+    HostRows rows(c, (size_t)n * (LPS_MLP_IN + 1));
+    if (rows.st) return rows.st;
     const hipStream_t s = c->stream;
-    if (hipMemcpy(dx, x, sizeof(float) * LPS_MLP_IN * (size_t)n, hipMemcpyHostToDevice) != hipSuccess ||
-        hipMemcpy(dt, t, sizeof(float) * n, hipMemcpyHostToDevice) != hipSuccess ||
-        hipMemsetAsync(c->d_grad, 0, sizeof(float) * LPS_MLP_PARAMS, s) != hipSuccess ||
-        hipMemsetAsync(c->d_loss, 0, sizeof(float), s) != hipSuccess)
-        st = LPS_ERR_HIP;
-    if (!st) {
-        const lps_dev::RowMap rm{nullptr, 0u, 1u, 0u, n};
-        lps_dev::launch_mlp_grad(s, mlp_args(c), dx, dt, rm, n, over_weight, c->d_grad, c->d_loss);
-        float l = 0.f;
-        if (hipMemcpyAsync(grad, c->d_grad, sizeof(float) * LPS_MLP_PARAMS, hipMemcpyDeviceToHost, s) != hipSuccess ||
-            hipMemcpyAsync(&l, c->d_loss, sizeof(float), hipMemcpyDeviceToHost, s) != hipSuccess ||
-            hipMemsetAsync(c->d_grad, 0, sizeof(float) * LPS_MLP_PARAMS, s) != hipSuccess ||
-            hipStreamSynchronize(s) != hipSuccess)
-            st = LPS_ERR_HIP;
-        if (loss) *loss = l;
-    }
-    dfree(dx);
-    dfree(dt);
-    return st;
+    float* dx = rows.p;
+    float* dt = rows.p + (size_t)n * LPS_MLP_IN;
+    HIPC(hipMemcpyAsync(dx, x, sizeof(float) * LPS_MLP_IN * (size_t)n, hipMemcpyHostToDevice, s));
+    HIPC(hipMemcpyAsync(dt, t, sizeof(float) * n, hipMemcpyHostToDevice, s));
+    HIPC(hipMemsetAsync(c->d_loss, 0, sizeof(float), s));
+    const lps_dev::RowMap rm{nullptr, 0u, 1u, 0u, n};
+    lps_dev::launch_mlp_grad(s, mlp_args(c), dx, dt, rm, n, over_weight, c->d_part, c->d_grad, c->d_loss);
+    HIPC(hipGetLastError());
+    float l = 0.f;
+    HIPC(hipMemcpyAsync(grad, c->d_grad, sizeof(float) * LPS_MLP_PARAMS, hipMemcpyDeviceToHost, s));
+    HIPC(hipMemcpyAsync(&l, c->d_loss, sizeof(float), hipMemcpyDeviceToHost, s));
+    HIPC(hipStreamSynchronize(s));
+    if (loss) *loss = l;
+    return LPS_OK;
 }
 
 int lps_mlp_grad_noalloc(lps_ctx* c, const float* x, const float* t, uint32_t n, float over_weight, float* grad,
@@ -2032,15 +2057,15 @@ int lps_mlp_grad_noalloc(lps_ctx* c, const float* x, const float* t, uint32_t n,
     float* dg = reinterpret_cast<float*>(base + LPS_NOALLOC_X_BYTES + LPS_NOALLOC_T_BYTES);
     float* dl = reinterpret_cast<float*>(base + LPS_NOALLOC_X_BYTES + LPS_NOALLOC_T_BYTES + LPS_NOALLOC_G_BYTES);
     const hipStream_t s = c->stream;
-    // the accumulators keep the previous call's sums: clear them (a fill
-    // kernel, so the call stays free of memset nodes)
-    lps_dev::launch_fill_zero(s, dg, LPS_MLP_PARAMS);
+    float* dp = reinterpret_cast<float*>(base + LPS_NOALLOC_PART);
+    // the loss keeps the previous call's sum: clear it (a fill kernel, so the
+    // call stays free of memset nodes)
     lps_dev::launch_fill_zero(s, dl, 1u);
     HIPC(hipGetLastError());
     HIPC(hipMemcpyAsync(dx, x, sizeof(float) * LPS_MLP_IN * (size_t)n, hipMemcpyHostToDevice, s));
     HIPC(hipMemcpyAsync(dt, t, sizeof(float) * n, hipMemcpyHostToDevice, s));
     const lps_dev::RowMap rm{nullptr, 0u, 1u, 0u, n};
-    lps_dev::launch_mlp_grad(s, mlp_args(c), dx, dt, rm, n, over_weight, dg, dl);
+    lps_dev::launch_mlp_grad(s, mlp_args(c), dx, dt, rm, n, over_weight, dp, dg, dl);
     HIPC(hipGetLastError());
     float l = 0.f;
     HIPC(hipMemcpyAsync(grad, dg, sizeof(float) * LPS_MLP_PARAMS, hipMemcpyDeviceToHost, s));

@@ -99,6 +99,11 @@ struct StepReport {
     uint32_t status, steps_ok, cells_needed;  // of DevGrid, at the end of the last step
 };
 
+// Gradient sums of the blocks of a batch: at most this many blocks, a row of
+// LPS_MLP_PARAMS sums and the loss each, padded to whole groups of 64.
+#define LPS_GRAD_BLOCKS 256u
+#define LPS_GRAD_STRIDE ((LPS_MLP_PARAMS + 1u + 63u) / 64u * 64u)
+
 // Per-block partial record: orderable-uint min xyz, max xyz, non-finite flag,
 // then the block's kinetic and potential energy (float bits), one spare word.
 #define LPS_BBOX_PART 10

@@ -162,7 +162,10 @@ struct RowMap {
     const uint32_t* idx;
     uint64_t start, mul, add, rows;
     __host__ __device__ uint32_t row(uint32_t s) const {
-        return idx ? idx[s] : (uint32_t)(((start + s) * mul + add) % rows);
+        if (idx) return idx[s];
+        // the identity (a plain batch) needs no 64-bit remainder
+        if (mul == 1u && add == 0u) return (uint32_t)(start + s);
+        return (uint32_t)(((start + s) * mul + add) % rows);
     }
 };
 // y_i = pscale * tscale * MLP(features_i) (0 when not finite) and seed_i =
@@ -184,11 +187,16 @@ void launch_mlp_pack(hipStream_t s, const MlpArgs& m, void* packed);
 void launch_mlp_forward(hipStream_t s, const void* packed, const float* x, uint32_t n, float* y);
 // p[0..n) = 0 with a kernel (no memset node)
 void launch_fill_zero(hipStream_t s, float* p, uint32_t n);
+// gradient of n rows (written) and their loss (added); part: LPS_GRAD_BLOCKS * LPS_GRAD_STRIDE floats of scratch
 void launch_mlp_grad(hipStream_t s, const MlpArgs& m, const float* x, const float* t, const RowMap& rm, uint32_t n,
-                     float over_weight, float* grad, float* loss);
-void launch_adam(hipStream_t s, float* params, float* grad, float* m1, float* m2, uint32_t count, float lr,
-                 float b1, float b2, float eps, uint32_t step);
-void launch_feature_stats(hipStream_t s, const float* x, uint64_t n, uint32_t cols, double* acc);
+                     float over_weight, float* part, float* grad, float* loss);
+// the same followed by one Adam step on params (m.params)
+void launch_train_step(hipStream_t s, const MlpArgs& m, const float* x, const float* t, const RowMap& rm, uint32_t n,
+                       float over_weight, float* part, float* loss, float* params, float* m1, float* m2, float lr,
+                       float b1, float b2, float eps, uint32_t step);
+// sums and sums of squares: of the 16 columns of n rows (16 + 16 doubles), of n values (2 doubles)
+void launch_feature_stats(hipStream_t s, const float* x, uint64_t n, double* acc);
+void launch_target_stats(hipStream_t s, const float* t, uint64_t n, double* acc);
 void launch_collect(hipStream_t s, const float* feat, uint32_t fs, const float* press, float pscale, uint32_t n,
                     uint32_t stride, uint32_t offset, uint32_t count, float* X, float* T, uint64_t base);
 // also applies the loop rule of correction k (block 0) and answers host_flag;

@@ -6,7 +6,8 @@
 // (lane l holds rows 4*(l/16)..+3 of column l%16) is exactly the B operand of
 // the next layer (lane l holds K rows 4*(l/16)..+3 of column l%16), so the
 // forward pass needs no data movement between layers.  The weight-gradient
-// products reduce over particles and take their operands from LDS transposes.
+// products reduce over particles; for them each layer is also evaluated the
+// other way round (k_mlp_grad).
 //
 // BF16: inputs (after normalisation), weights and hidden activations are
 // rounded to BF16 (round to nearest even); biases, accumulators, the output
@@ -69,77 +70,6 @@ __device__ __forceinline__ bf16x4 load4(const unsigned short* p) {
     return r;
 }
 
-struct alignas(16) MlpSmem {
-    unsigned short w1[HID * IN];    // [neuron][feature]
-    unsigned short w2[HID * HID];   // [out][in]
-    unsigned short w2t[HID * HID];  // [in][out]
-    float b1[HID], b2[HID], w3[HID];
-    float mean[IN], istd[IN];
-    float b3;
-};
-
-__device__ void load_weights(MlpSmem& S, const MlpArgs& m, bool transposed) {
-    for (uint32_t k = threadIdx.x; k < HID * IN; k += blockDim.x) S.w1[k] = f2bf(m.params[OFF_W1 + k]);
-    for (uint32_t k = threadIdx.x; k < HID * HID; k += blockDim.x) {
-        const unsigned short w = f2bf(m.params[OFF_W2 + k]);
-        S.w2[k] = w;
-        if (transposed) S.w2t[(k % HID) * HID + k / HID] = w;
-    }
-    for (uint32_t k = threadIdx.x; k < HID; k += blockDim.x) {
-        S.b1[k] = m.params[OFF_B1 + k];
-        S.b2[k] = m.params[OFF_B2 + k];
-        S.w3[k] = rbf(m.params[OFF_W3 + k]);
-    }
-    for (uint32_t k = threadIdx.x; k < IN; k += blockDim.x) {
-        S.mean[k] = m.fscale[k];
-        S.istd[k] = m.fscale[IN + k];
-    }
-    if (threadIdx.x == 0) S.b3 = m.params[OFF_B3];
-}
-
-// Forward pass of one group of 16 samples (column l%16 of the tiles).
-struct Fwd {
-    bf16x4 x;        // input tile (B layout): features 4*(l/16)..+3 of sample l%16
-    f32x4 y1[4];     // layer-1 pre-activations, neuron tiles
-    bf16x4 h1[4];
-    f32x4 y2[4];
-    bf16x4 h2[4];
-    float y;         // output (identical in the four lane groups of a sample)
-};
-
-__device__ __forceinline__ void forward(const MlpSmem& S, const float* __restrict__ xrow, bool valid, Fwd& F) {
-    const uint32_t l = threadIdx.x & 63u, g = l >> 4, r16 = l & 15u;
-    for (int r = 0; r < 4; r++) {
-        const uint32_t f = 4u * g + (uint32_t)r;
-        const float v = valid ? (xrow[f] - S.mean[f]) * S.istd[f] : 0.f;
-        F.x[r] = (short)f2bf(v);
-    }
-    for (int mt = 0; mt < 4; mt++) {
-        const bf16x4 a = load4(&S.w1[(mt * 16 + r16) * IN + 4 * g]);
-        F.y1[mt] = mfma(a, F.x, f32x4{0.f, 0.f, 0.f, 0.f});
-        for (int r = 0; r < 4; r++) {
-            const float v = F.y1[mt][r] + S.b1[mt * 16 + 4 * g + r];
-            F.y1[mt][r] = v;
-            F.h1[mt][r] = (short)f2bf(fmaxf(v, 0.f));
-        }
-    }
-    for (int mt = 0; mt < 4; mt++) {
-        f32x4 acc{0.f, 0.f, 0.f, 0.f};
-        for (int kt = 0; kt < 4; kt++) acc = mfma(load4(&S.w2[(mt * 16 + r16) * HID + kt * 16 + 4 * g]), F.h1[kt], acc);
-        for (int r = 0; r < 4; r++) {
-            const float v = acc[r] + S.b2[mt * 16 + 4 * g + r];
-            F.y2[mt][r] = v;
-            F.h2[mt][r] = (short)f2bf(fmaxf(v, 0.f));
-        }
-    }
-    float part = 0.f;
-    for (int mt = 0; mt < 4; mt++)
-        for (int r = 0; r < 4; r++) part += S.w3[mt * 16 + 4 * g + r] * bf2f((unsigned short)F.h2[mt][r]);
-    part += __shfl_xor(part, 16, 64);
-    part += __shfl_xor(part, 32, 64);
-    F.y = part + S.b3;
-}
-
 // The inference weights in BF16, packed once per change of the FP32 master
 // copy (k_mlp_pack) so that the seed kernel copies them instead of converting
 // them in every block.  The weight matrices are stored as MFMA A-operand
@@ -158,9 +88,7 @@ struct alignas(16) MlpPacked {
 };
 static_assert(sizeof(MlpPacked) % 16 == 0, "packed weights are copied as uint4");
 
-// Inference of one group of 16 samples (column l%16), the output only: the
-// arithmetic of forward() (same products, order and roundings) without
-// keeping the pre-activations and hidden tiles the gradient needs.
+// Inference of one group of 16 samples (column l%16), the output only.
 // xin holds features 4*(l/16)..+3 of the lane's sample.
 __device__ __forceinline__ float infer(const MlpPacked& S, const float4& xin, bool valid) {
     const uint32_t l = threadIdx.x & 63u, g = l >> 4;
@@ -345,169 +273,358 @@ __global__ void k_fill_zero(float* __restrict__ p, uint32_t n) {
 
 // Gradient of the weighted mean squared error mean(w d^2), d = y - t/tscale,
 // w = over_weight where d > 0 and 1 elsewhere, over a batch of n rows of x / t
-// (row of sample s given by rm) with respect to the FP32 parameters, added to
-// grad; loss gets the batch's loss.  The
-// forward uses the BF16-rounded values (straight-through).  Each block sums
-// its samples' gradients in LDS, then adds them to grad with global atomics.
-__global__ __launch_bounds__(LPS_BLOCK) void k_mlp_grad(MlpArgs m, const float* __restrict__ x,
-                                                        const float* __restrict__ t, RowMap rm, uint32_t n,
-                                                        float inv_n, float over_weight, float* __restrict__ grad,
-                                                        float* __restrict__ loss) {
-    __shared__ MlpSmem S;
-    // load4 reads 8 bytes at a time: every staging array is 16-byte aligned
-    __shared__ __align__(16) float G[LPS_MLP_PARAMS];
-    __shared__ __align__(16) unsigned short T_[LPS_BLOCK / 64][HID * 16];   // dY2 [neuron][sample]
-    __shared__ __align__(16) unsigned short U_[LPS_BLOCK / 64][HID * 16];   // H1  [neuron][sample]
-    __shared__ __align__(16) unsigned short D_[LPS_BLOCK / 64][HID * 16];   // dY1 [neuron][sample]
-    __shared__ __align__(16) unsigned short V_[LPS_BLOCK / 64][IN * 16];    // X   [feature][sample]
-    __shared__ float s_loss;
-    load_weights(S, m, true);
-    for (uint32_t k = threadIdx.x; k < LPS_MLP_PARAMS; k += blockDim.x) G[k] = 0.f;
-    if (threadIdx.x == 0) s_loss = 0.f;
-    __syncthreads();
-    const uint32_t w = threadIdx.x >> 6, l = threadIdx.x & 63u, g = l >> 4, r16 = l & 15u;
-    unsigned short* T = T_[w];
-    unsigned short* U = U_[w];
-    unsigned short* D = D_[w];
-    unsigned short* V = V_[w];
-    f32x4 dw2[4][4], dw1[4];
-    for (int a = 0; a < 4; a++) {
-        dw1[a] = f32x4{0.f, 0.f, 0.f, 0.f};
-        for (int b = 0; b < 4; b++) dw2[a][b] = f32x4{0.f, 0.f, 0.f, 0.f};
-    }
-    float gw3[16], gb2[16], gb1[16];
-    for (int k = 0; k < 16; k++) gw3[k] = gb2[k] = gb1[k] = 0.f;
-    float gb3 = 0.f, lsum = 0.f;
-    // block-uniform trip count: the loop body holds barriers
-    for (uint32_t bb = blockIdx.x * LPS_BLOCK; bb < n; bb += gridDim.x * LPS_BLOCK)
-    for (uint32_t grp = 0; grp < 4; grp++) {
-        const uint32_t s = bb + w * 64u + grp * 16u + r16;
-        const bool valid = s < n;
-        const uint32_t row = valid ? rm.row(s) : 0u;
-        Fwd F;
-        forward(S, x + (size_t)row * IN, valid, F);
-        const float tn = valid ? t[row] / m.tscale : 0.f;
-        const float d = valid ? F.y - tn : 0.f;
-        const float wd = d > 0.f ? over_weight : 1.f;  // over-predictions weigh more
-        const float dy = 2.f * wd * d * inv_n;
-        if (g == 0u) lsum += wd * d * d;
-        // output layer
-        if (g == 0u) gb3 += dy;
-        bf16x4 dy2b[4];
-        for (int mt = 0; mt < 4; mt++)
-            for (int r = 0; r < 4; r++) {
-                const int nn = mt * 16 + 4 * (int)g + r;
-                gw3[mt * 4 + r] += dy * bf2f((unsigned short)F.h2[mt][r]);
-                const float dy2 = F.y2[mt][r] > 0.f ? S.w3[nn] * dy : 0.f;
-                gb2[mt * 4 + r] += dy2;
-                dy2b[mt][r] = (short)f2bf(dy2);
-            }
-        // dH1 = W2^T dY2, dY1 = dH1 * relu'(Y1)
-        bf16x4 dy1b[4];
-        for (int mt = 0; mt < 4; mt++) {
-            f32x4 acc{0.f, 0.f, 0.f, 0.f};
-            for (int kt = 0; kt < 4; kt++)
-                acc = mfma(load4(&S.w2t[(mt * 16 + r16) * HID + kt * 16 + 4 * g]), dy2b[kt], acc);
-            for (int r = 0; r < 4; r++) {
-                const float dy1 = F.y1[mt][r] > 0.f ? acc[r] : 0.f;
-                gb1[mt * 4 + r] += dy1;
-                dy1b[mt][r] = (short)f2bf(dy1);
-            }
-        }
-        // stage [neuron][sample] tiles for the weight gradients
-        for (int mt = 0; mt < 4; mt++)
-            for (int r = 0; r < 4; r++) {
-                const int nn = mt * 16 + 4 * (int)g + r;
-                T[nn * 16 + r16] = (unsigned short)dy2b[mt][r];
-                U[nn * 16 + r16] = (unsigned short)F.h1[mt][r];
-                D[nn * 16 + r16] = (unsigned short)dy1b[mt][r];
-            }
-        for (int r = 0; r < 4; r++) V[(4 * g + r) * 16 + r16] = (unsigned short)F.x[r];
-        __syncthreads();
-        // dW2 += dY2 H1^T  (K = samples); A[o][s] = T, B[s][i] = U^T
-        for (int mt = 0; mt < 4; mt++) {
-            const bf16x4 a = load4(&T[(mt * 16 + r16) * 16 + 4 * g]);
-            for (int nt = 0; nt < 4; nt++) dw2[mt][nt] = mfma(a, load4(&U[(nt * 16 + r16) * 16 + 4 * g]), dw2[mt][nt]);
-        }
-        // dW1 += dY1 X^T; A[n][s] = D, B[s][f] = V^T
-        {
-            const bf16x4 b = load4(&V[r16 * 16 + 4 * g]);
-            for (int mt = 0; mt < 4; mt++) dw1[mt] = mfma(load4(&D[(mt * 16 + r16) * 16 + 4 * g]), b, dw1[mt]);
-        }
-        __syncthreads();
-    }
-    // reduce per-sample sums over the 16 samples of a lane group, then into LDS
-    for (int k = 0; k < 16; k++) {
-        float a = gw3[k], b = gb2[k], c = gb1[k];
-        for (int off = 1; off < 16; off <<= 1) {
-            a += __shfl_xor(a, off, 64);
-            b += __shfl_xor(b, off, 64);
-            c += __shfl_xor(c, off, 64);
-        }
-        if (r16 == 0u) {
-            const int nn = (k / 4) * 16 + 4 * (int)g + (k % 4);
-            atomicAdd(&G[OFF_W3 + nn], a);
-            atomicAdd(&G[OFF_B2 + nn], b);
-            atomicAdd(&G[OFF_B1 + nn], c);
-        }
-    }
-    for (int off = 1; off < 16; off <<= 1) gb3 += __shfl_xor(gb3, off, 64);
-    if (l == 0u) atomicAdd(&G[OFF_B3], gb3);
-    for (int off = 1; off < 64; off <<= 1) lsum += __shfl_xor(lsum, off, 64);
-    if (l == 0u) atomicAdd(&s_loss, lsum);
-    for (int mt = 0; mt < 4; mt++)
-        for (int r = 0; r < 4; r++) {
-            const int o = mt * 16 + 4 * (int)g + r;
-            for (int nt = 0; nt < 4; nt++) atomicAdd(&G[OFF_W2 + o * HID + nt * 16 + (int)r16], dw2[mt][nt][r]);
-            atomicAdd(&G[OFF_W1 + o * IN + (int)r16], dw1[mt][r]);
-        }
-    __syncthreads();
-    for (uint32_t k = threadIdx.x; k < LPS_MLP_PARAMS; k += blockDim.x)
-        if (G[k] != 0.f) atomicAdd(&grad[k], G[k]);
-    if (threadIdx.x == 0 && loss) atomicAdd(loss, s_loss * inv_n);
+// (row of sample s given by rm) with respect to the FP32 parameters: each
+// block's sums to its row of `part` (then the block's loss), which k_grad_sum
+// or k_adam adds up.  The forward uses the BF16-rounded values
+// (straight-through).
+//
+// Every product runs on the matrix cores without moving a value between lanes.
+// A 16x16 result tile leaves its rows in 4 (l/16) + r and its columns in l%16,
+// an operand its contracted index in the former and its free one in the
+// latter, so a tile serves the next product only if that contracts the tile's
+// rows.  Forward and backward contract neurons, the weight gradients samples.
+// So each layer is evaluated both ways round, with the operands swapped:
+// "P" tiles hold neurons in rows (they feed the next layer's product), "Q"
+// tiles samples in rows (they feed the weight gradients, and a bias or output
+// gradient is a sum over a lane's own four values).  32 samples at a time, so
+// that every contraction is 32 long (16 features excepted).
+//
+// Bound by the latency of its one wave per SIMD and the fetch of its straight
+// code: the weights live in registers (as fragments), the loop has no LDS
+// traffic but the biases, and the blocks' sums leave without atomics.  19 us
+// for 65,536 rows, and 4 us for the sums or Adam; with one orientation and
+// transposes through LDS (weights in rows 128 bytes apart, all in one bank) and
+// atomic sums it took 73 and 5.  The MFMA work alone is about 1 us.
+struct alignas(16) GradSmem {
+    // fp32 parameters, W2's rows padded to 68 floats (a fragment's 16 rows then
+    // lie in different banks); after the loop the waves' sums in the same layout
+    static constexpr int W2S = HID + 4;
+    struct Copy {
+        float w1[HID * IN], b1[HID], w2[HID * W2S], b2[HID], w3[HID], b3, loss;
+        float pad_[2];
+    } c[LPS_BLOCK / 64];
+};
+
+// Element k of the parameters (the loss after them) in a copy.
+__device__ __forceinline__ uint32_t grad_at(uint32_t k) {
+    if (k < OFF_W2) return k;
+    if (k < OFF_B2) return OFF_W2 + (k - OFF_W2) / HID * GradSmem::W2S + (k - OFF_W2) % HID;
+    return k + HID * (GradSmem::W2S - HID);
 }
 
-// Adam on the FP32 master parameters (bias-corrected); the gradient buffer is
-// cleared for the next batch.
-__global__ void k_adam(float* __restrict__ params, float* __restrict__ grad, float* __restrict__ m1,
-                       float* __restrict__ m2, uint32_t count, float lr, float b1, float b2, float eps, float c1,
-                       float c2) {
-    const uint32_t k = blockIdx.x * blockDim.x + threadIdx.x;
-    if (k >= count) return;
-    const float gk = grad[k];
+typedef __attribute__((ext_vector_type(8))) __bf16 bf16x8;
+
+__device__ __forceinline__ f32x4 mfma32(bf16x8 a, bf16x8 b, f32x4 c) {
+    return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0);
+}
+// two 16-long halves of a contraction (in the same order on both operands)
+__device__ __forceinline__ bf16x8 cat(bf16x4 lo, bf16x4 hi) {
+    struct { bf16x4 a, b; } v{lo, hi};
+    return __builtin_bit_cast(bf16x8, v);
+}
+__device__ __forceinline__ float relu_bf(float f) { return rbf(fmaxf(f, 0.f)); }
+
+__global__ __launch_bounds__(LPS_BLOCK) __attribute__((amdgpu_waves_per_eu(1, 1))) void k_mlp_grad(
+    MlpArgs m, const float* __restrict__ x, const float* __restrict__ t, RowMap rm, uint32_t n, float inv_n,
+    float over_weight, float* __restrict__ part) {
+    __shared__ GradSmem S;
+    const uint32_t w = threadIdx.x >> 6, l = threadIdx.x & 63u, g = l >> 4, c = l & 15u;
+    GradSmem::Copy& P = S.c[0];
+    float* copy = reinterpret_cast<float*>(&P);
+    {
+        // every load before the first store (one memory round trip)
+        constexpr uint32_t IT = (LPS_MLP_PARAMS + LPS_BLOCK - 1u) / LPS_BLOCK;
+        float v[IT];
+#pragma unroll
+        for (uint32_t q = 0; q < IT; q++) v[q] = m.params[min(threadIdx.x + q * LPS_BLOCK, (uint32_t)LPS_MLP_PARAMS - 1u)];
+#pragma unroll
+        for (uint32_t q = 0; q < IT; q++) {
+            const uint32_t k = threadIdx.x + q * LPS_BLOCK;
+            if (k < LPS_MLP_PARAMS) copy[grad_at(k)] = k >= OFF_W3 && k < OFF_B3 ? rbf(v[q]) : v[q];
+        }
+    }
+    __syncthreads();
+    // fragments: W1 and W2 by row (A of the P products, B of the Q ones), W2
+    // by column for the backward product
+    bf16x4 w1f[4];
+    bf16x8 w2f[4][2], w2t[4][2];
+    for (int a = 0; a < 4; a++) {
+        const float* q = &P.w1[(16 * a + c) * IN + 4 * g];
+        w1f[a] = f2bf4(q[0], q[1], q[2], q[3]);
+        for (int h = 0; h < 2; h++) {
+            const float* u0 = &P.w2[(16 * a + c) * GradSmem::W2S + 32 * h + 4 * g];
+            w2f[a][h] = cat(f2bf4(u0[0], u0[1], u0[2], u0[3]), f2bf4(u0[16], u0[17], u0[18], u0[19]));
+            const float* v0 = &P.w2[(32 * h + 4 * g) * GradSmem::W2S + 16 * a + c];
+            constexpr int R = GradSmem::W2S;
+            w2t[a][h] = cat(f2bf4(v0[0], v0[R], v0[2 * R], v0[3 * R]),
+                            f2bf4(v0[16 * R], v0[17 * R], v0[18 * R], v0[19 * R]));
+        }
+    }
+    const float b3 = P.b3;
+    float b1q[4], b2q[4], w3q[4];
+    for (int a = 0; a < 4; a++) {
+        b1q[a] = P.b1[16 * a + c];
+        b2q[a] = P.b2[16 * a + c];
+        w3q[a] = P.w3[16 * a + c];
+    }
+    float mean[4], istd[4];
+    for (int r = 0; r < 4; r++) {
+        mean[r] = m.fscale[4 * g + r];
+        istd[r] = m.fscale[IN + 4 * g + r];
+    }
+    const float meanq = m.fscale[c], istdq = m.fscale[IN + c];
+    const f32x4 zero{0.f, 0.f, 0.f, 0.f};
+    f32x4 dw2[4][4], dw1[4];
+    float gw3[4], gb2[4], gb1[4], gb3 = 0.f, lsum = 0.f;
+    for (int a = 0; a < 4; a++) {
+        dw1[a] = zero;
+        gw3[a] = gb2[a] = gb1[a] = 0.f;
+        for (int b = 0; b < 4; b++) dw2[a][b] = zero;
+    }
+    for (uint32_t s0 = (blockIdx.x * (LPS_BLOCK / 64) + w) * 32u; s0 < n; s0 += gridDim.x * (LPS_BLOCK / 64) * 32u) {
+        // both groups' rows first: features by quad (P) and by feature (Q)
+        float4 xin[2];
+        float xq[2][4], tn[2];
+        bool valid[2];
+        for (int u = 0; u < 2; u++) {
+            const uint32_t s = s0 + 16u * u + c;
+            valid[u] = s < n;
+            const uint32_t row = valid[u] ? rm.row(s) : 0u;
+            xin[u] = *reinterpret_cast<const float4*>(x + (size_t)row * IN + 4u * g);
+            tn[u] = t[row];
+            for (int r = 0; r < 4; r++) {
+                const uint32_t rq = (uint32_t)__shfl((int)row, 4 * (int)g + r, 64);
+                xq[u][r] = x[(size_t)rq * IN + c];
+            }
+        }
+        bf16x4 xb[2], h1q[2][4], dy2b[2][4], dy1b[2][4];
+        for (int u = 0; u < 2; u++) {
+            // samples past the end have zero features and no gradient
+            const float xi[4] = {xin[u].x, xin[u].y, xin[u].z, xin[u].w};
+            float v[4];
+            for (int r = 0; r < 4; r++) v[r] = valid[u] ? (xi[r] - mean[r]) * istd[r] : 0.f;
+            const bf16x4 xp = f2bf4(v[0], v[1], v[2], v[3]);
+            for (int r = 0; r < 4; r++) v[r] = s0 + 16u * u + 4u * g + r < n ? (xq[u][r] - meanq) * istdq : 0.f;
+            xb[u] = f2bf4(v[0], v[1], v[2], v[3]);
+            // layer 1, P and Q
+            bf16x4 h1p[4];
+            f32x4 y1q[4];
+            for (int a = 0; a < 4; a++) {
+                const f32x4 y = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(w1f[a], xp, zero, 0, 0, 0);
+                const float* b1 = &P.b1[16 * a + 4 * g];
+                h1p[a] = f2bf4(fmaxf(y[0] + b1[0], 0.f), fmaxf(y[1] + b1[1], 0.f), fmaxf(y[2] + b1[2], 0.f),
+                               fmaxf(y[3] + b1[3], 0.f));
+                y1q[a] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(xp, w1f[a], zero, 0, 0, 0);
+                for (int r = 0; r < 4; r++) y1q[a][r] += b1q[a];
+                h1q[u][a] = f2bf4(fmaxf(y1q[a][0], 0.f), fmaxf(y1q[a][1], 0.f), fmaxf(y1q[a][2], 0.f),
+                                  fmaxf(y1q[a][3], 0.f));
+            }
+            const bf16x8 h1a = cat(h1p[0], h1p[1]), h1b = cat(h1p[2], h1p[3]);
+            // layer 2 and the output, P
+            f32x4 y2p[4];
+            float y = 0.f;
+            for (int a = 0; a < 4; a++) {
+                y2p[a] = mfma32(w2f[a][1], h1b, mfma32(w2f[a][0], h1a, zero));
+                const float* b2 = &P.b2[16 * a + 4 * g];
+                const float* w3 = &P.w3[16 * a + 4 * g];
+                for (int r = 0; r < 4; r++) {
+                    y2p[a][r] += b2[r];
+                    y += w3[r] * relu_bf(y2p[a][r]);
+                }
+            }
+            y += __shfl_xor(y, 16, 64);
+            y += __shfl_xor(y, 32, 64);
+            const float d = valid[u] ? y + b3 - tn[u] / m.tscale : 0.f;
+            const float wd = d > 0.f ? over_weight : 1.f;  // over-predictions weigh more
+            const float dy = 2.f * wd * d * inv_n;
+            if (g == 0u) {
+                lsum += wd * d * d;
+                gb3 += dy;
+            }
+            float dyq[4];
+            for (int r = 0; r < 4; r++) dyq[r] = __shfl(dy, 4 * (int)g + r, 64);
+            // dY2, P
+            bf16x4 dy2p[4];
+            for (int a = 0; a < 4; a++) {
+                const float* w3 = &P.w3[16 * a + 4 * g];
+                float q[4];
+                for (int r = 0; r < 4; r++) q[r] = y2p[a][r] > 0.f ? w3[r] * dy : 0.f;
+                dy2p[a] = f2bf4(q[0], q[1], q[2], q[3]);
+            }
+            const bf16x8 da = cat(dy2p[0], dy2p[1]), db = cat(dy2p[2], dy2p[3]);
+            for (int a = 0; a < 4; a++) {
+                // layer 2 and dY2, Q
+                f32x4 y2 = mfma32(h1b, w2f[a][1], mfma32(h1a, w2f[a][0], zero));
+                float q[4];
+                for (int r = 0; r < 4; r++) {
+                    const float v2 = y2[r] + b2q[a];
+                    gw3[a] += dyq[r] * relu_bf(v2);
+                    q[r] = v2 > 0.f ? w3q[a] * dyq[r] : 0.f;
+                    gb2[a] += q[r];
+                }
+                dy2b[u][a] = f2bf4(q[0], q[1], q[2], q[3]);
+                // dY1 = (W2^T dY2) relu'(Y1), Q
+                const f32x4 e = mfma32(db, w2t[a][1], mfma32(da, w2t[a][0], zero));
+                for (int r = 0; r < 4; r++) {
+                    q[r] = y1q[a][r] > 0.f ? e[r] : 0.f;
+                    gb1[a] += q[r];
+                }
+                dy1b[u][a] = f2bf4(q[0], q[1], q[2], q[3]);
+            }
+        }
+        // weight gradients over the 32 samples
+        bf16x8 hb[4];
+        for (int a = 0; a < 4; a++) hb[a] = cat(h1q[0][a], h1q[1][a]);
+        const bf16x8 xx = cat(xb[0], xb[1]);
+        for (int a = 0; a < 4; a++) {
+            const bf16x8 d2 = cat(dy2b[0][a], dy2b[1][a]);
+            for (int b = 0; b < 4; b++) dw2[a][b] = mfma32(d2, hb[b], dw2[a][b]);
+            dw1[a] = mfma32(cat(dy1b[0][a], dy1b[1][a]), xx, dw1[a]);
+        }
+    }
+    __syncthreads();  // the parameters' copy becomes the first wave's sums
+    GradSmem::Copy& G = S.c[w];
+    for (int a = 0; a < 4; a++) {
+        for (int r = 0; r < 4; r++) {
+            const int o = 16 * a + 4 * (int)g + r;
+            for (int b = 0; b < 4; b++) G.w2[o * GradSmem::W2S + 16 * b + (int)c] = dw2[a][b][r];
+            G.w1[o * IN + (int)c] = dw1[a][r];
+        }
+        for (float* v : {&gw3[a], &gb2[a], &gb1[a]}) {
+            *v += __shfl_xor(*v, 16, 64);
+            *v += __shfl_xor(*v, 32, 64);
+        }
+        if (g == 0u) {
+            G.w3[16 * a + c] = gw3[a];
+            G.b2[16 * a + c] = gb2[a];
+            G.b1[16 * a + c] = gb1[a];
+        }
+    }
+    for (int off = 1; off < 16; off <<= 1) {
+        gb3 += __shfl_xor(gb3, off, 64);
+        lsum += __shfl_xor(lsum, off, 64);
+    }
+    if (l == 0u) {
+        G.b3 = gb3;
+        G.loss = lsum * inv_n;
+    }
+    __syncthreads();
+    float* __restrict__ out = part + (size_t)blockIdx.x * LPS_GRAD_STRIDE;
+    for (uint32_t k = threadIdx.x; k <= LPS_MLP_PARAMS; k += LPS_BLOCK) {
+        float v = 0.f;
+        for (uint32_t q = 0; q < LPS_BLOCK / 64; q++) v += reinterpret_cast<const float*>(&S.c[q])[grad_at(k)];
+        out[k] = v;
+    }
+}
+
+// Sum of element k over the blocks' rows of `part`: a workgroup takes 64
+// elements, its 16 waves every sixteenth row each.  The sum on every wave's
+// lane of the element; all 1024 threads call it.
+constexpr uint32_t LPS_SUM_WAVES = 16u;
+__device__ __forceinline__ float part_sum(const float* __restrict__ part, uint32_t nb) {
+    __shared__ float s[LPS_SUM_WAVES][64];
+    const uint32_t l = threadIdx.x & 63u, w = threadIdx.x >> 6;
+    float v = 0.f;
+#pragma unroll 8
+    for (uint32_t b = w; b < nb; b += LPS_SUM_WAVES) v += part[(size_t)b * LPS_GRAD_STRIDE + blockIdx.x * 64u + l];
+    s[w][l] = v;
+    __syncthreads();
+    v = 0.f;
+    for (uint32_t q = 0; q < LPS_SUM_WAVES; q++) v += s[q][l];
+    return v;
+}
+
+// The gradient, and the batch's loss added to loss.
+__global__ __launch_bounds__(LPS_SUM_WAVES * 64) void k_grad_sum(const float* __restrict__ part, uint32_t nb,
+                                                                 float* __restrict__ grad, float* __restrict__ loss) {
+    const uint32_t k = blockIdx.x * 64u + (threadIdx.x & 63u);
+    const float v = part_sum(part, nb);
+    if (threadIdx.x >= 64u) return;
+    if (k < LPS_MLP_PARAMS) grad[k] = v;
+    else if (k == LPS_MLP_PARAMS) *loss += v;
+}
+
+// Adam on the FP32 master parameters (bias-corrected) with the blocks' sums of
+// the batch; the batch's loss is added to loss.
+__global__ __launch_bounds__(LPS_SUM_WAVES * 64) void k_adam(float* __restrict__ params,
+                                                             const float* __restrict__ part, uint32_t nb,
+                                                             float* __restrict__ loss, float* __restrict__ m1,
+                                                             float* __restrict__ m2, float lr, float b1, float b2,
+                                                             float eps, float c1, float c2) {
+    const uint32_t k = blockIdx.x * 64u + (threadIdx.x & 63u);
+    const float gk = part_sum(part, nb);
+    if (threadIdx.x >= 64u) return;
+    if (k == LPS_MLP_PARAMS) *loss += gk;
+    if (k >= LPS_MLP_PARAMS) return;
     const float a = b1 * m1[k] + (1.f - b1) * gk;
     const float b = b2 * m2[k] + (1.f - b2) * gk * gk;
     m1[k] = a;
     m2[k] = b;
     params[k] -= lr * (a / c1) / (sqrtf(b / c2) + eps);
-    grad[k] = 0.f;
 }
 
-// Per-column sums of x and x^2 (double) over n rows of `cols` (<= 16)
-// columns, added to acc[0..cols) and acc[cols..2 cols).
-__global__ __launch_bounds__(LPS_BLOCK) void k_feature_stats(const float* __restrict__ x, uint64_t n, uint32_t cols,
+// Per-column sums of x and x^2 (double) over n rows of IN columns, added to
+// acc[0..IN) and acc[IN..2 IN).  A lane takes four columns of a row (one
+// 16-byte load), so a wave reads 16 whole rows; lanes of the same columns are
+// added across the wave, waves in LDS.
+__global__ __launch_bounds__(LPS_BLOCK) void k_feature_stats(const float* __restrict__ x, uint64_t n,
                                                              double* __restrict__ acc) {
-    __shared__ double s[2 * IN];
-    if (threadIdx.x < 2 * IN) s[threadIdx.x] = 0.0;
-    __syncthreads();
-    double a[IN], b[IN];
-    for (int f = 0; f < IN; f++) a[f] = b[f] = 0.0;
-    for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (uint64_t)gridDim.x * blockDim.x)
-        for (int f = 0; f < IN; f++)
-            if ((uint32_t)f < cols) {
-                const double v = x[i * cols + f];
-                a[f] += v;
-                b[f] += v * v;
-            }
-    for (int f = 0; f < IN; f++)
-        if ((uint32_t)f < cols) {
-            atomicAdd(&s[f], a[f]);
-            atomicAdd(&s[IN + f], b[f]);
+    __shared__ double s[LPS_BLOCK / 64][2 * IN];
+    static_assert(IN == 16, "four lanes per row");
+    const uint32_t q = threadIdx.x & 3u, l = threadIdx.x & 63u;
+    double a[4] = {0.0, 0.0, 0.0, 0.0}, b[4] = {0.0, 0.0, 0.0, 0.0};
+    const uint64_t step = (uint64_t)gridDim.x * (LPS_BLOCK / 4);
+#pragma unroll 4
+    for (uint64_t i = (uint64_t)blockIdx.x * (LPS_BLOCK / 4) + threadIdx.x / 4u; i < n; i += step) {
+        const float4 v = reinterpret_cast<const float4*>(x)[i * 4u + q];
+        const double d[4] = {v.x, v.y, v.z, v.w};
+        for (int f = 0; f < 4; f++) {
+            a[f] += d[f];
+            b[f] += d[f] * d[f];
+        }
+    }
+    for (int f = 0; f < 4; f++)
+        for (int off = 4; off < 64; off <<= 1) {
+            a[f] += __shfl_xor(a[f], off, 64);
+            b[f] += __shfl_xor(b[f], off, 64);
+        }
+    if (l < 4u)
+        for (int f = 0; f < 4; f++) {
+            s[threadIdx.x >> 6][4u * q + f] = a[f];
+            s[threadIdx.x >> 6][IN + 4u * q + f] = b[f];
         }
     __syncthreads();
-    if (threadIdx.x < cols) {
-        atomicAdd(&acc[threadIdx.x], s[threadIdx.x]);
-        atomicAdd(&acc[cols + threadIdx.x], s[IN + threadIdx.x]);
+    if (threadIdx.x < 2 * IN) {
+        double v = 0.0;
+        for (int w = 0; w < LPS_BLOCK / 64; w++) v += s[w][threadIdx.x];
+        atomicAdd(&acc[threadIdx.x], v);
+    }
+}
+
+// Sums of t and t^2 (double) over n values, added to acc[0] and acc[1].
+__global__ __launch_bounds__(LPS_BLOCK) void k_target_stats(const float* __restrict__ t, uint64_t n,
+                                                            double* __restrict__ acc) {
+    __shared__ double s[LPS_BLOCK / 64][2];
+    double a = 0.0, b = 0.0;
+#pragma unroll 4
+    for (uint64_t i = (uint64_t)blockIdx.x * LPS_BLOCK + threadIdx.x; i < n; i += (uint64_t)gridDim.x * LPS_BLOCK) {
+        const double v = t[i];
+        a += v;
+        b += v * v;
+    }
+    for (int off = 1; off < 64; off <<= 1) {
+        a += __shfl_xor(a, off, 64);
+        b += __shfl_xor(b, off, 64);
+    }
+    if ((threadIdx.x & 63u) == 0u) {
+        s[threadIdx.x >> 6][0] = a;
+        s[threadIdx.x >> 6][1] = b;
+    }
+    __syncthreads();
+    if (threadIdx.x < 2u) {
+        double v = 0.0;
+        for (int w = 0; w < LPS_BLOCK / 64; w++) v += s[w][threadIdx.x];
+        atomicAdd(&acc[threadIdx.x], v);
     }
 }
 
@@ -561,19 +678,38 @@ void launch_mlp_forward(hipStream_t s, const void* packed, const float* x, uint3
     k_mlp_forward<<<mlp_grid(n), LPS_BLOCK, 0, s>>>(static_cast<const MlpPacked*>(packed), x, n, y);
 }
 
+namespace {
+// blocks of k_mlp_grad: 128 samples each (two rounds of 32 per wave for 65,536
+// rows), one per CU at most
+uint32_t grad_blocks(uint32_t n) {
+    const uint32_t nb = n / 128u + (n % 128u ? 1u : 0u);
+    return nb < LPS_GRAD_BLOCKS ? nb : LPS_GRAD_BLOCKS;
+}
+}  // namespace
+
 void launch_mlp_grad(hipStream_t s, const MlpArgs& m, const float* x, const float* t, const RowMap& rm, uint32_t n,
-                     float over_weight, float* grad, float* loss) {
-    k_mlp_grad<<<mlp_grid(n), LPS_BLOCK, 0, s>>>(m, x, t, rm, n, 1.f / (float)n, over_weight, grad, loss);
+                     float over_weight, float* part, float* grad, float* loss) {
+    const uint32_t nb = grad_blocks(n);
+    k_mlp_grad<<<nb, LPS_BLOCK, 0, s>>>(m, x, t, rm, n, 1.f / (float)n, over_weight, part);
+    k_grad_sum<<<LPS_GRAD_STRIDE / 64, LPS_SUM_WAVES * 64, 0, s>>>(part, nb, grad, loss);
 }
 
-void launch_adam(hipStream_t s, float* params, float* grad, float* m1, float* m2, uint32_t count, float lr, float b1,
-                 float b2, float eps, uint32_t step) {
+void launch_train_step(hipStream_t s, const MlpArgs& m, const float* x, const float* t, const RowMap& rm, uint32_t n,
+                       float over_weight, float* part, float* loss, float* params, float* m1, float* m2, float lr,
+                       float b1, float b2, float eps, uint32_t step) {
+    const uint32_t nb = grad_blocks(n);
     const float c1 = 1.f - powf(b1, (float)step), c2 = 1.f - powf(b2, (float)step);
-    k_adam<<<(count + 255u) / 256u, 256, 0, s>>>(params, grad, m1, m2, count, lr, b1, b2, eps, c1, c2);
+    k_mlp_grad<<<nb, LPS_BLOCK, 0, s>>>(m, x, t, rm, n, 1.f / (float)n, over_weight, part);
+    k_adam<<<LPS_GRAD_STRIDE / 64, LPS_SUM_WAVES * 64, 0, s>>>(params, part, nb, loss, m1, m2, lr, b1, b2, eps, c1,
+                                                              c2);
 }
 
-void launch_feature_stats(hipStream_t s, const float* x, uint64_t n, uint32_t cols, double* acc) {
-    k_feature_stats<<<256, LPS_BLOCK, 0, s>>>(x, n, cols, acc);
+void launch_feature_stats(hipStream_t s, const float* x, uint64_t n, double* acc) {
+    k_feature_stats<<<512, LPS_BLOCK, 0, s>>>(x, n, acc);
+}
+
+void launch_target_stats(hipStream_t s, const float* t, uint64_t n, double* acc) {
+    k_target_stats<<<256, LPS_BLOCK, 0, s>>>(t, n, acc);
 }
 
 void launch_collect(hipStream_t s, const float* feat, uint32_t fs, const float* press, float pscale, uint32_t n,
