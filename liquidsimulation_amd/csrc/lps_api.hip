@@ -538,21 +538,27 @@ lps_dev::PhysArgs phys_args(lps_ctx* c, const SimConst& k) {
 void enqueue_grid(lps_ctx* c) {
     const hipStream_t s = c->stream;
     const uint32_t n = c->n;
-    {
+    if (scenes(c).count == 1u && n <= LPS_SORT_BLOCKS * LPS_BLOCK) {
         Timed t(c, "grid_setup");
-        lps_dev::launch_grid_setup(s, c->grid, scenes(c), c->bbox_part, c->der.h, c->cell_cap, c->h_energy);
-    }
-    {
-        Timed t(c, "keys");
-        lps_dev::launch_keys(s, c->pos[c->cur], n, c->grid, scenes(c), c->keys, c->rank, c->cell_count);
-    }
-    {
-        Timed t(c, "cell_table");
-        lps_dev::launch_cell_table(s, c->cell_count, c->grid, c->tile_sum, c->cell_lb, c->cell_cap);
-    }
-    {
-        Timed t(c, "place");
-        lps_dev::launch_place(s, c->keys, c->rank, n, c->grid, c->cell_lb, c->placed);
+        lps_dev::launch_sort_one(s, c->grid, scenes(c), c->bbox_part, c->der.h, c->cell_cap, c->h_energy,
+                                 c->pos[c->cur], n, c->cell_count, c->cell_lb, c->placed);
+    } else {
+        {
+            Timed t(c, "grid_setup");
+            lps_dev::launch_grid_setup(s, c->grid, scenes(c), c->bbox_part, c->der.h, c->cell_cap, c->h_energy);
+        }
+        {
+            Timed t(c, "keys");
+            lps_dev::launch_keys(s, c->pos[c->cur], n, c->grid, scenes(c), c->keys, c->rank, c->cell_count);
+        }
+        {
+            Timed t(c, "cell_table");
+            lps_dev::launch_cell_table(s, c->cell_count, c->grid, c->tile_sum, c->cell_lb, c->cell_cap);
+        }
+        {
+            Timed t(c, "place");
+            lps_dev::launch_place(s, c->keys, c->rank, n, c->grid, c->cell_lb, c->placed);
+        }
     }
     {
         Timed t(c, "reorder");

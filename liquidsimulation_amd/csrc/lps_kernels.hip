@@ -951,22 +951,53 @@ __global__ __launch_bounds__(LPS_BLOCK) void k_scene_energy(lps_dev::Scenes S, c
     scene_energy_block(S, part, blockIdx.x, out);
 }
 
-// Grid parameters of each scene (SPHSolver.cpp:1031-1040), one block per
-// scene over the partial boxes of its particle blocks.  min starts at FLT_MAX
-// and max at FLT_MIN as in the reference (SPHSolver.cpp:1013-1014).
-__device__ __forceinline__ void scene_grid_block(const lps_dev::Scenes& S, const uint32_t* __restrict__ part,
-                                                 float h, uint32_t sidx, double* __restrict__ energy) {
+// Grid of a scene (SPHSolver.cpp:1031-1040) from the reduced words of its
+// blocks' records, to *sg and to the caller.
+struct SceneBox {
+    float off[3];
+    uint32_t gsize[3], cells, bad;
+};
+__device__ __forceinline__ SceneBox scene_box(SceneGrid* sg, const uint32_t (&r)[7], float h) {
+    SceneBox b;
+    b.bad = r[6] ? 1u : 0u;
+    const float gs = h * 1.f;
+    uint64_t cells = 1;
+    for (int a = 0; a < 3; a++) {
+        const float mn = o2f(r[a]), mx = o2f(r[3 + a]);
+        sg->bbox_min[a] = mn;
+        sg->bbox_max[a] = mx;
+        sg->offset[a] = b.off[a] = -mn;
+        const float ex = (mx - mn) / gs;
+        if (!(ex < 2.0e9f)) {
+            b.bad = b.bad ? b.bad : 2u;
+            b.gsize[a] = 1u;
+        } else {
+            b.gsize[a] = (uint32_t)((int)ex + 1);
+        }
+        sg->gsize[a] = b.gsize[a];
+        cells *= b.gsize[a];
+    }
+    if (cells >= 0x7FFFFFFFull) b.bad = b.bad ? b.bad : 2u;
+    sg->cells = b.cells = b.bad ? 1u : (uint32_t)cells;
+    sg->bad = b.bad;
+    return b;
+}
+
+// The records' identity: min starts at FLT_MAX and max at FLT_MIN as in the
+// reference (SPHSolver.cpp:1013-1014).
+__device__ __forceinline__ uint32_t box_start(int a) { return a < 3 ? f2o(FLT_MAX) : a < 6 ? f2o(FLT_MIN) : 0u; }
+
+// Grid of each scene, one block per scene over the partial boxes of its
+// particle blocks; thread 0 returns it.
+__device__ __forceinline__ SceneBox scene_grid_block(const lps_dev::Scenes& S, const uint32_t* __restrict__ part,
+                                                     float h, uint32_t sidx, double* __restrict__ energy) {
     // the energy of the state entering this step, for the host
     if (energy) scene_energy_block(S, part, sidx, energy);
     __shared__ uint32_t s_r[7][LPS_BLOCK / 64];
     const SceneInfo si = S.info[sidx];
     const uint32_t nparts = si.padded / LPS_BLOCK;
     uint32_t r[7];
-    for (int a = 0; a < 3; a++) {
-        r[a] = f2o(FLT_MAX);
-        r[3 + a] = f2o(FLT_MIN);
-    }
-    r[6] = 0u;
+    for (int a = 0; a < 7; a++) r[a] = box_start(a);
 #pragma unroll 8
     for (uint32_t k = threadIdx.x; k < nparts; k += LPS_BLOCK) {
         const uint32_t* q = part + (si.block0 + k) * LPS_BBOX_PART;
@@ -980,32 +1011,12 @@ __device__ __forceinline__ void scene_grid_block(const lps_dev::Scenes& S, const
     if (lane_id() == 0)
         for (int a = 0; a < 7; a++) s_r[a][threadIdx.x >> 6] = r[a];
     __syncthreads();
-    if (threadIdx.x != 0) return;
+    SceneBox b{};
+    if (threadIdx.x != 0) return b;
     for (int a = 0; a < 7; a++)
         for (uint32_t k = 1; k < LPS_BLOCK / 64; k++) r[a] = (a < 3) ? min(r[a], s_r[a][k]) : max(r[a], s_r[a][k]);
-    SceneGrid* sg = S.grid + sidx;  // written by thread 0 only
-    uint32_t bad = r[6] ? 1u : 0u;
-    float mn[3], mx[3];
-    const float gs = h * 1.f;
-    uint64_t cells = 1;
-    for (int a = 0; a < 3; a++) {
-        mn[a] = o2f(r[a]);
-        mx[a] = o2f(r[3 + a]);
-        sg->bbox_min[a] = mn[a];
-        sg->bbox_max[a] = mx[a];
-        sg->offset[a] = -mn[a];
-        const float ex = (mx[a] - mn[a]) / gs;
-        if (!(ex < 2.0e9f)) {
-            bad = bad ? bad : 2u;
-            sg->gsize[a] = 1u;
-        } else {
-            sg->gsize[a] = (uint32_t)((int)ex + 1);
-        }
-        cells *= sg->gsize[a];
-    }
-    if (cells >= 0x7FFFFFFFull) bad = bad ? bad : 2u;
-    sg->cells = bad ? 1u : (uint32_t)cells;
-    sg->bad = bad;
+    b = scene_box(S.grid + sidx, r, h);
+    return b;
 }
 
 __global__ __launch_bounds__(LPS_BLOCK) void k_scene_grid(lps_dev::Scenes S, const uint32_t* __restrict__ part,
@@ -1013,36 +1024,23 @@ __global__ __launch_bounds__(LPS_BLOCK) void k_scene_grid(lps_dev::Scenes S, con
     scene_grid_block(S, part, h, blockIdx.x, energy);
 }
 
-// Cell numbering across scenes (scene s owns cells [cell_base, cell_base +
-// cells] including its empty-slot cell), capacity check, and the per-step
-// reset of the loop state.  Thread 0 reads every scene's grid.
-__device__ __forceinline__ void grid_finish_block(DevGrid* g, const lps_dev::Scenes& S, float h,
-                                                  uint32_t cell_cap) {
-    const uint32_t t = threadIdx.x;
-    for (uint32_t b = t; b < S.nblocks; b += LPS_BLOCK) S.act_list[b] = b;
-    for (uint32_t sidx = t; sidx < S.count; sidx += LPS_BLOCK) {
-        SceneGrid* sg = S.grid + sidx;
-        sg->stop_iter = 0u;
-        sg->best_bits = 0u;
-        sg->best_k = 0u;
-        sg->best_buf = 0u;
-        sg->stall = 0u;
-        sg->converged = 0u;
-        sg->final_bits = 0u;
-        sg->final_buf = 0u;
-        sg->buf_of[1] = 0u;
-    }
-    for (uint32_t e = t; e < S.count * 2u * LPS_ERR_SUBS; e += LPS_BLOCK) S.err[e * LPS_ERR_STRIDE] = 0u;
-    if (t != 0) return;
-    uint32_t status = 0u;
-    uint64_t total = 0;
-    for (uint32_t sidx = 0; sidx < S.count; sidx++) {
-        SceneGrid* sg = S.grid + sidx;
-        if (sg->bad == 1u) status = LPS_ERR_NONFINITE;
-        if (sg->bad == 2u && !status) status = LPS_ERR_GRID_OVERFLOW;
-        sg->cell_base = (uint32_t)min(total, (uint64_t)0xFFFFFFFFull);
-        total += (uint64_t)sg->cells + 1u;
-    }
+// The per-step reset of the loop state of a scene.
+__device__ __forceinline__ void reset_loop(SceneGrid* sg) {
+    sg->stop_iter = 0u;
+    sg->best_bits = 0u;
+    sg->best_k = 0u;
+    sg->best_buf = 0u;
+    sg->stall = 0u;
+    sg->converged = 0u;
+    sg->final_bits = 0u;
+    sg->final_buf = 0u;
+    sg->buf_of[1] = 0u;
+}
+
+// The step's global state, for `total` cells (with every scene's empty-slot
+// cell); returns the step's status.
+__device__ __forceinline__ uint32_t start_step(DevGrid* g, const lps_dev::Scenes& S, float h, uint32_t status,
+                                               uint64_t total, uint32_t cell_cap) {
     g->spacing = h * 1.f;
     g->cells_needed = total > 0xFFFFFFFFull ? 0xFFFFFFFFu : (uint32_t)total;
     if (!status && total > (uint64_t)cell_cap) status = LPS_ERR_GRID_OVERFLOW;
@@ -1058,21 +1056,59 @@ __device__ __forceinline__ void grid_finish_block(DevGrid* g, const lps_dev::Sce
     g->act_count[1] = 0u;
     g->list_of[1] = 0u;
     if (!status) g->steps_ok += 1u;
+    return status;
 }
 
+__device__ __forceinline__ uint32_t box_status(bool nonfinite, bool too_large) {
+    return nonfinite ? LPS_ERR_NONFINITE : too_large ? LPS_ERR_GRID_OVERFLOW : 0u;
+}
+
+// Cell numbering across scenes (scene s owns cells [cell_base, cell_base +
+// cells] including its empty-slot cell), capacity check, and the per-step
+// reset of the loop state: a thread per scene and one scan over them.  One
+// thread that walked the scenes took 21 us for 64 of them (a memory round trip
+// each) where this takes 5.
 __global__ __launch_bounds__(LPS_BLOCK) void k_grid_finish(DevGrid* g, lps_dev::Scenes S, float h,
                                                            uint32_t cell_cap) {
-    grid_finish_block(g, S, h, cell_cap);
+    static_assert(LPS_MAX_SCENES <= LPS_BLOCK, "a thread per scene");
+    __shared__ unsigned long long s_sum[LPS_BLOCK / 64];
+    const uint32_t t = threadIdx.x, w = t >> 6;
+    SceneGrid* sg = S.grid + t;
+    const bool own = t < S.count;
+    const uint32_t bad = own ? sg->bad : 0u;
+    const unsigned long long cells = own ? (unsigned long long)sg->cells + 1u : 0u;
+    for (uint32_t b = t; b < S.nblocks; b += LPS_BLOCK) S.act_list[b] = b;
+    for (uint32_t e = t; e < S.count * 2u * LPS_ERR_SUBS; e += LPS_BLOCK) S.err[e * LPS_ERR_STRIDE] = 0u;
+    if (own) reset_loop(sg);
+    unsigned long long upto = cells;
+    for (uint32_t off = 1; off < 64u; off <<= 1) {
+        const unsigned long long y = __shfl_up(upto, off, 64);
+        if (lane_id() >= off) upto += y;
+    }
+    if (lane_id() == 63u) s_sum[w] = upto;
+    const uint32_t status = box_status(__syncthreads_or(bad == 1u), __syncthreads_or(bad == 2u));
+    unsigned long long total = 0u;
+    for (uint32_t k = 0; k < LPS_BLOCK / 64; k++) {
+        if (k < w) upto += s_sum[k];
+        total += s_sum[k];
+    }
+    if (own) sg->cell_base = (uint32_t)min(upto - cells, 0xFFFFFFFFull);
+    if (t == 0u) start_step(g, S, h, status, total, cell_cap);
 }
 
-// Both of the above for a single scene, in one block: thread 0 writes the
-// scene's grid and then reads it (one launch less per step).
+// Both of the above for a single scene, in one block (one launch less per
+// step).
 __global__ __launch_bounds__(LPS_BLOCK) void k_grid_one(DevGrid* g, lps_dev::Scenes S,
                                                         const uint32_t* __restrict__ part, float h,
                                                         uint32_t cell_cap, double* __restrict__ energy) {
-    scene_grid_block(S, part, h, 0u, energy);
-    __syncthreads();
-    grid_finish_block(g, S, h, cell_cap);
+    const uint32_t t = threadIdx.x;
+    for (uint32_t b = t; b < S.nblocks; b += LPS_BLOCK) S.act_list[b] = b;
+    if (t < 2u * LPS_ERR_SUBS) S.err[t * LPS_ERR_STRIDE] = 0u;
+    const SceneBox b = scene_grid_block(S, part, h, 0u, energy);
+    if (t != 0u) return;
+    reset_loop(S.grid);
+    S.grid->cell_base = 0u;
+    start_step(g, S, h, box_status(b.bad == 1u, b.bad == 2u), (uint64_t)b.cells + 1u, cell_cap);
 }
 
 // ---- sort by cell: a counting sort
@@ -1097,8 +1133,43 @@ __global__ __launch_bounds__(LPS_BLOCK) void k_grid_one(DevGrid* g, lps_dev::Sce
 // Its cost grows with the square of a cell's particles in k_reorder, as every
 // stencil pass's does.
 
-// Cell keys (calcGridIndices, SPHKernels.cl:66-82) within the scene's grid,
-// offset by the scene's first cell; empty slots get the scene's empty-slot
+// A particle's cell (calcGridIndices, SPHKernels.cl:66-82).
+__device__ __forceinline__ uint32_t cell_key(const GridView& G, const float4& p) {
+    const uint32_t xg = (uint32_t)truncf((p.x + G.off0) / G.gs);
+    const uint32_t yg = (uint32_t)truncf((p.y + G.off1) / G.gs);
+    const uint32_t zg = (uint32_t)truncf((p.z + G.off2) / G.gs);
+    return G.base + xg + (uint32_t)G.gx * yg + G.gxy * zg;
+}
+
+// The same with y = RN(1 / gs) for a cell size in [2^-78, 2^40): the quotients
+// are the IEEE ones for numerators of at least 2^-80, and below one for
+// smaller ones either way (no numerator is negative).
+__device__ __forceinline__ uint32_t cell_key_quick(const GridView& G, const float4& p, float y) {
+    const uint32_t xg = cvt_u32_sat(lps_div::div_rn(p.x + G.off0, G.gs, y));
+    const uint32_t yg = cvt_u32_sat(lps_div::div_rn(p.y + G.off1, G.gs, y));
+    const uint32_t zg = cvt_u32_sat(lps_div::div_rn(p.z + G.off2, G.gs, y));
+    return G.base + xg + (uint32_t)G.gx * yg + G.gxy * zg;
+}
+
+// Counts a wave's keys and returns each one's place of arrival in its cell.
+// The particles are in the last step's sorted order, so most of a cell's lie
+// in consecutive lanes: the first lane of a run of equal keys counts the whole
+// run.
+__device__ __forceinline__ uint32_t count_key(uint32_t* count, uint32_t key, uint32_t lane) {
+    const uint32_t before = (uint32_t)__shfl_up((int)key, 1, 64);
+    const uint64_t heads = __ballot(lane == 0u || key != before);
+    const uint64_t upto = ~0ull >> (63u - lane);
+    const uint32_t head = 63u - (uint32_t)__clzll((long long)(heads & upto));
+    uint32_t base = 0u;
+    if (lane == head) {
+        const uint64_t later = heads & ~upto;
+        const uint32_t end = later ? (uint32_t)__ffsll((long long)later) - 1u : 64u;
+        base = atomicAdd(&count[key], end - lane);
+    }
+    return (uint32_t)__shfl((int)base, (int)head, 64) + lane - head;
+}
+
+// Keys within the scene's grid, offset by the scene's first cell; empty slots get the scene's empty-slot
 // cell so they follow its particles.  run[i] is the place of arrival in the
 // cell, count[cell] the counts.
 __global__ __launch_bounds__(LPS_BLOCK) void k_keys(const float4* __restrict__ pos, const DevGrid* g,
@@ -1110,28 +1181,9 @@ __global__ __launch_bounds__(LPS_BLOCK) void k_keys(const float4* __restrict__ p
     const BlockScene B = block_scene(S, lb);
     const SceneGrid* sg = S.grid + B.s;
     const GridView G = grid_view(g, sg);
-    uint32_t key = G.base + sg->cells;
-    if (i < B.info.slot0 + B.info.count) {
-        const uint32_t xg = (uint32_t)truncf((p.x + G.off0) / G.gs);
-        const uint32_t yg = (uint32_t)truncf((p.y + G.off1) / G.gs);
-        const uint32_t zg = (uint32_t)truncf((p.z + G.off2) / G.gs);
-        key = G.base + xg + (uint32_t)G.gx * yg + G.gxy * zg;
-    }
+    const uint32_t key = i < B.info.slot0 + B.info.count ? cell_key(G, p) : G.base + sg->cells;
     keys[i] = key;
-    // the particles are in the last step's sorted order, so most of a cell's
-    // lie in consecutive lanes: the first lane of a run of equal keys counts
-    // the whole run
-    const uint32_t before = (uint32_t)__shfl_up((int)key, 1, 64);
-    const uint64_t heads = __ballot(lane == 0u || key != before);
-    const uint64_t upto = ~0ull >> (63u - lane);
-    const uint32_t head = 63u - (uint32_t)__clzll((long long)(heads & upto));
-    uint32_t base = 0u;
-    if (lane == head) {
-        const uint64_t later = heads & ~upto;
-        const uint32_t end = later ? (uint32_t)__ffsll((long long)later) - 1u : 64u;
-        base = atomicAdd(&count[key], end - lane);
-    }
-    rank[i] = (uint32_t)__shfl((int)base, (int)head, 64) + lane - head;
+    rank[i] = count_key(count, key, lane);
 }
 
 // Particles of each tile of LPS_SCAN_TILE cells.
@@ -1217,6 +1269,180 @@ __global__ __launch_bounds__(LPS_BLOCK) void k_place(const uint32_t* __restrict_
     const uint32_t key = keys[i], r = rank[i];
     if (step_dead(g)) return;
     placed[cell_lb[key] + r] = make_uint2(i, key);
+}
+
+// Everything above for a single scene of up to LPS_SORT_BLOCKS particle blocks,
+// in one workgroup: grid, keys, cell table and placement need only its own
+// barriers between them instead of a launch each, which is what such a scene's
+// step waits for (each of the five kernels is a chain of two or three memory
+// round trips).  The cells are counted and summed in LDS, or in the global
+// counts (zero between steps) when the grid has more of them than fit.
+// Per step, five launches -> one: 11.8 -> 4.4 us of kernels at 512 particles,
+// 13.0 -> 5.6 at 1,080, 14.2 -> 11.2 at 16,128, beside the four launches.  One
+// compute unit then does all of its arithmetic (with IEEE divisions and the
+// runs of k_keys the last figure was 16.6); more blocks would not fit its
+// registers, which hold the positions and keys of 16 particles a thread.
+constexpr uint32_t SORT_WG = 1024u, SORT_WAVES = SORT_WG / 64u, SORT_CELLS = 32768u;
+constexpr uint32_t SORT_ITEMS = LPS_SORT_BLOCKS * LPS_BLOCK / SORT_WG;
+
+__device__ __forceinline__ uint32_t wave_scan_u32(uint32_t v) {
+    const uint32_t lane = lane_id();
+    for (uint32_t off = 1; off < 64u; off <<= 1) {
+        const uint32_t y = (uint32_t)__shfl_up((int)v, (int)off, 64);
+        if (lane >= off) v += y;
+    }
+    return v;
+}
+
+// count: `entries` counters, zero up to whole multiples of 256 per wave where
+// IN_LDS (the counts turn into the table there); global counts are cleared.
+template <bool IN_LDS>
+__device__ __forceinline__ void sort_cells(uint32_t* count, uint32_t entries, const GridView& G, uint32_t empty_cell,
+                                           uint32_t particles, uint32_t n, const float4 (&p)[SORT_ITEMS],
+                                           uint32_t* s_wave, uint32_t* __restrict__ cell_lb,
+                                           uint2* __restrict__ placed) {
+    const uint32_t t = threadIdx.x, lane = lane_id(), w = t >> 6;
+    uint32_t key[SORT_ITEMS], rank[SORT_ITEMS];
+    const bool quick = G.gs >= 0x1p-78f && G.gs < 0x1p40f;
+    const float y = lps_div::rcp_rn(G.gs);
+#pragma unroll
+    for (uint32_t k = 0; k < SORT_ITEMS; k++) {
+        const uint32_t i = k * SORT_WG + t;
+        if (k * SORT_WG >= n) break;
+        if (i >= n) continue;  // whole waves: n is whole blocks
+        const uint32_t cell = quick ? cell_key_quick(G, p[k], y) : cell_key(G, p[k]);
+        key[k] = i < particles ? cell : empty_cell;
+        rank[k] = IN_LDS ? atomicAdd(&count[key[k]], 1u) : count_key(count, key[k], lane);
+    }
+    if (!IN_LDS) __threadfence();
+    __syncthreads();
+    // each wave sums its stretch of cells, then turns it into table entries
+    const uint32_t stretch = (entries + SORT_WAVES * 256u - 1u) / (SORT_WAVES * 256u) * 256u;
+    const uint32_t c0 = w * stretch + lane * 4u, c1 = min((w + 1u) * stretch, entries);
+    auto cells4 = [&](uint32_t c) {
+        if constexpr (IN_LDS) {
+            return *reinterpret_cast<const uint4*>(count + c);
+        } else {
+            uint4 v = make_uint4(0u, 0u, 0u, 0u);
+            if (c < entries) v.x = count[c];
+            if (c + 1u < entries) v.y = count[c + 1u];
+            if (c + 2u < entries) v.z = count[c + 2u];
+            if (c + 3u < entries) v.w = count[c + 3u];
+            return v;
+        }
+    };
+    uint32_t sum = 0u;
+    for (uint32_t c = c0; c < c1; c += 256u) {
+        const uint4 v = cells4(c);
+        sum += v.x + v.y + v.z + v.w;
+    }
+    for (int off = 32; off > 0; off >>= 1) sum += (uint32_t)__shfl_xor((int)sum, off, 64);
+    if (lane == 0u) s_wave[w] = sum;
+    __syncthreads();
+    uint32_t run = 0u;
+    for (uint32_t k = 0; k < w; k++) run += s_wave[k];
+    for (uint32_t cw = w * stretch; cw < c1; cw += 256u) {  // the wave in step
+        const uint32_t c = cw + lane * 4u;
+        const uint4 v = c < c1 ? cells4(c) : make_uint4(0u, 0u, 0u, 0u);
+        const uint32_t own = v.x + v.y + v.z + v.w, upto = wave_scan_u32(own);
+        const uint32_t a = run + upto - own;
+        const uint4 lb = make_uint4(a, a + v.x, a + v.x + v.y, a + v.x + v.y + v.z);
+        run += (uint32_t)__builtin_amdgcn_readlane((int)upto, 63);
+        if (c + 3u < entries) {
+            *reinterpret_cast<uint4*>(cell_lb + c) = lb;
+        } else if (c < entries) {
+            cell_lb[c] = lb.x;
+            if (c + 1u < entries) cell_lb[c + 1u] = lb.y;
+            if (c + 2u < entries) cell_lb[c + 2u] = lb.z;
+        }
+        if constexpr (IN_LDS) {
+            if (c < c1) *reinterpret_cast<uint4*>(count + c) = lb;
+        } else if (c < entries) {
+            if (v.x) count[c] = 0u;
+            if (v.y) count[c + 1u] = 0u;
+            if (v.z) count[c + 2u] = 0u;
+            if (v.w) count[c + 3u] = 0u;
+        }
+    }
+    if (!IN_LDS) __threadfence();
+    __syncthreads();
+    const uint32_t* table = IN_LDS ? count : cell_lb;
+#pragma unroll
+    for (uint32_t k = 0; k < SORT_ITEMS; k++) {
+        const uint32_t i = k * SORT_WG + t;
+        if (k * SORT_WG >= n) break;
+        if (i < n) placed[table[key[k]] + rank[k]] = make_uint2(i, key[k]);
+    }
+}
+
+__global__ __launch_bounds__(SORT_WG) void k_sort_one(DevGrid* g, lps_dev::Scenes S,
+                                                      const uint32_t* __restrict__ part, float h, uint32_t cell_cap,
+                                                      double* __restrict__ energy, const float4* __restrict__ pos,
+                                                      uint32_t* count, uint32_t* cell_lb,
+                                                      uint2* __restrict__ placed, uint32_t n) {
+    static_assert(LPS_SORT_BLOCKS <= 64u, "a lane per record");
+    __shared__ __attribute__((aligned(16))) uint32_t s_cell[SORT_CELLS];
+    __shared__ uint32_t s_wave[SORT_WAVES];
+    __shared__ SceneBox s_box;
+    __shared__ uint32_t s_status;
+    const uint32_t t = threadIdx.x, lane = lane_id(), w = t >> 6;
+    // the positions load while the grid is formed
+    float4 p[SORT_ITEMS];
+#pragma unroll
+    for (uint32_t k = 0; k < SORT_ITEMS; k++) {
+        if (k * SORT_WG >= n) break;
+        p[k] = pos[min(k * SORT_WG + t, n - 1u)];
+    }
+    if (w == 0u) {
+        uint32_t r[7];
+        for (int a = 0; a < 7; a++) r[a] = lane < S.nblocks ? part[lane * LPS_BBOX_PART + a] : box_start(a);
+        for (int a = 0; a < 7; a++)
+            r[a] = a < 3 ? min(wave_min_u32(r[a]), box_start(a)) : max(wave_max_u32(r[a]), box_start(a));
+        if (lane == 0u) {
+            s_box = scene_box(S.grid, r, h);
+            S.grid->cell_base = 0u;
+            s_status = start_step(g, S, h, box_status(s_box.bad == 1u, s_box.bad == 2u), (uint64_t)s_box.cells + 1u,
+                                  cell_cap);
+        }
+    } else if (w == 1u) {
+        // the energy of the state entering this step, for the host
+        if (energy) {
+            const uint32_t* q = part + min(lane, S.nblocks - 1u) * LPS_BBOX_PART;
+            const double ke = wave_sum_f64(lane < S.nblocks ? (double)__uint_as_float(q[7]) : 0.0);
+            const double pe = wave_sum_f64(lane < S.nblocks ? (double)__uint_as_float(q[8]) : 0.0);
+            if (lane == 0u) {
+                energy[0] = ke;
+                energy[1] = pe;
+            }
+        }
+    } else if (w == 2u) {
+        if (lane < S.nblocks) S.act_list[lane] = lane;
+        if (lane < 2u * LPS_ERR_SUBS) S.err[lane * LPS_ERR_STRIDE] = 0u;
+        if (lane == 0u) reset_loop(S.grid);
+    }
+    reinterpret_cast<uint4*>(s_cell)[t] = make_uint4(0u, 0u, 0u, 0u);  // cells 0 .. 4095
+    __syncthreads();
+    if (s_status != 0u) return;
+    GridView G;
+    G.off0 = s_box.off[0];
+    G.off1 = s_box.off[1];
+    G.off2 = s_box.off[2];
+    G.gs = h * 1.f;
+    G.gx = (int)s_box.gsize[0];
+    G.gy = (int)s_box.gsize[1];
+    G.gz = (int)s_box.gsize[2];
+    G.gxy = s_box.gsize[0] * s_box.gsize[1];
+    G.base = 0u;
+    const uint32_t entries = s_box.cells + 2u;  // with the empty-slot cell and the end
+    const uint32_t particles = S.info[0].count;
+    if (entries <= SORT_CELLS) {
+        for (uint32_t c = SORT_WG + t; c * 4u < entries; c += SORT_WG)
+            reinterpret_cast<uint4*>(s_cell)[c] = make_uint4(0u, 0u, 0u, 0u);
+        if (entries > SORT_WG * 4u) __syncthreads();
+        sort_cells<true>(s_cell, entries, G, s_box.cells, particles, n, p, s_wave, cell_lb, placed);
+    } else {
+        sort_cells<false>(count, entries, G, s_box.cells, particles, n, p, s_wave, cell_lb, placed);
+    }
 }
 
 // The stable order within each cell, and the state gathered into it (the
@@ -3223,6 +3449,12 @@ void launch_grid_setup(hipStream_t s, DevGrid* g, const Scenes& sc, const uint32
         k_scene_grid<<<sc.count, LPS_BLOCK, 0, s>>>(sc, part, h, energy);
         k_grid_finish<<<1, LPS_BLOCK, 0, s>>>(g, sc, h, cell_cap);
     }
+}
+
+void launch_sort_one(hipStream_t s, DevGrid* g, const Scenes& sc, const uint32_t* part, float h, uint32_t cell_cap,
+                     double* energy, const float4* pos, uint32_t n, uint32_t* count, uint32_t* cell_lb,
+                     uint2* placed) {
+    k_sort_one<<<1, SORT_WG, 0, s>>>(g, sc, part, h, cell_cap, energy, pos, count, cell_lb, placed, n);
 }
 
 void launch_keys(hipStream_t s, const float4* pos, uint32_t n, const DevGrid* g, const Scenes& sc, uint32_t* keys,
