@@ -38,20 +38,70 @@ __device__ __forceinline__ uint32_t xcd_block(uint32_t nlogical) {
     return lb < nlogical ? lb : UINT_MAX;
 }
 
+// A value combined over the wave by a commutative operation, in the order of a
+// butterfly over lane distances 32, 16, 8, 4, 2, 1; every lane gets it, and
+// every lane has to be active.  The halves and rows are exchanged by the
+// permlane swaps; within a row, once the lanes at distance 8 (4) agree,
+// rotating by 8 (4) brings the butterfly's partner or its equal.  No LDS: with
+// __shfl_xor a step costs a trip through it (54 of them in the records that
+// end every integration): k_integrate 14.3 -> 11.5 us at 524,288 particles, 7.5 -> 6.3
+// at 151,219.
+template <int CTRL>
+__device__ __forceinline__ uint32_t row_move(uint32_t v) {
+    return (uint32_t)__builtin_amdgcn_mov_dpp((int)v, CTRL, 0xF, 0xF, true);
+}
+template <int STEP, class T>
+__device__ __forceinline__ void butterfly_pair(const T& v, T& a, T& b) {
+    constexpr int W = sizeof(T) / 4;
+    struct Words { uint32_t w[W]; };
+    const Words x = __builtin_bit_cast(Words, v);
+    Words y = x, z = x;
+    for (int k = 0; k < W; k++) {
+        if constexpr (STEP == 32) {
+            const auto r = __builtin_amdgcn_permlane32_swap(x.w[k], x.w[k], false, false);
+            y.w[k] = r[0];
+            z.w[k] = r[1];
+        } else if constexpr (STEP == 16) {
+            const auto r = __builtin_amdgcn_permlane16_swap(x.w[k], x.w[k], false, false);
+            y.w[k] = r[0];
+            z.w[k] = r[1];
+        } else {
+            // row_ror:8, row_ror:4, quad_perm [2,3,0,1], quad_perm [1,0,3,2]
+            constexpr int CTRL = STEP == 8 ? 0x128 : STEP == 4 ? 0x124 : STEP == 2 ? 0x4E : 0xB1;
+            z.w[k] = row_move<CTRL>(x.w[k]);
+        }
+    }
+    a = __builtin_bit_cast(T, y);
+    b = __builtin_bit_cast(T, z);
+}
+template <int STEP, class T, class Op>
+__device__ __forceinline__ T wave_reduce(T v, Op op) {
+    T a, b;
+    butterfly_pair<STEP>(v, a, b);
+    v = op(a, b);
+    if constexpr (STEP > 1) return wave_reduce<STEP / 2>(v, op);
+    else return v;
+}
+template <class T>
+__device__ __forceinline__ T wave_sum(T v) {
+    return wave_reduce<32>(v, [](T a, T b) { return a + b; });
+}
 __device__ __forceinline__ uint32_t wave_max_u32(uint32_t v) {
-    for (int off = 32; off > 0; off >>= 1) v = max(v, (uint32_t)__shfl_xor((int)v, off, 64));
-    return v;
+    return wave_reduce<32>(v, [](uint32_t a, uint32_t b) { return max(a, b); });
 }
 __device__ __forceinline__ uint32_t wave_min_u32(uint32_t v) {
-    for (int off = 32; off > 0; off >>= 1) v = min(v, (uint32_t)__shfl_xor((int)v, off, 64));
-    return v;
+    return wave_reduce<32>(v, [](uint32_t a, uint32_t b) { return min(a, b); });
 }
-__device__ __forceinline__ float wave_sum_f32(float v) {
-    for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
-    return v;
-}
-__device__ __forceinline__ double wave_sum_f64(double v) {
-    for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
+
+// Inclusive sum over the lanes up to each lane (every lane active): within
+// the rows, then the rows' last lanes to the rows after them.
+__device__ __forceinline__ uint32_t wave_scan_u32(uint32_t v) {
+    v += row_move<0x111>(v);  // row_shr:1, zero shifted in
+    v += row_move<0x112>(v);
+    v += row_move<0x114>(v);
+    v += row_move<0x118>(v);
+    v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x142, 0xA, 0xF, false);  // row_bcast:15 to rows 1, 3
+    v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x143, 0xC, 0xF, false);  // row_bcast:31 to rows 2, 3
     return v;
 }
 
@@ -863,7 +913,7 @@ __device__ __forceinline__ void bbox_partial(uint32_t* __restrict__ part, uint32
         mx[a] = wave_max_u32(fin ? f2o(v[a]) : 0u);
     }
     nf = wave_max_u32(nf);
-    const float wke = wave_sum_f32(valid ? ke : 0.f), wpe = wave_sum_f32(valid ? pe : 0.f);
+    const float wke = wave_sum(valid ? ke : 0.f), wpe = wave_sum(valid ? pe : 0.f);
     const uint32_t w = threadIdx.x >> 6;
     if (lane_id() == 0) {
         for (int a = 0; a < 3; a++) {
@@ -928,8 +978,8 @@ __device__ __forceinline__ void scene_energy_block(const lps_dev::Scenes& S, con
         ke += (double)__uint_as_float(q[7]);
         pe += (double)__uint_as_float(q[8]);
     }
-    ke = wave_sum_f64(ke);
-    pe = wave_sum_f64(pe);
+    ke = wave_sum(ke);
+    pe = wave_sum(pe);
     if (lane_id() == 0) {
         s_e[0][threadIdx.x >> 6] = ke;
         s_e[1][threadIdx.x >> 6] = pe;
@@ -1156,7 +1206,7 @@ __device__ __forceinline__ uint32_t cell_key_quick(const GridView& G, const floa
 // in consecutive lanes: the first lane of a run of equal keys counts the whole
 // run.
 __device__ __forceinline__ uint32_t count_key(uint32_t* count, uint32_t key, uint32_t lane) {
-    const uint32_t before = (uint32_t)__shfl_up((int)key, 1, 64);
+    const uint32_t before = row_move<0x138>(key);  // wave_shr:1
     const uint64_t heads = __ballot(lane == 0u || key != before);
     const uint64_t upto = ~0ull >> (63u - lane);
     const uint32_t head = 63u - (uint32_t)__clzll((long long)(heads & upto));
@@ -1203,7 +1253,7 @@ __global__ __launch_bounds__(LPS_BLOCK) void k_tile_sum(const uint32_t* __restri
     } else {
         for (uint32_t k = c; k < total; k++) v += count[k];
     }
-    for (int off = 32; off > 0; off >>= 1) v += (uint32_t)__shfl_xor((int)v, off, 64);
+    v = wave_sum(v);
     if (lane_id() == 0u) s[threadIdx.x >> 6] = v;
     __syncthreads();
     if (threadIdx.x == 0u) {
@@ -1236,12 +1286,8 @@ __global__ __launch_bounds__(LPS_BLOCK) void k_cell_scan(uint32_t* __restrict__ 
     uint32_t local = 0u;
 #pragma unroll
     for (uint32_t k = 0; k < LPS_SCAN_ITEMS; k++) local += v[k];
-    uint32_t incl = local;
-    for (int off = 1; off < 64; off <<= 1) {
-        const uint32_t y = (uint32_t)__shfl_up((int)incl, off, 64);
-        if (lane >= (uint32_t)off) incl += y;
-        pre += (uint32_t)__shfl_xor((int)pre, off, 64);
-    }
+    const uint32_t incl = wave_scan_u32(local);
+    pre = wave_sum(pre);
     if (lane == 63u) {
         s_pre[w] = pre;
         s_in[w] = incl;
@@ -1277,22 +1323,13 @@ __global__ __launch_bounds__(LPS_BLOCK) void k_place(const uint32_t* __restrict_
 // step waits for (each of the five kernels is a chain of two or three memory
 // round trips).  The cells are counted and summed in LDS, or in the global
 // counts (zero between steps) when the grid has more of them than fit.
-// Per step, five launches -> one: 11.8 -> 4.4 us of kernels at 512 particles,
-// 13.0 -> 5.6 at 1,080, 14.2 -> 11.2 at 16,128, beside the four launches.  One
+// Per step, five launches -> one: 11.8 -> 3.6 us of kernels at 512 particles,
+// 13.0 -> 5.2 at 1,080, 14.2 -> 10.9 at 16,128, beside the four launches.  One
 // compute unit then does all of its arithmetic (with IEEE divisions and the
 // runs of k_keys the last figure was 16.6); more blocks would not fit its
 // registers, which hold the positions and keys of 16 particles a thread.
 constexpr uint32_t SORT_WG = 1024u, SORT_WAVES = SORT_WG / 64u, SORT_CELLS = 32768u;
 constexpr uint32_t SORT_ITEMS = LPS_SORT_BLOCKS * LPS_BLOCK / SORT_WG;
-
-__device__ __forceinline__ uint32_t wave_scan_u32(uint32_t v) {
-    const uint32_t lane = lane_id();
-    for (uint32_t off = 1; off < 64u; off <<= 1) {
-        const uint32_t y = (uint32_t)__shfl_up((int)v, (int)off, 64);
-        if (lane >= off) v += y;
-    }
-    return v;
-}
 
 // count: `entries` counters, zero up to whole multiples of 256 per wave where
 // IN_LDS (the counts turn into the table there); global counts are cleared.
@@ -1336,7 +1373,7 @@ __device__ __forceinline__ void sort_cells(uint32_t* count, uint32_t entries, co
         const uint4 v = cells4(c);
         sum += v.x + v.y + v.z + v.w;
     }
-    for (int off = 32; off > 0; off >>= 1) sum += (uint32_t)__shfl_xor((int)sum, off, 64);
+    sum = wave_sum(sum);
     if (lane == 0u) s_wave[w] = sum;
     __syncthreads();
     uint32_t run = 0u;
@@ -1408,8 +1445,8 @@ __global__ __launch_bounds__(SORT_WG) void k_sort_one(DevGrid* g, lps_dev::Scene
         // the energy of the state entering this step, for the host
         if (energy) {
             const uint32_t* q = part + min(lane, S.nblocks - 1u) * LPS_BBOX_PART;
-            const double ke = wave_sum_f64(lane < S.nblocks ? (double)__uint_as_float(q[7]) : 0.0);
-            const double pe = wave_sum_f64(lane < S.nblocks ? (double)__uint_as_float(q[8]) : 0.0);
+            const double ke = wave_sum(lane < S.nblocks ? (double)__uint_as_float(q[7]) : 0.0);
+            const double pe = wave_sum(lane < S.nblocks ? (double)__uint_as_float(q[8]) : 0.0);
             if (lane == 0u) {
                 energy[0] = ke;
                 energy[1] = pe;
@@ -2606,8 +2643,11 @@ __device__ __forceinline__ void wave_lds_fence() {
 }
 
 __device__ __forceinline__ uint32_t max_over_teams(uint32_t v) {
-    v = max(v, (uint32_t)__shfl_xor((int)v, 16, 64));
-    return max(v, (uint32_t)__shfl_xor((int)v, 32, 64));
+    uint32_t a, b;
+    butterfly_pair<16>(v, a, b);
+    v = max(a, b);
+    butterfly_pair<32>(v, a, b);
+    return max(a, b);
 }
 
 // The stencil rows of a team's particle: lane r < 9 holds row r's first slot
