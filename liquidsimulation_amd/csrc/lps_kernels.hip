@@ -465,6 +465,28 @@ __device__ __forceinline__ void visit_row(const char* __restrict__ xb, const Com
     if (record) row[i] = first;
 }
 
+// The priority of a wave falls with the rows it has behind it, so the waves of
+// a SIMD reach the end of the stencil together: at 524,288 particles all of a
+// kernel's waves are resident from its start (eight per SIMD), and when the
+// older ones were served first (the default) the youngest ran on alone at the
+// end: wave ends were spread over 38 to 63 us.  k_pci_density 60.0 -> 56.8 us,
+// k_density 57.3 -> 52.4, k_pci_pressure (below, a level per z-plane) 52.0 ->
+// 47.7; at 2,097,152, with four rounds of waves, 197 -> 190, 186 -> 183, 163 ->
+// 161.  The staging of the tables stays at the lowest level: raised, its
+// barrier holds up working waves (k_pci_pressure 53.4).  k_forces, whose waves
+// take more than one round at 524,288 particles, gains nothing and has none.
+__device__ __forceinline__ void row_priority(uint32_t row) {
+    if (row < 2u) __builtin_amdgcn_s_setprio(3);
+    else if (row < 5u) __builtin_amdgcn_s_setprio(2);
+    else if (row < 7u) __builtin_amdgcn_s_setprio(1);
+    else __builtin_amdgcn_s_setprio(0);
+}
+__device__ __forceinline__ void plane_priority(uint32_t plane) {
+    if (plane == 0u) __builtin_amdgcn_s_setprio(2);
+    else if (plane == 1u) __builtin_amdgcn_s_setprio(1);
+    else __builtin_amdgcn_s_setprio(0);
+}
+
 template <int VB, class Acc, class Pre, class F>
 __device__ __forceinline__ void for_neighbors_masked(const GridView& G, const uint32_t* __restrict__ lb, float ax,
                                                      float ay, float az, const float4* __restrict__ xs, float px,
@@ -485,6 +507,7 @@ __device__ __forceinline__ void for_neighbors_masked(const GridView& G, const ui
             const int y = yg - 1 + (int)ry;
             if (y < 0 || y >= G.gy) continue;
             const uint32_t base = G.base + (uint32_t)G.gx * (uint32_t)y + G.gxy * (uint32_t)z;
+            row_priority(3u * rz + ry);
             visit_row<VB>(xb, CF, lb[base + (uint32_t)x0], lb[base + (uint32_t)x1 + 1u],
                           M.mask + (3u * rz + ry) * M.stride, i, replay, record, px, py, pz, s_max, s_relax,
                           accept_extra, pre, fn);
@@ -501,7 +524,7 @@ __device__ __forceinline__ void for_neighbors_masked(const GridView& G, const ui
 // are those of for_neighbors_masked in MC_REPLAY mode; a plane where some lane
 // of the wave has no recorded masks or a row longer than one window of 32
 // candidates is walked row by row as there.
-// SELF: the particle itself is visited too.
+// SELF: the particle itself is visited too (the force pass; no priorities).
 template <int VB, bool SELF, class Pre, class F>
 __device__ __forceinline__ void for_neighbors_planes(const GridView& G, const uint32_t* __restrict__ lb, float ax,
                                                      float ay, float az, const float4* __restrict__ xs, float px,
@@ -515,6 +538,7 @@ __device__ __forceinline__ void for_neighbors_planes(const GridView& G, const ui
     const bool replay = M.ok[i] != 0u;
     for (uint32_t rz = 0; rz < 3u; rz++) {
         const int z = zg - 1 + (int)rz;
+        if constexpr (!SELF) plane_priority(rz);
         if (z < 0 || z >= G.gz) continue;
         uint32_t b[3], m[3];
         bool merge = replay;
