@@ -2699,85 +2699,115 @@ __device__ __forceinline__ TeamRows team_rows(const GridView& G, const uint32_t*
 
 constexpr uint32_t LPS_PENDING = 128u;  // entries of a team's list in LDS
 
-// The candidates of a z-plane's three rows: 32 of each row in flight per team.
-struct TeamPlane {
-    uint32_t b[3], n[3];
-    float3 x[3][2];
+// The first 64 candidates of a row, four per lane of the team.
+struct TeamRow {
+    uint32_t b, n;
+    float3 x[4];
 };
 
+// Row R of the team's rows: its range, and its candidates' loads (a lane
+// without one reads its own particle, which is not taken).
 template <int R>
-__device__ __forceinline__ void team_load(TeamPlane& P, uint32_t b, uint32_t n, const char* __restrict__ xb,
+__device__ __forceinline__ void team_load(TeamRow& P, const TeamRows& rows, const char* __restrict__ xb,
                                           uint32_t own) {
     const uint32_t lane = team_lane();
-    P.b[R] = team_bcast<R>(b);
-    P.n[R] = team_bcast<R>(n);
-    // a lane without a candidate reads its own particle, which is not taken
-    const uint32_t at = (P.b[R] + lane) << 4;
-    P.x[R][0] = *reinterpret_cast<const float3*>(xb + (lane < P.n[R] ? at : own));
-    if (__any(P.n[R] > 16u)) P.x[R][1] = *reinterpret_cast<const float3*>(xb + (lane + 16u < P.n[R] ? at + 256u : own));
+    P.b = team_bcast<R>(rows.b);
+    P.n = team_bcast<R>(rows.n);
+    const uint32_t at = (P.b + lane) << 4;
+    auto load = [&](uint32_t k) {
+        P.x[k] = *reinterpret_cast<const float3*>(xb + (lane + 16u * k < P.n ? at + 256u * k : own));
+    };
+    load(0u);
+    if (__any(P.n > 16u)) load(1u);
+    if (__any(P.n > 32u)) {
+        load(2u);
+        load(3u);
+    }
 }
 
 // Appends the accepted candidates (slot, s2) of the team's particle to its
-// list in LDS, in visiting order (of 12.6 us of k_density_t at 16,000
-// particles the tests take 4.6 and the lists 2.5; numbering the candidates of
-// all rows took 8.8 us instead of 8.3 at 512 particles, 8.1 of predicted
-// density instead of 7.2 at 1,080, the same at 16,000; testing each cell's
-// candidates once for the wave's particles of that cell 14.4 instead of 12.6
-// at 16,000): each row 16 candidates at a time, a plane's
-// loads in flight while the plane before it is tested.  room() empties the
-// lists when some team's may run full; pend is the team's number of entries.
+// list in LDS, in visiting order, 16 candidates at a time, with the loads of
+// the next DEPTH - 1 rows in flight (the scan is half of a density pass's time).
+// With a plane's rows of 32 candidates in flight and longer rows read again in
+// turn, and a branch per 16 candidates: k_density_t 12.5 us now 11.5 at 16,000
+// particles (SPH), k_pci_density_t 10.1 now 8.6 (6.5 now 5.9 at 1,080).  The
+// time is the same for 3, 4 and 5 rows.  room() empties the lists when some team's may run full; pend is the
+// team's number of entries.  Not better: numbering the candidates of all rows
+// (8.8 us instead of 8.3 at 512 particles, 8.1 instead of 7.2 of predicted
+// density at 1,080), testing each cell's candidates once for the wave's
+// particles of that cell (14.4 instead of 12.6 at 16,000).
 template <class Room>
+struct TeamScan {
+    const char* __restrict__ xb;
+    uint32_t i;
+    float px, py, pz, s_max;
+    uint2* s_list;
+    uint32_t& pend;
+    Room& room;
+    uint32_t lane, shift, below;
+
+    // K candidates per lane (slots j0 + lane + 16 k below the row's end) in one
+    // stretch of code: rejected ones go to a spare entry of the lane's own
+    template <int K>
+    __device__ __forceinline__ void tests(const float3 (&x)[K], uint32_t j0, uint32_t left) {
+        uint32_t m[K];
+        float s2[K];
+        bool ok[K];
+#pragma unroll
+        for (int k = 0; k < K; k++) {
+            const float dx = x[k].x - px, dy = x[k].y - py, dz = x[k].z - pz;
+            s2[k] = dx * dx + dy * dy + dz * dz;
+            ok[k] = lane + 16u * (uint32_t)k < left && s2[k] <= s_max;
+            m[k] = (uint32_t)(__builtin_amdgcn_ballot_w64(ok[k]) >> shift) & 0xFFFFu;
+        }
+#pragma unroll
+        for (int k = 0; k < K; k++) {
+            const uint32_t at = ok[k] ? pend + (uint32_t)__popc(m[k] & below) : LPS_PENDING + lane;
+            s_list[at] = make_uint2(j0 + lane + 16u * (uint32_t)k, __float_as_uint(s2[k]));
+            pend += (uint32_t)__popc(m[k]);
+        }
+    }
+    __device__ __forceinline__ void row(const TeamRow& P) {
+        if (__any(pend > LPS_PENDING - 64u)) room();
+        if (!__any(P.n > 16u)) {
+            const float3 x[1] = {P.x[0]};
+            tests<1>(x, P.b, P.n);
+        } else if (!__any(P.n > 32u)) {
+            const float3 x[2] = {P.x[0], P.x[1]};
+            tests<2>(x, P.b, P.n);
+        } else {
+            tests<4>(P.x, P.b, P.n);
+            for (uint32_t o = 64u; __any(o < P.n); o += 32u) {
+                if (__any(pend > LPS_PENDING - 32u)) room();
+                const uint32_t at = (P.b + o + lane) << 4, left = o < P.n ? P.n - o : 0u;
+                const float3 x[2] = {*reinterpret_cast<const float3*>(xb + (lane < left ? at : i << 4)),
+                                     *reinterpret_cast<const float3*>(xb + (lane + 16u < left ? at + 256u : i << 4))};
+                tests<2>(x, P.b + o, left);
+            }
+        }
+    }
+    template <int R, int DEPTH>
+    __device__ __forceinline__ void rows_from(const TeamRows& rows, TeamRow (&P)[DEPTH]) {
+        row(P[R % DEPTH]);
+        if constexpr (R + DEPTH < 9) team_load<R + DEPTH>(P[R % DEPTH], rows, xb, i << 4);
+        if constexpr (R < 8) rows_from<R + 1, DEPTH>(rows, P);
+    }
+    template <int R, int DEPTH>
+    __device__ __forceinline__ void first_loads(const TeamRows& rows, TeamRow (&P)[DEPTH]) {
+        team_load<R>(P[R], rows, xb, i << 4);
+        if constexpr (R + 1 < DEPTH) first_loads<R + 1, DEPTH>(rows, P);
+    }
+};
+
+template <int DEPTH, class Room>
 __device__ __forceinline__ void team_scan(const TeamRows& R, const float4* __restrict__ xs, uint32_t i, float px,
                                           float py, float pz, float s_max, uint2* s_list, uint32_t& pend, Room&& room) {
-    const uint32_t lane = team_lane(), shift = threadIdx.x & 48u, below = (1u << lane) - 1u;
-    const char* __restrict__ xb = reinterpret_cast<const char*>(xs);
-    auto test = [&](const float3& x, uint32_t j, bool in) {
-        const float dx = x.x - px, dy = x.y - py, dz = x.z - pz;
-        const float s2 = dx * dx + dy * dy + dz * dz;
-        const bool ok = in && s2 <= s_max;
-        const uint32_t m = (uint32_t)(__builtin_amdgcn_ballot_w64(ok) >> shift) & 0xFFFFu;
-        if (ok) s_list[pend + (uint32_t)__popc(m & below)] = make_uint2(j, __float_as_uint(s2));
-        pend += (uint32_t)__popc(m);
-    };
-    uint32_t b = R.b, n = R.n;
-    TeamPlane P, N;
-    team_load<0>(P, b, n, xb, i << 4);
-    team_load<1>(P, b, n, xb, i << 4);
-    team_load<2>(P, b, n, xb, i << 4);
-    for (uint32_t rz = 0; rz < 3u; rz++) {
-        if (rz < 2u) {
-            // the next plane's rows to lanes 0 to 2 (row_shl 3)
-            b = (uint32_t)__builtin_amdgcn_mov_dpp((int)b, 0x103, 0xF, 0xF, true);
-            n = (uint32_t)__builtin_amdgcn_mov_dpp((int)n, 0x103, 0xF, 0xF, true);
-            team_load<0>(N, b, n, xb, i << 4);
-            team_load<1>(N, b, n, xb, i << 4);
-            team_load<2>(N, b, n, xb, i << 4);
-        }
-        const uint32_t longest = max(max(P.n[0], P.n[1]), P.n[2]);
-        if (!__any(longest > 32u)) {
-            if (__any(pend > LPS_PENDING - 96u)) room();
-#pragma unroll
-            for (int r = 0; r < 3; r++) {
-                test(P.x[r][0], P.b[r] + lane, lane < P.n[r]);
-                if (__any(P.n[r] > 16u)) test(P.x[r][1], P.b[r] + lane + 16u, lane + 16u < P.n[r]);
-            }
-        } else {
-            for (uint32_t r = 0; r < 3u; r++) {
-                const uint32_t rb = r == 0u ? P.b[0] : r == 1u ? P.b[1] : P.b[2];
-                const uint32_t rn = r == 0u ? P.n[0] : r == 1u ? P.n[1] : P.n[2];
-                for (uint32_t o = 0u; __any(o < rn); o += 32u) {
-                    if (__any(pend > LPS_PENDING - 32u)) room();
-                    const bool in0 = o + lane < rn, in1 = o + lane + 16u < rn;
-                    const uint32_t j0 = in0 ? rb + o + lane : i, j1 = in1 ? rb + o + lane + 16u : i;
-                    const float3 x0 = *reinterpret_cast<const float3*>(xb + (j0 << 4));
-                    const float3 x1 = *reinterpret_cast<const float3*>(xb + (j1 << 4));
-                    test(x0, j0, in0);
-                    test(x1, j1, in1);
-                }
-            }
-        }
-        P = N;
-    }
+    const uint32_t lane = team_lane();
+    TeamScan<std::decay_t<Room>> scan{reinterpret_cast<const char*>(xs), i,    px,   py,   pz, s_max, s_list, pend,
+                                      room,                              lane, threadIdx.x & 48u, (1u << lane) - 1u};
+    TeamRow P[DEPTH];
+    scan.template first_loads<0, DEPTH>(R, P);
+    scan.template rows_from<0, DEPTH>(R, P);
 }
 
 // The exact table index from s2 = d^2 (no threshold table).
@@ -2861,7 +2891,7 @@ __device__ __forceinline__ float team_density(const TeamRows& R, const float4* _
         done += pend;
         pend = 0u;
     };
-    team_scan(R, xs, i, px, py, pz, c.s_max, s_list, pend, flush);
+    team_scan<4>(R, xs, i, px, py, pz, c.s_max, s_list, pend, flush);
     flush();
     if (valid && lane == 0u) L.count[i] = done;
     return sum.v[0];
@@ -2912,7 +2942,7 @@ __device__ __forceinline__ void team_replay(const lps_dev::NbLists& L, uint32_t 
         wave_lds_fence();
         pend = 0u;
     };
-    team_scan(R, xs, i, px, py, pz, c.s_max, s_list, pend, flush);
+    team_scan<2>(R, xs, i, px, py, pz, c.s_max, s_list, pend, flush);
     flush();
 }
 
@@ -2938,7 +2968,7 @@ __global__ __launch_bounds__(LPS_BLOCK) void k_density_t(const float4* __restric
     W.load(tables);
     const BlockScene B = block_scene(S, lb / LPS_TEAM);
     __shared__ float sW[LPS_TABLE_SIZE];
-    __shared__ uint2 s_list[LPS_BLOCK / LPS_TEAM][LPS_PENDING];
+    __shared__ uint2 s_list[LPS_BLOCK / LPS_TEAM][LPS_PENDING + LPS_TEAM];
     if (status != 0u) return;
     const GridView G = grid_view(g, S.grid + B.s);
     const bool valid = i < B.info.slot0 + B.info.count;
@@ -2998,7 +3028,7 @@ __global__ __launch_bounds__(LPS_BLOCK) void k_forces_t(
     const float ri = xi.w;
     // snx, sny, snz, lc, vfx, vfy, vfz, then (features) nb, dv
     constexpr int NT = FEAT ? 9 : 7;
-    __shared__ uint2 s_list[LPS_BLOCK / LPS_TEAM][LPS_PENDING];
+    __shared__ uint2 s_list[LPS_BLOCK / LPS_TEAM][LPS_PENDING + LPS_TEAM];
     __shared__ __align__(16) float s_t[LPS_BLOCK / LPS_TEAM][NT * LPS_TEAM];
     TeamSum<NT> sum;
     team_replay<NT>(L, valid ? listed : 0u, nb0, [&]() { return team_rows(G, cell_lb, xi.x, xi.y, xi.z, valid); },
@@ -3108,7 +3138,7 @@ __global__ __launch_bounds__(LPS_BLOCK) void k_pressure_sph_t(const float4* __re
     const bool fastdiv = c.s_max < 0x1p78f;  // accepted pairs have d < 2^40
     const bool nocheck = fastdiv && g->odd_state == 0u;
     const bool qidx = index_q_ok(c.div);
-    __shared__ uint2 s_list[LPS_BLOCK / LPS_TEAM][LPS_PENDING];
+    __shared__ uint2 s_list[LPS_BLOCK / LPS_TEAM][LPS_PENDING + LPS_TEAM];
     TeamSum<3> sum;
     team_replay<3>(L, valid ? listed : 0u, nb0, [&]() { return team_rows(G, cell_lb, xi.x, xi.y, xi.z, valid); },
                    posrho, i, xi.x, xi.y, xi.z, c, s_list[threadIdx.x / LPS_TEAM], nullptr,
@@ -3145,13 +3175,14 @@ __global__ __launch_bounds__(LPS_BLOCK) void k_pci_density_t(
     SimConst c, const float* __restrict__ tables, float* __restrict__ rho_pred, float* __restrict__ press,
     float4* __restrict__ xq, uint32_t k, float* __restrict__ feat, const float4* __restrict__ posrho,
     lps_dev::Scenes S, lps_dev::NbMasks mk, lps_dev::NbLists nl, uint32_t nlogical) {
-    if (step_dead(g) || g->running == 0u) return;
-    const uint32_t L = g->list_of[k % LPS_MAX_ITER_SLOTS];
+    // checked once the slot's own loads are on their way
+    const uint32_t status = g->status, running = g->running;
+    const uint32_t L = g->list_of[k % LPS_MAX_ITER_SLOTS] & 1u;  // unset in a dead step
     uint32_t s0 = 0u;
     const uint32_t lb = active_piece<LPS_BLOCK / LPS_TEAM>(g, S, L, blockIdx.x, s0);
     if (lb == UINT_MAX) return;
     __shared__ float sW[LPS_TABLE_SIZE];
-    __shared__ uint2 s_list[LPS_BLOCK / LPS_TEAM][LPS_PENDING];
+    __shared__ uint2 s_list[LPS_BLOCK / LPS_TEAM][LPS_PENDING + LPS_TEAM];
     __shared__ uint32_t s_max[LPS_BLOCK / 64];
     TableSlice<LPS_BLOCK, LPS_TABLE_SIZE> W;
     W.load(tables);
@@ -3161,7 +3192,12 @@ __global__ __launch_bounds__(LPS_BLOCK) void k_pci_density_t(
     const float4 xa = pos[i];
     const float4 xi = xpred[i];
     const BlockScene B = block_scene(S, lb);
-    const GridView G = grid_view(g, S.grid + B.s);
+    const SceneGrid* sg = S.grid + B.s;
+    const size_t ob = (size_t)sg->buf_of[k % LPS_MAX_ITER_SLOTS] * mk.stride;
+    const size_t old = (size_t)sg->buf_of[(k - 1u) % LPS_MAX_ITER_SLOTS] * mk.stride;
+    const GridView G = grid_view(g, sg);
+    if (status != 0u || running == 0u) return;
+    const float pold = k == 1u ? 0.f : press[old + i];
     const bool valid = i < B.info.slot0 + B.info.count;
     const TeamRows R = team_rows(G, cell_lb, xa.x, xa.y, xa.z, valid);
     W.store(sW);
@@ -3178,10 +3214,6 @@ __global__ __launch_bounds__(LPS_BLOCK) void k_pci_density_t(
                 dp *= c.npf;
                 e *= c.npf;
             }
-            const SceneGrid* sg = S.grid + B.s;
-            const size_t ob = (size_t)sg->buf_of[k % LPS_MAX_ITER_SLOTS] * mk.stride;
-            const float pold =
-                k == 1u ? 0.f : press[(size_t)sg->buf_of[(k - 1u) % LPS_MAX_ITER_SLOTS] * mk.stride + i];
             const float p = pold + dp;
             rho_pred[ob + i] = rp;
             press[ob + i] = p;
@@ -3222,9 +3254,10 @@ __global__ __launch_bounds__(LPS_BLOCK) void k_pci_pressure_t(
         if (blockIdx.x == 0) loop_rule_block(g, S, k, rule, c0.rest_density, host_flag);
         return;
     }
-    if (step_dead(g)) return;
+    const uint32_t status = g->status;  // checked with the stop below
     uint32_t s0 = 0u;
-    const uint32_t lb = active_piece<LPS_BLOCK / LPS_TEAM>(g, S, g->list_of[k % LPS_MAX_ITER_SLOTS], blockIdx.x - LPS_RULE_BLOCKS, s0);
+    const uint32_t lb = active_piece<LPS_BLOCK / LPS_TEAM>(g, S, g->list_of[k % LPS_MAX_ITER_SLOTS] & 1u,
+                                                                   blockIdx.x - LPS_RULE_BLOCKS, s0);
     if (lb == UINT_MAX) return;
     // the slot's own state loads while the tables are staged; the
     // predicted-density pass's (prediction, p / rho*^2)
@@ -3240,7 +3273,9 @@ __global__ __launch_bounds__(LPS_BLOCK) void k_pci_pressure_t(
     const bool is_first = first[i] != 0;
     const BlockScene B = block_scene(S, lb);
     const uint32_t stop = S.grid[B.s].stop_iter;
-    if (stop != 0u && stop < k) return;
+    const size_t ob = (size_t)S.grid[B.s].buf_of[k % LPS_MAX_ITER_SLOTS] * mk.stride;
+    if (status != 0u || (stop != 0u && stop < k)) return;
+    const float ri = rho_pred[ob + i];
     const bool fastdiv = c0.s_max < 0x1p78f;
     const bool nocheck = fastdiv && g->tiny_pred == 0u;
     const bool qidx = index_q_ok(c0.div);
@@ -3255,7 +3290,7 @@ __global__ __launch_bounds__(LPS_BLOCK) void k_pci_pressure_t(
     const GridView G = grid_view(g, S.grid + B.s);
     const SimConst c = scene_const(c0, B.info);
     const float tf = xi.w;
-    __shared__ uint2 s_list[LPS_BLOCK / LPS_TEAM][LPS_PENDING];
+    __shared__ uint2 s_list[LPS_BLOCK / LPS_TEAM][LPS_PENDING + LPS_TEAM];
     TeamSum<3> sum;
     team_replay<3>(nl, valid ? listed : 0u, nb0, [&]() { return team_rows(G, cell_lb, xa.x, xa.y, xa.z, valid); }, xq,
                    i, xi.x, xi.y, xi.z, c, s_list[threadIdx.x / LPS_TEAM], nullptr, [](uint32_t) { return 0; },
@@ -3276,8 +3311,6 @@ __global__ __launch_bounds__(LPS_BLOCK) void k_pci_pressure_t(
     float acc[3];
     sum.get(acc);
     if (!valid || team_lane() != 0u) return;
-    const size_t ob = (size_t)S.grid[B.s].buf_of[k % LPS_MAX_ITER_SLOTS] * mk.stride;
-    const float ri = rho_pred[ob + i];
     const float4 f4 = make_float4((-acc[0]) * c.mass * ri, (-acc[1]) * c.mass * ri, (-acc[2]) * c.mass * ri, 0.f);
     fp[ob + i] = f4;
     const float4 xn = predict(make_float4(xr.x, xr.y, xr.z, 0.f), vi, vhi, is_first, f.x + f4.x,

@@ -53,3 +53,18 @@ def test_ragged_counts(gpu, method, n):
 @pytest.mark.parametrize("dims", [(40, 32, 32), (41, 32, 32)])
 def test_around_the_team_limit(gpu, dims):
     _both(scenes.small_block(*dims, s=0.016, jitter_amp=2e-4, seed=3, method=METHOD_PCISPH), 4)
+
+
+@pytest.mark.parametrize("method", [METHOD_SPH, METHOD_PCISPH])
+# a row's candidates are read 16, 32 or 64 at a time, then 32 by 32
+@pytest.mark.parametrize("n", [16, 17, 32, 33, 64, 65, 96, 97, 129])
+def test_row_lengths(gpu, method, n):
+    sc = scenes.small_block(7, 7, 7, seed=n, method=method)
+    # n particles of one cell, and a sparse row beside them
+    rng = np.random.default_rng(n)
+    h = sc.params.particle_radius * sc.params.kernel_radius_factor
+    crowd = sc.x.mean(0) + rng.random((n, 3)) * 0.9 * h
+    line = sc.x.mean(0) + np.array([0.0, 1.2, 0.0]) * h + np.linspace(-2.0, 2.0, 9)[:, None] * [h, 0.0, 0.0]
+    sc.x = np.concatenate([crowd, line]).astype(np.float32)
+    sc.v = np.zeros_like(sc.x)
+    _both(sc, 2)
