@@ -1619,11 +1619,12 @@ __global__ __launch_bounds__(LPS_BLOCK) void k_density(const float4* __restrict_
 
 // accumulateNonPressureForces (SPHKernels.cl:256-349); for PCISPH also the
 // first prediction of the correction loop (pciInit + pciIntegrate +
-// pciHandleCollisions with fp = 0, SPHKernels.cl:661-735).  Held one wave per
-// SIMD above what the compiler picks (7 and 6 waves: 102.3 and 110.1 µs
-// against 103.3 and 113.4 at 524k); at eight it spills inside the plane loop.
+// pciHandleCollisions with fp = 0, SPHKernels.cl:661-735).  Six waves per SIMD
+// (80 registers) against 7 (72, two spilled) and 8 (64): 64.5, 66.9 and 62.2 us
+// at 524,288 particles, 236, 237 and 258 at 2,097,152, 42.1, 44.2 and 46.3 at
+// 151,219.
 template <bool FEAT>
-__global__ __launch_bounds__(LPS_BLOCK) __attribute__((amdgpu_waves_per_eu(FEAT ? 6 : 7))) void k_forces(
+__global__ __launch_bounds__(LPS_BLOCK) __attribute__((amdgpu_waves_per_eu(6))) void k_forces(
     const float4* __restrict__ posrho, const float4* __restrict__ vel, const float4* __restrict__ vh,
     const uint8_t* __restrict__ first, DevGrid* g, const uint32_t* __restrict__ cell_lb, SimConst c0,
     const float* __restrict__ tables, const lps_box* __restrict__ boxes0, const lps_sphere* __restrict__ spheres0,
