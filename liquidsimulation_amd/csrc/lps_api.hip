@@ -154,6 +154,7 @@ struct lps_ctx {
     uint2* placed = nullptr;                    // (index, key) in the cells' slots, by arrival
     uint32_t *skeys = nullptr, *perm = nullptr;
     uint32_t* bbox_part = nullptr;
+    bool records_valid = true;  // bbox_part holds the current state's records
     float4 *posrho = nullptr, *force = nullptr, *fp = nullptr, *xpred[2] = {};
     float4* xq = nullptr;  // predicted-density pass: (prediction, p / rho*^2) [cap_n + LPS_STENCIL_PAD]
     float *press = nullptr, *q = nullptr, *rho_pred = nullptr;
@@ -533,14 +534,34 @@ lps_dev::PhysArgs phys_args(lps_ctx* c, const SimConst& k) {
     return a;
 }
 
+// Whether one workgroup sorts the state, and whether its SPH steps integrate in
+// the pressure pass: the sort takes the box from the positions then, and the
+// blocks' records (the boxes and energies of larger scenes and of lps_get_energy)
+// are not written.  That saves a launch and costs the sort's one compute unit a
+// pass over the positions: 512 particles 56.5 -> 54.2 us a frame, 10,000 84.6 ->
+// 83.0, 16,000 43.9 -> 44.4 us a step, so it stops between the last two.
+bool sort_in_one(const lps_ctx* c) { return c->h_sinfo.size() == 1u && c->n <= LPS_SORT_BLOCKS * LPS_BLOCK; }
+bool move_with_pressure(const lps_ctx* c) {
+    return c->params.method == LPS_METHOD_SPH && sort_in_one(c) && c->n <= LPS_MOVE_BLOCKS * LPS_BLOCK &&
+           stencil_lanes(c) == 16u;
+}
+
+// The records of the current state, where the last steps left them out.
+void ensure_records(lps_ctx* c) {
+    if (c->records_valid) return;
+    lps_dev::launch_bbox(c->stream, c->pos[c->cur], c->vel[c->cur], c->der.mass, 0u, scenes(c), c->bbox_part);
+    c->records_valid = true;
+}
+
 // Grid build of one step: keys, cell table, placement, reorder (state flips to
 // the other buffer).
 void enqueue_grid(lps_ctx* c) {
     const hipStream_t s = c->stream;
     const uint32_t n = c->n;
-    if (scenes(c).count == 1u && n <= LPS_SORT_BLOCKS * LPS_BLOCK) {
+    const bool no_records = move_with_pressure(c);
+    if (sort_in_one(c)) {
         Timed t(c, "grid_setup");
-        lps_dev::launch_sort_one(s, c->grid, scenes(c), c->bbox_part, c->der.h, c->cell_cap, c->h_energy,
+        lps_dev::launch_sort_one(s, c->grid, scenes(c), no_records ? nullptr : c->bbox_part, c->der.h, c->cell_cap, c->h_energy,
                                  c->pos[c->cur], n, c->cell_count, c->cell_lb, c->placed);
     } else {
         {
@@ -779,11 +800,15 @@ StepResult enqueue_step(lps_ctx* c, float dt, bool seeded, bool feat_on) {
             Timed t(c, "forces");
             lps_dev::launch_forces(s, a, nullptr, nullptr, nullptr);
         }
-        {
+        if (move_with_pressure(c)) {
             Timed t(c, "pressure_sph");
-            lps_dev::launch_pressure_sph(s, a, c->q);
-        }
-        {
+            lps_dev::launch_pressure_move(s, a, c->q, c->pprev[c->cur], c->press, c->report);
+            c->records_valid = false;
+        } else {
+            {
+                Timed t(c, "pressure_sph");
+                lps_dev::launch_pressure_sph(s, a, c->q);
+            }
             Timed t(c, "integrate");
             lps_dev::launch_integrate(s, a, nullptr, c->pprev[c->cur], c->press, c->bbox_part, c->report);
         }
@@ -1218,6 +1243,7 @@ int lps_set_scenes(lps_ctx* c, uint32_t nscenes, const uint32_t* counts, const f
         c->h_part_cap = parts;
     }
     lps_dev::launch_unpack(s, rows, c->der.mass, scenes(c), state_arrays(c, 0), c->bbox_part);
+    c->records_valid = true;
     HIPC(hipGetLastError());
     HIPC(hipMemcpyAsync(c->h_part, c->bbox_part, sizeof(uint32_t) * parts, hipMemcpyDeviceToHost, s));
     HIPC(hipStreamSynchronize(s));
@@ -1308,8 +1334,12 @@ int lps_add_particles(lps_ctx* c, const float* x, const float* v, const float* v
     c->feat_valid = c->seed_valid = false;
     if ((st = upload_scenes(c))) return st;
     // the blocks before the first new slot keep their records (unless the
-    // storage grew, and the records with it)
-    lps_dev::launch_bbox(s, c->pos[b], c->vel[b], c->der.mass, grown ? 0u : old / LPS_BLOCK, scenes(c), c->bbox_part);
+    // storage grew, and the records with it, or there were none)
+    if (grown) c->records_valid = false;
+    if (c->records_valid)
+        lps_dev::launch_bbox(s, c->pos[b], c->vel[b], c->der.mass, old / LPS_BLOCK, scenes(c), c->bbox_part);
+    else if (!move_with_pressure(c))
+        ensure_records(c);
     HIPC(hipGetLastError());
     HIPC(hipStreamSynchronize(s));
     c->e_prev_valid = false;
@@ -1418,6 +1448,7 @@ int lps_step(lps_ctx* c, float dt, uint32_t nsteps, lps_step_stats* stats) {
     // A failed step leaves the state as it was (its kernels no-op and the
     // reorder copies the identity), so after a grid overflow the cell table is
     // grown and the remaining steps are issued again.
+    if (!move_with_pressure(c)) ensure_records(c);
     // every call that enqueued steps has waited for the last one's report
     const uint32_t base = c->report->steps_ok;
     uint32_t completed = 0;
@@ -1498,8 +1529,9 @@ int lps_get_energy(lps_ctx* c, double* kinetic, double* potential, uint32_t nsce
     if (c->n_real == 0) return LPS_ERR_STATE;
     HIPC(hipStreamSynchronize(c->stream));
     // the current state's per-block records were written by the last
-    // integration or particle upload
+    // integration or particle upload, or are written now
     std::vector<double> keep(c->h_energy, c->h_energy + 2 * (size_t)nscenes);
+    ensure_records(c);
     lps_dev::launch_scene_energy(c->stream, scenes(c), c->bbox_part, c->h_energy);
     HIPC(hipGetLastError());
     HIPC(hipStreamSynchronize(c->stream));
@@ -1580,6 +1612,7 @@ int lps_autotune(lps_ctx* c, float dt, uint32_t steps, lps_tuning* chosen) {
             cp(c->vh[b], sh, sizeof(float4) * n); cp(c->first[b], sf, n);
             cp(c->id[b], si, sizeof(uint32_t) * n); cp(c->pprev[b], spp, sizeof(float) * n);
             cp(c->bbox_part, sb, sizeof(uint32_t) * nparts);
+            c->records_valid = true;
         }
         if (e == hipSuccess) e = hipStreamSynchronize(s);
         return e;
@@ -1590,6 +1623,7 @@ int lps_autotune(lps_ctx* c, float dt, uint32_t steps, lps_tuning* chosen) {
     c->coll_stride = 0;  // no training rows from trial steps
     const WarmFallback wf0 = c->wf;
     const uint64_t steps0 = c->steps;
+    ensure_records(c);
     if (copy_all(true) != hipSuccess) st = LPS_ERR_HIP;
     // graphs x lookahead x correction-kernel workgroup size (the particle
     // block of 256 slots run as 1, 2 or 4 workgroups) with one lane per

@@ -127,7 +127,7 @@ void launch_scene_energy(hipStream_t s, const Scenes& sc, const uint32_t* part, 
 void launch_grid_setup(hipStream_t s, DevGrid* g, const Scenes& sc, const uint32_t* part, float h, uint32_t cell_cap,
                        double* energy);
 // a single scene of at most LPS_SORT_BLOCKS blocks: launch_grid_setup to launch_place in one launch (keys and ranks
-// stay in it)
+// stay in it); part null: the scene's box from the positions, no energy
 void launch_sort_one(hipStream_t s, DevGrid* g, const Scenes& sc, const uint32_t* part, float h, uint32_t cell_cap,
                      double* energy, const float4* pos, uint32_t n, uint32_t* count, uint32_t* cell_lb,
                      uint2* placed);
@@ -144,6 +144,9 @@ void launch_reorder(hipStream_t s, const ReorderArgs& a);
 void launch_density(hipStream_t s, const PhysArgs& a, float* press, float* q);
 void launch_forces(hipStream_t s, const PhysArgs& a, float4* xpred, const float* pprev, float* feat);
 void launch_pressure_sph(hipStream_t s, const PhysArgs& a, const float* q);
+// the same and the integration, with 16 lanes per particle; leaves the blocks' records as they were
+void launch_pressure_move(hipStream_t s, const PhysArgs& a, const float* q, float* pprev, const float* press,
+                          StepReport* report);
 // rho_pred and press: three buffers of a.mk.stride slots each; correction k
 // writes the scene's buffer buf_of[k % 64] (and reads the previous pressure
 // from buf_of[(k - 1) % 64]); xq receives (prediction xyz, p / rho*^2), the

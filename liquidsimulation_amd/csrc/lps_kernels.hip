@@ -1352,6 +1352,8 @@ __global__ __launch_bounds__(LPS_BLOCK) void k_place(const uint32_t* __restrict_
 // compute unit then does all of its arithmetic (with IEEE divisions and the
 // runs of k_keys the last figure was 16.6); more blocks would not fit its
 // registers, which hold the positions and keys of 16 particles a thread.
+// RECORDS: the box (and the energy) from the blocks' records, else from the
+// positions.
 constexpr uint32_t SORT_WG = 1024u, SORT_WAVES = SORT_WG / 64u, SORT_CELLS = 32768u;
 constexpr uint32_t SORT_ITEMS = LPS_SORT_BLOCKS * LPS_BLOCK / SORT_WG;
 
@@ -1436,6 +1438,7 @@ __device__ __forceinline__ void sort_cells(uint32_t* count, uint32_t entries, co
     }
 }
 
+template <bool RECORDS>
 __global__ __launch_bounds__(SORT_WG) void k_sort_one(DevGrid* g, lps_dev::Scenes S,
                                                       const uint32_t* __restrict__ part, float h, uint32_t cell_cap,
                                                       double* __restrict__ energy, const float4* __restrict__ pos,
@@ -1454,9 +1457,44 @@ __global__ __launch_bounds__(SORT_WG) void k_sort_one(DevGrid* g, lps_dev::Scene
         if (k * SORT_WG >= n) break;
         p[k] = pos[min(k * SORT_WG + t, n - 1u)];
     }
+    const uint32_t particles = S.info[0].count;
+    __shared__ uint32_t s_red[7][SORT_WAVES];
+    if constexpr (!RECORDS) {
+        uint32_t r[7];
+        auto box = [&](bool finite_only) {
+            for (int a = 0; a < 6; a++) r[a] = a < 3 ? 0xFFFFFFFFu : 0u;
+#pragma unroll
+            for (uint32_t k = 0; k < SORT_ITEMS; k++) {
+                if (k * SORT_WG >= n) break;
+                const bool valid = k * SORT_WG + t < particles;
+                const float v[3] = {p[k].x, p[k].y, p[k].z};
+                for (int a = 0; a < 3; a++) {
+                    const bool in = valid && (!finite_only || isfinite(v[a]));
+                    // f2o in three operations
+                    const uint32_t u = __float_as_uint(v[a]), o = u ^ ((uint32_t)((int)u >> 31) | 0x80000000u);
+                    r[a] = min(r[a], in ? o : 0xFFFFFFFFu);
+                    r[3 + a] = max(r[3 + a], in ? o : 0u);
+                }
+            }
+            for (int a = 0; a < 6; a++) r[a] = a < 3 ? wave_min_u32(r[a]) : wave_max_u32(r[a]);
+        };
+        // f2o puts infinities and NaN past the finite values at either end; a
+        // wave that finds some takes them out
+        box(false);
+        r[6] = 0u;
+        for (int a = 0; a < 3; a++) r[6] |= r[a] <= 0x007FFFFFu || r[3 + a] >= 0xFF800000u ? 1u : 0u;
+        if (__any(r[6] != 0u)) box(true);
+        if (lane == 0u)
+            for (int a = 0; a < 7; a++) s_red[a][w] = r[a];
+        __syncthreads();
+    }
     if (w == 0u) {
         uint32_t r[7];
-        for (int a = 0; a < 7; a++) r[a] = lane < S.nblocks ? part[lane * LPS_BBOX_PART + a] : box_start(a);
+        if constexpr (RECORDS) {
+            for (int a = 0; a < 7; a++) r[a] = lane < S.nblocks ? part[lane * LPS_BBOX_PART + a] : box_start(a);
+        } else {
+            for (int a = 0; a < 7; a++) r[a] = s_red[a][lane % SORT_WAVES];
+        }
         for (int a = 0; a < 7; a++)
             r[a] = a < 3 ? min(wave_min_u32(r[a]), box_start(a)) : max(wave_max_u32(r[a]), box_start(a));
         if (lane == 0u) {
@@ -1467,7 +1505,7 @@ __global__ __launch_bounds__(SORT_WG) void k_sort_one(DevGrid* g, lps_dev::Scene
         }
     } else if (w == 1u) {
         // the energy of the state entering this step, for the host
-        if (energy) {
+        if (RECORDS && energy) {
             const uint32_t* q = part + min(lane, S.nblocks - 1u) * LPS_BBOX_PART;
             const double ke = wave_sum(lane < S.nblocks ? (double)__uint_as_float(q[7]) : 0.0);
             const double pe = wave_sum(lane < S.nblocks ? (double)__uint_as_float(q[8]) : 0.0);
@@ -1495,7 +1533,6 @@ __global__ __launch_bounds__(SORT_WG) void k_sort_one(DevGrid* g, lps_dev::Scene
     G.gxy = s_box.gsize[0] * s_box.gsize[1];
     G.base = 0u;
     const uint32_t entries = s_box.cells + 2u;  // with the empty-slot cell and the end
-    const uint32_t particles = S.info[0].count;
     if (entries <= SORT_CELLS) {
         for (uint32_t c = SORT_WG + t; c * 4u < entries; c += SORT_WG)
             reinterpret_cast<uint4*>(s_cell)[c] = make_uint4(0u, 0u, 0u, 0u);
@@ -2953,6 +2990,47 @@ __device__ __forceinline__ uint32_t team_particle(uint32_t lb) {
     return lb * (LPS_BLOCK / LPS_TEAM) + threadIdx.x / LPS_TEAM;
 }
 
+// integrate (SPHKernels.cl:424-455) + handleCollisions (SPHKernels.cl:457-486)
+// of particle i under the force f; its new position and velocity.
+struct Moved {
+    float3 p;
+    float4 v;
+};
+__device__ __forceinline__ Moved move_particle(uint32_t i, const float3& x, const float4& f, float rho,
+                                               const float4& h4, bool is_first, const SimConst& c,
+                                               const lps_box* boxes, const lps_sphere* spheres,
+                                               const lps_plane* planes, float4* __restrict__ pos,
+                                               float4* __restrict__ vel, float4* __restrict__ vh,
+                                               uint8_t* __restrict__ first) {
+    Moved m;
+    m.p = x;
+    const float ax = f.x / rho, ay = f.y / rho, az = f.z / rho;
+    float3 hv = make_float3(h4.x, h4.y, h4.z);
+    if (is_first) {
+        const float4 v4 = vel[i];
+        hv.x = v4.x - ax * c.dt / 2.f;
+        hv.y = v4.y - ay * c.dt / 2.f;
+        hv.z = v4.z - az * c.dt / 2.f;
+        first[i] = 0;
+    }
+    const float3 old = hv;
+    hv.x += ax * c.dt; hv.y += ay * c.dt; hv.z += az * c.dt;
+    m.p.x += hv.x * c.dt; m.p.y += hv.y * c.dt; m.p.z += hv.z * c.dt;
+    collide_all(m.p, hv, c, boxes, spheres, planes);
+    vh[i] = make_float4(hv.x, hv.y, hv.z, 0.f);
+    pos[i] = make_float4(m.p.x, m.p.y, m.p.z, 0.f);
+    m.v = make_float4((old.x + hv.x) / 2.f, (old.y + hv.y) / 2.f, (old.z + hv.z) / 2.f, 0.f);
+    vel[i] = m.v;
+    return m;
+}
+
+// What the host reads once the stream has drained.
+__device__ __forceinline__ void write_report(StepReport* __restrict__ report, const DevGrid* g) {
+    report->status = g->status;
+    report->steps_ok = g->steps_ok;
+    report->cells_needed = g->cells_needed;
+}
+
 // k_density with a team per particle.
 __global__ __launch_bounds__(LPS_BLOCK) void k_density_t(const float4* __restrict__ pos, DevGrid* g, float4* __restrict__ vel,
                                                          lps_dev::Scenes S, const uint32_t* __restrict__ cell_lb,
@@ -3110,13 +3188,28 @@ __global__ __launch_bounds__(LPS_BLOCK) void k_forces_t(
     }
 }
 
-// k_pressure_sph with a team per particle.
+// k_pressure_sph with a team per particle.  MOVE: also the step's integration,
+// with the report to the host but without the blocks' records (a team's
+// workgroup has 16 particles, a record 256 slots), for scenes whose sort takes
+// the box from the positions (k_pressure_sph_t 4.2 and k_integrate 3.2 -> 5.6 us at
+// 512 particles, and a launch; the sort 3.8 -> 4.3).
+struct Motion {
+    float4 *pos, *vel, *vh;
+    uint8_t* first;
+    float* pprev;
+    const float* press;
+    const lps_box* boxes;
+    const lps_sphere* spheres;
+    const lps_plane* planes;
+    StepReport* report;
+};
+template <bool MOVE>
 __global__ __launch_bounds__(LPS_BLOCK) void k_pressure_sph_t(const float4* __restrict__ posrho,
                                                               const float* __restrict__ q, const DevGrid* g,
-                                                              const uint32_t* __restrict__ cell_lb, SimConst c,
+                                                              const uint32_t* __restrict__ cell_lb, SimConst c0,
                                                               const float* __restrict__ tables,
                                                               float4* __restrict__ force, lps_dev::Scenes S,
-                                                              lps_dev::NbLists L, uint32_t nlogical) {
+                                                              lps_dev::NbLists L, Motion M, uint32_t nlogical) {
     const uint32_t status = g->status;
     const uint32_t lb = xcd_block(nlogical);
     if (lb == UINT_MAX) return;
@@ -3125,7 +3218,17 @@ __global__ __launch_bounds__(LPS_BLOCK) void k_pressure_sph_t(const float4* __re
     const float4 xi = posrho[i];
     const float tf = q[i];
     const uint32_t listed = L.count[i];
+    float4 f = force[i], h4{};
+    float pi = 0.f;
+    bool is_first = false;
+    if constexpr (MOVE) {
+        h4 = M.vh[i];
+        is_first = M.first[i] != 0;
+        pi = M.press[i];
+        if (lb == 0u && threadIdx.x == 0u) write_report(M.report, g);
+    }
     const BlockScene B = block_scene(S, lb / LPS_TEAM);
+    const SimConst c = scene_const(c0, B.info);
     __shared__ float sP1[LPS_TABLE_SIZE];
     {
         TableSlice<LPS_BLOCK, LPS_TABLE_SIZE> a;
@@ -3161,11 +3264,15 @@ __global__ __launch_bounds__(LPS_BLOCK) void k_pressure_sph_t(const float4* __re
     float acc[3];
     sum.get(acc);
     if (!valid || team_lane() != 0u) return;
-    float4 f = force[i];
     f.x += (-acc[0]) * c.mass * xi.w;
     f.y += (-acc[1]) * c.mass * xi.w;
     f.z += (-acc[2]) * c.mass * xi.w;
     force[i] = f;
+    if constexpr (MOVE) {
+        move_particle(i, make_float3(xi.x, xi.y, xi.z), f, xi.w, h4, is_first, c, M.boxes + B.info.box0,
+                      M.spheres + B.info.sphere0, M.planes + B.info.plane0, M.pos, M.vel, M.vh, M.first);
+        M.pprev[i] = pi;
+    }
 }
 
 // k_pci_density with a team per particle: a workgroup of 256 threads takes a
@@ -3334,12 +3441,7 @@ __global__ __launch_bounds__(LPS_BLOCK) void k_integrate(
     const uint32_t lb = xcd_block(nlogical);
     if (lb == UINT_MAX) return;
     const bool dead = step_dead(g);
-    // what the host reads once the stream has drained
-    if (lb == 0u && threadIdx.x == 0u) {
-        report->status = g->status;
-        report->steps_ok = g->steps_ok;
-        report->cells_needed = g->cells_needed;
-    }
+    if (lb == 0u && threadIdx.x == 0u) write_report(report, g);
     const uint32_t i = lb * LPS_BLOCK + threadIdx.x;
     // the slot's own state loads before its scene's constants arrive (every
     // slot of a block lies within the allocated slots)
@@ -3367,24 +3469,9 @@ __global__ __launch_bounds__(LPS_BLOCK) void k_integrate(
                 const float4 a = fp[ob + i];
                 f.x += a.x; f.y += a.y; f.z += a.z;
             }
-            const float ax = f.x / rho, ay = f.y / rho, az = f.z / rho;
-            float3 hv = make_float3(h4.x, h4.y, h4.z);
-            if (is_first) {
-                const float4 v4 = vel[i];
-                hv.x = v4.x - ax * c.dt / 2.f;
-                hv.y = v4.y - ay * c.dt / 2.f;
-                hv.z = v4.z - az * c.dt / 2.f;
-                first[i] = 0;
-            }
-            const float3 old = hv;
-            hv.x += ax * c.dt; hv.y += ay * c.dt; hv.z += az * c.dt;
-            p.x += hv.x * c.dt; p.y += hv.y * c.dt; p.z += hv.z * c.dt;
-            collide_all(p, hv, c, boxes, spheres, planes);
-            vh[i] = make_float4(hv.x, hv.y, hv.z, 0.f);
-            pos[i] = make_float4(p.x, p.y, p.z, 0.f);
-            const float4 vn = make_float4((old.x + hv.x) / 2.f, (old.y + hv.y) / 2.f, (old.z + hv.z) / 2.f, 0.f);
-            vel[i] = vn;
-            particle_energy(c.mass, c.gravity, p.x, p.y, p.z, vn.x, vn.y, vn.z, ke, pe);
+            const Moved m = move_particle(i, p, f, rho, h4, is_first, c, boxes, spheres, planes, pos, vel, vh, first);
+            p = m.p;
+            particle_energy(c.mass, c.gravity, p.x, p.y, p.z, m.v.x, m.v.y, m.v.z, ke, pe);
             if (pprev) pprev[i] = press[ob + i];
         } else {
             const float4 vo = vel[i];
@@ -3552,7 +3639,10 @@ void launch_grid_setup(hipStream_t s, DevGrid* g, const Scenes& sc, const uint32
 void launch_sort_one(hipStream_t s, DevGrid* g, const Scenes& sc, const uint32_t* part, float h, uint32_t cell_cap,
                      double* energy, const float4* pos, uint32_t n, uint32_t* count, uint32_t* cell_lb,
                      uint2* placed) {
-    k_sort_one<<<1, SORT_WG, 0, s>>>(g, sc, part, h, cell_cap, energy, pos, count, cell_lb, placed, n);
+    if (part)
+        k_sort_one<true><<<1, SORT_WG, 0, s>>>(g, sc, part, h, cell_cap, energy, pos, count, cell_lb, placed, n);
+    else
+        k_sort_one<false><<<1, SORT_WG, 0, s>>>(g, sc, part, h, cell_cap, energy, pos, count, cell_lb, placed, n);
 }
 
 void launch_keys(hipStream_t s, const float4* pos, uint32_t n, const DevGrid* g, const Scenes& sc, uint32_t* keys,
@@ -3627,8 +3717,8 @@ void launch_pressure_sph(hipStream_t s, const PhysArgs& a, const float* q) {
     const uint32_t nl = cdiv(a.c.n, LPS_BLOCK);
     if (a.lanes == LPS_TEAM) {
         const uint32_t nt = nl * LPS_TEAM;
-        k_pressure_sph_t<<<xcd_grid(nt), LPS_BLOCK, 0, s>>>(a.posrho, q, a.g, a.cell_lb, a.c, a.tables, a.force, a.sc,
-                                                           a.nl, nt);
+        k_pressure_sph_t<false><<<xcd_grid(nt), LPS_BLOCK, 0, s>>>(a.posrho, q, a.g, a.cell_lb, a.c, a.tables, a.force,
+                                                                  a.sc, a.nl, Motion{}, nt);
         return;
     }
     if (a.lanes == LPS_QUAD) {
@@ -3700,6 +3790,14 @@ void launch_pci_pressure(hipStream_t s, const PhysArgs& a, const float4* xq, con
     if (threads == 64u) pci_pressure_wg<64>(s, a, xq, rho_pred, fp, xpred_next, k, rule, host_flag);
     else if (threads == 128u) pci_pressure_wg<128>(s, a, xq, rho_pred, fp, xpred_next, k, rule, host_flag);
     else pci_pressure_wg<LPS_BLOCK>(s, a, xq, rho_pred, fp, xpred_next, k, rule, host_flag);
+}
+
+void launch_pressure_move(hipStream_t s, const PhysArgs& a, const float* q, float* pprev, const float* press,
+                          StepReport* report) {
+    const uint32_t nt = cdiv(a.c.n, LPS_BLOCK) * LPS_TEAM;
+    const Motion m{a.pos, a.vel, a.vh, a.first, pprev, press, a.boxes, a.spheres, a.planes, report};
+    k_pressure_sph_t<true><<<xcd_grid(nt), LPS_BLOCK, 0, s>>>(a.posrho, q, a.g, a.cell_lb, a.c, a.tables, a.force, a.sc,
+                                                             a.nl, m, nt);
 }
 
 void launch_integrate(hipStream_t s, const PhysArgs& a, const float4* fp, float* pprev, const float* press,
