@@ -237,30 +237,36 @@ __global__ __launch_bounds__(LPS_BLOCK) __attribute__((amdgpu_waves_per_eu(4))) 
         // the first correction's pressure buffer of this scene
         const size_t ob = (size_t)sc.grid[s].buf_of[1] * fs;
         __syncthreads();
+        // lane l finishes slot l of the wave; its values load during the
+        // inference (the groups' 16 first lanes finishing each group in turn
+        // waited for them four times: 23.8 us, now 19.9 at 524,288 particles)
+        const uint32_t p = bb + w * 64u + l;
+        const bool own = p < end;
+        const uint32_t q = own ? p : bb;
+        const float p1 = clamp_nonneg ? press[ob + q] : 0.f, before = clamp_nonneg ? pprev[q] : 0.f;
+        const float rp = rho_pred[ob + q];
+        float y = 0.f;  // infer gives every row of lanes the group's outputs
         for (uint32_t grp = 0; grp < 4; grp++) {
-            const uint32_t p = bb + w * 64u + grp * 16u + (l & 15u);
-            const float y = infer(S, xin[grp], p < end);
-            if (p < end && (l >> 4) == 0u) {
-                float v = y * tscale * pscale;
-                if (!isfinite(v)) v = 0.f;
-                seed[p] = v;
-                if (clamp_nonneg) {
-                    // With negative pressures disabled the loop never lowers
-                    // a pressure, so the seed stays within an envelope: at
-                    // least the zero start's own first-correction pressure
-                    // p1 (which the loop would reach anyway), at most kappa
-                    // times the particle's previous applied pressure unless
-                    // p1 is larger.  An over-prediction then shrinks by kappa
-                    // per step instead of feeding itself through the
-                    // previous-pressure feature.
-                    v = fmaxf(press[ob + p], fminf(v, kappa * pprev[p]));
-                }
-                const float rp = rho_pred[ob + p];
-                press[ob + p] = v;
-                // the pressure pass reads p / rho*^2 from the w slot of the prediction copy
-                reinterpret_cast<float*>(xq)[4u * p + 3u] = v / (rp * rp);
-            }
+            const float yg = infer(S, xin[grp], bb + w * 64u + grp * 16u + (l & 15u) < end);
+            if (grp == l >> 4) y = yg;
         }
+        if (!own) return;
+        float v = y * tscale * pscale;
+        if (!isfinite(v)) v = 0.f;
+        seed[p] = v;
+        if (clamp_nonneg) {
+            // With negative pressures disabled the loop never lowers a
+            // pressure, so the seed stays within an envelope: at least the
+            // zero start's own first-correction pressure p1 (which the loop
+            // would reach anyway), at most kappa times the particle's previous
+            // applied pressure unless p1 is larger.  An over-prediction then
+            // shrinks by kappa per step instead of feeding itself through the
+            // previous-pressure feature.
+            v = fmaxf(p1, fminf(v, kappa * before));
+        }
+        press[ob + p] = v;
+        // the pressure pass reads p / rho*^2 from the w slot of the prediction copy
+        reinterpret_cast<float*>(xq)[4u * p + 3u] = v / (rp * rp);
     }
 }
 
