@@ -496,15 +496,15 @@ bool several_lanes(const lps_ctx* c) { return c->lanes == 4u || (c->lanes == 0u 
 
 // How many lanes: a team of 16, or a quad.  Microseconds per step of a dam
 // break, 16 lanes against 4 (and 1):
-//   SPH     4,394 particles 44 : 82,  16,000 50 : 92 (171),  65,536 85 : 109
-//           (155),  128,000 129 : 153 (158): teams at every size they may run
-//   PCISPH  4,394 121 : 231,  16,000 223 : 377 (618),  31,250 486 : 567 (893),
-//           65,536 905 : 709 (905): teams up to 160 particle blocks, where the
-//           two cross; a team's density pass costs more per particle, and
-//           PCISPH runs one per correction
+//   SPH     4,394 particles 31 : 69,  16,000 42 : 82 (140),  65,536 82 : 98
+//           (130),  128,000 131 : 133 (134): teams at every size they may run
+//   PCISPH  4,394 95 : 214,  16,000 172 : 362 (553),  43,904 458 : 567,
+//           54,000 522 : 583,  65,536 649 : 639 (826): teams up to 240
+//           particle blocks, before the two cross; a team's density pass costs
+//           more per particle, and PCISPH runs one per correction
 uint32_t stencil_lanes(const lps_ctx* c) {
     if (!several_lanes(c)) return 1u;
-    const uint32_t most = c->params.method == LPS_METHOD_SPH ? LPS_TEAM_BLOCKS : 160u;
+    const uint32_t most = c->params.method == LPS_METHOD_SPH ? LPS_TEAM_BLOCKS : 240u;
     return c->n / LPS_BLOCK <= most ? 16u : 4u;
 }
 
@@ -1628,7 +1628,7 @@ int lps_autotune(lps_ctx* c, float dt, uint32_t steps, lps_tuning* chosen) {
     // graphs x lookahead x correction-kernel workgroup size (the particle
     // block of 256 slots run as 1, 2 or 4 workgroups) with one lane per
     // particle; below 2048 particle blocks also graphs x lookahead with a
-    // quad per particle (where the workgroup size does not apply); with
+    // several lanes per particle (where the workgroup size does not apply); with
     // several scenes and at least 512 blocks also the automatic lanes (one
     // lane, and quads in the corrections that run fewer than 512 blocks)
     struct Cand { bool g; uint32_t l, t, q; float ms; };

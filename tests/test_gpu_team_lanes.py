@@ -68,3 +68,9 @@ def test_row_lengths(gpu, method, n):
     sc.x = np.concatenate([crowd, line]).astype(np.float32)
     sc.v = np.zeros_like(sc.x)
     _both(sc, 2)
+
+
+# 240 particle blocks (PCISPH: the last with a team) and 241 (a quad)
+@pytest.mark.parametrize("dims", [(48, 40, 32), (47, 41, 32)])
+def test_around_the_pcisph_limit(gpu, dims):
+    _both(scenes.small_block(*dims, s=0.016, jitter_amp=2e-4, seed=3, method=METHOD_PCISPH), 4)
