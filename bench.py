@@ -53,7 +53,7 @@ HBM_PEAK_GBS = 8000.0
 # own state read or written once, FP32 SoA (vec3 = 12 B, scalar = 4 B);
 # neighbour re-reads not counted.  Per PCISPH correction 108 B = predicted
 # density + pressure update + error max (24 B) + pressure force + re-prediction
-# (84 B); fixed part 348 B at three radix passes.
+# (84 B); fixed part 348 B at three passes of the reference's radix sort.
 ALGO_BYTES = {
     "pci_density": 24.0,
     "pci_pressure": 84.0,

@@ -207,7 +207,7 @@ void launch_feature_stats(hipStream_t s, const float* x, uint64_t n, double* acc
 void launch_target_stats(hipStream_t s, const float* t, uint64_t n, double* acc);
 void launch_collect(hipStream_t s, const float* feat, uint32_t fs, const float* press, float pscale, uint32_t n,
                     uint32_t stride, uint32_t offset, uint32_t count, float* X, float* T, uint64_t base);
-// also applies the loop rule of correction k (block 0) and answers host_flag;
+// also applies the loop rule of correction k (its first workgroup) and answers host_flag;
 // xq is the predicted-density pass's (prediction, p / rho*^2)
 void launch_pci_pressure(hipStream_t s, const PhysArgs& a, const float4* xq, const float* rho_pred, float4* fp,
                          float4* xpred_next, uint32_t k, const LoopRule& rule, uint32_t* host_flag, uint32_t threads);

@@ -1,15 +1,15 @@
 // lps_kernels.hip -- hand-written gfx950 kernels of the SPH/PCISPH step.
 //
 // One launch per phase of PhysicSolver::update (LiquidPhysics/src/PhysicSolver.cpp:12-21):
-//   grid      k_grid_one (or k_scene_grid + k_grid_finish), k_keys, k_cell_scan,
-//             k_place, k_reorder
+//   grid      k_grid_one (or k_scene_grid + k_grid_finish), k_keys, k_tile_sum,
+//             k_cell_scan, k_place (a small single scene: k_sort_one), k_reorder
 //   density   k_density
 //   forces    k_forces (+ first PCISPH prediction)
 //   pressure  SPH: k_pressure_sph;  PCISPH: {k_pci_density, k_pci_pressure (+ the
-//             loop rule in block 0, + next prediction)} per correction
-//   integrate k_integrate (+ collisions, + bounding box of the next step)
+//             loop rule in a workgroup of its own, + next prediction)} per correction
+//   integrate (small SPH scenes: within k_pressure_sph_t) k_integrate (+ collisions, + bounding box of the next step)
 // Particle kernels run 256 threads (4 wave64) per block, one particle per thread
-// (the *_q variants of the stencil kernels: a quad of threads per particle),
+// (the *_t and *_q variants of the stencil kernels: 16 or 4 threads per particle),
 // with a block index remapped so each of the 8 XCDs works on a contiguous range
 // of the cell-sorted particles and keeps its neighbours in its own L2.
 #include <hip/hip_runtime.h>
@@ -2195,7 +2195,8 @@ __global__ __launch_bounds__(LPS_BLOCK) void k_pressure_sph_q(const float4* __re
 // adds its maximum to one of the scene's sixteen sub-maxima of correction k
 // (thousands of workgroups ending together on one word waited for each other's
 // atomics: 65.4 -> 61.7 us at 524,288 particles, 219 -> 194 in the 64-scene
-// ensemble); block 0 of the pressure pass that follows applies the loop rule (loop_rule_block).
+// ensemble); the first workgroup of the pressure pass that follows applies the loop
+// rule (loop_rule_block).
 template <bool FEAT, int WG>
 __global__ __launch_bounds__(WG) void k_pci_density(
     const float4* __restrict__ pos, const float4* __restrict__ xpred, DevGrid* g, const uint32_t* __restrict__ cell_lb,
@@ -2434,9 +2435,8 @@ __device__ void loop_rule_block(DevGrid* g, const lps_dev::Scenes& S, uint32_t k
 
 // pciCalcPressureForce (SPHKernels.cl:806-878) followed by the next
 // prediction (pciIntegrate + pciHandleCollisions) from f + fp.  Held to eight
-// waves per SIMD (64 VGPRs): the compiler then spills a few values that live
-// across the whole stencil, outside its loops, and the pass runs 61.7 µs per
-// launch at 524k particles against 68.7 µs at the seven waves it would pick.
+// waves per SIMD (59 VGPRs, no spills; it issues at 99 % of the VALU peak at
+// 524,288 particles).
 template <int WG>
 __global__ __launch_bounds__(WG) __attribute__((amdgpu_waves_per_eu(WG >= 128 ? 8 : 1))) void k_pci_pressure(
     const float4* __restrict__ pos, const float4* __restrict__ xq, const float* __restrict__ rho_pred, DevGrid* g,
@@ -2664,14 +2664,13 @@ __global__ __launch_bounds__(LPS_BLOCK) void k_pci_pressure_q(
 // walking the nine rows of the stencil one after the other, as the one-lane
 // kernels do, waits for the cell table, the candidates and the kept
 // candidates' data in every row.  A team waits for each of them once.  Times
-// per launch, quads -> teams: density 18.7 -> 9.8, forces 18.6 -> 5.2, SPH
-// pressure 16.7 -> 4.8 us at 512 particles; 22.5 -> 13.0, 26.9 -> 7.7, 24.1 ->
-// 6.8 us in the 16k SPH dam break; predicted density 19.0 -> 12.4, its
-// pressure pass 17.0 -> 8.1 us in the 16k PCISPH one.
+// per launch, quads -> teams: density 18.7 -> 7.7, forces 18.6 -> 5.2, SPH
+// pressure 16.7 -> 4.4 us at 512 particles; 22.5 -> 11.5, 26.9 -> 6.9, 24.1 ->
+// 5.9 us in the 16k SPH dam break; predicted density 19.0 -> 8.6, its
+// pressure pass 17.0 -> 5.9 us in the 16k PCISPH one.
 // * lanes 0 to 8 load the ranges of the nine rows together;
-// * the density passes test the rows' candidates 16 at a time, a z-plane's
-//   loads in flight while the plane before it is tested, with the exact
-//   squared distance, and append the accepted ones in order (ballot and bit
+// * the density passes test the rows' candidates 16 at a time, with the loads
+//   of the next three rows in flight, by the exact squared distance, and append the accepted ones in order (ballot and bit
 //   count) to the team's list in LDS;
 // * the lists are also recorded in memory, so the passes over the same
 //   positions (forces, pressure) start from the list itself: one load gives
