@@ -49,7 +49,7 @@ def test_ragged_counts(gpu, method, n):
     _both(sc, 5)
 
 
-# 160 particle blocks (PCISPH: the last with a team) and 161 (a quad)
+# 160 and 161 particle blocks
 @pytest.mark.parametrize("dims", [(40, 32, 32), (41, 32, 32)])
 def test_around_the_team_limit(gpu, dims):
     _both(scenes.small_block(*dims, s=0.016, jitter_amp=2e-4, seed=3, method=METHOD_PCISPH), 4)
