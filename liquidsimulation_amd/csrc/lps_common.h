@@ -86,7 +86,8 @@ struct DevGrid {
     uint32_t converged;      // every scene met the tolerance
     uint32_t tiny_pred;      // a prediction of this step has a coordinate in (0, 2^-56)
     uint32_t odd_state;      // a nonzero coordinate or velocity component of the step's state is below the
-                             // magnitude of Derived::tiny_key, or a density outside [2^-78, 2^40)
+                             // magnitude of Derived::tiny_key, a velocity not finite (its particle's pair with
+                             // itself is then no zero), or a density outside [2^-78, 2^40)
     // Correction kernels run only the particle blocks of scenes whose loop
     // is still running.  Two block lists alternate; list_of[k % 64] names the
     // list of correction k (both of its passes).  Entries are written once per

@@ -1578,7 +1578,8 @@ __global__ __launch_bounds__(LPS_BLOCK) void k_reorder(
         // empty slots follow all particles of their scene before and after
         // the sort: they keep their places
         d = i;
-        if (key != G.base + sg->cells) {
+        const bool real = key != G.base + sg->cells;
+        if (real) {
             const uint32_t b = cell_lb[key], e = cell_lb[key + 1u];
             d = b;
             // four of the cell's entries at a time (the last one repeats,
@@ -1596,10 +1597,12 @@ __global__ __launch_bounds__(LPS_BLOCK) void k_reorder(
         cq[d] = quantize(p.x, p.y, p.z, G, compact_scale(G));
         skeys_out[d] = key;
         perm_out[d] = i;
-        // the shared-reciprocal quotients of the force passes need checks then
+        // the force passes then check their quotients' numerators and look
+        // for the pair of a particle with itself (an empty slot may hold
+        // anything and decides nothing)
         const uint32_t least = min(min(min(lps_div::num_key(p.x), lps_div::num_key(p.y)), lps_div::num_key(p.z)),
                                    min(min(lps_div::num_key(v.x), lps_div::num_key(v.y)), lps_div::num_key(v.z)));
-        if (least < tiny_key) g->odd_state = 1u;
+        if (real && (least < tiny_key || !(fabsf(v.x) + fabsf(v.y) + fabsf(v.z) < INFINITY))) g->odd_state = 1u;
     }
     pos_out[d] = p;
     vel_out[d] = v;
@@ -1694,17 +1697,21 @@ __global__ __launch_bounds__(LPS_BLOCK) __attribute__((amdgpu_waves_per_eu(6))) 
     auto walk = [&](auto quick) {
         for_neighbors_planes<2, true>(G, cell_lb, xi.x, xi.y, xi.z, posrho, xi.x, xi.y, xi.z, c.s_max, c.s_relax, mk, i,
                                       [&](uint32_t j) { return vel[j]; },
-                                      [&](uint32_t, const float4& xj, float s2, const float4& vj, const float3& dl) {
+                                      [&](uint32_t j, const float4& xj, float s2, const float4& vj, const float3& dl) {
             const uint32_t idx = table_index(s2, sT, c.inv_div);
             const float w1 = sW1[idx], wv = sV2[idx];
             // the numerators of every quotient by rho_j; x_i - x_j = -dl but
             // for the sign of a zero, which the sums cannot tell (they start
-            // at +0), and the self pair's velocity terms are +0
+            // at +0), and the self pair's velocity terms are 0 while its
+            // velocity is finite
             const float dvx = vj.x - vi.x, dvy = vj.y - vi.y, dvz = vj.z - vi.z;
             float n[8] = {-dl.x * w1, -dl.y * w1, -dl.z * w1, sW2[idx], dvx * wv, dvy * wv, dvz * wv, 0.f};
             constexpr int NQ = FEAT ? 8 : 7;
             if constexpr (FEAT) n[7] = (dvx * -dl.x + dvy * -dl.y + dvz * -dl.z) * w1;
             force_quotients<decltype(quick)::value, NQ>(n, xj.w, vj.w);
+            if constexpr (!decltype(quick)::value) {
+                if (j == i) n[4] = n[5] = n[6] = n[7] = 0.f;
+            }
             snx += n[0];
             sny += n[1];
             snz += n[2];
