@@ -155,6 +155,7 @@ struct lps_ctx {
     uint32_t *skeys = nullptr, *perm = nullptr;
     uint32_t* bbox_part = nullptr;
     bool records_valid = true;  // bbox_part holds the current state's records
+    bool records_present = true;  // ... and all of them with the present mass and gravity
     float4 *posrho = nullptr, *force = nullptr, *fp = nullptr, *xpred[2] = {};
     float4* xq = nullptr;  // predicted-density pass: (prediction, p / rho*^2) [cap_n + LPS_STENCIL_PAD]
     float *press = nullptr, *q = nullptr, *rho_pred = nullptr;
@@ -550,7 +551,7 @@ bool move_with_pressure(const lps_ctx* c) {
 void ensure_records(lps_ctx* c) {
     if (c->records_valid) return;
     lps_dev::launch_bbox(c->stream, c->pos[c->cur], c->vel[c->cur], c->der.mass, 0u, scenes(c), c->bbox_part);
-    c->records_valid = true;
+    c->records_valid = c->records_present = true;
 }
 
 // Grid build of one step: keys, cell table, placement, reorder (state flips to
@@ -811,6 +812,7 @@ StepResult enqueue_step(lps_ctx* c, float dt, bool seeded, bool feat_on) {
             }
             Timed t(c, "integrate");
             lps_dev::launch_integrate(s, a, nullptr, c->pprev[c->cur], c->press, c->bbox_part, c->report);
+            c->records_present = true;
         }
         c->last_fp_valid = 0;
         c->feat_valid = c->seed_valid = false;
@@ -856,6 +858,7 @@ StepResult enqueue_step(lps_ctx* c, float dt, bool seeded, bool feat_on) {
     {
         Timed t(c, "integrate");
         lps_dev::launch_integrate(s, a, c->fp, c->pprev[c->cur], c->press, c->bbox_part, c->report);
+        c->records_present = true;
     }
     if (feat_on && res.ok && c->coll_stride > 0 && c->coll_rows < c->coll_cap) {
         // training rows: every stride-th particle's features and the
@@ -1114,6 +1117,9 @@ int lps_set_params(lps_ctx* c, const lps_params* p) {
     if (!c) return LPS_ERR_INVALID;
     int st = check_params(p);
     if (st) return st;
+    // the state keeps the energies of the parameters it was reached with
+    ensure_records(c);
+    c->records_present = false;
     c->params = *p;
     c->epoch++;
     lps_compute_derived(&c->params, &c->der);
@@ -1243,7 +1249,7 @@ int lps_set_scenes(lps_ctx* c, uint32_t nscenes, const uint32_t* counts, const f
         c->h_part_cap = parts;
     }
     lps_dev::launch_unpack(s, rows, c->der.mass, scenes(c), state_arrays(c, 0), c->bbox_part);
-    c->records_valid = true;
+    c->records_valid = c->records_present = true;
     HIPC(hipGetLastError());
     HIPC(hipMemcpyAsync(c->h_part, c->bbox_part, sizeof(uint32_t) * parts, hipMemcpyDeviceToHost, s));
     HIPC(hipStreamSynchronize(s));
@@ -1334,8 +1340,9 @@ int lps_add_particles(lps_ctx* c, const float* x, const float* v, const float* v
     c->feat_valid = c->seed_valid = false;
     if ((st = upload_scenes(c))) return st;
     // the blocks before the first new slot keep their records (unless the
-    // storage grew, and the records with it, or there were none)
-    if (grown) c->records_valid = false;
+    // storage grew, and the records with it, or there were none, or some are
+    // of other parameters)
+    if (grown || !c->records_present) c->records_valid = false;
     if (c->records_valid)
         lps_dev::launch_bbox(s, c->pos[b], c->vel[b], c->der.mass, old / LPS_BLOCK, scenes(c), c->bbox_part);
     else if (!move_with_pressure(c))
@@ -1585,6 +1592,8 @@ int lps_autotune(lps_ctx* c, float dt, uint32_t steps, lps_tuning* chosen) {
     const hipStream_t s = c->stream;
     const uint32_t n = c->n, cur = (uint32_t)c->cur;
     const size_t nparts = (size_t)LPS_BBOX_PART * lps_dev::bbox_parts(n);
+    ensure_records(c);
+    const bool present0 = c->records_present;
     // snapshot of everything the next step reads
     float4 *sp = nullptr, *sv = nullptr, *sh = nullptr;
     uint8_t* sf = nullptr;
@@ -1613,6 +1622,7 @@ int lps_autotune(lps_ctx* c, float dt, uint32_t steps, lps_tuning* chosen) {
             cp(c->id[b], si, sizeof(uint32_t) * n); cp(c->pprev[b], spp, sizeof(float) * n);
             cp(c->bbox_part, sb, sizeof(uint32_t) * nparts);
             c->records_valid = true;
+            c->records_present = present0;
         }
         if (e == hipSuccess) e = hipStreamSynchronize(s);
         return e;
@@ -1623,7 +1633,6 @@ int lps_autotune(lps_ctx* c, float dt, uint32_t steps, lps_tuning* chosen) {
     c->coll_stride = 0;  // no training rows from trial steps
     const WarmFallback wf0 = c->wf;
     const uint64_t steps0 = c->steps;
-    ensure_records(c);
     if (copy_all(true) != hipSuccess) st = LPS_ERR_HIP;
     // graphs x lookahead x correction-kernel workgroup size (the particle
     // block of 256 slots run as 1, 2 or 4 workgroups) with one lane per
