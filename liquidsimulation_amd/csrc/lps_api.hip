@@ -410,8 +410,11 @@ uint64_t scene_cell_bound(const lps_ctx* c, const SceneInfo& si, const std::vect
 }
 
 int ensure_cells(lps_ctx* c, uint32_t cap) {
-    if (cap <= c->cell_cap && c->cell_lb) return LPS_OK;
+    if (cap <= c->cell_cap) return LPS_OK;
     c->epoch++;
+    // no cells until all three arrays are there: a step then reports an
+    // overflow on the device before it touches them, and asks again
+    c->cell_cap = 0;
     int st;
     if ((st = dalloc(&c->cell_lb, (size_t)cap + 1))) return st;
     if ((st = dalloc(&c->cell_count, (size_t)cap + 1))) return st;
@@ -951,6 +954,16 @@ int ensure_scenes(lps_ctx* c, uint32_t nscenes, uint32_t nblocks) {
     return LPS_OK;
 }
 
+// After a call that failed with the state half replaced: a context without
+// particles, which every call refuses that would run on it.
+int without_particles(lps_ctx* c, int st) {
+    c->n = c->n_real = 0;
+    c->have_step = false;
+    c->feat_valid = c->seed_valid = false;
+    c->records_valid = c->records_present = true;
+    return st;
+}
+
 lps_dev::StateArrays state_arrays(const lps_ctx* c, int b) {
     return lps_dev::StateArrays{c->pos[b], c->vel[b], c->vh[b], c->first[b], c->id[b], c->pprev[b]};
 }
@@ -1255,7 +1268,7 @@ int lps_set_scenes(lps_ctx* c, uint32_t nscenes, const uint32_t* counts, const f
     HIPC(hipStreamSynchronize(s));
     uint64_t cells = 0;
     for (uint32_t k = 0; k < nscenes; k++) cells += scene_cell_bound(c, c->h_sinfo[k], c->s_boxes[k]) + 1u;
-    if ((st = ensure_cells(c, (uint32_t)std::min<uint64_t>(cells, 0x7FFFFFF0ull)))) return st;
+    if ((st = ensure_cells(c, (uint32_t)std::min<uint64_t>(cells, 0x7FFFFFF0ull)))) return without_particles(c, st);
     c->e_prev_valid = false;
     c->wf.prev_seeded = -1;  // a new state: its first step pairs with no earlier one
     return LPS_OK;

@@ -1,0 +1,90 @@
+"""CPU tests of the library's host code where an allocation fails: the library
+runs over a stand-in for the HIP runtime (fake_hip.cpp) in a process of its
+own.  What a failed call left behind must not reach the device: later calls
+either report an error or find everything they launch with in place."""
+import os
+import subprocess
+import sys
+import textwrap
+
+import pytest
+
+HERE = os.path.dirname(os.path.abspath(__file__))
+ROOT = os.path.dirname(HERE)
+
+PRELUDE = """
+import ctypes as C, sys
+F = C.CDLL({fake!r}, C.RTLD_GLOBAL)  # before the library, which then binds to it
+F.fake_bytes.restype = C.c_size_t
+sys.path.insert(0, {root!r})
+sys.modules["torch"] = None  # it would bring the real runtime
+import numpy as np
+from liquidsimulation_amd._lib import LPSError
+from liquidsimulation_amd.abi import Box, Colliders, METHOD_PCISPH, METHOD_SPH, Params, WARM_LEARNED
+from liquidsimulation_amd.solver import Ensemble, PCISPHSolver, SPHSolver
+OOM, STATE = 3, 7
+def status(call, *a):
+    try:
+        call(*a)
+    except LPSError as e:
+        return e.status
+    return 0
+def rows(n):
+    return np.zeros((n, 3), np.float32)
+def box(half):
+    return Colliders(boxes=[Box(center=(0.0, 0.0, 0.0), half=(half,) * 3, boundary=True)])
+"""
+
+
+@pytest.fixture(scope="module")
+def run(tmp_path_factory):
+    from liquidsimulation_amd import _lib
+    if not os.path.exists(_lib.LIB_PATH):
+        pytest.skip("liblps.so is not built")
+    fake = str(tmp_path_factory.mktemp("fake") / "libfake_hip.so")
+    subprocess.run(["g++", "-shared", "-fPIC", "-O1", "-std=c++17", "-D__HIP_PLATFORM_AMD__", "-I/opt/rocm/include",
+                    "-I", os.path.join(ROOT, "include"), "-I", os.path.join(ROOT, "liquidsimulation_amd", "csrc"),
+                    "-o", fake, os.path.join(HERE, "fake_hip.cpp")], check=True, capture_output=True)
+
+    def go(body):
+        code = PRELUDE.format(fake=fake, root=ROOT) + textwrap.dedent(body)
+        r = subprocess.run([sys.executable, "-c", code], capture_output=True, text=True, timeout=120)
+        assert r.returncode == 0, r.stdout + r.stderr
+    return go
+
+
+# 12,000 particles are sorted by one workgroup, 17,000 in several launches
+@pytest.mark.parametrize("n", [12000, 17000])
+# the three allocations of the cell table
+@pytest.mark.parametrize("which", [0, 1, 2])
+def test_cell_table_growth_fails_in_an_upload(run, n, which):
+    run(f"""
+    s = SPHSolver(Params(method=METHOD_SPH))
+    s.set_colliders(box(0.5)); s.set_particles(rows({n})); s.set_colliders(box(0.5)); s.set_particles(rows({n}))
+    s.update(1e-3, 2)
+    s.set_colliders(box(2.0))
+    F.fake_fail_malloc({which})
+    assert status(s.set_particles, rows({n})) == OOM
+    F.fake_fail_malloc(-1)
+    assert status(s.update, 1e-3, 1) == STATE  # the table no longer fits the scene
+    s.set_particles(rows({n}))
+    s.update(1e-3, 2)
+    assert F.fake_null_launches() == 0
+    """)
+
+
+@pytest.mark.parametrize("n", [12000, 17000])
+@pytest.mark.parametrize("which", [0, 1, 2])
+def test_cell_table_growth_fails_in_a_step(run, n, which):
+    run(f"""
+    s = SPHSolver(Params(method=METHOD_SPH))
+    s.set_particles(rows({n}))
+    s.update(1e-3, 2)
+    F.fake_overflow(1 << 20)
+    F.fake_fail_malloc({which})
+    assert status(s.update, 1e-3, 1) == OOM
+    F.fake_fail_malloc(-1)
+    F.fake_overflow(1 << 20)  # it still needs them
+    s.update(1e-3, 2)
+    assert F.fake_null_launches() == 0
+    """)
