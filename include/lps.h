@@ -133,7 +133,9 @@ int lps_index_thresholds(const lps_params* params, float* thr /* [LPS_TABLE_SIZE
  * whole particle blocks of 256 slots is at most LPS_MAX_PARTICLES (so
  * n <= 2^28 - 256); other counts are refused with LPS_ERR_INVALID before any
  * array is read.  The same bound holds for the slots of all scenes together
- * (lps_set_scenes) and after lps_add_particles. */
+ * (lps_set_scenes) and after lps_add_particles.  Where one of the three fails
+ * with LPS_ERR_OOM or LPS_ERR_HIP after it began to replace the state, the
+ * context is left without particles (LPS_ERR_STATE from lps_step). */
 #define LPS_MAX_PARTICLES ((1u << 28) - 1u)
 int lps_set_particles(lps_ctx* ctx, const float* x, const float* v, const float* vhalf,
                       const uint8_t* first, uint32_t n);

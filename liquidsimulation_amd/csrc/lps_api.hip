@@ -425,8 +425,9 @@ int ensure_cells(lps_ctx* c, uint32_t cap) {
 }
 
 int ensure_particles(lps_ctx* c, uint32_t n) {
-    if (n <= c->cap_n && c->pos[0]) return LPS_OK;
+    if (n <= c->cap_n) return LPS_OK;
     c->epoch++;
+    c->cap_n = 0;  // until all of them are there
     int st;
     for (int b = 0; b < 2; b++) {
         if ((st = dalloc(&c->pos[b], (size_t)n + LPS_STENCIL_PAD))) return st;
@@ -1023,6 +1024,68 @@ int gather_applied(lps_ctx* c, const T* dev3, std::vector<T>& full) {
     return LPS_OK;
 }
 
+// lps_set_scenes for valid counts: `total` particles in n slots.
+int replace_scenes(lps_ctx* c, uint32_t nscenes, const uint32_t* counts, const float* gravity, const float* x,
+                   const float* v, const float* vhalf, const uint8_t* first, uint32_t n, uint32_t total) {
+    const hipStream_t s = c->stream;
+    HIPC(hipStreamSynchronize(s));
+    int st = ensure_particles(c, n);
+    if (st) return st;
+    // captured graphs hold the sizes and the arrays' addresses
+    if (n != c->n || nscenes != c->h_sinfo.size()) c->epoch++;
+    // layout; colliders of scenes that existed before are kept
+    c->h_sinfo.assign(nscenes, SceneInfo{});
+    c->s_boxes.resize(nscenes);
+    c->s_spheres.resize(nscenes);
+    c->s_planes.resize(nscenes);
+    if (gravity) c->s_gravity.assign(gravity, gravity + 3 * nscenes);
+    else c->s_gravity.clear();
+    uint32_t slot = 0;
+    for (uint32_t k = 0; k < nscenes; k++) {
+        SceneInfo& si = c->h_sinfo[k];
+        si.slot0 = slot;
+        si.count = counts[k];
+        si.padded = (counts[k] + LPS_BLOCK - 1u) / LPS_BLOCK * LPS_BLOCK;
+        si.block0 = slot / LPS_BLOCK;
+        slot += si.padded;
+    }
+    if ((st = ensure_scenes(c, nscenes, n / LPS_BLOCK))) return st;
+    c->n = n;
+    c->n_real = total;
+    c->next_id = total;
+    c->cur = 0;
+    c->have_step = false;
+    if ((st = upload_scenes(c))) return st;
+    if (nscenes > 1u) {
+        std::vector<uint32_t> bscene(n / LPS_BLOCK);
+        for (uint32_t k = 0; k < nscenes; k++)
+            for (uint32_t b = 0; b < c->h_sinfo[k].padded / LPS_BLOCK; b++) bscene[c->h_sinfo[k].block0 + b] = k;
+        HIPC(hipMemcpy(c->d_bscene, bscene.data(), sizeof(uint32_t) * (n / LPS_BLOCK), hipMemcpyHostToDevice));
+    }
+    // the caller's rows as they are, then into the state arrays on the device
+    lps_dev::Rows rows;
+    if ((st = upload_rows(c, x, v, vhalf, first, total, &rows))) return st;
+    const size_t parts = (size_t)LPS_BBOX_PART * (n / LPS_BLOCK);
+    if (parts > c->h_part_cap) {
+        if (c->h_part) (void)hipHostFree(c->h_part);
+        c->h_part = nullptr;
+        c->h_part_cap = 0;
+        HIPC(hipHostMalloc((void**)&c->h_part, sizeof(uint32_t) * parts, hipHostMallocDefault));
+        c->h_part_cap = parts;
+    }
+    lps_dev::launch_unpack(s, rows, c->der.mass, scenes(c), state_arrays(c, 0), c->bbox_part);
+    c->records_valid = c->records_present = true;
+    HIPC(hipGetLastError());
+    HIPC(hipMemcpyAsync(c->h_part, c->bbox_part, sizeof(uint32_t) * parts, hipMemcpyDeviceToHost, s));
+    HIPC(hipStreamSynchronize(s));
+    uint64_t cells = 0;
+    for (uint32_t k = 0; k < nscenes; k++) cells += scene_cell_bound(c, c->h_sinfo[k], c->s_boxes[k]) + 1u;
+    if ((st = ensure_cells(c, (uint32_t)std::min<uint64_t>(cells, 0x7FFFFFF0ull)))) return st;
+    c->e_prev_valid = false;
+    c->wf.prev_seeded = -1;  // a new state: its first step pairs with no earlier one
+    return LPS_OK;
+}
+
 }  // namespace
 
 // ================================================================= C ABI ==
@@ -1214,64 +1277,8 @@ int lps_set_scenes(lps_ctx* c, uint32_t nscenes, const uint32_t* counts, const f
     if (gravity)
         for (uint32_t k = 0; k < 3 * nscenes; k++)
             if (!std::isfinite(gravity[k])) return LPS_ERR_INVALID;
-    const uint32_t n = (uint32_t)slots;
-    const hipStream_t s = c->stream;
-    HIPC(hipStreamSynchronize(s));
-    int st = ensure_particles(c, n);
-    if (st) return st;
-    // captured graphs hold the sizes and the arrays' addresses
-    if (n != c->n || nscenes != c->h_sinfo.size()) c->epoch++;
-    // layout; colliders of scenes that existed before are kept
-    c->h_sinfo.assign(nscenes, SceneInfo{});
-    c->s_boxes.resize(nscenes);
-    c->s_spheres.resize(nscenes);
-    c->s_planes.resize(nscenes);
-    if (gravity) c->s_gravity.assign(gravity, gravity + 3 * nscenes);
-    else c->s_gravity.clear();
-    uint32_t slot = 0;
-    for (uint32_t k = 0; k < nscenes; k++) {
-        SceneInfo& si = c->h_sinfo[k];
-        si.slot0 = slot;
-        si.count = counts[k];
-        si.padded = (counts[k] + LPS_BLOCK - 1u) / LPS_BLOCK * LPS_BLOCK;
-        si.block0 = slot / LPS_BLOCK;
-        slot += si.padded;
-    }
-    if ((st = ensure_scenes(c, nscenes, n / LPS_BLOCK))) return st;
-    c->n = n;
-    c->n_real = (uint32_t)total;
-    c->next_id = (uint32_t)total;
-    c->cur = 0;
-    c->have_step = false;
-    if ((st = upload_scenes(c))) return st;
-    if (nscenes > 1u) {
-        std::vector<uint32_t> bscene(n / LPS_BLOCK);
-        for (uint32_t k = 0; k < nscenes; k++)
-            for (uint32_t b = 0; b < c->h_sinfo[k].padded / LPS_BLOCK; b++) bscene[c->h_sinfo[k].block0 + b] = k;
-        HIPC(hipMemcpy(c->d_bscene, bscene.data(), sizeof(uint32_t) * (n / LPS_BLOCK), hipMemcpyHostToDevice));
-    }
-    // the caller's rows as they are, then into the state arrays on the device
-    lps_dev::Rows rows;
-    if ((st = upload_rows(c, x, v, vhalf, first, (uint32_t)total, &rows))) return st;
-    const size_t parts = (size_t)LPS_BBOX_PART * (n / LPS_BLOCK);
-    if (parts > c->h_part_cap) {
-        if (c->h_part) (void)hipHostFree(c->h_part);
-        c->h_part = nullptr;
-        c->h_part_cap = 0;
-        HIPC(hipHostMalloc((void**)&c->h_part, sizeof(uint32_t) * parts, hipHostMallocDefault));
-        c->h_part_cap = parts;
-    }
-    lps_dev::launch_unpack(s, rows, c->der.mass, scenes(c), state_arrays(c, 0), c->bbox_part);
-    c->records_valid = c->records_present = true;
-    HIPC(hipGetLastError());
-    HIPC(hipMemcpyAsync(c->h_part, c->bbox_part, sizeof(uint32_t) * parts, hipMemcpyDeviceToHost, s));
-    HIPC(hipStreamSynchronize(s));
-    uint64_t cells = 0;
-    for (uint32_t k = 0; k < nscenes; k++) cells += scene_cell_bound(c, c->h_sinfo[k], c->s_boxes[k]) + 1u;
-    if ((st = ensure_cells(c, (uint32_t)std::min<uint64_t>(cells, 0x7FFFFFF0ull)))) return without_particles(c, st);
-    c->e_prev_valid = false;
-    c->wf.prev_seeded = -1;  // a new state: its first step pairs with no earlier one
-    return LPS_OK;
+    const int st = replace_scenes(c, nscenes, counts, gravity, x, v, vhalf, first, (uint32_t)slots, (uint32_t)total);
+    return st ? without_particles(c, st) : LPS_OK;
 }
 
 int lps_set_particles(lps_ctx* c, const float* x, const float* v, const float* vhalf, const uint8_t* first,
@@ -1322,7 +1329,7 @@ int lps_add_particles(lps_ctx* c, const float* x, const float* v, const float* v
         if (e == hipSuccess) e = hipStreamSynchronize(s);
         if (e != hipSuccess || (st = ensure_particles(c, (uint32_t)cap))) {
             release();
-            return e != hipSuccess ? hip_status(e) : st;
+            return e != hipSuccess ? hip_status(e) : without_particles(c, st);
         }
         c->cur = 0;
         grown = true;
@@ -1331,12 +1338,12 @@ int lps_add_particles(lps_ctx* c, const float* x, const float* v, const float* v
         cp(c->id[0], si, sizeof(uint32_t) * old); cp(c->pprev[0], spp, sizeof(float) * old);
         if (e == hipSuccess) e = hipStreamSynchronize(s);
         release();
-        if (e != hipSuccess) return hip_status(e);
+        if (e != hipSuccess) return without_particles(c, hip_status(e));
     }
     // the new particles take slots old .. total - 1 of the current state
     const int b = c->cur;
     const uint32_t nslots = (uint32_t)slots;
-    if ((st = ensure_scenes(c, 1u, nslots / LPS_BLOCK))) return st;
+    if ((st = ensure_scenes(c, 1u, nslots / LPS_BLOCK))) return without_particles(c, st);
     if (nslots != c->n) c->epoch++;  // captured graphs hold the number of slots
     lps_dev::Rows rows;
     if ((st = upload_rows(c, x, v, vhalf, first, n, &rows))) return st;
@@ -1351,7 +1358,7 @@ int lps_add_particles(lps_ctx* c, const float* x, const float* v, const float* v
     c->have_step = false;
     c->last_fp_valid = 0;
     c->feat_valid = c->seed_valid = false;
-    if ((st = upload_scenes(c))) return st;
+    if ((st = upload_scenes(c))) return without_particles(c, st);
     // the blocks before the first new slot keep their records (unless the
     // storage grew, and the records with it, or there were none, or some are
     // of other parameters)

@@ -19,7 +19,7 @@ namespace {
 std::map<const void*, std::string> g_names;
 struct Config { dim3 grid, block; size_t shared; hipStream_t stream; } g_config;
 int g_fail_in = -1;          // allocations until the one that fails (-1: none)
-int g_plain_its = 3, g_seeded_its = 3;  // corrections of a step without and with the seed
+int g_plain_its = 4, g_seeded_its = 4;  // corrections of a step without and with the seed
 bool g_seeded = false;
 uint32_t g_overflow_cells = 0;  // cells the next step needs, as a grid overflow (0: it succeeds)
 uint32_t g_cell_cap = 0;
@@ -142,7 +142,11 @@ hipError_t hipGetDeviceProperties(hipDeviceProp_t* p, int) {
 hipError_t hipGetLastError() { return hipSuccess; }
 hipError_t hipGetSymbolAddress(void** p, const void*) { *p = nullptr; return hipErrorInvalidSymbol; }
 hipError_t hipStreamCreateWithFlags(hipStream_t* s, unsigned) { *s = reinterpret_cast<hipStream_t>(&g_config); return hipSuccess; }
-hipError_t hipStreamDestroy(hipStream_t) { return hipSuccess; }
+hipError_t hipStreamDestroy(hipStream_t) {  // a context ends
+    g_report = nullptr;
+    g_now = StepReport{0u, 0u, 0u};
+    return hipSuccess;
+}
 hipError_t hipStreamQuery(hipStream_t) { return hipSuccess; }
 hipError_t hipStreamSynchronize(hipStream_t) {
     if (g_report) *g_report = g_now;

@@ -88,3 +88,52 @@ def test_cell_table_growth_fails_in_a_step(run, n, which):
     s.update(1e-3, 2)
     assert F.fake_null_launches() == 0
     """)
+
+
+# every allocation of a larger upload, and past the last
+@pytest.mark.parametrize("method", ["METHOD_SPH", "METHOD_PCISPH"])
+def test_upload_fails_at_any_allocation(run, method):
+    run(f"""
+    failed = 0
+    for which in range(60):
+        s = Ensemble(Params(method={method}))
+        s.set_tuning(False)
+        s.set_scenes([rows(300)]); s.update(1e-3, 2)
+        F.fake_fail_malloc(which)
+        st = status(s.set_scenes, [rows(9000), rows(20000)])
+        F.fake_fail_malloc(-1)
+        assert st in (0, OOM)
+        failed += st == OOM
+        assert status(s.update, 1e-3, 1) == (STATE if st else 0)
+        assert status(s.get_energy) == (STATE if st else 0)
+        s.set_scenes([rows(400), rows(500)]); s.update(1e-3, 2)
+        s.set_scenes([rows(9000), rows(20000)]); s.update(1e-3, 2)
+        s.close()
+    assert 35 < failed < 60
+    assert F.fake_null_launches() == 0
+    """)
+
+
+def test_append_fails_at_any_allocation(run):
+    run("""
+    lost = kept = 0
+    for which in range(60):
+        s = SPHSolver(Params(method=METHOD_SPH))
+        s.set_particles(rows(300)); s.update(1e-3, 2)
+        F.fake_fail_malloc(which)
+        st = status(s.add_particles, rows(20000))
+        F.fake_fail_malloc(-1)
+        if st == 0:
+            s.update(1e-3, 1)
+        else:
+            assert st == OOM
+            # the state survives where the copy of it could not be made
+            st = status(s.update, 1e-3, 1)
+            assert st in (0, STATE)
+            lost += st == STATE
+            kept += st == 0
+            s.set_particles(rows(300)); s.update(1e-3, 2)
+        s.close()
+    assert lost > 30 and kept == 6
+    assert F.fake_null_launches() == 0
+    """)
