@@ -1487,7 +1487,12 @@ int lps_step(lps_ctx* c, float dt, uint32_t nsteps, lps_step_stats* stats) {
         const bool feat_on = capture_features(c, seeded);
         if (feat_on) {
             int st = ensure_feat(c);
-            if (st) return st;
+            if (st) {
+                // steps of this call may be on their way: the next call's
+                // count starts from their report
+                (void)hipStreamSynchronize(c->stream);
+                return st;
+            }
         }
         StepResult last;
         for (uint32_t b = 0; b < batch; b++) {

@@ -137,3 +137,24 @@ def test_append_fails_at_any_allocation(run):
     assert lost > 30 and kept == 6
     assert F.fake_null_launches() == 0
     """)
+
+
+def test_steps_in_flight_when_a_call_fails_are_not_the_next_ones(run):
+    """A seeded probe step in the middle of a call cannot allocate the network's
+    features.  The steps before it are still on their way (the stand-in reports
+    them when the stream is waited for); the next call counts its own only."""
+    run("""
+    s = PCISPHSolver(Params(method=METHOD_PCISPH, warm_start=WARM_LEARNED))
+    s.set_tuning(False)
+    s.set_warm_start_weights(np.zeros(5313, np.float32), np.ones(32, np.float32), 1.0)
+    s.set_particles(rows(300))
+    F.fake_iterations(4, 5)
+    s.set_params(s.params.replace(max_iterations=8))
+    st = s.update(1e-3, 20)  # the probe (step 16) is the cheaper one: the seed goes off
+    assert [x.warm_start_used for x in st] == [1] * 15 + [0] * 5
+    s.set_particles(rows(3000))  # larger: the features are allocated at the next probe (step 32)
+    F.fake_fail_malloc(0)
+    assert status(s.update, 1e-3, 20) == OOM
+    F.fake_fail_malloc(-1)
+    s.update(1e-3, 3)
+    """)
