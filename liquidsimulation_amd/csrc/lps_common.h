@@ -84,7 +84,11 @@ struct DevGrid {
     uint32_t iterations;     // corrections run this step (max over scenes)
     uint32_t final_err;      // max over scenes of the last correction's max |e| (float bits)
     uint32_t converged;      // every scene met the tolerance
-    uint32_t tiny_pred;      // a prediction of this step has a coordinate in (0, 2^-56)
+    // A prediction has a coordinate in (0, 2^-56); word k & 1 for correction
+    // k's (and perhaps an earlier one's).  The pressure pass of correction k
+    // reads its word while it writes the other: the waves of a workgroup, which
+    // stage tables by it, all read the same.
+    uint32_t tiny_pred[2];
     uint32_t odd_state;      // a nonzero coordinate or velocity component of the step's state is below the
                              // magnitude of Derived::tiny_key, a velocity not finite (its particle's pair with
                              // itself is then no zero), or a density outside [2^-78, 2^40)

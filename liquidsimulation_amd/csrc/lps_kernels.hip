@@ -1124,7 +1124,7 @@ __device__ __forceinline__ uint32_t start_step(DevGrid* g, const lps_dev::Scenes
     g->iterations = 0u;
     g->final_err = 0u;
     g->converged = 0u;
-    g->tiny_pred = 0u;
+    g->tiny_pred[0] = g->tiny_pred[1] = 0u;
     g->odd_state = 0u;
     g->act_count[0] = S.nblocks;
     g->act_count[1] = 0u;
@@ -1763,7 +1763,7 @@ __global__ __launch_bounds__(LPS_BLOCK) __attribute__((amdgpu_waves_per_eu(6))) 
                                   planes);
         xpred[i] = xp;
         mk.cq[i] = quantize(xp.x, xp.y, xp.z, G, compact_scale(G));
-        if (lps_div::tiny_coord(xp.x, xp.y, xp.z)) g->tiny_pred = 1u;
+        if (lps_div::tiny_coord(xp.x, xp.y, xp.z)) g->tiny_pred[1] = 1u;
         if constexpr (FEAT) {
             const float ex = xp.x - xo.x, ey = xp.y - xo.y, ez = xp.z - xo.z;
             feat[(size_t)10 * mk.stride + i] = sqrtf(ex * ex + ey * ey + ez * ez) / c.h;
@@ -2137,7 +2137,7 @@ __global__ __launch_bounds__(LPS_BLOCK) void k_forces_q(
                                   boxes0 + B.info.box0, spheres0 + B.info.sphere0, planes0 + B.info.plane0);
         xpred[i] = xp;
         mk.cq[i] = quantize(xp.x, xp.y, xp.z, G, compact_scale(G));
-        if (lps_div::tiny_coord(xp.x, xp.y, xp.z)) g->tiny_pred = 1u;
+        if (lps_div::tiny_coord(xp.x, xp.y, xp.z)) g->tiny_pred[1] = 1u;
         if constexpr (FEAT) {
             const float ex = xp.x - xo.x, ey = xp.y - xo.y, ez = xp.z - xo.z;
             feat[(size_t)10 * mk.stride + i] = sqrtf(ex * ex + ey * ey + ez * ez) / c.h;
@@ -2476,7 +2476,7 @@ __global__ __launch_bounds__(WG) __attribute__((amdgpu_waves_per_eu(WG >= 128 ? 
     // the quotient d / div and needs no thresholds (one instantiation of the
     // stencil per case, so the pair loop carries no mode test)
     const bool fastdiv = c0.s_max < 0x1p78f;
-    const bool quick = fastdiv && g->tiny_pred == 0u && index_q_ok(c0.div);
+    const bool quick = fastdiv && g->tiny_pred[k & 1u] == 0u && index_q_ok(c0.div);
     __shared__ float sP1[LPS_TABLE_SIZE], sT[LPS_THR_SIZE];
     stage_table<WG>(sP1, tables + 3 * LPS_TABLE_SIZE, sT, tables, !quick);
     __syncthreads();
@@ -2518,7 +2518,7 @@ __global__ __launch_bounds__(WG) __attribute__((amdgpu_waves_per_eu(WG >= 128 ? 
                               f.y + f4.y, f.z + f4.z, xr.w, c, boxes, spheres, planes);
     xpred_next[i] = xn;
     mk.cq[i] = quantize(xn.x, xn.y, xn.z, G, compact_scale(G));
-    if (lps_div::tiny_coord(xn.x, xn.y, xn.z)) g->tiny_pred = 1u;
+    if (lps_div::tiny_coord(xn.x, xn.y, xn.z)) g->tiny_pred[(k + 1u) & 1u] = 1u;
 }
 
 // k_pci_density with a quad per particle: a workgroup of 256 threads takes a
@@ -2623,7 +2623,7 @@ __global__ __launch_bounds__(LPS_BLOCK) void k_pci_pressure_q(
     const uint32_t stop = S.grid[B.s].stop_iter;
     if (stop != 0u && stop < k) return;
     const bool fastdiv = c0.s_max < 0x1p78f;
-    const bool nocheck = fastdiv && g->tiny_pred == 0u;
+    const bool nocheck = fastdiv && g->tiny_pred[k & 1u] == 0u;
     const bool qidx = index_q_ok(c0.div);
     __shared__ float sP1[LPS_TABLE_SIZE], sT[LPS_THR_SIZE];
     // the thresholds serve only the pairs without the quotient index
@@ -2662,7 +2662,7 @@ __global__ __launch_bounds__(LPS_BLOCK) void k_pci_pressure_q(
                               planes0 + B.info.plane0);
     xpred_next[i] = xn;
     mk.cq[i] = quantize(xn.x, xn.y, xn.z, G, compact_scale(G));
-    if (lps_div::tiny_coord(xn.x, xn.y, xn.z)) g->tiny_pred = 1u;
+    if (lps_div::tiny_coord(xn.x, xn.y, xn.z)) g->tiny_pred[(k + 1u) & 1u] = 1u;
 }
 
 // ===================================================== team stencils ====
@@ -3186,7 +3186,7 @@ __global__ __launch_bounds__(LPS_BLOCK) void k_forces_t(
         const float4 xp = predict(xo, vi, vhi, is_first, fx + 0.f, fy + 0.f, fz + 0.f, ri, c,
                                   boxes0 + B.info.box0, spheres0 + B.info.sphere0, planes0 + B.info.plane0);
         xpred[i] = xp;
-        if (lps_div::tiny_coord(xp.x, xp.y, xp.z)) g->tiny_pred = 1u;
+        if (lps_div::tiny_coord(xp.x, xp.y, xp.z)) g->tiny_pred[1] = 1u;
         if constexpr (FEAT) {
             const float ex = xp.x - xo.x, ey = xp.y - xo.y, ez = xp.z - xo.z;
             feat[(size_t)10 * mk.stride + i] = sqrtf(ex * ex + ey * ey + ez * ez) / c.h;
@@ -3391,7 +3391,7 @@ __global__ __launch_bounds__(LPS_BLOCK) void k_pci_pressure_t(
     if (status != 0u || (stop != 0u && stop < k)) return;
     const float ri = rho_pred[ob + i];
     const bool fastdiv = c0.s_max < 0x1p78f;
-    const bool nocheck = fastdiv && g->tiny_pred == 0u;
+    const bool nocheck = fastdiv && g->tiny_pred[k & 1u] == 0u;
     const bool qidx = index_q_ok(c0.div);
     __shared__ float sP1[LPS_TABLE_SIZE];
     {
@@ -3431,7 +3431,7 @@ __global__ __launch_bounds__(LPS_BLOCK) void k_pci_pressure_t(
                               f.y + f4.y, f.z + f4.z, xr.w, c, boxes0 + B.info.box0, spheres0 + B.info.sphere0,
                               planes0 + B.info.plane0);
     xpred_next[i] = xn;
-    if (lps_div::tiny_coord(xn.x, xn.y, xn.z)) g->tiny_pred = 1u;
+    if (lps_div::tiny_coord(xn.x, xn.y, xn.z)) g->tiny_pred[(k + 1u) & 1u] = 1u;
 }
 
 // integrate (SPHKernels.cl:424-455) + pciAddPressureForce (SPHKernels.cl:880-890)
