@@ -141,6 +141,7 @@ struct lps_ctx {
     uint32_t next_id = 0;   // id of the next particle added (ids number particles in order of arrival)
     uint32_t cap_n = 0;     // allocated slot capacity
     uint32_t cell_cap = 0;  // allocated cell-table entries (plus one sentinel)
+    bool wide_grid = false; // since the upload, a step had more cells than one workgroup sorts into
     int cur = 0;            // which state buffer holds the sorted state
     uint64_t steps = 0;
     bool have_step = false; // a step has produced grid/fields
@@ -382,10 +383,12 @@ int upload_tables(lps_ctx* c) {
 // Cell-count bound of one scene: particles end every step inside each
 // BOUNDARY box shrunk by the particle radius, so that box bounds the grid; the
 // first step's grid comes from the initial positions, whose bounds (over the
-// finite coordinates) are in the records of the scene's particle blocks.
-uint64_t scene_cell_bound(const lps_ctx* c, const SceneInfo& si, const std::vector<lps_box>& boxes) {
+// finite coordinates) are in the records of the scene's particle blocks; first:
+// about that grid's cells.
+uint64_t scene_cell_bound(const lps_ctx* c, const SceneInfo& si, const std::vector<lps_box>& boxes, double* first) {
     const float h = c->der.h;
     uint64_t init = 1, bound = 0;
+    *first = 1.0;
     float mn[3] = {INFINITY, INFINITY, INFINITY}, mx[3] = {-INFINITY, -INFINITY, -INFINITY};
     for (uint32_t b = si.block0; b < si.block0 + si.padded / LPS_BLOCK; b++)
         for (int a = 0; a < 3; a++) {
@@ -397,6 +400,7 @@ uint64_t scene_cell_bound(const lps_ctx* c, const SceneInfo& si, const std::vect
     for (int a = 0; a < 3; a++) {
         const double ex = mx[a] >= mn[a] ? ((double)mx[a] - (double)mn[a]) / (double)h : 0.0;
         init *= (uint64_t)std::min(ex, 4.0e9) + 2;
+        *first *= std::floor(ex) + 1.0;
     }
     init = std::min<uint64_t>(init, 0x7FFFFFF0ull);
     for (const lps_box& b : boxes) {
@@ -545,7 +549,9 @@ lps_dev::PhysArgs phys_args(lps_ctx* c, const SimConst& k) {
 // are not written.  That saves a launch and costs the sort's one compute unit a
 // pass over the positions: 512 particles 56.5 -> 54.2 us a frame, 10,000 84.6 ->
 // 83.0, 16,000 43.9 -> 44.4 us a step, so it stops between the last two.
-bool sort_in_one(const lps_ctx* c) { return c->h_sinfo.size() == 1u && c->n <= LPS_SORT_BLOCKS * LPS_BLOCK; }
+bool sort_in_one(const lps_ctx* c) {
+    return c->h_sinfo.size() == 1u && c->n <= LPS_SORT_BLOCKS * LPS_BLOCK && !c->wide_grid;
+}
 bool move_with_pressure(const lps_ctx* c) {
     return c->params.method == LPS_METHOD_SPH && sort_in_one(c) && c->n <= LPS_MOVE_BLOCKS * LPS_BLOCK &&
            stencil_lanes(c) == 16u;
@@ -558,6 +564,11 @@ void ensure_records(lps_ctx* c) {
     c->records_valid = c->records_present = true;
 }
 
+void set_wide_grid(lps_ctx* c, bool wide) {
+    if (c->wide_grid != wide) c->epoch++;  // captured graphs hold the sort
+    c->wide_grid = wide;
+}
+
 // Grid build of one step: keys, cell table, placement, reorder (state flips to
 // the other buffer).
 void enqueue_grid(lps_ctx* c) {
@@ -567,7 +578,7 @@ void enqueue_grid(lps_ctx* c) {
     if (sort_in_one(c)) {
         Timed t(c, "grid_setup");
         lps_dev::launch_sort_one(s, c->grid, scenes(c), no_records ? nullptr : c->bbox_part, c->der.h, c->cell_cap, c->h_energy,
-                                 c->pos[c->cur], n, c->cell_count, c->cell_lb, c->placed);
+                                 c->pos[c->cur], n, c->cell_lb, c->placed);
     } else {
         {
             Timed t(c, "grid_setup");
@@ -1079,7 +1090,10 @@ int replace_scenes(lps_ctx* c, uint32_t nscenes, const uint32_t* counts, const f
     HIPC(hipMemcpyAsync(c->h_part, c->bbox_part, sizeof(uint32_t) * parts, hipMemcpyDeviceToHost, s));
     HIPC(hipStreamSynchronize(s));
     uint64_t cells = 0;
-    for (uint32_t k = 0; k < nscenes; k++) cells += scene_cell_bound(c, c->h_sinfo[k], c->s_boxes[k]) + 1u;
+    double first_cells = 0.0;
+    for (uint32_t k = 0; k < nscenes; k++) cells += scene_cell_bound(c, c->h_sinfo[k], c->s_boxes[k], &first_cells) + 1u;
+    // a first step that could not take the one-workgroup sort need not try
+    set_wide_grid(c, nscenes == 1u && first_cells >= (double)LPS_SORT_CELLS);
     if ((st = ensure_cells(c, (uint32_t)std::min<uint64_t>(cells, 0x7FFFFFF0ull)))) return st;
     c->e_prev_valid = false;
     c->wf.prev_seeded = -1;  // a new state: its first step pairs with no earlier one
@@ -1519,12 +1533,22 @@ int lps_step(lps_ctx* c, float dt, uint32_t nsteps, lps_step_stats* stats) {
             if (warm_ready(c)) ws_record(c, seeded, last.iterations, last.converged != 0);
             continue;
         }
+        const bool e_valid = c->e_prev_valid;
         c->e_prev_valid = false;
         HIPC(hipStreamSynchronize(c->stream));
         completed = c->report->steps_ok - base;
         const uint32_t status = c->report->status;
         if (status == LPS_ERR_GRID_OVERFLOW) {
             const uint32_t need = c->report->cells_needed;
+            if (sort_in_one(c) && need > LPS_SORT_CELLS) {
+                // once per upload at most; nothing to grow where the table holds them
+                set_wide_grid(c, true);
+                ensure_records(c);
+                if (need <= c->cell_cap) {
+                    c->e_prev_valid = e_valid;
+                    continue;
+                }
+            }
             if (need >= 0x7FFFFFF0u || ++retries > 8) return LPS_ERR_GRID_OVERFLOW;
             int st = ensure_cells(c, need + need / 4 + 64);
             if (st) return st;
@@ -1652,7 +1676,7 @@ int lps_autotune(lps_ctx* c, float dt, uint32_t steps, lps_tuning* chosen) {
         if (e == hipSuccess) e = hipStreamSynchronize(s);
         return e;
     };
-    const bool g0 = c->graphs_on;
+    const bool g0 = c->graphs_on, wide0 = c->wide_grid;
     const uint32_t l0 = c->lookahead, t0 = c->corr_threads, q0 = c->lanes;
     const uint32_t coll0 = c->coll_stride;
     c->coll_stride = 0;  // no training rows from trial steps
@@ -1711,6 +1735,7 @@ int lps_autotune(lps_ctx* c, float dt, uint32_t steps, lps_tuning* chosen) {
     c->steps = steps0;
     c->e_prev_valid = false;
     c->coll_stride = coll0;
+    set_wide_grid(c, wide0);  // trial steps may have spread further
     if (copy_all(false) != hipSuccess && !st) st = LPS_ERR_HIP;
     c->have_step = false;
     if (e0) (void)hipEventDestroy(e0);

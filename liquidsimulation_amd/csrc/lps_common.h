@@ -14,6 +14,7 @@
 #define LPS_SCAN_ITEMS 4       // cells per thread in the cell-table scan
 #define LPS_SCAN_TILE (LPS_BLOCK * LPS_SCAN_ITEMS)
 #define LPS_SORT_BLOCKS 64u     // particle blocks of a single scene up to which one workgroup sorts it
+#define LPS_SORT_CELLS 32767u   // and the cells it may have, the empty slots' among them (their counts stay in LDS)
 #define LPS_MOVE_BLOCKS 48u     // of those, up to which an SPH step integrates in its pressure pass
 #define LPS_MAX_ITER_SLOTS 64   // per-correction slots (buffers, block lists, host flags), used as a ring
 // Maximum error of a correction: sub-maxima per scene, 64 bytes apart, in two

@@ -126,11 +126,11 @@ void launch_scene_energy(hipStream_t s, const Scenes& sc, const uint32_t* part, 
 // to energy[2 * scene .. + 1] when energy is given
 void launch_grid_setup(hipStream_t s, DevGrid* g, const Scenes& sc, const uint32_t* part, float h, uint32_t cell_cap,
                        double* energy);
-// a single scene of at most LPS_SORT_BLOCKS blocks: launch_grid_setup to launch_place in one launch (keys and ranks
-// stay in it); part null: the scene's box from the positions, no energy
+// a single scene of at most LPS_SORT_BLOCKS blocks: launch_grid_setup to launch_place in one launch (keys, ranks and
+// counts stay in it); more than LPS_SORT_CELLS cells are a grid overflow; part null: the scene's box from the
+// positions, no energy
 void launch_sort_one(hipStream_t s, DevGrid* g, const Scenes& sc, const uint32_t* part, float h, uint32_t cell_cap,
-                     double* energy, const float4* pos, uint32_t n, uint32_t* count, uint32_t* cell_lb,
-                     uint2* placed);
+                     double* energy, const float4* pos, uint32_t n, uint32_t* cell_lb, uint2* placed);
 // cell keys, places of arrival in the cells, and the particles per cell (zero before; launch_cell_table clears
 // them); n: slots (whole blocks)
 void launch_keys(hipStream_t s, const float4* pos, uint32_t n, const DevGrid* g, const Scenes& sc, uint32_t* keys,

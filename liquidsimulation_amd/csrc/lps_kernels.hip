@@ -1345,8 +1345,12 @@ __global__ __launch_bounds__(LPS_BLOCK) void k_place(const uint32_t* __restrict_
 // in one workgroup: grid, keys, cell table and placement need only its own
 // barriers between them instead of a launch each, which is what such a scene's
 // step waits for (each of the five kernels is a chain of two or three memory
-// round trips).  The cells are counted and summed in LDS, or in the global
-// counts (zero between steps) when the grid has more of them than fit.
+// round trips).  The cells are counted and summed in LDS; a grid with more of
+// them than fit is reported as too large, and the host takes the other kernels,
+// whose time hardly depends on the cells: with the counts in memory instead,
+// a step of 512 SPH particles in 32,768 cells took 47 us against 36 (in 29,791,
+// with LDS, 28 against 35), in 305,252 cells 167 against 36, of 15,488
+// particles 65 against 41 (41 against 41) and 186 against 42.
 // Per step, five launches -> one: 11.8 -> 3.6 us of kernels at 512 particles,
 // 13.0 -> 5.2 at 1,080, 14.2 -> 10.9 at 16,128, beside the four launches.  One
 // compute unit then does all of its arithmetic (with IEEE divisions and the
@@ -1354,12 +1358,11 @@ __global__ __launch_bounds__(LPS_BLOCK) void k_place(const uint32_t* __restrict_
 // registers, which hold the positions and keys of 16 particles a thread.
 // RECORDS: the box (and the energy) from the blocks' records, else from the
 // positions.
-constexpr uint32_t SORT_WG = 1024u, SORT_WAVES = SORT_WG / 64u, SORT_CELLS = 32768u;
+constexpr uint32_t SORT_WG = 1024u, SORT_WAVES = SORT_WG / 64u, SORT_CELLS = LPS_SORT_CELLS + 1u;
 constexpr uint32_t SORT_ITEMS = LPS_SORT_BLOCKS * LPS_BLOCK / SORT_WG;
 
-// count: `entries` counters, zero up to whole multiples of 256 per wave where
-// IN_LDS (the counts turn into the table there); global counts are cleared.
-template <bool IN_LDS>
+// count: `entries` counters in LDS, zero up to whole multiples of 256 per wave;
+// they turn into the table.
 __device__ __forceinline__ void sort_cells(uint32_t* count, uint32_t entries, const GridView& G, uint32_t empty_cell,
                                            uint32_t particles, uint32_t n, const float4 (&p)[SORT_ITEMS],
                                            uint32_t* s_wave, uint32_t* __restrict__ cell_lb,
@@ -1372,28 +1375,16 @@ __device__ __forceinline__ void sort_cells(uint32_t* count, uint32_t entries, co
     for (uint32_t k = 0; k < SORT_ITEMS; k++) {
         const uint32_t i = k * SORT_WG + t;
         if (k * SORT_WG >= n) break;
-        if (i >= n) continue;  // whole waves: n is whole blocks
+        if (i >= n) continue;
         const uint32_t cell = quick ? cell_key_quick(G, p[k], y) : cell_key(G, p[k]);
         key[k] = i < particles ? cell : empty_cell;
-        rank[k] = IN_LDS ? atomicAdd(&count[key[k]], 1u) : count_key(count, key[k], lane);
+        rank[k] = atomicAdd(&count[key[k]], 1u);
     }
-    if (!IN_LDS) __threadfence();
     __syncthreads();
     // each wave sums its stretch of cells, then turns it into table entries
     const uint32_t stretch = (entries + SORT_WAVES * 256u - 1u) / (SORT_WAVES * 256u) * 256u;
     const uint32_t c0 = w * stretch + lane * 4u, c1 = min((w + 1u) * stretch, entries);
-    auto cells4 = [&](uint32_t c) {
-        if constexpr (IN_LDS) {
-            return *reinterpret_cast<const uint4*>(count + c);
-        } else {
-            uint4 v = make_uint4(0u, 0u, 0u, 0u);
-            if (c < entries) v.x = count[c];
-            if (c + 1u < entries) v.y = count[c + 1u];
-            if (c + 2u < entries) v.z = count[c + 2u];
-            if (c + 3u < entries) v.w = count[c + 3u];
-            return v;
-        }
-    };
+    auto cells4 = [&](uint32_t c) { return *reinterpret_cast<const uint4*>(count + c); };
     uint32_t sum = 0u;
     for (uint32_t c = c0; c < c1; c += 256u) {
         const uint4 v = cells4(c);
@@ -1418,23 +1409,14 @@ __device__ __forceinline__ void sort_cells(uint32_t* count, uint32_t entries, co
             if (c + 1u < entries) cell_lb[c + 1u] = lb.y;
             if (c + 2u < entries) cell_lb[c + 2u] = lb.z;
         }
-        if constexpr (IN_LDS) {
-            if (c < c1) *reinterpret_cast<uint4*>(count + c) = lb;
-        } else if (c < entries) {
-            if (v.x) count[c] = 0u;
-            if (v.y) count[c + 1u] = 0u;
-            if (v.z) count[c + 2u] = 0u;
-            if (v.w) count[c + 3u] = 0u;
-        }
+        if (c < c1) *reinterpret_cast<uint4*>(count + c) = lb;
     }
-    if (!IN_LDS) __threadfence();
     __syncthreads();
-    const uint32_t* table = IN_LDS ? count : cell_lb;
 #pragma unroll
     for (uint32_t k = 0; k < SORT_ITEMS; k++) {
         const uint32_t i = k * SORT_WG + t;
         if (k * SORT_WG >= n) break;
-        if (i < n) placed[table[key[k]] + rank[k]] = make_uint2(i, key[k]);
+        if (i < n) placed[count[key[k]] + rank[k]] = make_uint2(i, key[k]);
     }
 }
 
@@ -1442,8 +1424,8 @@ template <bool RECORDS>
 __global__ __launch_bounds__(SORT_WG) void k_sort_one(DevGrid* g, lps_dev::Scenes S,
                                                       const uint32_t* __restrict__ part, float h, uint32_t cell_cap,
                                                       double* __restrict__ energy, const float4* __restrict__ pos,
-                                                      uint32_t* count, uint32_t* cell_lb,
-                                                      uint2* __restrict__ placed, uint32_t n) {
+                                                      uint32_t* __restrict__ cell_lb, uint2* __restrict__ placed,
+                                                      uint32_t n) {
     static_assert(LPS_SORT_BLOCKS <= 64u, "a lane per record");
     __shared__ __attribute__((aligned(16))) uint32_t s_cell[SORT_CELLS];
     __shared__ uint32_t s_wave[SORT_WAVES];
@@ -1532,15 +1514,11 @@ __global__ __launch_bounds__(SORT_WG) void k_sort_one(DevGrid* g, lps_dev::Scene
     G.gz = (int)s_box.gsize[2];
     G.gxy = s_box.gsize[0] * s_box.gsize[1];
     G.base = 0u;
-    const uint32_t entries = s_box.cells + 2u;  // with the empty-slot cell and the end
-    if (entries <= SORT_CELLS) {
-        for (uint32_t c = SORT_WG + t; c * 4u < entries; c += SORT_WG)
-            reinterpret_cast<uint4*>(s_cell)[c] = make_uint4(0u, 0u, 0u, 0u);
-        if (entries > SORT_WG * 4u) __syncthreads();
-        sort_cells<true>(s_cell, entries, G, s_box.cells, particles, n, p, s_wave, cell_lb, placed);
-    } else {
-        sort_cells<false>(count, entries, G, s_box.cells, particles, n, p, s_wave, cell_lb, placed);
-    }
+    const uint32_t entries = s_box.cells + 2u;  // with the empty-slot cell and the end; cell_cap holds them to SORT_CELLS
+    for (uint32_t c = SORT_WG + t; c * 4u < entries; c += SORT_WG)
+        reinterpret_cast<uint4*>(s_cell)[c] = make_uint4(0u, 0u, 0u, 0u);
+    if (entries > SORT_WG * 4u) __syncthreads();
+    sort_cells(s_cell, entries, G, s_box.cells, particles, n, p, s_wave, cell_lb, placed);
 }
 
 // The stable order within each cell, and the state gathered into it (the
@@ -3643,12 +3621,12 @@ void launch_grid_setup(hipStream_t s, DevGrid* g, const Scenes& sc, const uint32
 }
 
 void launch_sort_one(hipStream_t s, DevGrid* g, const Scenes& sc, const uint32_t* part, float h, uint32_t cell_cap,
-                     double* energy, const float4* pos, uint32_t n, uint32_t* count, uint32_t* cell_lb,
-                     uint2* placed) {
+                     double* energy, const float4* pos, uint32_t n, uint32_t* cell_lb, uint2* placed) {
+    cell_cap = cell_cap < LPS_SORT_CELLS ? cell_cap : LPS_SORT_CELLS;
     if (part)
-        k_sort_one<true><<<1, SORT_WG, 0, s>>>(g, sc, part, h, cell_cap, energy, pos, count, cell_lb, placed, n);
+        k_sort_one<true><<<1, SORT_WG, 0, s>>>(g, sc, part, h, cell_cap, energy, pos, cell_lb, placed, n);
     else
-        k_sort_one<false><<<1, SORT_WG, 0, s>>>(g, sc, part, h, cell_cap, energy, pos, count, cell_lb, placed, n);
+        k_sort_one<false><<<1, SORT_WG, 0, s>>>(g, sc, part, h, cell_cap, energy, pos, cell_lb, placed, n);
 }
 
 void launch_keys(hipStream_t s, const float4* pos, uint32_t n, const DevGrid* g, const Scenes& sc, uint32_t* keys,

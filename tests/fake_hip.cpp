@@ -80,7 +80,7 @@ hipError_t hipLaunchKernel(const void* f, dim3, dim3, void** args, size_t, hipSt
     } else if (is("k_sort_one")) {
         g_cell_cap = arg<uint32_t>(args, 4);
         need(args, 6, 6);
-        if (g_cell_cap) need(args, 7, 9);  // with no cells it reports an overflow and stops
+        if (g_cell_cap) need(args, 7, 8);  // with no cells it reports an overflow and stops
     } else if (is("k_keys")) {
         need(args, 0, 0);
         if (g_cell_cap) need(args, 3, 5);
