@@ -162,6 +162,7 @@ struct lps_ctx {
     float *press = nullptr, *q = nullptr, *rho_pred = nullptr;
     uint32_t *mk_mask = nullptr, *mk_ok = nullptr;  // recorded candidate masks [LPS_MC_ROWS][cap_n], flags
     uint32_t *nb_list = nullptr, *nb_count = nullptr;  // recorded neighbour lists of the team kernels
+    uint32_t cap_lists = 0;                            // slots they hold
     uint2* mk_cq = nullptr;                         // compact predictions [cap_n + LPS_STENCIL_PAD]
     uint32_t *cell_count = nullptr, *cell_lb = nullptr, *tile_sum = nullptr;  // counts are zero between steps
     float* tables = nullptr;
@@ -460,15 +461,27 @@ int ensure_particles(lps_ctx* c, uint32_t n) {
     if ((st = dalloc(&c->mk_mask, (size_t)LPS_MC_ROWS * n))) return st;
     if ((st = dalloc(&c->mk_ok, n))) return st;
     if ((st = dalloc(&c->mk_cq, (size_t)n + LPS_STENCIL_PAD))) return st;
-    const size_t nt = std::min<size_t>(n, (size_t)LPS_TEAM_BLOCKS * LPS_BLOCK);
-    if ((st = dalloc(&c->nb_list, nt * LPS_NB_LIST))) return st;
-    if ((st = dalloc(&c->nb_count, nt))) return st;
     // every replaying pass follows its recording pass; until then no slot
     // counts as recorded
     HIPC(hipMemsetAsync(c->mk_ok, 0, sizeof(uint32_t) * n, c->stream));
     dfree(c->feat);
     dfree(c->seed);
     c->cap_n = n;
+    return LPS_OK;
+}
+
+// The neighbour lists (512 bytes a slot) of a state that may run 16 lanes per
+// particle; larger ones never read them.
+int ensure_lists(lps_ctx* c, uint32_t n) {
+    const uint32_t most = LPS_TEAM_BLOCKS * LPS_BLOCK;
+    if (n > most || n <= c->cap_lists) return LPS_OK;
+    c->epoch++;
+    c->cap_lists = 0;
+    const uint32_t nt = std::min(c->cap_n, most);
+    int st;
+    if ((st = dalloc(&c->nb_list, (size_t)nt * LPS_NB_LIST))) return st;
+    if ((st = dalloc(&c->nb_count, nt))) return st;
+    c->cap_lists = nt;
     return LPS_OK;
 }
 
@@ -1041,6 +1054,7 @@ int replace_scenes(lps_ctx* c, uint32_t nscenes, const uint32_t* counts, const f
     const hipStream_t s = c->stream;
     HIPC(hipStreamSynchronize(s));
     int st = ensure_particles(c, n);
+    if (!st) st = ensure_lists(c, n);
     if (st) return st;
     // captured graphs hold the sizes and the arrays' addresses
     if (n != c->n || nscenes != c->h_sinfo.size()) c->epoch++;
@@ -1357,7 +1371,8 @@ int lps_add_particles(lps_ctx* c, const float* x, const float* v, const float* v
     // the new particles take slots old .. total - 1 of the current state
     const int b = c->cur;
     const uint32_t nslots = (uint32_t)slots;
-    if ((st = ensure_scenes(c, 1u, nslots / LPS_BLOCK))) return without_particles(c, st);
+    if ((st = ensure_lists(c, nslots)) || (st = ensure_scenes(c, 1u, nslots / LPS_BLOCK)))
+        return without_particles(c, st);
     if (nslots != c->n) c->epoch++;  // captured graphs hold the number of slots
     lps_dev::Rows rows;
     if ((st = upload_rows(c, x, v, vhalf, first, n, &rows))) return st;

@@ -86,6 +86,9 @@ hipError_t hipLaunchKernel(const void* f, dim3, dim3, void** args, size_t, hipSt
         if (g_cell_cap) need(args, 3, 5);
     } else if (is("k_reorder")) {
         need(args, 2, 16);
+    } else if (is("k_density_t")) {  // its neighbour lists
+        for (int k = 0; k < 2; k++)
+            if (!static_cast<void**>(args[10])[k]) g_null_launches++;
     } else if (is("k_mlp_seed")) {
         g_seeded = true;
     } else if (is("k_pci_pressure")) {

@@ -158,3 +158,25 @@ def test_steps_in_flight_when_a_call_fails_are_not_the_next_ones(run):
     F.fake_fail_malloc(-1)
     s.update(1e-3, 3)
     """)
+
+
+def test_neighbour_lists_only_where_a_team_may_run(run):
+    """A state of 600 particle blocks takes less than 400 bytes a slot; the lists
+    of 16 lanes per particle (512 bytes a slot) come with a state that these
+    may run for."""
+    run("""
+    before = F.fake_bytes()
+    s = SPHSolver(Params(method=METHOD_SPH))
+    s.set_particles(rows(153600)); s.update(1e-3, 2)
+    large = F.fake_bytes() - before
+    assert large < 153600 * 400
+    s.set_particles(rows(300)); s.update(1e-3, 2)
+    assert 131072 * 512 < F.fake_bytes() - before - large < 131072 * 520
+    s.add_particles(rows(120000)); s.update(1e-3, 2)
+    s.add_particles(rows(60000)); s.update(1e-3, 2)
+    t = SPHSolver(Params(method=METHOD_SPH))
+    t.set_particles(rows(300)); t.update(1e-3, 2)
+    t.add_particles(rows(300)); t.update(1e-3, 2)
+    t.add_particles(rows(3000)); t.update(1e-3, 2)
+    assert F.fake_null_launches() == 0
+    """)
