@@ -1,11 +1,13 @@
 """GPU tests of states with infinite or NaN components: a velocity that no
 other particle sees (the leapfrog advances the half-step velocity, so the step
-replaces it) leaves the step equal to the oracle's, whatever the lanes."""
+replaces it) leaves the step equal to the oracle's, whatever the lanes, and a
+position fails the step and keeps the state."""
 import numpy as np
 import pytest
 
 from liquidsimulation_amd import scenes
 from liquidsimulation_amd.abi import METHOD_PCISPH, METHOD_SPH
+from liquidsimulation_amd._lib import LPSError
 from liquidsimulation_amd.solver import solver_for
 from tests.helpers import ulp_diff
 
@@ -44,3 +46,32 @@ def test_nonfinite_velocity_of_a_lone_particle(gpu, oracle, method, lanes, value
     assert np.isfinite(p["x"]).all() and np.isfinite(p["v"]).all()
     for k, ref in (("x", st.x), ("v", st.v), ("vhalf", st.vh)):
         assert ulp_diff(p[k], ref) == 0, k
+
+
+# one particle of the first, a middle and the last (partly filled) wave
+@pytest.mark.parametrize("n,at", [(1, 0), (500, 0), (500, 123), (500, 499), (5000, 2600), (5000, 4999)])
+@pytest.mark.parametrize("value", [0x7F800000, 0xFF800000, 0x7FC00000, 0xFFC00000, 0x7F800001, 0xFFFFFFFF])
+def test_nonfinite_position_fails_the_step_and_keeps_the_state(gpu, n, at, value):
+    """Infinities and NaN of either sign, found by the box from the positions
+    (0 lanes: the automatic choice) or from the blocks' records: the status,
+    and the state as it was, with the next state's steps unharmed."""
+    sc = scenes.small_block(18, 18, 18, seed=3, method=METHOD_SPH)
+    x = sc.x[:n].copy()
+    x.view(np.uint32)[at, at % 3] = value
+    v = np.full_like(x, 0.25)
+    for lanes in (0, 1):
+        s = solver_for(sc.params)
+        s.set_tuning(True, 1, 256, lanes)
+        s.set_colliders(sc.colliders)
+        s.set_particles(x, v, v)
+        with pytest.raises(LPSError) as e:
+            s.update(sc.dt, 3)
+        assert e.value.status == 4  # LPS_ERR_NONFINITE
+        p = s.get_particles()
+        np.testing.assert_array_equal(p["x"].view(np.uint32), x.view(np.uint32))
+        for k, ref in (("v", v), ("vhalf", v), ("first", np.ones(n)), ("id", np.arange(n))):
+            np.testing.assert_array_equal(p[k], ref, err_msg=k)
+        s.set_particles(sc.x[:n], v)
+        s.update(sc.dt, 3)
+        assert np.isfinite(s.get_particles()["x"]).all()
+        s.close()
