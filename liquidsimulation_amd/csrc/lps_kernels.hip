@@ -1375,10 +1375,11 @@ __device__ __forceinline__ void sort_cells(uint32_t* count, uint32_t entries, co
     for (uint32_t k = 0; k < SORT_ITEMS; k++) {
         const uint32_t i = k * SORT_WG + t;
         if (k * SORT_WG >= n) break;
-        if (i >= n) continue;
-        const uint32_t cell = quick ? cell_key_quick(G, p[k], y) : cell_key(G, p[k]);
-        key[k] = i < particles ? cell : empty_cell;
-        rank[k] = atomicAdd(&count[key[k]], 1u);
+        if (i < n) {
+            const uint32_t cell = quick ? cell_key_quick(G, p[k], y) : cell_key(G, p[k]);
+            key[k] = i < particles ? cell : empty_cell;
+            rank[k] = atomicAdd(&count[key[k]], 1u);
+        }
     }
     __syncthreads();
     // each wave sums its stretch of cells, then turns it into table entries
