@@ -49,9 +49,11 @@ if ROOT not in sys.path:
 
 HBM_PEAK_GBS = 8000.0
 
-# Algorithmic (compulsory) bytes per particle for each kernel: every particle's
-# own state read or written once, FP32 SoA (vec3 = 12 B, scalar = 4 B);
-# neighbour re-reads not counted.  Per PCISPH correction 108 B = predicted
+# Algorithmic bytes per particle for each kernel of the reference's algorithm:
+# every particle's own state read or written once, FP32 SoA (vec3 = 12 B,
+# scalar = 4 B); neighbour re-reads not counted.  Its sort moves each key once
+# per radix pass, the counting sort here once in all, so the fixed part is no
+# lower bound for this library.  Per PCISPH correction 108 B = predicted
 # density + pressure update + error max (24 B) + pressure force + re-prediction
 # (84 B); fixed part 348 B at three passes of the reference's radix sort.
 ALGO_BYTES = {
@@ -65,7 +67,7 @@ ALGO_BYTES = {
 
 
 def step_bytes(k: float, passes: int = 3) -> float:
-    """Compulsory bytes per particle-step: 300 + 16P fixed + 108 per correction."""
+    """Bytes per particle-step of the reference's algorithm: 300 + 16P fixed (P radix passes) + 108 per correction."""
     return 300.0 + 16.0 * passes + 108.0 * k
 
 

@@ -519,7 +519,11 @@ bool several_lanes(const lps_ctx* c) { return c->lanes == 4u || (c->lanes == 0u 
 // How many lanes: a team of 16, or a quad.  Microseconds per step of a dam
 // break, 16 lanes against 4 (and 1):
 //   SPH     4,394 particles 31 : 69,  16,000 42 : 82 (140),  65,536 82 : 98
-//           (130),  128,000 131 : 133 (134): teams at every size they may run
+//           (130),  128,000 131 : 133 (134): teams at every size they may run;
+//           with a wider kernel the more so (radius 5 to 8 particle radii, 150
+//           to 500 neighbours, quads and one lane as of the build before the
+//           teams: 16,000 particles 70 : 232 and 260 : 709, 128,000 287 : 540
+//           and 1371 : 1680)
 //   PCISPH  4,394 95 : 214,  16,000 172 : 362 (553),  43,904 458 : 567,
 //           54,000 522 : 583,  65,536 649 : 639 (826): teams up to 240
 //           particle blocks, before the two cross; a team's density pass costs
@@ -560,8 +564,10 @@ lps_dev::PhysArgs phys_args(lps_ctx* c, const SimConst& k) {
 // the pressure pass: the sort takes the box from the positions then, and the
 // blocks' records (the boxes and energies of larger scenes and of lps_get_energy)
 // are not written.  That saves a launch and costs the sort's one compute unit a
-// pass over the positions: 512 particles 56.5 -> 54.2 us a frame, 10,000 84.6 ->
-// 83.0, 16,000 43.9 -> 44.4 us a step, so it stops between the last two.
+// pass over the positions.  Microseconds a step, separate -> moved: 512 particles
+// 29.2 -> 28.0, 2,880 33.3 -> 31.7, 7,200 35.8 -> 34.9, 10,098 38.8 -> 38.6,
+// 11,970 (47 blocks) 40.1 -> 39.8, 13,357 (53) 42.0 -> 42.4, 15,600 43.0 -> 43.4:
+// it stops between the last but two.
 bool sort_in_one(const lps_ctx* c) {
     return c->h_sinfo.size() == 1u && c->n <= LPS_SORT_BLOCKS * LPS_BLOCK && !c->wide_grid;
 }

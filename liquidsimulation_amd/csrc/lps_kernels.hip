@@ -1244,7 +1244,7 @@ __device__ __forceinline__ uint32_t count_key(uint32_t* count, uint32_t key, uin
 }
 
 // Keys within the scene's grid, offset by the scene's first cell; empty slots get the scene's empty-slot
-// cell so they follow its particles.  run[i] is the place of arrival in the
+// cell so they follow its particles.  rank[i] is the place of arrival in the
 // cell, count[cell] the counts.
 __global__ __launch_bounds__(LPS_BLOCK) void k_keys(const float4* __restrict__ pos, const DevGrid* g,
                                                     lps_dev::Scenes S, uint32_t* __restrict__ keys,
@@ -1351,11 +1351,12 @@ __global__ __launch_bounds__(LPS_BLOCK) void k_place(const uint32_t* __restrict_
 // a step of 512 SPH particles in 32,768 cells took 47 us against 36 (in 29,791,
 // with LDS, 28 against 35), in 305,252 cells 167 against 36, of 15,488
 // particles 65 against 41 (41 against 41) and 186 against 42.
-// Per step, five launches -> one: 11.8 -> 3.6 us of kernels at 512 particles,
-// 13.0 -> 5.2 at 1,080, 14.2 -> 10.9 at 16,128, beside the four launches.  One
-// compute unit then does all of its arithmetic (with IEEE divisions and the
-// runs of k_keys the last figure was 16.6); more blocks would not fit its
-// registers, which hold the positions and keys of 16 particles a thread.
+// Per step, five launches -> one (averages over 100 steps of PCISPH blocks):
+// 11.9 -> 4.2 us of kernels at 512 particles, 11.9 -> 4.6 at 1,080, 13.2 -> 11.1
+// at 16,000, beside the four launches.  One compute unit then does all of its
+// arithmetic (with IEEE divisions and the runs of k_keys the last figure was
+// 16.6); more blocks would not fit its registers, which hold the positions and
+// keys of 16 particles a thread.
 // RECORDS: the box (and the energy) from the blocks' records, else from the
 // positions.
 constexpr uint32_t SORT_WG = 1024u, SORT_WAVES = SORT_WG / 64u, SORT_CELLS = LPS_SORT_CELLS + 1u;
@@ -1799,11 +1800,11 @@ __global__ __launch_bounds__(LPS_BLOCK) void k_pressure_sph(const float4* __rest
 }
 
 // ===================================================== quad stencils ====
-// Small scenes leave most of the chip idle while every lane walks a long
-// neighbour list alone: the 16k SPH dam break's compressed fluid gives a
-// particle hundreds of candidates, and its 63 particle blocks fill a quarter
-// of the SIMDs with one wave each.  The quad kernels give a particle the four
-// lanes of a quad.  Pass 1 tests every fourth candidate of a window on each
+// Scenes of a few hundred particle blocks leave much of the chip idle while
+// every lane walks a neighbour list alone: 65,536 PCISPH particles are 256
+// blocks, one wave on every SIMD, and take 826 us a step with one lane, 639
+// with a quad and 649 with a team of 16 (which wins in smaller scenes, below).
+// The quad kernels give a particle the four lanes of a quad.  Pass 1 tests every fourth candidate of a window on each
 // lane, and the quad ORs the four masks.  Pass 2 hands the quad's next four
 // kept candidates to its four lanes in order; each lane computes the terms
 // of its candidate, and every lane of the quad then adds the four terms in
@@ -3176,8 +3177,8 @@ __global__ __launch_bounds__(LPS_BLOCK) void k_forces_t(
 // k_pressure_sph with a team per particle.  MOVE: also the step's integration,
 // with the report to the host but without the blocks' records (a team's
 // workgroup has 16 particles, a record 256 slots), for scenes whose sort takes
-// the box from the positions (k_pressure_sph_t 4.2 and k_integrate 3.2 -> 5.6 us at
-// 512 particles, and a launch; the sort 3.8 -> 4.3).
+// the box from the positions (k_pressure_sph_t 4.6 and k_integrate 3.4 -> 6.0 us at
+// 512 particles, and a launch; the sort 4.2 -> 4.3).
 struct Motion {
     float4 *pos, *vel, *vh;
     uint8_t* first;
