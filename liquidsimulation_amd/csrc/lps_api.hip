@@ -264,6 +264,11 @@ int hip_status(hipError_t e) {
         if (e_ != hipSuccess) return hip_status(e_); \
     } while (0)
 
+// For calls that ask for the last error after their launches: one left by an
+// earlier call, which reported it then, or by another user of the runtime in
+// this thread is not theirs.
+void forget_error() { (void)hipGetLastError(); }
+
 template <class T>
 int dalloc(T** p, size_t count) {
     if (*p) {
@@ -1058,6 +1063,7 @@ int gather_applied(lps_ctx* c, const T* dev3, std::vector<T>& full) {
 int replace_scenes(lps_ctx* c, uint32_t nscenes, const uint32_t* counts, const float* gravity, const float* x,
                    const float* v, const float* vhalf, const uint8_t* first, uint32_t n, uint32_t total) {
     const hipStream_t s = c->stream;
+    forget_error();
     HIPC(hipStreamSynchronize(s));
     int st = ensure_particles(c, n);
     if (!st) st = ensure_lists(c, n);
@@ -1334,6 +1340,7 @@ int lps_add_particles(lps_ctx* c, const float* x, const float* v, const float* v
         if (!std::isfinite(x[k]) || (v && !std::isfinite(v[k])) || (vhalf && !std::isfinite(vhalf[k])))
             return LPS_ERR_INVALID;
     const hipStream_t s = c->stream;
+    forget_error();
     HIPC(hipStreamSynchronize(s));
     int st;
     bool grown = false;
@@ -1425,6 +1432,7 @@ int lps_copy_positions_device(lps_ctx* c, float* dst, uint32_t stride, uint32_t 
     } else {
         (void)hipGetLastError();
     }
+    forget_error();
     lps_dev::launch_export_positions(c->stream, c->pos[c->cur], c->n, scenes(c), dst, stride);
     HIPC(hipGetLastError());
     HIPC(hipStreamSynchronize(c->stream));
@@ -1477,6 +1485,7 @@ int lps_get_particles(lps_ctx* c, float* x, float* v, float* vhalf, uint8_t* fir
     dev.vhalf = vhalf ? rows + 6 * (size_t)n : nullptr;
     dev.id = id ? words : nullptr;
     dev.first = first ? reinterpret_cast<uint8_t*>(words + n) : nullptr;
+    forget_error();
     lps_dev::launch_pack(s, state_arrays(c, c->cur), scenes(c), dev);
     HIPC(hipGetLastError());
     const struct { void* to; const void* from; size_t bytes; } part[] = {
@@ -1608,6 +1617,7 @@ int lps_get_energy(lps_ctx* c, double* kinetic, double* potential, uint32_t nsce
     // the current state's per-block records were written by the last
     // integration or particle upload, or are written now
     std::vector<double> keep(c->h_energy, c->h_energy + 2 * (size_t)nscenes);
+    forget_error();
     ensure_records(c);
     lps_dev::launch_scene_energy(c->stream, scenes(c), c->bbox_part, c->h_energy);
     HIPC(hipGetLastError());
@@ -1887,6 +1897,7 @@ int lps_mlp_set_weights(lps_ctx* c, const float* params, const float* feature_sc
         if (!std::isfinite(params[k])) return LPS_ERR_INVALID;
     for (uint32_t k = 0; k < 2 * LPS_MLP_IN; k++)
         if (!std::isfinite(feature_scale[k])) return LPS_ERR_INVALID;
+    forget_error();
     if (!c->d_mlp) HIPC(hipMalloc((void**)&c->d_mlp, sizeof(float) * (LPS_MLP_PARAMS + 2 * LPS_MLP_IN)));
     if (!c->d_mlp_packed) HIPC(hipMalloc((void**)&c->d_mlp_packed, lps_dev::mlp_packed_bytes()));
     c->mlp_w.assign(params, params + LPS_MLP_PARAMS);
@@ -2054,6 +2065,7 @@ int lps_mlp_train(lps_ctx* c, const lps_mlp_train_cfg* cfg, float* epoch_loss) {
         !(cfg->beta1 >= 0.f && cfg->beta1 < 1.f) || !(cfg->beta2 >= 0.f && cfg->beta2 < 1.f) || !(cfg->eps > 0.f))
         return LPS_ERR_INVALID;
     if (c->coll_rows == 0) return LPS_ERR_STATE;
+    forget_error();
     int st = ensure_train_buffers(c);
     if (st) return st;
     const hipStream_t s = c->stream;
@@ -2143,6 +2155,7 @@ int lps_mlp_grad(lps_ctx* c, const float* x, const float* t, uint32_t n, float o
     if (!c || !x || !t || !grad || n == 0 || !(over_weight > 0.f) || !std::isfinite(over_weight))
         return LPS_ERR_INVALID;
     if (!c->mlp_loaded) return LPS_ERR_STATE;
+    forget_error();
     int st = ensure_train_buffers(c);
     if (st) return st;
     HostRows rows(c, (size_t)n * (LPS_MLP_IN + 1));
@@ -2178,6 +2191,7 @@ int lps_mlp_grad_noalloc(lps_ctx* c, const float* x, const float* t, uint32_t n,
     float* dl = reinterpret_cast<float*>(base + LPS_NOALLOC_X_BYTES + LPS_NOALLOC_T_BYTES + LPS_NOALLOC_G_BYTES);
     const hipStream_t s = c->stream;
     float* dp = reinterpret_cast<float*>(base + LPS_NOALLOC_PART);
+    forget_error();
     // the loss keeps the previous call's sum: clear it (a fill kernel, so the
     // call stays free of memset nodes)
     lps_dev::launch_fill_zero(s, dl, 1u);

@@ -24,10 +24,13 @@ bool g_seeded = false;
 uint32_t g_overflow_cells = 0;  // cells the next step needs, as a grid overflow (0: it succeeds)
 uint32_t g_cell_cap = 0;
 uint32_t g_null_launches = 0;
+hipError_t g_last = hipSuccess;  // as the runtime keeps it: the last error, until it is asked for
 size_t g_bytes = 0;
 std::map<void*, size_t> g_sizes;
 StepReport* g_report = nullptr;
 StepReport g_now{0u, 0u, 0u};
+
+hipError_t failed(hipError_t e) { return g_last = e; }
 
 template <class T>
 T arg(void** args, int k) { return *static_cast<T*>(args[k]); }
@@ -50,6 +53,7 @@ void finish_step(StepReport* r) {
 extern "C" {
 void fake_fail_malloc(int in) { g_fail_in = in; }
 void fake_iterations(int plain, int seeded) { g_plain_its = plain; g_seeded_its = seeded; }
+void fake_leave_error() { failed(hipErrorInvalidValue); }
 void fake_overflow(uint32_t cells) { g_overflow_cells = cells; }
 uint32_t fake_null_launches() { return g_null_launches; }
 size_t fake_bytes() { return g_bytes; }
@@ -111,11 +115,11 @@ hipError_t hipLaunchKernel(const void* f, dim3, dim3, void** args, size_t, hipSt
 
 hipError_t hipMalloc(void** p, size_t n) {
     *p = nullptr;
-    if (g_fail_in >= 0 && g_fail_in-- == 0) return hipErrorOutOfMemory;
+    if (g_fail_in >= 0 && g_fail_in-- == 0) return failed(hipErrorOutOfMemory);
     *p = std::calloc(n, 1);
     g_sizes[*p] = n;
     g_bytes += n;
-    return *p ? hipSuccess : hipErrorOutOfMemory;
+    return *p ? hipSuccess : failed(hipErrorOutOfMemory);
 }
 hipError_t hipFree(void* p) {
     g_bytes -= g_sizes[p];
@@ -142,8 +146,12 @@ hipError_t hipGetDeviceProperties(hipDeviceProp_t* p, int) {
     p->multiProcessorCount = 256;
     return hipSuccess;
 }
-hipError_t hipGetLastError() { return hipSuccess; }
-hipError_t hipGetSymbolAddress(void** p, const void*) { *p = nullptr; return hipErrorInvalidSymbol; }
+hipError_t hipGetLastError() {
+    const hipError_t e = g_last;
+    g_last = hipSuccess;
+    return e;
+}
+hipError_t hipGetSymbolAddress(void** p, const void*) { *p = nullptr; return failed(hipErrorInvalidSymbol); }
 hipError_t hipStreamCreateWithFlags(hipStream_t* s, unsigned) { *s = reinterpret_cast<hipStream_t>(&g_config); return hipSuccess; }
 hipError_t hipStreamDestroy(hipStream_t) {  // a context ends
     g_report = nullptr;
@@ -155,5 +163,5 @@ hipError_t hipStreamSynchronize(hipStream_t) {
     if (g_report) *g_report = g_now;
     return hipSuccess;
 }
-hipError_t hipStreamBeginCapture(hipStream_t, hipStreamCaptureMode) { return hipErrorNotSupported; }
+hipError_t hipStreamBeginCapture(hipStream_t, hipStreamCaptureMode) { return failed(hipErrorNotSupported); }
 }

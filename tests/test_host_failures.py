@@ -180,3 +180,21 @@ def test_neighbour_lists_only_where_a_team_may_run(run):
     t.add_particles(rows(3000)); t.update(1e-3, 2)
     assert F.fake_null_launches() == 0
     """)
+
+
+def test_an_error_left_by_another_call_is_not_this_ones(run):
+    """The runtime keeps a thread's last error until it is asked for it; calls
+    that ask after their launches must not take one that was there before."""
+    run("""
+    def each(*calls):
+        for call in calls:
+            F.fake_leave_error()  # as another library's failed call would
+            call()
+    s = PCISPHSolver(Params(method=METHOD_PCISPH))
+    s.set_tuning(False)
+    each(lambda: s.set_particles(rows(300)), lambda: s.update(1e-3, 2), lambda: s.add_particles(rows(20)),
+         s.get_particles, s.get_energy, lambda: s.set_params(s.params), lambda: s.set_colliders(box(0.5)),
+         lambda: s.set_warm_start_weights(np.zeros(5313, np.float32), np.ones(32, np.float32), 1.0),
+         lambda: s.mlp_forward(np.zeros((9, 16))), lambda: s.mlp_grad(np.zeros((9, 16)), np.zeros(9)),
+         lambda: s.update(1e-3, 2), s.get_fields)
+    """)
