@@ -1832,6 +1832,7 @@ int lps_get_grid(lps_ctx* c, lps_grid_info* info, uint32_t* keys, uint32_t* perm
     }
     if (cell_start || cell_end) {
         const uint32_t m = std::min(cap, cells);
+        if (m > c->cell_cap) return LPS_ERR_STATE;  // of a failed step, which the table was too small for
         std::vector<uint32_t> lb((size_t)m + 1);
         HIPC(hipMemcpy(lb.data(), c->cell_lb, sizeof(uint32_t) * ((size_t)m + 1), hipMemcpyDeviceToHost));
         for (uint32_t k = 0; k < m; k++) {

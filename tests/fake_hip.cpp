@@ -83,6 +83,7 @@ hipError_t hipLaunchKernel(const void* f, dim3, dim3, void** args, size_t, hipSt
         g_cell_cap = arg<uint32_t>(args, 4);
     } else if (is("k_sort_one")) {
         g_cell_cap = arg<uint32_t>(args, 4);
+        if (g_overflow_cells) static_cast<SceneGrid**>(args[1])[1]->cells = g_overflow_cells - 1u;
         need(args, 6, 6);
         if (g_cell_cap) need(args, 7, 8);  // with no cells it reports an overflow and stops
     } else if (is("k_keys")) {

@@ -198,3 +198,16 @@ def test_an_error_left_by_another_call_is_not_this_ones(run):
          lambda: s.mlp_forward(np.zeros((9, 16))), lambda: s.mlp_grad(np.zeros((9, 16)), np.zeros(9)),
          lambda: s.update(1e-3, 2), s.get_fields)
     """)
+
+
+def test_cell_arrays_of_a_step_whose_table_could_not_grow(run):
+    run("""
+    s = SPHSolver(Params(method=METHOD_SPH))
+    s.set_particles(rows(300)); s.update(1e-3, 2); s.get_grid()
+    F.fake_overflow(1 << 20)
+    F.fake_fail_malloc(0)
+    assert status(s.update, 1e-3, 1) == OOM
+    F.fake_fail_malloc(-1)
+    assert status(s.get_grid) == STATE  # there is no table of so many cells to read
+    s.get_particles()
+    """)
